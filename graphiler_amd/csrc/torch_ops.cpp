@@ -1202,9 +1202,11 @@ torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::T
   int rc = typed_rows(q, pairs.dst_by_type, att_t, q_pair);
   if (rc == GA_EUNSUPPORTED) return per_edge();
   check_ga(rc, "ga_segment_mm_gather");
+  // both passes share the scratch; the bytes are not monotonic in the number of items
+  // (longer runs from a threshold on), so the pairs are asked for as well
   torch::Tensor ws = graph->workspace(std::max(
-      {ga_gat_workspace_bytes(e, hid, heads), ga_softmax_workspace_bytes(P, heads),
-       ga_spmm_workspace_bytes(P, hid)}));
+      {ga_gat_workspace_bytes(e, hid, heads), ga_gat_workspace_bytes(P, hid, heads),
+       ga_softmax_workspace_bytes(P, heads), ga_spmm_workspace_bytes(P, hid)}));
   torch::Tensor v_pair = torch::empty({P, hid}, k.options());
   torch::Tensor lse = torch::empty({P, heads}, k.options().dtype(at::kFloat));
   rc = ga_dot_attention_sum(pairs.pair_pointer.data_ptr<int>(), pairs.pair_of_slot.data_ptr<int>(),

@@ -1025,9 +1025,11 @@ def relation_pair_attention(k, q, v, relation_att, relation_msg, relation_scale,
         return y
 
     q_pair = typed_rows(q, pairs.dst_by_type, att_t)
+    # both passes share the scratch; the bytes are not monotonic in the number of items
+    # (longer runs from a threshold on), so the pairs are asked for as well
     ws = graph.workspace(max(lib.ga_softmax_workspace_bytes(e, heads),
-                             lib.ga_spmm_workspace_bytes(e, hid),
-                             lib.ga_gat_workspace_bytes(e, hid, heads)))
+                             max(lib.ga_spmm_workspace_bytes(i, hid) for i in (e, P)),
+                             max(lib.ga_gat_workspace_bytes(i, hid, heads) for i in (e, P))))
     # scores, softmax inside every pair and the pair's weighted sum of value rows in one
     # pass; the pairs of a destination are then weighed by the softmax of their
     # log-sum-exps (the softmax-weighted sum of per-"edge" rows, with the pairs as the

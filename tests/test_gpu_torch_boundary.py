@@ -366,3 +366,30 @@ def test_sum_with_row_wise_tail(setup, device):
         ops.SpMMScaled(x, None, 3, True, sg)
     with pytest.raises(RuntimeError, match="rows"):
         ops.SpMMScaled(x, None, 0, False, sg)
+
+
+def test_relation_pair_attention_scratch_on_many_pairs(device):
+    """The scratch of the row reductions is not monotonic in the number of items (runs get
+    longer from a threshold on): just under 2^20 pairs of just over 2^21 edges of 256
+    features need more of it than the edges do.  Both front ends ask for the larger."""
+    torch_boundary.load()
+    from graphiler_amd import ops as pyops
+    from graphiler_amd.graph import sort_edges_by_type
+    rng = np.random.default_rng(5)
+    n, te, heads, d = 10_400, 100, 16, 16
+    dst, et = (a.ravel() for a in np.meshgrid(np.arange(n), np.arange(te)))     # 1.04 M pairs
+    extra = rng.integers(0, dst.size, 20_000)
+    dst = np.concatenate([dst, dst, dst[extra]])
+    et = np.concatenate([et, et, et[extra]])
+    src, dst, et, _ = sort_edges_by_type(rng.integers(0, n, dst.size), dst, et)
+    assert dst.size >= 1 << 21 and n * te < 1 << 20
+    g = prepare_graph(src, dst, n, device=device, etype_of=et, num_etypes=te)
+    k, q, v = (torch.randn(n, heads * d, device=device) for _ in range(3))
+    att, msg = (torch.randn(te, heads, d, d, device=device) / 4 for _ in range(2))
+    got = pyops.relation_pair_attention(k, q, v, att, msg, None, g, factor=0.25)
+    score = pyops.SegmentMMEdgeDot(k, att, 0, q, 1, g) * 0.25
+    want = pyops.edge_softmax_sum(score, pyops.SegmentMMEdgeGather(v, msg, 0, g), g)
+    assert_close(got.cpu().numpy(), want.cpu().numpy(), 2 * TOL_F32, "many pairs")
+    same = torch.ops.my_ops.relation_pair_attention(k, q, v, att, msg, None, 4.0,
+                                                    torch_boundary.script_graph(g))
+    assert torch.equal(got, same)
