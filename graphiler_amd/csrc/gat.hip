@@ -62,13 +62,15 @@ __device__ __forceinline__ float lanes_sum(float v, int lanes) {
 // the store sits at five places of the run loop, under divergence, so its length is
 // paid once per closed row and wavefront, not per element.
 constexpr int kActRuntime = -1;
-template <typename T, int VEC, int MODE = kGatNode, bool SPREAD = false, int ACT = kActRuntime>
+template <typename T, int VEC, int MODE = kGatNode, bool SPREAD = false, int ACT = kActRuntime,
+          int GL = 0>
 struct GatPolicy {
   static constexpr bool EDGE = MODE == kGatEdge;
   typedef T out_t;
   static constexpr int kVec = VEC;
   static constexpr int kState = VEC + 2;
   static constexpr bool kSpread = SPREAD;
+  static constexpr int kGL = GL;
   struct Args {
     const int32_t *nbr;   // kGatEdge: the edge-id column, or null when slot = edge id
     const float *el;      // kGatEdge: per-edge logits (E, heads); kGatFromZ: a_l (heads*dph)
@@ -140,6 +142,81 @@ struct GatPolicy {
     float al[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) al[v] = MODE == kGatFromZ ? A.el[f0 + v] : 0.0f;
+    if constexpr (GL > 0) {
+      typedef GroupCol<GL> Col;
+      const int sub = threadIdx.x & (GL - 1);
+      GroupIds<GL> ids, next;
+      ids.load(row_of_slot, A.nbr, a, b, sub);
+      for (int64_t j = a; j < b; j += kUnroll) {
+        // the columns of the next batch arrive under this batch's gathers
+        next.load(row_of_slot, A.nbr, j + kUnroll, b, sub);
+        typename IO::raw_t x[kUnroll];
+        float sv;                   // lane i holds the logit of slot (i & 7)
+        if constexpr (MODE == kGatEdge) {
+          if constexpr (GL == 16) {     // lanes 8 .. 15 hold the indices
+            sv = A.el[(int64_t)(sub & 8 ? ids.row : 0) * A.heads + h];
+            const float o = other_half(sv);
+            sv = sub & 8 ? sv : o;
+          } else {
+            sv = A.el[(int64_t)ids.idx * A.heads + h];
+          }
+        } else if constexpr (GL == 16) {    // one load for both terms, each from its half
+          sv = (sub & 8 ? A.el : A.er)[(int64_t)ids.row * A.heads + h];
+          sv = leaky(sv + other_half(sv), A.slope);
+        } else {
+          sv = leaky(A.el[(int64_t)ids.idx * A.heads + h] + A.er[(int64_t)ids.row * A.heads + h],
+                     A.slope);
+        }
+        static_for<kUnroll>([&](auto t) {
+          x[t] = IO::load(A.z + (int64_t)ids.template index_of<t>() * feat + f0, ln);
+        });
+        const bool one_row = j + kUnroll <= b && ids.template row_of<0>() == cur &&
+                             ids.template row_of<kUnroll - 1>() == cur;
+        if (one_row) {
+          // whole batch inside the open row (rows are sorted): one rescale
+          const float nm = fmaxf(st[VEC], Col::max(sv));
+          const float ref = finite_or_zero(nm);
+          const float sc = __expf(st[VEC] - ref);
+          st[VEC + 1] *= sc;
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) st[v] *= sc;
+          st[VEC] = nm;
+          const float pv = __expf(sv - ref);    // one exponential per slot, not per slot and lane
+          st[VEC + 1] += Col::sum(pv);
+          static_for<kUnroll>([&](auto t) {
+            const float p = Col::template get<t>(pv);
+            float xf[VEC];
+            IO::widen(x[t], xf);
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) st[v] = fmaf(p, xf[v], st[v]);
+          });
+        } else {
+          static_for<kUnroll>([&](auto t) {
+            if (j + t < b) {
+              const int r = ids.template row_of<t>();
+              if (r != cur) {
+                close_segment();
+                cur = r;
+                init(st);
+              }
+              const float s = Col::template get<t>(sv);
+              const float nm = fmaxf(st[VEC], s);
+              const float ref = finite_or_zero(nm);
+              const float sc = __expf(st[VEC] - ref);
+              const float p = __expf(s - ref);
+              st[VEC + 1] = st[VEC + 1] * sc + p;
+              float xf[VEC];
+              IO::widen(x[t], xf);
+#pragma unroll
+              for (int v = 0; v < VEC; ++v) st[v] = fmaf(p, xf[v], st[v] * sc);
+              st[VEC] = nm;
+            }
+          });
+        }
+        ids = next;
+      }
+      return;
+    }
     for (int64_t j = a; j < b; j += kUnroll) {
       int r[kUnroll], g[kUnroll];
       float s[kUnroll];
@@ -352,7 +429,8 @@ int launch_dot_attn(const int32_t *pointer, const int32_t *row_of_slot, const in
                         stream, ws_bytes);
 }
 
-template <typename T, int VEC, int MODE = kGatNode, bool SPREAD = false, int ACT = kActRuntime>
+template <typename T, int VEC, int MODE = kGatNode, bool SPREAD = false, int ACT = kActRuntime,
+          int GL = 0>
 int launch_gat(const int32_t *pointer, const int32_t *row_of_slot,
                const int32_t *nbr, const float *el, const float *er,
                const void *z, void *out, int64_t n_rows, int64_t n_edges,
@@ -373,7 +451,20 @@ int launch_gat(const int32_t *pointer, const int32_t *row_of_slot,
                                                         n_rows, n_edges, heads, dim, slope, ws, stream,
                                                         ws_bytes, act, size_only);
   }
-  typedef GatPolicy<T, VEC, MODE, SPREAD, ACT> P;
+  if constexpr (GL == 0 && VEC > 1 && MODE != kGatFromZ) {
+    // lane groups of eight lanes and more share the columns and the logits they form from
+    // them, where the sharing lanes lie in one head
+    const int share = heads == 1 ? 16 : dim % (16 * VEC) == 0 ? 16 : dim % (8 * VEC) == 0 ? 8 : 0;
+    const int lanes = (heads * dim + VEC - 1) / VEC;
+#define GA_GAT_GL(N)                                                                            \
+  return launch_gat<T, VEC, MODE, SPREAD, ACT, N>(pointer, row_of_slot, nbr, el, er, z, out,    \
+                                                  n_rows, n_edges, heads, dim, slope, ws, stream, \
+                                                  ws_bytes, act, size_only)
+    if (lanes > 8 && share == 16) GA_GAT_GL(16);
+    if (lanes > 4 && lanes <= 8 && share >= 8) GA_GAT_GL(8);
+#undef GA_GAT_GL
+  }
+  typedef GatPolicy<T, VEC, MODE, SPREAD, ACT, GL> P;
   const bool ids_vec = aligned(row_of_slot, 16) && (!nbr || aligned(nbr, 16));
   const int head_lanes = dim / VEC;
   if (MODE == kGatFromZ &&

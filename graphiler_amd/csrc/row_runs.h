@@ -28,7 +28,12 @@
 //                               a policy with further outputs writes them here
 //   kSpread                     lane layout (see above); such a policy's Args carry
 //                               `stride_shift`, which the launcher sets to log2(tpr)
+//   kGL                         how the lanes of a group share the slot-indexed columns
+//                               (GroupCol below); 0: every lane reads them for itself
 #pragma once
+
+#include <type_traits>
+#include <utility>
 
 #include "common.h"
 
@@ -39,7 +44,7 @@ constexpr int kUnroll = 8;
 static_assert(kUnroll == 8, "load_ids8 reads two int4");
 
 // Eight consecutive int32 of a slot-indexed column starting at slot j (a
-// multiple of 8: runs start at multiples of 32).  Two 16-byte loads when the
+// multiple of 8, as every run's start is).  Two 16-byte loads when the
 // column is 16-byte aligned and the batch is whole; otherwise element loads
 // clamped to the run's last slot.
 __device__ __forceinline__ void load_ids8(const int32_t *__restrict__ p, int64_t j, int64_t b,
@@ -54,6 +59,99 @@ __device__ __forceinline__ void load_ids8(const int32_t *__restrict__ p, int64_t
     for (int t = 0; t < kUnroll; ++t) out[t] = p[j + t < b ? j + t : b - 1];
   }
 }
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): an unrolled loop
+// whose index may be used where a constant is required (DPP controls).
+template <class F, int... I>
+__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+  static_for_impl(std::forward<F>(f), std::make_integer_sequence<int, N>{});
+}
+
+// A batch of kUnroll slot-indexed values held once per lane group instead of once per
+// lane.  What bounds a gather of rows that hit the caches is the address unit: it
+// takes the lanes of a 16-byte load four at a time whether or not they read the same
+// words, so the two 16-byte loads per column and batch that every lane would issue
+// for itself cost as much as four of the eight row gathers.  Here lane i of a group
+// reads one value with a 4-byte load, and a batch's values reach the other lanes by
+// DPP moves.  GL = 16 stands for every group of 16 lanes or more (each 16 lanes of a
+// larger group hold a copy), GL = 8 for groups of eight.  30 M edges, 64 fp32 features,
+// a 2 MB table: copy_u 427 -> 350 us (18 -> 22 TB/s of rows), the fused GAT aggregation
+// 538 -> 427 us; from tables that miss the L2s (above 12 MB) the two are level.  Groups
+// of four lanes keep the 16-byte loads: two values per lane were slower (16 features:
+// 180 -> 206 us).
+template <int GL>
+struct GroupCol {
+  static_assert(GL == 8 || GL == 16, "lanes that share a batch");
+  // value of slot T, in every lane of the group
+  template <int T>
+  static __device__ __forceinline__ int get(int v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, v, 0x150 + T, 0xF, 0xF, true);     // row_newbcast:T
+    if constexpr (GL == 16) return lo;
+    // the upper eight lanes of a row of 16 are a group of their own
+    else return __builtin_amdgcn_update_dpp(lo, v, 0x150 + 8 + T, 0xF, 0xC, false);
+  }
+  template <int T>
+  static __device__ __forceinline__ float get(float v) {
+    return __int_as_float(get<T>(__float_as_int(v)));
+  }
+  // sum / maximum over the batch: every eight lanes hold all of it
+  static __device__ __forceinline__ float sum(float v) { return row8_sum(v); }
+  static __device__ __forceinline__ float max(float v) {
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true)));
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true)));
+    return fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xF, 0xF, true)));
+  }
+  // slot (sub & 7) of the batch at j, clamped to the run's last slot
+  static __device__ __forceinline__ int64_t slot(int64_t j, int64_t b, int sub) {
+    const int64_t jj = j + (sub & (kUnroll - 1));
+    return jj < b ? jj : b - 1;
+  }
+};
+__device__ __forceinline__ int other_half(int v) {    // the value of the lane eight away, of 16
+  return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xF, 0xF, true);                   // row_ror:8
+}
+__device__ __forceinline__ float other_half(float v) {
+  return __int_as_float(other_half(__float_as_int(v)));
+}
+
+// The row ids and the gather indices of a batch.  With 16 lanes or more one load
+// serves both columns: lanes 0 .. 7 of every 16 hold the rows, lanes 8 .. 15 the
+// indices.  `index` may be null: the slots themselves are the indices.
+template <int GL>
+struct GroupIds {
+  typedef GroupCol<GL> Col;
+  int row;              // GL = 16: rows | indices
+  int idx;              // GL = 16: unused
+  __device__ __forceinline__ void load(const int32_t *__restrict__ rows,
+                                       const int32_t *__restrict__ index, int64_t j, int64_t b,
+                                       int sub) {
+    const int64_t jj = Col::slot(j, b, sub);
+    if constexpr (GL == 16) {
+      if (index) row = (sub & 8 ? index : rows)[jj];
+      else row = sub & 8 ? (int)jj : rows[jj];
+    } else {
+      row = rows[jj];
+      idx = index ? index[jj] : (int)jj;
+    }
+  }
+  template <int T>
+  __device__ __forceinline__ int row_of() const { return Col::template get<T>(row); }
+  template <int T>
+  __device__ __forceinline__ int index_of() const {
+    if constexpr (GL == 16) return Col::template get<8 + T>(row);
+    else return Col::template get<T>(idx);
+  }
+  __device__ __forceinline__ int my_row(int sub) const {       // row of slot (sub & 7)
+    if constexpr (GL == 16) {
+      const int other = other_half(row);
+      return sub & 8 ? other : row;
+    } else return row;
+  }
+};
 
 struct RunGeom {
   int64_t n_edges;
@@ -129,7 +227,12 @@ __global__ __launch_bounds__(kBlock) void runs_kernel(
   const int64_t k = (int64_t)blockIdx.x * G + grp;
   const int flane = (int)blockIdx.y * tpr + lane;   // feature lane index
   const int f0 = lane_first_feature<Policy>((int)blockIdx.y, lane, geo.tpr_shift);
-  const bool live = k < geo.n_runs && f0 < geo.feat;
+  // lanes past the row's features take part in the walk where the group's lanes read the
+  // columns for one another (on the features of the row's last lane), but store nothing
+  const bool lane_live = f0 < geo.feat;
+  const bool live = k < geo.n_runs && (Policy::kGL > 0 || lane_live);
+  const int f0w = Policy::kGL > 0 && !lane_live
+                      ? (Policy::kSpread ? 0 : geo.feat - Policy::kVec) : f0;
 
   float *my_a = lds_state + ((grp * 2 + 0) * tpr + lane) * SF;
   float *my_b = lds_state + ((grp * 2 + 1) * tpr + lane) * SF;
@@ -154,13 +257,13 @@ __global__ __launch_bounds__(kBlock) void runs_kernel(
         row_a = cur;
 #pragma unroll
         for (int i = 0; i < SF; ++i) my_a[i] = st[i];
-      } else {
+      } else if (Policy::kGL == 0 || lane_live) {
         Policy::emit(args, out, cur, geo.feat, f0, st);
       }
       first_seg = false;
     };
 
-    Policy::walk(args, row_of_slot, a, b, f0, geo.feat, st, cur, close_segment);
+    Policy::walk(args, row_of_slot, a, b, f0w, geo.feat, st, cur, close_segment);
 
     const bool continues = b < geo.n_edges && row_of_slot[b] == cur;
     if (first_seg && began_before) {
@@ -174,7 +277,7 @@ __global__ __launch_bounds__(kBlock) void runs_kernel(
       row_b = cur;
 #pragma unroll
       for (int i = 0; i < SF; ++i) my_b[i] = st[i];
-    } else {
+    } else if (Policy::kGL == 0 || lane_live) {
       Policy::emit(args, out, cur, geo.feat, f0, st);
     }
   }
@@ -186,7 +289,7 @@ __global__ __launch_bounds__(kBlock) void runs_kernel(
     flags[grp].row_b = row_b;
   }
   __syncthreads();
-  if (!live) return;
+  if (!live || !lane_live) return;
 
   auto state_of = [&](int g, int slot) -> const float * {
     return lds_state + ((g * 2 + slot) * tpr + lane) * SF;
@@ -367,6 +470,9 @@ inline size_t runs_workspace_bytes(int64_t n_edges, int64_t feat,
   return (size_t)n_wg * 2 * (size_t)slots * state_floats_per_feature * sizeof(float);
 }
 
+// `line_slices`: the feature row is taken in slices of eight lanes (one 128-byte line
+// of 16-byte lanes), one slice after the other over all runs, instead of whole: the
+// part of the table that the caches have to hold shrinks with the slice.
 // `partial_bytes`: capacity of `partial`.  The launch needs two partial rows per
 // workgroup of the layout actually chosen (never more than runs_workspace_bytes)
 // and returns GA_EWORKSPACE, having launched nothing, when that does not fit.
@@ -376,12 +482,13 @@ template <class Policy>
 int launch_runs(typename Policy::Args args, const int32_t *pointer,
                 const int32_t *row_of_slot, void *out, int64_t n_rows,
                 int64_t n_edges, int feat, float *partial, hipStream_t stream,
-                size_t partial_bytes = SIZE_MAX, size_t *size_only = nullptr) {
+                size_t partial_bytes = SIZE_MAX, size_t *size_only = nullptr,
+                bool line_slices = false) {
   constexpr int VEC = Policy::kVec;
   constexpr int SF = Policy::kState;
   RunGeom geo;
   const int lanes = (feat + VEC - 1) / VEC;
-  geo.tpr_shift = ilog2_ceil((uint64_t)(lanes > kWave ? kWave : lanes));
+  geo.tpr_shift = line_slices ? 3 : ilog2_ceil((uint64_t)(lanes > kWave ? kWave : lanes));
   const int tpr = 1 << geo.tpr_shift;
   const int ftiles = (lanes + tpr - 1) / tpr;
   geo.run_shift = run_shift_for(n_edges, feat);

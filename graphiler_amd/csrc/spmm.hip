@@ -55,13 +55,14 @@ __device__ __forceinline__ float bin_apply(float x, float w) {
 // walk over the slots, once per unrolled position, and a choice made there at run time
 // triples the loop's code.
 template <typename T, int VEC, int RED, int BOP, bool SPREAD = false, bool EPI = false,
-          int ACT = GA_ACT_NONE>
+          int ACT = GA_ACT_NONE, int GL = 0>
 struct SpmmPolicy {
   static constexpr bool HASW = BOP != 0;
   typedef T out_t;
   static constexpr int kVec = VEC;
   static constexpr int kState = VEC + (EPI ? 1 : 0);
   static constexpr bool kSpread = SPREAD;
+  static constexpr int kGL = GL;
   struct Args {
     const int32_t *gidx;  // row of `u` gathered per slot (neighbour id, or edge
                           // id for copy_e); nullptr: the slot index itself
@@ -134,6 +135,69 @@ struct SpmmPolicy {
     typedef RowIO<T, VEC, SPREAD> IO;
     const typename IO::lane_t ln = IO::lane(A.stride_shift, feat - f0);
     const int h = HASW && !SPREAD ? f0 / A.dph : 0;
+    if constexpr (GL > 0) {
+      typedef GroupCol<GL> Col;
+      const int sub = threadIdx.x & (GL - 1);
+      GroupIds<GL> ids, next;
+      int e = 0, e_next = 0;              // edge ids of the weights
+      auto load_cols = [&](int64_t j, GroupIds<GL> &I, int &E) {
+        I.load(row_of_slot, A.gidx, j, b, sub);
+        if constexpr (HASW) {
+          const int64_t jj = Col::slot(j, b, sub);
+          E = A.eid ? A.eid[jj] : (int)jj;
+        }
+      };
+      load_cols(a, ids, e);
+      for (int64_t j = a; j < b; j += kUnroll) {
+        // the columns of the next batch arrive under this batch's gathers
+        load_cols(j + kUnroll, next, e_next);
+        typename IO::raw_t x[kUnroll];
+        float ww[kUnroll], rsv = 1.0f;
+        if constexpr (HASW) {
+          const float wv = A.w[(int64_t)e * A.heads + h];    // the lanes are in one head
+          static_for<kUnroll>([&](auto t) { ww[t] = Col::template get<t>(wv); });
+        }
+        static_for<kUnroll>([&](auto t) {
+          x[t] = IO::load(A.u + (int64_t)ids.template index_of<t>() * feat + f0, ln);
+        });
+        if constexpr (EPI) {
+          if (A.row_scale) rsv = A.row_scale[ids.my_row(sub)];
+        }
+        const bool one_row = j + kUnroll <= b && ids.template row_of<0>() == cur &&
+                             ids.template row_of<kUnroll - 1>() == cur;
+        if (one_row) {                    // rows are sorted: the whole batch is the open row's
+#pragma unroll
+          for (int t = 0; t < kUnroll; ++t) {
+            float xf[VEC];
+            IO::widen(x[t], xf);
+#pragma unroll
+            for (int v = 0; v < VEC; ++v)
+              st[v] = red_apply<RED>(st[v], bin_apply<BOP>(xf[v], ww[t]));
+          }
+          if constexpr (EPI) st[VEC] = Col::template get<0>(rsv);
+        } else {
+          static_for<kUnroll>([&](auto t) {
+            if (j + t < b) {
+              const int r = ids.template row_of<t>();
+              if (r != cur) {
+                close_segment();
+                cur = r;
+                init(st);
+              }
+              float xf[VEC];
+              IO::widen(x[t], xf);
+#pragma unroll
+              for (int v = 0; v < VEC; ++v)
+                st[v] = red_apply<RED>(st[v], bin_apply<BOP>(xf[v], ww[t]));
+              if constexpr (EPI) st[VEC] = Col::template get<t>(rsv);
+            }
+          });
+        }
+        ids = next;
+        e = e_next;
+      }
+      return;
+    }
     for (int64_t j = a; j < b; j += kUnroll) {
       int r[kUnroll], g[kUnroll], e[kUnroll];
       float ww[kUnroll];
@@ -182,19 +246,54 @@ struct SpmmPolicy {
   }
 };
 
+// Rows of whole 128-byte lines, gathered by node, are taken a line at a time where the
+// table is several times the 4 MB of an L2 and a row has enough slots to hide the second
+// walk over the columns: the line that is gathered leaves the L2 room for that many more
+// of the often-gathered rows.  R-MAT, 64 fp32 features, one slice -> two: 232,965 nodes
+// 114.6 M edges 2.01 -> 1.93 ms (L2 misses 99 M -> 84 M lines), 11.6 M edges 269 -> 238 us;
+// with seven edges per node (169,343 nodes) the second walk costs more, 39 -> 58 us.
+template <typename T, int VEC, int BOP, bool SPREAD>
+bool line_slices(const int32_t *gidx, const int32_t *eid, int64_t n_rows, int64_t n_edges,
+                 int feat) {
+  return BOP == 0 && !SPREAD && VEC * sizeof(T) == 16 && gidx && gidx != eid &&
+         feat % (8 * VEC) == 0 && n_edges >= 32 * n_rows &&
+         n_rows * feat * (int64_t)sizeof(T) >= ((int64_t)16 << 20);
+}
+
 template <typename T, int VEC, int RED, int BOP, bool SPREAD, bool EPI = false,
-          int ACT = GA_ACT_NONE>
+          int ACT = GA_ACT_NONE, int GL = 0>
 int launch_spmm(const int32_t *pointer, const int32_t *row_of_slot,
                 const int32_t *gidx, const int32_t *eid, const void *u,
                 const float *w, void *out, int64_t n_rows, int64_t n_edges,
                 int feat, int heads, float *partial, hipStream_t stream,
                 const float *row_scale = nullptr, size_t partial_bytes = SIZE_MAX) {
-  typedef SpmmPolicy<T, VEC, RED, BOP, SPREAD, EPI, ACT> P;
+  if constexpr (GL == 0 && VEC > 1 && (BOP == 0 || BOP == GA_U_MUL_E)) {
+    // lane groups of eight lanes and more share the columns they read; with edge data
+    // only where the sharing lanes lie in one head (otherwise the edge datum is a read
+    // per slot and lane again: four heads of 16, 875 k edges, 38 us either way)
+    const int lanes = (feat + VEC - 1) / VEC;
+    const int head_lanes = BOP == 0 || heads == 1 ? 16 : feat / heads % (16 * VEC) == 0 ? 16
+                           : feat / heads % (8 * VEC) == 0 ? 8 : 0;
+#define GA_SPMM_GL(N)                                                                         \
+  return launch_spmm<T, VEC, RED, BOP, SPREAD, EPI, ACT, N>(pointer, row_of_slot, gidx, eid, u, \
+                                                            w, out, n_rows, n_edges, feat,    \
+                                                            heads, partial, stream, row_scale, \
+                                                            partial_bytes)
+    if (lanes > 8 && head_lanes == 16 &&
+        !line_slices<T, VEC, BOP, SPREAD>(gidx, eid, n_rows, n_edges, feat))
+      GA_SPMM_GL(16);
+    if (lanes > 4 && (lanes <= 8 ? head_lanes >= 8
+                                 : line_slices<T, VEC, BOP, SPREAD>(gidx, eid, n_rows, n_edges, feat)))
+      GA_SPMM_GL(8);
+#undef GA_SPMM_GL
+  }
+  typedef SpmmPolicy<T, VEC, RED, BOP, SPREAD, EPI, ACT, GL> P;
   const bool ids_vec = aligned(row_of_slot, 16) && (!gidx || aligned(gidx, 16)) &&
                        (!eid || aligned(eid, 16));
   typename P::Args args{gidx, eid, (const T *)u, w, heads, feat / heads, ids_vec, 0, row_scale};
   return launch_runs<P>(args, pointer, row_of_slot, out, n_rows, n_edges, feat,
-                        partial, stream, partial_bytes);
+                        partial, stream, partial_bytes, nullptr,
+                        GL == 8 && feat > 8 * VEC);
 }
 
 // ---- sums of rows of at most eight features: one or two lanes per slot --------
@@ -520,6 +619,7 @@ struct SpmmArgPolicy {
   static constexpr int kVec = VEC;
   static constexpr int kState = 2 * VEC;
   static constexpr bool kSpread = false;
+  static constexpr int kGL = 0;
   struct Args {
     const int32_t *gidx;  // row of `u` gathered per slot; nullptr: the slot index
     const int32_t *eid;   // edge id per slot; nullptr: the slot index
