@@ -11,7 +11,13 @@ int run_shift_for(int64_t n_edges, int64_t feat) {
   // aim at >= 16k wavefronts of work, between 32 and 1024 slots per run
   int64_t per_run = (n_edges << lane_shift) / 64 / 16384;
   int shift = per_run < 1 ? 0 : ilog2_floor((uint64_t)per_run);
-  if (shift < 5) shift = 5;
+  // (32 slots amortise a run's start) -- down to 8 where that leaves under 2k wavefronts
+  // for the 1,024 SIMDs: a run is a chain of dependent batches of eight slots, and a
+  // small graph takes as long as its chain
+  if (shift < 5) {
+    const int64_t few = (n_edges << lane_shift) / 64 / 2048;
+    shift = few < 8 ? 3 : few < 32 ? ilog2_floor((uint64_t)few) : 5;
+  }
   if (shift > 10) shift = 10;
   return shift;
 }
