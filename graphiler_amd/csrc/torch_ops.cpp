@@ -207,6 +207,7 @@ struct DGLGraph : torch::CustomClassHolder {
   // with library sorts and scans; `valid` is false when the slots are not so grouped.
   struct RelationPairs {
     int64_t num_pairs = 0;
+    int64_t max_slots = 0;             // slots of the largest pair
     torch::Tensor pair_pointer, pair_of_slot, pair_dst, dst_pointer, type_pointer;   // int32
     torch::Tensor by_type, dst_by_type;                                              // int64
     torch::Tensor rank, rank_of_slot;                                                // int32
@@ -240,8 +241,9 @@ struct DGLGraph : torch::CustomClassHolder {
           torch::Tensor rank = torch::empty_like(by_type);
           rank.index_copy_(0, by_type, torch::arange(P, i64));
           pairs_.num_pairs = P;
-          pairs_.pair_pointer =
-              torch::cat({starts, torch::full({1}, num_edges, i64)}).to(at::kInt).contiguous();
+          torch::Tensor bounds = torch::cat({starts, torch::full({1}, num_edges, i64)});
+          pairs_.max_slots = torch::diff(bounds).max().item<int64_t>();
+          pairs_.pair_pointer = bounds.to(at::kInt).contiguous();
           pairs_.pair_of_slot = pair_of_slot.to(at::kInt).contiguous();
           pairs_.pair_dst = pair_dst.to(at::kInt).contiguous();
           pairs_.dst_pointer = torch::searchsorted(pair_dst.contiguous(),
@@ -1198,8 +1200,29 @@ torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::T
                                 y.data_ptr(), nullptr, nullptr, nullptr, nullptr, nullptr, P, heads,
                                 d, d, dt, stream);
   };
+  // products, scores, softmax inside every pair and weighted sum in one pass where its
+  // shape fits
+  torch::Tensor m_pair = torch::empty({P, hid}, k.options());
+  torch::Tensor lse = torch::empty({P, heads}, k.options().dtype(at::kFloat));
+  int rc = ga_pair_attention(pairs.type_pointer.data_ptr<int>(), graph->num_etypes,
+                             pairs.by_type.data_ptr<int64_t>(), pairs.dst_by_type.data_ptr<int64_t>(),
+                             pairs.pair_pointer.data_ptr<int>(),
+                             graph->in_node_indices.data_ptr<int>(), q.data_ptr(), k.data_ptr(),
+                             v.data_ptr(), att_t.data_ptr(), relation_msg.data_ptr(),
+                             m_pair.data_ptr(), lse.data_ptr<float>(), P, pairs.max_slots, heads, d,
+                             dt, stream);
+  if (rc != GA_EUNSUPPORTED) {
+    check_ga(rc, "ga_pair_attention");
+    torch::Tensor ws = graph->workspace(ga_gat_workspace_bytes(P, hid, heads));
+    torch::Tensor out = torch::empty({n, hid}, k.options());
+    check_ga(ga_edge_softmax_sum(pairs.dst_pointer.data_ptr<int>(), pairs.pair_dst.data_ptr<int>(),
+                                 nullptr, lse.data_ptr<float>(), m_pair.data_ptr(), out.data_ptr(),
+                                 n, P, heads, d, dt, ws.data_ptr(), (size_t)ws.numel(), stream),
+             "ga_edge_softmax_sum");
+    return out;
+  }
   torch::Tensor q_pair = torch::empty({P, hid}, k.options());
-  int rc = typed_rows(q, pairs.dst_by_type, att_t, q_pair);
+  rc = typed_rows(q, pairs.dst_by_type, att_t, q_pair);
   if (rc == GA_EUNSUPPORTED) return per_edge();
   check_ga(rc, "ga_segment_mm_gather");
   // both passes share the scratch; the bytes are not monotonic in the number of items
@@ -1208,7 +1231,6 @@ torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::T
       {ga_gat_workspace_bytes(e, hid, heads), ga_gat_workspace_bytes(P, hid, heads),
        ga_softmax_workspace_bytes(P, heads), ga_spmm_workspace_bytes(P, hid)}));
   torch::Tensor v_pair = torch::empty({P, hid}, k.options());
-  torch::Tensor lse = torch::empty({P, heads}, k.options().dtype(at::kFloat));
   rc = ga_dot_attention_sum(pairs.pair_pointer.data_ptr<int>(), pairs.pair_of_slot.data_ptr<int>(),
                             graph->in_node_indices.data_ptr<int>(),
                             pairs.rank_of_slot.data_ptr<int>(), k.data_ptr(), q_pair.data_ptr(),
@@ -1218,7 +1240,6 @@ torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::T
   if (rc == GA_EUNSUPPORTED) return per_edge();
   check_ga(rc, "ga_dot_attention_sum");
   // (the log-sum-exps were written in by_type order, the row order of m_pair)
-  torch::Tensor m_pair = torch::empty({P, hid}, k.options());
   check_ga(typed_rows(v_pair, pairs.by_type, relation_msg, m_pair), "ga_segment_mm_gather");
   torch::Tensor out = torch::empty({n, hid}, k.options());
   check_ga(ga_edge_softmax_sum(pairs.dst_pointer.data_ptr<int>(), pairs.pair_dst.data_ptr<int>(),

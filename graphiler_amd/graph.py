@@ -241,6 +241,7 @@ class RelationPairs:
     Pairs are numbered in slot order (by destination, then relation); ``by_type``
     lists them by relation (stable), which is the row order the typed products need."""
     num_pairs: int
+    max_slots: int                  # slots of the largest pair
     pair_pointer: torch.Tensor      # (P + 1) int32: first slot of every pair
     pair_of_slot: torch.Tensor      # (E) int32
     pair_dst: torch.Tensor          # (P) int32, ascending
@@ -273,9 +274,11 @@ def _build_relation_pairs(g: "DGLGraph") -> Optional[RelationPairs]:
     by_type = torch.argsort(pair_type, stable=True)
     rank = torch.empty_like(by_type)
     rank[by_type] = torch.arange(n_pairs, device=dev)
+    bounds = torch.cat([starts, starts.new_tensor([n_edges])])
     return RelationPairs(
         num_pairs=n_pairs,
-        pair_pointer=torch.cat([starts, starts.new_tensor([n_edges])]).int().contiguous(),
+        max_slots=int(torch.diff(bounds).max().item()),
+        pair_pointer=bounds.int().contiguous(),
         pair_of_slot=pair_of_slot.int().contiguous(),
         pair_dst=pair_dst.int().contiguous(),
         dst_pointer=torch.searchsorted(pair_dst.contiguous(),

@@ -517,6 +517,26 @@ int ga_dot_attention_sum(const int32_t *pointer, const int32_t *row_of_slot,
                          int64_t n_rows, int64_t n_edges, int64_t heads, int64_t dim, int dtype,
                          void *workspace, size_t workspace_bytes, ga_stream_t stream);
 
+/* The per-relation part of an HGT layer (examples/HGT/HGT.py:35-53) over the (destination,
+ * relation) pairs of a graph, in one pass; pairs are numbered in slot order, row r of the
+ * by_type order is pair by_type[r]:
+ *   qp       = q[dst_by_type[r], :] @ att[type(r)]                    (per head)
+ *   s_i      = <k[nbr[i], h, :], qp[h, :]>   for the slots pair_pointer[p] <= i < pair_pointer[p + 1]
+ *   lse[p]   = log sum_i exp(s_i),   m[p, :] = (sum_i softmax_p(s)_i v[nbr[i], :]) @ msg[type(r)]
+ * type_pointer (n_types + 1) int32 over the by_type order; by_type, dst_by_type (n_pairs)
+ * int64; pair_pointer (n_pairs + 1) int32, no pair empty; att, msg (n_types, heads, dim, dim),
+ * q, k, v (*, heads*dim), m (n_pairs, heads*dim) `dtype`; lse (n_pairs, heads) fp32.
+ * max_slots: the slots of the largest pair (the caller's claim, used to choose only).
+ * GA_EUNSUPPORTED, having launched nothing, for pairs above 256 slots, heads*dim other than
+ * 64 and 128, dim other than 8, 16, 32 and 64, rows not 16-byte aligned: the caller then
+ * runs ga_segment_mm_gather, ga_dot_attention_sum and ga_segment_mm_gather. */
+int ga_pair_attention(const int32_t *type_pointer, int64_t n_types, const int64_t *by_type,
+                      const int64_t *dst_by_type, const int32_t *pair_pointer,
+                      const int32_t *nbr, const void *q, const void *k, const void *v,
+                      const void *att, const void *msg, void *m, float *lse, int64_t n_pairs,
+                      int64_t max_slots, int64_t heads, int64_t dim, int dtype,
+                      ga_stream_t stream);
+
 /* The softmax-weighted reduction with per-edge operands:
  *   a = softmax_v(logit[e, h] over the in-edges e of v),
  *   out[v, h, :] = sum_e a_e * m[e, h, :]
