@@ -17,7 +17,12 @@
 // softmax.  As three launches the pairs' rows crossed memory four more times (qp and vp
 // written and read back) and the matrix cores and the gathers never ran together.
 //
-// Bound: the gathered key and value rows, 2 F b bytes per edge.  A lane group walks a pair
+// Bound: the gathered key and value rows, 2 F b bytes per edge, at the rate the caches
+// behind the L2s deliver.  4.76 M edges in 1.95 M pairs of 64 fp32 features: 194 + 650 +
+// 226 us as three launches, 660 us here (3.4 GB, 5.2 TB/s); 2 M edges in 270 k pairs, 8
+// heads of 16 in bf16: 38 + 159 + 40 -> 140 us.  Five wavefronts per SIMD (96 registers)
+// hide more of the gathers than the four it takes by itself (251 -> 238 us for that layer;
+// six spill nothing but load less at once: 251).  A lane group walks a pair
 // alone, so the rule of the dispatch refuses graphs with very large pairs (the host knows
 // the largest): those run as separate passes over equal runs of slots.
 #include "common.h"
@@ -121,7 +126,7 @@ __device__ __forceinline__ float head_sum(float v) {     // over LANES adjacent 
 }
 
 template <typename T, int F, int D>
-__global__ __launch_bounds__(kBlock) void pair_attn_kernel(PairArgs A) {
+__global__ __launch_bounds__(kBlock, 5) void pair_attn_kernel(PairArgs A) {
   constexpr int VEC = 16 / (int)sizeof(T);
   constexpr int LPR = F / VEC;                    // lanes per row
   constexpr int G = kBlock / LPR;                 // lane groups
@@ -290,9 +295,11 @@ __global__ __launch_bounds__(kBlock) void pair_attn_kernel(PairArgs A) {
 
 template <typename T, int F, int D>
 int launch_pairs(PairArgs &A, int64_t n_pairs, hipStream_t s) {
-  // four tiles share a load of the weights where that leaves several workgroups per CU
+  // four tiles share a load of the weights on large pair lists (30.5 k tiles of 64 fp32
+  // features: 606 us with two, 584 with four for the layer); on 4.2 k tiles a workgroup per
+  // tile fills the chip more evenly (239 -> 216 us for the layer)
   const int64_t tiles = (n_pairs + kPairRows - 1) / kPairRows;
-  const int64_t steps = tiles >= 16384 ? 4 : tiles >= 4096 ? 2 : 1;
+  const int64_t steps = tiles >= 16384 ? 4 : 1;
   A.chunk_rows = (int)steps * kPairRows;
   const int64_t grid = (n_pairs + A.chunk_rows - 1) / A.chunk_rows + A.n_types;
   if (grid > 0x7fffffff) return GA_EUNSUPPORTED;
