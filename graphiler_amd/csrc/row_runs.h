@@ -470,9 +470,6 @@ inline size_t runs_workspace_bytes(int64_t n_edges, int64_t feat,
   return (size_t)n_wg * 2 * (size_t)slots * state_floats_per_feature * sizeof(float);
 }
 
-// `line_slices`: the feature row is taken in slices of eight lanes (one 128-byte line
-// of 16-byte lanes), one slice after the other over all runs, instead of whole: the
-// part of the table that the caches have to hold shrinks with the slice.
 // `partial_bytes`: capacity of `partial`.  The launch needs two partial rows per
 // workgroup of the layout actually chosen (never more than runs_workspace_bytes)
 // and returns GA_EWORKSPACE, having launched nothing, when that does not fit.
@@ -482,13 +479,12 @@ template <class Policy>
 int launch_runs(typename Policy::Args args, const int32_t *pointer,
                 const int32_t *row_of_slot, void *out, int64_t n_rows,
                 int64_t n_edges, int feat, float *partial, hipStream_t stream,
-                size_t partial_bytes = SIZE_MAX, size_t *size_only = nullptr,
-                bool line_slices = false) {
+                size_t partial_bytes = SIZE_MAX, size_t *size_only = nullptr) {
   constexpr int VEC = Policy::kVec;
   constexpr int SF = Policy::kState;
   RunGeom geo;
   const int lanes = (feat + VEC - 1) / VEC;
-  geo.tpr_shift = line_slices ? 3 : ilog2_ceil((uint64_t)(lanes > kWave ? kWave : lanes));
+  geo.tpr_shift = ilog2_ceil((uint64_t)(lanes > kWave ? kWave : lanes));
   const int tpr = 1 << geo.tpr_shift;
   const int ftiles = (lanes + tpr - 1) / tpr;
   geo.run_shift = run_shift_for(n_edges, feat);

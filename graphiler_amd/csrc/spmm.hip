@@ -252,20 +252,6 @@ struct SpmmPolicy {
   }
 };
 
-// Rows of whole 128-byte lines, gathered by node, are taken a line at a time where the
-// table is several times the 4 MB of an L2 and a row has enough slots to hide the second
-// walk over the columns: the line that is gathered leaves the L2 room for that many more
-// of the often-gathered rows.  R-MAT, 64 fp32 features, one slice -> two: 232,965 nodes
-// 114.6 M edges 2.01 -> 1.93 ms (L2 misses 99 M -> 84 M lines), 11.6 M edges 269 -> 238 us;
-// with seven edges per node (169,343 nodes) the second walk costs more, 39 -> 58 us.
-template <typename T, int VEC, int BOP, bool SPREAD>
-bool line_slices(const int32_t *gidx, const int32_t *eid, int64_t n_rows, int64_t n_edges,
-                 int feat) {
-  return BOP == 0 && !SPREAD && VEC * sizeof(T) == 16 && gidx && gidx != eid &&
-         feat % (8 * VEC) == 0 && n_edges >= 32 * n_rows &&
-         n_rows * feat * (int64_t)sizeof(T) >= ((int64_t)16 << 20);
-}
-
 template <typename T, int VEC, int RED, int BOP, bool SPREAD, bool EPI = false,
           int ACT = GA_ACT_NONE, int GL = 0>
 int launch_spmm(const int32_t *pointer, const int32_t *row_of_slot,
@@ -285,12 +271,8 @@ int launch_spmm(const int32_t *pointer, const int32_t *row_of_slot,
                                                             w, out, n_rows, n_edges, feat,    \
                                                             heads, partial, stream, row_scale, \
                                                             partial_bytes)
-    if (lanes > 8 && head_lanes == 16 &&
-        !line_slices<T, VEC, BOP, SPREAD>(gidx, eid, n_rows, n_edges, feat))
-      GA_SPMM_GL(16);
-    if (lanes > 4 && (lanes <= 8 ? head_lanes >= 8
-                                 : line_slices<T, VEC, BOP, SPREAD>(gidx, eid, n_rows, n_edges, feat)))
-      GA_SPMM_GL(8);
+    if (lanes > 8 && head_lanes == 16) GA_SPMM_GL(16);
+    if (lanes > 4 && lanes <= 8 && head_lanes >= 8) GA_SPMM_GL(8);
 #undef GA_SPMM_GL
   }
   typedef SpmmPolicy<T, VEC, RED, BOP, SPREAD, EPI, ACT, GL> P;
@@ -298,8 +280,7 @@ int launch_spmm(const int32_t *pointer, const int32_t *row_of_slot,
                        (!eid || aligned(eid, 16));
   typename P::Args args{gidx, eid, (const T *)u, w, heads, feat / heads, ids_vec, 0, row_scale};
   return launch_runs<P>(args, pointer, row_of_slot, out, n_rows, n_edges, feat,
-                        partial, stream, partial_bytes, nullptr,
-                        GL == 8 && feat > 8 * VEC);
+                        partial, stream, partial_bytes);
 }
 
 // ---- sums of rows of at most eight features: one or two lanes per slot --------

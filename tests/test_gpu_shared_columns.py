@@ -1,6 +1,6 @@
 """Row reductions whose lane groups read the slot-indexed columns for one another
-(groups of 8 lanes and of 16 and more), rows taken a line at a time, and the short runs
-of small graphs: widths around the lane counts where the layouts change, against the oracle."""
+(groups of 8 lanes and of 16 and more), dense graphs with tables of several times an L2,
+and the short runs of small graphs: widths around the lane counts where the layouts change, against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -84,9 +84,9 @@ def test_heads_with_and_without_a_shared_batch(device, heads, dim, bf16):
     assert_close(got.float().cpu().numpy().reshape(n, -1), ref.reshape(n, -1), tol, "gat")
 
 
-# 32 edges per node and a table of 16 MB: from here on rows are taken a line at a time
+# 32 edges per node and a table of 16 MB, several times an L2
 @pytest.mark.parametrize("feat,bf16", [(64, False), (128, False), (192, True), (256, True)])
-def test_rows_taken_a_line_at_a_time(device, feat, bf16):
+def test_dense_graph_with_a_large_table(device, feat, bf16):
     rng = np.random.default_rng(feat)
     n = (16 << 20) // (feat * (2 if bf16 else 4)) + 1
     edges = 32 * n
@@ -99,8 +99,8 @@ def test_rows_taken_a_line_at_a_time(device, feat, bf16):
     ref = oracle.spmm(*adj, x)
     dx = _dev(x, device, bf16)
     got = ops.SpMMSrc(dx, [1], False, None, g).float().cpu().numpy()
-    assert_close(got, ref, TOL_BF16 if bf16 else TOL_F32, f"line slices F={feat}")
+    assert_close(got, ref, TOL_BF16 if bf16 else TOL_F32, f"large table F={feat}")
     scale = rng.standard_normal(n).astype(np.float32)
     got = ops.spmm_scaled(dx, g, row_scale=_dev(scale, device), activation="relu")
     assert_close(got.float().cpu().numpy(), np.maximum(ref * scale[:, None], 0),
-                 TOL_BF16 if bf16 else TOL_F32, f"line slices, scaled F={feat}")
+                 TOL_BF16 if bf16 else TOL_F32, f"large table, scaled F={feat}")
