@@ -148,8 +148,6 @@ struct GatPolicy {
       GroupIds<GL> ids, next;
       ids.load(row_of_slot, A.nbr, a, b, sub);
       for (int64_t j = a; j < b; j += kUnroll) {
-        // the columns of the next batch arrive under this batch's gathers
-        next.load(row_of_slot, A.nbr, j + kUnroll, b, sub);
         typename IO::raw_t x[kUnroll];
         float sv;                   // lane i holds the logit of slot (i & 7)
         if constexpr (MODE == kGatEdge) {
@@ -170,6 +168,11 @@ struct GatPolicy {
         static_for<kUnroll>([&](auto t) {
           x[t] = IO::load(A.z + (int64_t)ids.template index_of<t>() * feat + f0, ln);
         });
+        // the columns of the next batch arrive while this batch's rows are added; asked for
+        // after the gathers (GroupIds)
+        __builtin_amdgcn_sched_barrier(0);
+        next.load(row_of_slot, A.nbr, j + kUnroll, b, sub);
+        __builtin_amdgcn_sched_barrier(0);
         const bool one_row = j + kUnroll <= b && ids.template row_of<0>() == cur &&
                              ids.template row_of<kUnroll - 1>() == cur;
         if (one_row) {

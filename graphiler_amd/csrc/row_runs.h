@@ -121,6 +121,11 @@ __device__ __forceinline__ float other_half(float v) {
 // The row ids and the gather indices of a batch.  With 16 lanes or more one load
 // serves both columns: lanes 0 .. 7 of every 16 hold the rows, lanes 8 .. 15 the
 // indices.  `index` may be null: the slots themselves are the indices.
+// A batch's columns are asked for one batch ahead and after the gathers of the batch before:
+// loads return in order, so in front of them the rows would wait for a streaming load
+// (10 M uniform edges, 64 fp32 features: 392 us with lanes reading for themselves, 397 with
+// the load in front, 390 behind; 2 M edges with the rows in the L2, 128 features: 1.25 -> 1.26
+// times the speed).
 template <int GL>
 struct GroupIds {
   typedef GroupCol<GL> Col;

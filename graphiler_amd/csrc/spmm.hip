@@ -155,8 +155,6 @@ struct SpmmPolicy {
       };
       load_cols(a, ids, e);
       for (int64_t j = a; j < b; j += kUnroll) {
-        // the columns of the next batch arrive under this batch's gathers
-        load_cols(j + kUnroll, next, e_next);
         typename IO::raw_t x[kUnroll];
         float ww[kUnroll], rsv = 1.0f;
         if constexpr (HASW) {
@@ -169,6 +167,11 @@ struct SpmmPolicy {
         if constexpr (EPI) {
           if (A.row_scale) rsv = A.row_scale[ids.my_row(sub)];
         }
+        // the columns of the next batch arrive while this batch's rows are added; asked for
+        // after the gathers (GroupIds)
+        __builtin_amdgcn_sched_barrier(0);
+        load_cols(j + kUnroll, next, e_next);
+        __builtin_amdgcn_sched_barrier(0);
         const bool one_row = j + kUnroll <= b && ids.template row_of<0>() == cur &&
                              ids.template row_of<kUnroll - 1>() == cur;
         if (one_row) {                    // rows are sorted: the whole batch is the open row's
