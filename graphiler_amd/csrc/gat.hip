@@ -456,15 +456,16 @@ int launch_gat(const int32_t *pointer, const int32_t *row_of_slot,
   }
   if constexpr (GL == 0 && VEC > 1 && MODE != kGatFromZ) {
     // lane groups of eight lanes and more share the columns and the logits they form from
-    // them, where the sharing lanes lie in one head
-    const int share = heads == 1 ? 16 : dim % (16 * VEC) == 0 ? 16 : dim % (8 * VEC) == 0 ? 8 : 0;
+    // them, where the sharing lanes lie in one head (two fp32 heads of 32 are eight lanes
+    // each: they keep their own reads)
+    const bool one_head = heads == 1;
     const int lanes = (heads * dim + VEC - 1) / VEC;
 #define GA_GAT_GL(N)                                                                            \
   return launch_gat<T, VEC, MODE, SPREAD, ACT, N>(pointer, row_of_slot, nbr, el, er, z, out,    \
                                                   n_rows, n_edges, heads, dim, slope, ws, stream, \
                                                   ws_bytes, act, size_only)
-    if (lanes > 8 && share == 16) GA_GAT_GL(16);
-    if (lanes > 4 && lanes <= 8 && share >= 8) GA_GAT_GL(8);
+    if (lanes > 8 && (one_head || dim % (16 * VEC) == 0)) GA_GAT_GL(16);
+    if (lanes > 4 && lanes <= 8 && one_head) GA_GAT_GL(8);
 #undef GA_GAT_GL
   }
   typedef GatPolicy<T, VEC, MODE, SPREAD, ACT, GL> P;

@@ -262,20 +262,41 @@ int launch_spmm(const int32_t *pointer, const int32_t *row_of_slot,
                 const float *w, void *out, int64_t n_rows, int64_t n_edges,
                 int feat, int heads, float *partial, hipStream_t stream,
                 const float *row_scale = nullptr, size_t partial_bytes = SIZE_MAX) {
+  // Lane groups that read the columns for one another (GroupCol).  Always where a lane's
+  // features lie apart or the row gets a factor: there the lanes' own reads are four-byte
+  // loads per slot and lane (41 features, R-MAT, 11.6 M edges: copy_u 1.07, scaled 1.40
+  // times the speed).  Otherwise only where it was not slower on any of eight graphs (10 k
+  // to 12 M edges, R-MAT and uniform; speed against lanes that read for themselves):
+  //   copy_u, fp32   groups of 16 and more 0.98 .. 1.34; of eight: sums 0.98 .. 1.1, max
+  //                  and min 0.96 .. 1.08 and so not
+  //   copy_u, bf16   eight features a lane keep the vector units busy, and the exchange adds
+  //                  to that: sums 0.93 .. 1.1 up to 16 lanes, 0.97 .. 1.2 above; max 0.90
+  //                  .. 1.2 and so not
+  //   u_mul_e        groups of 16 and more 0.96 .. 1.5; of eight 0.91 .. 1.15 and so not
+  //   copy_e         the rows stream, the columns are little beside them: fp32 0.95 .. 1.1,
+  //                  bf16 0.92 .. 1.03, and so not
+  // With edge data the sharing lanes have to lie in one head (four heads of 16, 875 k
+  // edges: 38 us either way): heads narrower than 16 lanes keep their own reads.
   if constexpr (GL == 0 && VEC > 1 && (BOP == 0 || BOP == GA_U_MUL_E)) {
-    // lane groups of eight lanes and more share the columns they read; with edge data
-    // only where the sharing lanes lie in one head (otherwise the edge datum is a read
-    // per slot and lane again: four heads of 16, 875 k edges, 38 us either way)
+    constexpr bool kPlain = !SPREAD && !EPI, kHalf = sizeof(T) == 2;
+    constexpr bool kShare16 = !kPlain || BOP != 0 || !kHalf || RED == GA_SUM;
+    constexpr bool kShare8 = !kPlain || (BOP == 0 && !kHalf && RED == GA_SUM);
     const int lanes = (feat + VEC - 1) / VEC;
-    const int head_lanes = BOP == 0 || heads == 1 ? 16 : feat / heads % (16 * VEC) == 0 ? 16
-                           : feat / heads % (8 * VEC) == 0 ? 8 : 0;
+    const bool streams = kPlain && BOP == 0 && (!gidx || gidx == eid);      // copy_e
+    const bool one_head = BOP == 0 || heads == 1;
 #define GA_SPMM_GL(N)                                                                         \
   return launch_spmm<T, VEC, RED, BOP, SPREAD, EPI, ACT, N>(pointer, row_of_slot, gidx, eid, u, \
                                                             w, out, n_rows, n_edges, feat,    \
                                                             heads, partial, stream, row_scale, \
                                                             partial_bytes)
-    if (lanes > 8 && head_lanes == 16) GA_SPMM_GL(16);
-    if (lanes > 4 && lanes <= 8 && head_lanes >= 8) GA_SPMM_GL(8);
+    if constexpr (kShare16) {
+      if (lanes > (kPlain && BOP == 0 && kHalf ? 16 : 8) && !streams &&
+          (one_head || feat / heads % (16 * VEC) == 0))
+        GA_SPMM_GL(16);
+    }
+    if constexpr (kShare8) {
+      if (lanes > 4 && lanes <= 8 && !streams && one_head) GA_SPMM_GL(8);
+    }
 #undef GA_SPMM_GL
   }
   typedef SpmmPolicy<T, VEC, RED, BOP, SPREAD, EPI, ACT, GL> P;
