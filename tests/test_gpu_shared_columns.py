@@ -84,6 +84,34 @@ def test_heads_with_and_without_a_shared_batch(device, heads, dim, bf16):
     assert_close(got.float().cpu().numpy().reshape(n, -1), ref.reshape(n, -1), tol, "gat")
 
 
+# rows over one run of eight slots, over as many runs as a word of flags has bits and one less
+# and more, over all runs of a workgroup: the chain inside a workgroup from every lane-group width
+@pytest.mark.parametrize("feat", [1, 3, 5, 8, 12, 20, 64, 100])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_rows_over_many_runs(device, feat, bf16):
+    rng = np.random.default_rng(feat)
+    lengths = np.array([1, 7, 8, 9, 16, 17, 31, 33, 503, 511, 512, 513, 520, 1017, 1024, 1033,
+                        1543, 2040, 2048, 2049, 5000, 0, 3, 64 * 8 + 4, 2, 127])
+    lengths = np.concatenate([rng.permutation(lengths), rng.permutation(lengths)])
+    n, edges = lengths.size, int(lengths.sum())
+    dst = np.repeat(np.arange(n), lengths)
+    src = rng.integers(0, n, edges)
+    g = prepare_graph(src, dst, n, device=device)
+    arr = build_graph_arrays(src, dst, n)
+    adj = (arr.in_pointer, arr.in_node_indices, arr.in_edge_indices)
+    x = rng.standard_normal((n, feat), dtype=np.float32)
+    x = to_bf16_f32(x) if bf16 else x
+    el, er = (rng.standard_normal((n, 1), dtype=np.float32) for _ in range(2))
+    dx, tol = _dev(x, device, bf16), TOL_BF16 if bf16 else TOL_F32
+    host = lambda t: t.float().cpu().numpy()
+    for reduce in ("sum", "max"):
+        ref = oracle.spmm(*adj, x, op="copy_u", reduce=reduce)
+        assert_close(host(ops.spmm(g, "copy_u", reduce, dx)), ref, tol, f"{reduce} F={feat}")
+    ref = oracle.gat_aggregate(arr.in_pointer, arr.in_node_indices, el, er, x, heads=1, slope=0.2)
+    got = ops.gat_aggregate(_dev(el, device), _dev(er, device), dx, g, 0.2)
+    assert_close(host(got), ref, tol, f"gat F={feat}")
+
+
 # 32 edges per node and a table of 16 MB, several times an L2
 @pytest.mark.parametrize("feat,bf16", [(64, False), (128, False), (192, True), (256, True)])
 def test_dense_graph_with_a_large_table(device, feat, bf16):
