@@ -209,7 +209,7 @@ __global__ __launch_bounds__(kBlock, 5) void pair_attn_kernel(PairArgs A) {
         l = 0.0f;
       };
       int pos = slot0[r], end = slot1[r];
-      int ids = A.nbr[min(pos + (lane & 3), end - 1)];
+      int ids = A.nbr[pos + min(lane & 3, end - 1 - pos)];
       open_row();
       while (true) {
         const int cnt = end - pos;         // at least one
@@ -219,7 +219,7 @@ __global__ __launch_bounds__(kBlock, 5) void pair_attn_kernel(PairArgs A) {
           if (nr < r_end) { npos = slot0[nr]; nend = slot1[nr]; }
         }
         // sources of the next batch, whichever row it belongs to
-        const int ids_next = nr < r_end ? A.nbr[min(npos + (lane & 3), nend - 1)] : 0;
+        const int ids_next = nr < r_end ? A.nbr[npos + min(lane & 3, nend - 1 - npos)] : 0;
         const int g[kPairBatch] = {
             __builtin_amdgcn_update_dpp(0, ids, 0x00, 0xF, 0xF, true),      // quad_perm: lane t
             __builtin_amdgcn_update_dpp(0, ids, 0x55, 0xF, 0xF, true),
