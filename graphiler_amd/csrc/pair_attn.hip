@@ -9,22 +9,26 @@
 //
 // The pairs of a destination are weighed by the softmax of their lse afterwards.
 //
-// A workgroup takes chunks of 64 pairs of one relation.  The 64 rows stay in one LDS tile
-// from the gathered queries to the stored messages: every wavefront owns a quarter of the
-// columns, keeps its columns of both relation matrices in registers for the whole chunk
-// and multiplies all 64 rows with them; between the two products a lane group per row (16
-// bytes per lane) walks the pair's slots, gathering keys and values, with an online
-// softmax.  As three launches the pairs' rows crossed memory four more times (qp and vp
-// written and read back) and the matrix cores and the gathers never ran together.
+// A workgroup takes a tile of up to 64 pairs of one relation.  The 64 rows stay in LDS from
+// the gathered queries to the stored messages: every wavefront owns a quarter of the
+// columns and multiplies all rows with its columns of a relation matrix; between the two
+// products a lane group per row (16 bytes per lane) walks the pair's slots, gathering keys
+// and values, with an online softmax.  As three launches the pairs' rows crossed memory four
+// more times (qp and vp written and read back) and the matrix cores and the gathers never
+// ran together.
+//
+// A matrix's columns are loaded for its product alone: the walk needs neither, and held
+// across it (and several tiles per workgroup, whose addresses stay live as well) they made
+// 12 of the 16 builds spill at five wavefronts per SIMD and left fp32 rows of 128 features
+// at two or three.  72 to 107 registers now, nothing spilled, five to seven wavefronts (four
+// where the tile's 35 KB of LDS allow no more).
 //
 // Bound: the gathered key and value rows, 2 F b bytes per edge, at the rate the caches
-// behind the L2s deliver.  4.76 M edges in 1.95 M pairs of 64 fp32 features: 194 + 650 +
-// 226 us as three launches, 660 us here (3.4 GB, 5.2 TB/s); 2 M edges in 270 k pairs, 8
-// heads of 16 in bf16: 38 + 159 + 40 -> 140 us.  Five wavefronts per SIMD (96 registers)
-// hide more of the gathers than the four it takes by itself (251 -> 238 us for that layer;
-// six spill nothing but load less at once: 251).  A lane group walks a pair
-// alone, so the rule of the dispatch refuses graphs with very large pairs (the host knows
-// the largest): those run as separate passes over equal runs of slots.
+// behind the L2s deliver.  The whole pair form (this pass, the transposed matrices, the sum
+// of the pairs) as three launches -> matrices held -> now, us:
+//   4.68 M edges, 1.95 M pairs: 1 x 64 fp32 1183 -> 809 -> 709, 8 x 16 bf16 1234 -> 699 -> 671,
+//     2 x 64 fp32 2619 -> 1653 -> 1343, 2 x 64 bf16 1199 -> 875 -> 697
+//   300 k edges, 100 k pairs: 1 x 64 fp32 99 -> 67 -> 59, 8 x 16 bf16 107 -> 63 -> 59
 #include "common.h"
 #include "typed_chunks.h"
 
@@ -49,8 +53,18 @@ struct PairArgs {
   void *m;                          // (P, F), pair order
   float *lse;                       // (P, heads), pair order
   int n_types;
-  int chunk_rows;
 };
+
+// Element of the (heads, D, D) matrices of a type that lane (col, lk) of a block holds
+// first, and whether its s-th row belongs to the column's head (D < 16: two heads a block).
+template <int D>
+__device__ __forceinline__ uint32_t first(int col, int lk) {
+  return (uint32_t)((D < 16 ? col & ~15 : col / D * D) + 4 * lk) * D + col % D;
+}
+template <int D>
+__device__ __forceinline__ bool in_block(int col, int lk, int s) {
+  return D >= 16 || ((col & ~15) + 4 * lk + s) / D == col / D;
+}
 
 // One 16 x 16 block of a product, k blocks of 16: the wavefront's weights and the
 // multiplication of 16 tile rows.  D < 16: the block diagonal of two heads.
@@ -62,15 +76,11 @@ struct Block<float, D> {
   static constexpr int KB = D < 16 ? 1 : D / 16;
   float w[KB][4];
   __device__ __forceinline__ void load(const float *W, int col, int lk) {   // W: (heads, D, D) of the type
-    const int head = col / D;
-    const int k0 = D < 16 ? col & ~15 : head * D;
+    const uint32_t at = first<D>(col, lk);
 #pragma unroll
     for (int b = 0; b < KB; ++b)
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int kk = k0 + 16 * b + 4 * lk + s;
-        w[b][s] = kk / D == head ? W[(int64_t)kk * D + col % D] : 0.0f;
-      }
+      for (int s = 0; s < 4; ++s) w[b][s] = in_block<D>(col, lk, s) ? W[at + (16 * b + s) * D] : 0.0f;
   }
   __device__ __forceinline__ floatx4 mma(const float *row, int k0, int lk) const {
     floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -91,16 +101,12 @@ struct Block<bf16_t, D> {
   static constexpr int KB = D < 16 ? 1 : D / 16;
   uint2 w[KB];
   __device__ __forceinline__ void load(const bf16_t *W, int col, int lk) {
-    const int head = col / D;
-    const int k0 = D < 16 ? col & ~15 : head * D;
+    const uint32_t at = first<D>(col, lk);
 #pragma unroll
     for (int b = 0; b < KB; ++b) {
       uint32_t e[4];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int kk = k0 + 16 * b + 4 * lk + s;
-        e[s] = kk / D == head ? W[(int64_t)kk * D + col % D] : 0u;
-      }
+      for (int s = 0; s < 4; ++s) e[s] = in_block<D>(col, lk, s) ? W[at + (16 * b + s) * D] : 0u;
       w[b] = make_uint2(e[0] | (e[1] << 16), e[2] | (e[3] << 16));
     }
   }
@@ -126,7 +132,7 @@ __device__ __forceinline__ float head_sum(float v) {     // over LANES adjacent 
 }
 
 template <typename T, int F, int D>
-__global__ __launch_bounds__(kBlock, 5) void pair_attn_kernel(PairArgs A) {
+__global__ __launch_bounds__(kBlock, F == 128 && sizeof(T) == 4 ? 4 : 5) void pair_attn_kernel(PairArgs A) {
   constexpr int VEC = 16 / (int)sizeof(T);
   constexpr int LPR = F / VEC;                    // lanes per row
   constexpr int G = kBlock / LPR;                 // lane groups
@@ -143,20 +149,23 @@ __global__ __launch_bounds__(kBlock, 5) void pair_attn_kernel(PairArgs A) {
   const T *const q = (const T *)A.q, *const k = (const T *)A.k, *const v = (const T *)A.v;
 
   int type, row0, row1;
-  if (!locate_chunk(A.type_pointer, A.n_types, A.chunk_rows, blockIdx.x, type, row0, row1)) return;
+  if (!locate_chunk(A.type_pointer, A.n_types, kPairRows, blockIdx.x, type, row0, row1)) return;
+
+  type = __builtin_amdgcn_readfirstlane(type);
+  row0 = __builtin_amdgcn_readfirstlane(row0);
+  row1 = __builtin_amdgcn_readfirstlane(row1);
 
   const int tid = threadIdx.x;
   const int lane64 = tid & (kWave - 1), wave = tid / kWave;
   const int lr = lane64 & 15, lk = lane64 >> 4;
   const int grp = tid / LPR, lane = tid % LPR, f0 = lane * VEC;
 
-  Block<T, D> wa[CB], wm[CB];
+  // the wavefront's columns of a relation matrix
+  auto columns = [&](const void *W, Block<T, D> (&w)[CB]) {
 #pragma unroll
-  for (int c = 0; c < CB; ++c) {
-    const int col = (wave * CB + c) * 16 + lr;
-    wa[c].load((const T *)A.att + (int64_t)type * F * D, col, lk);
-    wm[c].load((const T *)A.msg + (int64_t)type * F * D, col, lk);
-  }
+    for (int c = 0; c < CB; ++c)
+      w[c].load((const T *)W + (int64_t)type * F * D, (wave * CB + c) * 16 + lr, lk);
+  };
   // the tile's rows times the wavefront's columns, in place
   auto product = [&](const Block<T, D> (&w)[CB]) {
     floatx4 acc[CB][kPairRows / 16];
@@ -165,8 +174,11 @@ __global__ __launch_bounds__(kBlock, 5) void pair_attn_kernel(PairArgs A) {
       const int col0 = (wave * CB + c) * 16;
       const int k0 = D < 16 ? col0 : col0 / D * D;
 #pragma unroll
-      for (int b = 0; b < kPairRows / 16; ++b)
+      for (int b = 0; b < kPairRows / 16; ++b) {
         acc[c][b] = w[c].mma(tile + (16 * b + lr) * LD, k0, lk);
+        // heads of 64: the rows of all blocks at once would take 64 registers more
+        if constexpr (D == 64) __builtin_amdgcn_sched_barrier(0);
+      }
     }
     __syncthreads();                       // every wavefront has read all rows
 #pragma unroll
@@ -179,129 +191,128 @@ __global__ __launch_bounds__(kBlock, 5) void pair_attn_kernel(PairArgs A) {
     __syncthreads();
   };
 
-  for (int base = row0; base < row1; base += kPairRows) {
-    const int n = min(kPairRows, row1 - base);
-    if (tid < kPairRows) {
-      const int p = (int)A.by_type[base + min(tid, n - 1)];
-      pair_of[tid] = p;
-      slot0[tid] = A.pair_pointer[p];
-      slot1[tid] = A.pair_pointer[p + 1];
-    }
+  const int n = row1 - row0;             // at most kPairRows
+  if (tid < kPairRows) {
+    const int p = (int)A.by_type[row0 + min(tid, n - 1)];
+    pair_of[tid] = p;
+    slot0[tid] = A.pair_pointer[p];
+    slot1[tid] = A.pair_pointer[p + 1];
+  }
 #pragma unroll
-    for (int i = 0; i < RPG; ++i) {        // rows past the last one repeat it
-      const int r = grp + i * G;
-      const int64_t d = A.dst_by_type[base + min(r, n - 1)];
-      *reinterpret_cast<raw_t *>(tile + r * LD + f0) = IO::load(q + d * F + f0);
-    }
+  for (int i = 0; i < RPG; ++i) {        // rows past the last one repeat it
+    const int r = grp + i * G;
+    const int64_t d = A.dst_by_type[row0 + min(r, n - 1)];
+    *reinterpret_cast<raw_t *>(tile + r * LD + f0) = IO::load(q + d * F + f0);
+  }
+  {
+    Block<T, D> w[CB];
+    columns(A.att, w);
     __syncthreads();
-    product(wa);
+    product(w);
+  }
 
-    // ---- attention inside the pairs: rows grp * RPG .. of the tile, one after another ----
-    int r = grp * RPG;
-    const int r_end = min(r + RPG, n);
-    if (r < r_end) {
-      float qf[VEC], acc[VEC], m = -INFINITY, l = 0.0f;
-      auto open_row = [&]() {
-        IO::widen(*reinterpret_cast<const raw_t *>(tile + r * LD + f0), qf);
+  // ---- attention inside the pairs: every G-th row of the tile, one after another (large
+  // pairs lie side by side where the relation's popular destinations do) ----
+  int r = grp;
+  if (r < n) {
+    float qf[VEC], acc[VEC], m = -INFINITY, l = 0.0f;
+    auto open_row = [&]() {
+      IO::widen(*reinterpret_cast<const raw_t *>(tile + r * LD + f0), qf);
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) acc[e] = 0.0f;
-        m = -INFINITY;
-        l = 0.0f;
-      };
-      int pos = slot0[r], end = slot1[r];
-      int ids = A.nbr[pos + min(lane & 3, end - 1 - pos)];
-      open_row();
-      while (true) {
-        const int cnt = end - pos;         // at least one
-        int nr = r, npos = pos + kPairBatch, nend = end;
-        if (cnt <= kPairBatch) {
-          nr = r + 1;
-          if (nr < r_end) { npos = slot0[nr]; nend = slot1[nr]; }
-        }
-        // sources of the next batch, whichever row it belongs to
-        const int ids_next = nr < r_end ? A.nbr[npos + min(lane & 3, nend - 1 - npos)] : 0;
-        const int g[kPairBatch] = {
-            __builtin_amdgcn_update_dpp(0, ids, 0x00, 0xF, 0xF, true),      // quad_perm: lane t
-            __builtin_amdgcn_update_dpp(0, ids, 0x55, 0xF, 0xF, true),
-            __builtin_amdgcn_update_dpp(0, ids, 0xAA, 0xF, 0xF, true),
-            __builtin_amdgcn_update_dpp(0, ids, 0xFF, 0xF, 0xF, true)};
-        raw_t kx[kPairBatch], vx[kPairBatch];
-#pragma unroll
-        for (int t = 0; t < kPairBatch; ++t) {
-          kx[t] = vx[t] = raw_t{};
-          if (t < cnt) {
-            kx[t] = IO::load(k + (int64_t)g[t] * F + f0);
-            vx[t] = IO::load(v + (int64_t)g[t] * F + f0);
-          }
-        }
-        float s[kPairBatch], bm = -INFINITY;
-#pragma unroll
-        for (int t = 0; t < kPairBatch; ++t) {
-          float kf[VEC], d = 0.0f;
-          IO::widen(kx[t], kf);
-#pragma unroll
-          for (int e = 0; e < VEC; ++e) d = fmaf(kf[e], qf[e], d);
-          d = head_sum<HL>(d);
-          s[t] = t < cnt ? d : -INFINITY;
-          bm = fmaxf(bm, s[t]);
-        }
-        // exponentials from 0 while every score is -inf (see the fused GAT aggregation)
-        const float nm = fmaxf(m, bm);
-        const float ref = nm == -INFINITY ? 0.0f : nm;
-        const float sc = __expf(m - ref);
-        l *= sc;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) acc[e] *= sc;
-        m = nm;
-#pragma unroll
-        for (int t = 0; t < kPairBatch; ++t) {
-          if (t < cnt) {
-            const float p = __expf(s[t] - ref);
-            l += p;
-            float vf[VEC];
-            IO::widen(vx[t], vf);
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) acc[e] = fmaf(p, vf[e], acc[e]);
-          }
-        }
-        if (cnt <= kPairBatch) {           // the row is complete: over its own query row
-          const float inv = 1.0f / l;
-          float o[VEC];
-#pragma unroll
-          for (int e = 0; e < VEC; ++e) o[e] = acc[e] * inv;
-          IO::store(tile + r * LD + f0, o);
-          if (f0 % D == 0 || D < VEC) A.lse[(int64_t)pair_of[r] * H + f0 / D] = m + logf(l);
-          r = nr;
-          if (r >= r_end) break;
-          open_row();
-        }
-        pos = npos;
-        end = nend;
-        ids = ids_next;
+      for (int e = 0; e < VEC; ++e) acc[e] = 0.0f;
+      m = -INFINITY;
+      l = 0.0f;
+    };
+    int pos = slot0[r], end = slot1[r];
+    int ids = A.nbr[pos + min(lane & 3, end - 1 - pos)];
+    open_row();
+    while (true) {
+      const int cnt = end - pos;         // at least one
+      int nr = r, npos = pos + kPairBatch, nend = end;
+      if (cnt <= kPairBatch) {
+        nr = r + G;
+        if (nr < n) { npos = slot0[nr]; nend = slot1[nr]; }
       }
-    }
-    __syncthreads();
-    product(wm);
+      // sources of the next batch, whichever row it belongs to
+      const int ids_next = nr < n ? A.nbr[npos + min(lane & 3, nend - 1 - npos)] : 0;
+      const int g[kPairBatch] = {
+          __builtin_amdgcn_update_dpp(0, ids, 0x00, 0xF, 0xF, true),      // quad_perm: lane t
+          __builtin_amdgcn_update_dpp(0, ids, 0x55, 0xF, 0xF, true),
+          __builtin_amdgcn_update_dpp(0, ids, 0xAA, 0xF, 0xF, true),
+          __builtin_amdgcn_update_dpp(0, ids, 0xFF, 0xF, 0xF, true)};
+      raw_t kx[kPairBatch], vx[kPairBatch];
 #pragma unroll
-    for (int i = 0; i < RPG; ++i) {
-      const int row = grp + i * G;
-      if (row < n)
-        *reinterpret_cast<raw_t *>((T *)A.m + (int64_t)pair_of[row] * F + f0) =
-            *reinterpret_cast<const raw_t *>(tile + row * LD + f0);
+      for (int t = 0; t < kPairBatch; ++t) {
+        kx[t] = vx[t] = raw_t{};
+        if (t < cnt) {
+          kx[t] = IO::load(k + (int64_t)g[t] * F + f0);
+          vx[t] = IO::load(v + (int64_t)g[t] * F + f0);
+        }
+      }
+      float s[kPairBatch], bm = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < kPairBatch; ++t) {
+        float kf[VEC], d = 0.0f;
+        IO::widen(kx[t], kf);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) d = fmaf(kf[e], qf[e], d);
+        d = head_sum<HL>(d);
+        s[t] = t < cnt ? d : -INFINITY;
+        bm = fmaxf(bm, s[t]);
+      }
+      // exponentials from 0 while every score is -inf (see the fused GAT aggregation)
+      const float nm = fmaxf(m, bm);
+      const float ref = nm == -INFINITY ? 0.0f : nm;
+      const float sc = __expf(m - ref);
+      l *= sc;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) acc[e] *= sc;
+      m = nm;
+#pragma unroll
+      for (int t = 0; t < kPairBatch; ++t) {
+        if (t < cnt) {
+          const float p = __expf(s[t] - ref);
+          l += p;
+          float vf[VEC];
+          IO::widen(vx[t], vf);
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) acc[e] = fmaf(p, vf[e], acc[e]);
+        }
+      }
+      if (cnt <= kPairBatch) {           // the row is complete: over its own query row
+        const float inv = 1.0f / l;
+        float o[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) o[e] = acc[e] * inv;
+        IO::store(tile + r * LD + f0, o);
+        if (f0 % D == 0 || D < VEC) A.lse[(int64_t)pair_of[r] * H + f0 / D] = m + logf(l);
+        r = nr;
+        if (r >= n) break;
+        open_row();
+      }
+      pos = npos;
+      end = nend;
+      ids = ids_next;
     }
+  }
+  {
+    Block<T, D> w[CB];
+    columns(A.msg, w);
     __syncthreads();
+    product(w);
+  }
+#pragma unroll
+  for (int i = 0; i < RPG; ++i) {
+    const int row = grp + i * G;
+    if (row < n)
+      *reinterpret_cast<raw_t *>((T *)A.m + (int64_t)pair_of[row] * F + f0) =
+          *reinterpret_cast<const raw_t *>(tile + row * LD + f0);
   }
 }
 
 template <typename T, int F, int D>
 int launch_pairs(PairArgs &A, int64_t n_pairs, hipStream_t s) {
-  // four tiles share a load of the weights on large pair lists (30.5 k tiles of 64 fp32
-  // features: 606 us with two, 584 with four for the layer); on 4.2 k tiles a workgroup per
-  // tile fills the chip more evenly (239 -> 216 us for the layer)
-  const int64_t tiles = (n_pairs + kPairRows - 1) / kPairRows;
-  const int64_t steps = tiles >= 16384 ? 4 : 1;
-  A.chunk_rows = (int)steps * kPairRows;
-  const int64_t grid = (n_pairs + A.chunk_rows - 1) / A.chunk_rows + A.n_types;
+  const int64_t grid = (n_pairs + kPairRows - 1) / kPairRows + A.n_types;
   if (grid > 0x7fffffff) return GA_EUNSUPPORTED;
   hipLaunchKernelGGL((pair_attn_kernel<T, F, D>), dim3((unsigned)grid), dim3(kBlock), 0, s, A);
   return launch_status();
@@ -346,7 +357,7 @@ extern "C" int ga_pair_attention(const int32_t *type_pointer, int64_t n_types,
   if (!ga::aligned(q, 16) || !ga::aligned(k, 16) || !ga::aligned(v, 16) || !ga::aligned(m, 16))
     return GA_EUNSUPPORTED;
   ga::PairArgs A{type_pointer, by_type, dst_by_type, pair_pointer, nbr, q, k, v, att, msg, m, lse,
-                 (int)n_types, 0};
+                 (int)n_types};
   if (dtype == GA_F32)
     return ga::launch_pairs_dim<float>(A, n_pairs, heads * dim, dim, (hipStream_t)stream);
   return ga::launch_pairs_dim<ga::bf16_t>(A, n_pairs, heads * dim, dim, (hipStream_t)stream);

@@ -1,0 +1,28 @@
+"""Registers of the kernels that are held to a number of wavefronts: a build that spills
+them to memory is found here, without a GPU."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                    "graphiler_amd", "csrc")
+HIPCC = "/opt/rocm/bin/hipcc"
+
+
+@pytest.mark.skipif(not (os.path.exists(HIPCC) or shutil.which("hipcc")), reason="no hipcc")
+def test_pair_attention_builds_spill_nothing(tmp_path):
+    r = subprocess.run([HIPCC if os.path.exists(HIPCC) else "hipcc", "--offload-arch=gfx950", "-O3",
+                        "-std=c++17", "-fPIC", "-Xclang", "-target-feature", "-Xclang",
+                        "-packed-fp32-ops", "-Rpass-analysis=kernel-resource-usage", "-c",
+                        "pair_attn.hip", "-o", str(tmp_path / "pair_attn.o")],
+                       cwd=CSRC, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert "failed to meet occupancy" not in r.stderr
+    spills = [int(x) for x in re.findall(r"VGPRs Spill: (\d+)", r.stderr)]
+    waves = [int(x) for x in re.findall(r"Occupancy \[waves/SIMD\]: (\d+)", r.stderr)]
+    assert len(spills) == len(waves) == 16
+    assert not any(spills), spills
+    assert min(waves) >= 4, waves
