@@ -89,6 +89,7 @@ SIGNATURES = {
                                     _i64, _i64, _int, _vp, _sz, _vp]),
     "ga_pair_attention": (_int, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                  _i64, _i64, _i64, _i64, _int, _vp]),
+    "ga_pair_attention_preferred": (_int, [_i64, _i64, _i64, _i64, _i64, _int]),
     "ga_gat_static_scratch_needed": (_i64, [_i64, _i64, _i64, _int, _int]),
     "ga_gat_aggregate_static": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64,
                                        _i64, _i64, ctypes.c_float, _int, _vp]),

@@ -351,8 +351,8 @@ extern "C" int ga_pair_attention(const int32_t *type_pointer, int64_t n_types,
       !att || !msg || !m || !lse)
     return GA_EINVAL;
   if (!ga::aligned(lse, 4)) return GA_EALIGN;
-  // one lane group walks a pair: 256 slots are 64 dependent batches, some 50 us in which
-  // the rest of the grid runs; larger pairs would outlast it
+  // a lane group walks its rows alone (ga_pair_attention_preferred): 256 slots are 64
+  // dependent batches, some 50 us
   if (max_slots > 256) return GA_EUNSUPPORTED;
   if (!ga::aligned(q, 16) || !ga::aligned(k, 16) || !ga::aligned(v, 16) || !ga::aligned(m, 16))
     return GA_EUNSUPPORTED;
@@ -361,4 +361,35 @@ extern "C" int ga_pair_attention(const int32_t *type_pointer, int64_t n_types,
   if (dtype == GA_F32)
     return ga::launch_pairs_dim<float>(A, n_pairs, heads * dim, dim, (hipStream_t)stream);
   return ga::launch_pairs_dim<ga::bf16_t>(A, n_pairs, heads * dim, dim, (hipStream_t)stream);
+}
+
+// Where the pass beats the three launches, from what the host knows.  A lane group walks
+// rpg rows of a tile, four slots per dependent batch, and nobody helps it: the pass takes
+// the longer of its share of the traffic and that chain, and large pairs come on top --
+// taken as one and a half rows of the largest size on one group, between a lone large pair
+// and many side by side.  The three launches pay for the pairs' rows in memory and for
+// their own starts, but spread the slots evenly.  The figures (us; 0.72 per batch, 30 and
+// 33 per 100 k pairs and 1 M edges of 256-byte rows) are fitted to 500 to 1.95 M pairs of 1
+// to 256 slots; pair form against three launches, 1 x 64 fp32:
+//   500 pairs of 16 / 32 / 256      29 : 34,  40 : 34,  199 : 40 us    (7 tiles for 256 CUs)
+//   2,500 pairs of 16 / 32 / 100    30 : 36,  42 : 38,   91 : 48
+//   10,000 pairs of 32 / 64         41 : 48,  65 : 59
+//   40,000 pairs of 64 / 256       111 : 138, 359 : 378
+//   100,000 pairs of 3 on average, 0.3 % of 64 / 128 / 256   84 : 99, 115 : 99, 177 : 100
+//   1 M pairs of 3, 0.3 % of 128 / 256                      523 : 669, 656 : 696
+extern "C" int ga_pair_attention_preferred(int64_t n_pairs, int64_t n_edges, int64_t max_slots,
+                                           int64_t heads, int64_t dim, int dtype) {
+  if (n_pairs <= 0 || n_edges < n_pairs || heads <= 0 || dim <= 0 || max_slots > 256) return 0;
+  if (dtype != GA_F32 && dtype != GA_BF16) return 0;
+  if ((heads * dim != 64 && heads * dim != 128) || (dim != 8 && dim != 16 && dim != 32 && dim != 64))
+    return 0;
+  const double rpg = (double)(heads * dim * (dtype == GA_F32 ? 4 : 2)) / 64;    // rows per lane group
+  const double mean = (double)((n_edges / n_pairs + ga::kPairBatch - 1) / ga::kPairBatch);
+  const double most = (double)((max_slots + ga::kPairBatch - 1) / ga::kPairBatch);
+  const double p = 1e-3 * (double)n_pairs, e = 1e-3 * (double)n_edges, row = rpg / 4;
+  const double share = (0.30 * p + 0.033 * e) * row, chain = 0.72 * rpg * mean;
+  const double extra = most > mean ? 1.5 * 0.72 * (most - mean) : 0.0;
+  const double pass = 20.0 + (share > chain ? share : chain) + extra;
+  const double three = 36.0 + (0.43 * p + 0.033 * e) * row;
+  return pass < three;
 }

@@ -1144,9 +1144,10 @@ torch::Tensor dot_attention_sum(torch::Tensor k, torch::Tensor q, torch::Tensor 
 // relation, so with at least two edges per (destination, relation) pair they are applied
 // per pair instead of per edge:
 //   score = <k[src], q[dst] (s A)^T>,  out[v] = sum_pairs (sum_{e in pair} a_e v[src]) M
-// with one pass over the slots for scores, softmax inside the pair and weighted sum
-// (ga_dot_attention_sum), the pairs of a destination weighed by the softmax of their
-// log-sum-exps.  Graphs without such pairs and shapes outside those kernels run the
+// with both products, the scores, the softmax inside the pair and its weighted sum in one
+// pass (ga_pair_attention) or, where ga_pair_attention_preferred says no, in three launches
+// around ga_dot_attention_sum; the pairs of a destination are weighed by the softmax of
+// their log-sum-exps.  Graphs without such pairs and shapes outside those kernels run the
 // three per-edge operators.
 torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::Tensor v,
                                       torch::Tensor relation_att, torch::Tensor relation_msg,
@@ -1200,29 +1201,31 @@ torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::T
                                 y.data_ptr(), nullptr, nullptr, nullptr, nullptr, nullptr, P, heads,
                                 d, d, dt, stream);
   };
-  // products, scores, softmax inside every pair and weighted sum in one pass where its
-  // shape fits
-  torch::Tensor m_pair = torch::empty({P, hid}, k.options());
-  torch::Tensor lse = torch::empty({P, heads}, k.options().dtype(at::kFloat));
-  int rc = ga_pair_attention(pairs.type_pointer.data_ptr<int>(), graph->num_etypes,
-                             pairs.by_type.data_ptr<int64_t>(), pairs.dst_by_type.data_ptr<int64_t>(),
-                             pairs.pair_pointer.data_ptr<int>(),
-                             graph->in_node_indices.data_ptr<int>(), q.data_ptr(), k.data_ptr(),
-                             v.data_ptr(), att_t.data_ptr(), relation_msg.data_ptr(),
-                             m_pair.data_ptr(), lse.data_ptr<float>(), P, pairs.max_slots, heads, d,
-                             dt, stream);
-  if (rc != GA_EUNSUPPORTED) {
-    check_ga(rc, "ga_pair_attention");
-    torch::Tensor ws = graph->workspace(ga_gat_workspace_bytes(P, hid, heads));
-    torch::Tensor out = torch::empty({n, hid}, k.options());
-    check_ga(ga_edge_softmax_sum(pairs.dst_pointer.data_ptr<int>(), pairs.pair_dst.data_ptr<int>(),
-                                 nullptr, lse.data_ptr<float>(), m_pair.data_ptr(), out.data_ptr(),
-                                 n, P, heads, d, dt, ws.data_ptr(), (size_t)ws.numel(), stream),
-             "ga_edge_softmax_sum");
-    return out;
+  // products, scores, softmax inside every pair and weighted sum in one pass where that is
+  // the faster way
+  if (ga_pair_attention_preferred(P, e, pairs.max_slots, heads, d, dt)) {
+    torch::Tensor m_pair = torch::empty({P, hid}, k.options());
+    torch::Tensor lse = torch::empty({P, heads}, k.options().dtype(at::kFloat));
+    const int rc = ga_pair_attention(
+        pairs.type_pointer.data_ptr<int>(), graph->num_etypes, pairs.by_type.data_ptr<int64_t>(),
+        pairs.dst_by_type.data_ptr<int64_t>(), pairs.pair_pointer.data_ptr<int>(),
+        graph->in_node_indices.data_ptr<int>(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+        att_t.data_ptr(), relation_msg.data_ptr(), m_pair.data_ptr(), lse.data_ptr<float>(), P,
+        pairs.max_slots, heads, d, dt, stream);
+    if (rc != GA_EUNSUPPORTED) {
+      check_ga(rc, "ga_pair_attention");
+      torch::Tensor ws = graph->workspace(ga_gat_workspace_bytes(P, hid, heads));
+      torch::Tensor out = torch::empty({n, hid}, k.options());
+      check_ga(ga_edge_softmax_sum(pairs.dst_pointer.data_ptr<int>(), pairs.pair_dst.data_ptr<int>(),
+                                   nullptr, lse.data_ptr<float>(), m_pair.data_ptr(),
+                                   out.data_ptr(), n, P, heads, d, dt, ws.data_ptr(),
+                                   (size_t)ws.numel(), stream),
+               "ga_edge_softmax_sum");
+      return out;
+    }
   }
   torch::Tensor q_pair = torch::empty({P, hid}, k.options());
-  rc = typed_rows(q, pairs.dst_by_type, att_t, q_pair);
+  int rc = typed_rows(q, pairs.dst_by_type, att_t, q_pair);
   if (rc == GA_EUNSUPPORTED) return per_edge();
   check_ga(rc, "ga_segment_mm_gather");
   // both passes share the scratch; the bytes are not monotonic in the number of items
@@ -1231,6 +1234,7 @@ torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::T
       {ga_gat_workspace_bytes(e, hid, heads), ga_gat_workspace_bytes(P, hid, heads),
        ga_softmax_workspace_bytes(P, heads), ga_spmm_workspace_bytes(P, hid)}));
   torch::Tensor v_pair = torch::empty({P, hid}, k.options());
+  torch::Tensor lse = torch::empty({P, heads}, k.options().dtype(at::kFloat));
   rc = ga_dot_attention_sum(pairs.pair_pointer.data_ptr<int>(), pairs.pair_of_slot.data_ptr<int>(),
                             graph->in_node_indices.data_ptr<int>(),
                             pairs.rank_of_slot.data_ptr<int>(), k.data_ptr(), q_pair.data_ptr(),
@@ -1240,6 +1244,7 @@ torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::T
   if (rc == GA_EUNSUPPORTED) return per_edge();
   check_ga(rc, "ga_dot_attention_sum");
   // (the log-sum-exps were written in by_type order, the row order of m_pair)
+  torch::Tensor m_pair = torch::empty({P, hid}, k.options());
   check_ga(typed_rows(v_pair, pairs.by_type, relation_msg, m_pair), "ga_segment_mm_gather");
   torch::Tensor out = torch::empty({n, hid}, k.options());
   check_ga(ga_edge_softmax_sum(pairs.dst_pointer.data_ptr<int>(), pairs.pair_dst.data_ptr<int>(),

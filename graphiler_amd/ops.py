@@ -1024,28 +1024,29 @@ def relation_pair_attention(k, q, v, relation_att, relation_msg, relation_scale,
             stream), "ga_segment_mm_gather")
         return y
 
-    # products, scores, softmax inside every pair and weighted sum in one pass where its
-    # shape fits; the pairs of a destination are then weighed by the softmax of their
+    # products, scores, softmax inside every pair and weighted sum in one pass where that is
+    # the faster way; the pairs of a destination are then weighed by the softmax of their
     # log-sum-exps (the softmax-weighted sum of per-"edge" rows, with the pairs as the
     # edges), which makes the weights the softmax over all its in-edges
-    m_pair = torch.empty((P, hid), dtype=v.dtype, device=dev)            # pair order
-    lse = torch.empty((P, heads), dtype=torch.float32, device=dev)
-    rc = lib.ga_pair_attention(
-        pairs.type_pointer.data_ptr(), n_types, pairs.by_type.data_ptr(),
-        pairs.dst_by_type.data_ptr(), pairs.pair_pointer.data_ptr(),
-        graph.in_node_indices.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-        att_t.data_ptr(), relation_msg.data_ptr(), m_pair.data_ptr(), lse.data_ptr(), P,
-        pairs.max_slots, heads, d, dt, stream)
-    if rc != capi.GA_EUNSUPPORTED:
-        capi.check(rc, "ga_pair_attention")
-        ws = graph.workspace(lib.ga_gat_workspace_bytes(P, hid, heads))
-        out = torch.empty((n, hid), dtype=v.dtype, device=dev)
-        capi.check(lib.ga_edge_softmax_sum(
-            pairs.dst_pointer.data_ptr(), pairs.pair_dst.data_ptr(), None, lse.data_ptr(),
-            m_pair.data_ptr(), out.data_ptr(), n, P, heads, d, dt, ws.data_ptr(), ws.numel(),
-            stream), "ga_edge_softmax_sum")
-        return out
-    del m_pair, lse
+    if lib.ga_pair_attention_preferred(P, e, pairs.max_slots, heads, d, dt):
+        m_pair = torch.empty((P, hid), dtype=v.dtype, device=dev)            # pair order
+        lse = torch.empty((P, heads), dtype=torch.float32, device=dev)
+        rc = lib.ga_pair_attention(
+            pairs.type_pointer.data_ptr(), n_types, pairs.by_type.data_ptr(),
+            pairs.dst_by_type.data_ptr(), pairs.pair_pointer.data_ptr(),
+            graph.in_node_indices.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+            att_t.data_ptr(), relation_msg.data_ptr(), m_pair.data_ptr(), lse.data_ptr(), P,
+            pairs.max_slots, heads, d, dt, stream)
+        if rc != capi.GA_EUNSUPPORTED:
+            capi.check(rc, "ga_pair_attention")
+            ws = graph.workspace(lib.ga_gat_workspace_bytes(P, hid, heads))
+            out = torch.empty((n, hid), dtype=v.dtype, device=dev)
+            capi.check(lib.ga_edge_softmax_sum(
+                pairs.dst_pointer.data_ptr(), pairs.pair_dst.data_ptr(), None, lse.data_ptr(),
+                m_pair.data_ptr(), out.data_ptr(), n, P, heads, d, dt, ws.data_ptr(), ws.numel(),
+                stream), "ga_edge_softmax_sum")
+            return out
+        del m_pair, lse
     q_pair = typed_rows(q, pairs.dst_by_type, att_t)
     # both passes share the scratch; the bytes are not monotonic in the number of items
     # (longer runs from a threshold on), so the pairs are asked for as well

@@ -537,6 +537,12 @@ int ga_pair_attention(const int32_t *type_pointer, int64_t n_types, const int64_
                       int64_t max_slots, int64_t heads, int64_t dim, int dtype,
                       ga_stream_t stream);
 
+/* 1 where one pass of ga_pair_attention over these pairs is expected to be faster than the
+ * three launches it stands for, 0 otherwise and for shapes that it refuses (host arithmetic
+ * only).  It walks large pairs alone, so few pairs with many slots belong to the launches. */
+int ga_pair_attention_preferred(int64_t n_pairs, int64_t n_edges, int64_t max_slots,
+                                int64_t heads, int64_t dim, int dtype);
+
 /* The softmax-weighted reduction with per-edge operands:
  *   a = softmax_v(logit[e, h] over the in-edges e of v),
  *   out[v, h, :] = sum_e a_e * m[e, h, :]

@@ -277,3 +277,16 @@ def test_scaled_sum_and_projection_reject_bad_arguments_without_gpu():
     assert lin(one, one, one, None, 4, 8, 8, None) == capi.GA_EINVAL
     assert lin(one, one, odd, one, 4, 8, 8, None) == capi.GA_EALIGN
     assert lin(one, one, one, one, 4, 1 << 23, 8, None) == capi.GA_EUNSUPPORTED
+
+
+@pytest.mark.parametrize("n_pairs,n_edges,max_slots,want", [
+    (1_950_000, 4_681_010, 12, 1), (269_078, 2_000_000, 60, 1), (1_000, 1_000, 1, 1),
+    (10_000, 320_000, 32, 1), (40_000, 2_560_000, 64, 1), (1_000_000, 3_002_187, 256, 1),
+    # few pairs with many slots, large pairs on short lists
+    (500, 128_000, 256, 0), (2_500, 250_000, 100, 0), (10_000, 640_000, 64, 0),
+    (100_000, 302_475, 256, 0), (1_000_000, 3_000_000, 257, 0), (0, 0, 0, 0)])
+def test_pair_attention_rule(n_pairs, n_edges, max_slots, want):
+    lib = capi.load()
+    for heads, d, dt in ((1, 64, capi.GA_F32), (8, 16, capi.GA_BF16)):
+        assert lib.ga_pair_attention_preferred(n_pairs, n_edges, max_slots, heads, d, dt) == want
+    assert lib.ga_pair_attention_preferred(n_pairs, n_edges, max_slots, 4, 64, capi.GA_F32) == 0
