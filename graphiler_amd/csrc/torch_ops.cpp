@@ -242,7 +242,7 @@ struct DGLGraph : torch::CustomClassHolder {
           rank.index_copy_(0, by_type, torch::arange(P, i64));
           pairs_.num_pairs = P;
           torch::Tensor bounds = torch::cat({starts, torch::full({1}, num_edges, i64)});
-          pairs_.max_slots = torch::diff(bounds).max().item<int64_t>();
+          torch::Tensor largest = torch::diff(bounds).max();
           pairs_.pair_pointer = bounds.to(at::kInt).contiguous();
           pairs_.pair_of_slot = pair_of_slot.to(at::kInt).contiguous();
           pairs_.pair_dst = pair_dst.to(at::kInt).contiguous();
@@ -257,6 +257,7 @@ struct DGLGraph : torch::CustomClassHolder {
           pairs_.dst_by_type = pair_dst.index_select(0, by_type).contiguous();
           pairs_.rank = rank.to(at::kInt).contiguous();
           pairs_.rank_of_slot = rank.index_select(0, pair_of_slot).to(at::kInt).contiguous();
+          pairs_.max_slots = largest.item<int64_t>();     // behind all launches: the host waits once
           pairs_.valid = true;
         }
       }

@@ -272,12 +272,12 @@ def _build_relation_pairs(g: "DGLGraph") -> Optional[RelationPairs]:
     pair_dst = torch.div(pair_key, n_types, rounding_mode="floor")
     pair_type = pair_key - pair_dst * n_types
     by_type = torch.argsort(pair_type, stable=True)
-    rank = torch.empty_like(by_type)
-    rank[by_type] = torch.arange(n_pairs, device=dev)
-    bounds = torch.cat([starts, starts.new_tensor([n_edges])])
-    return RelationPairs(
+    rank = torch.empty_like(by_type).scatter_(0, by_type, torch.arange(n_pairs, device=dev))
+    bounds = torch.cat([starts, starts.new_full((1,), n_edges)])
+    largest = torch.diff(bounds).max()
+    pairs = RelationPairs(
         num_pairs=n_pairs,
-        max_slots=int(torch.diff(bounds).max().item()),
+        max_slots=0,
         pair_pointer=bounds.int().contiguous(),
         pair_of_slot=pair_of_slot.int().contiguous(),
         pair_dst=pair_dst.int().contiguous(),
@@ -289,6 +289,8 @@ def _build_relation_pairs(g: "DGLGraph") -> Optional[RelationPairs]:
         rank=rank.int().contiguous(),
         rank_of_slot=rank[pair_of_slot].int().contiguous(),
         dst_by_type=pair_dst[by_type].contiguous())
+    pairs.max_slots = int(largest.item())      # read behind all launches: the host waits once
+    return pairs
 
 
 def group_on_device(key: torch.Tensor, other: Optional[torch.Tensor], n_keys: int):
