@@ -3,7 +3,7 @@
 forwards at the benchmark configurations, with per-kernel roofline figures.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--configs c5,c2,c3,c4,c1]
-                    [--only KEY[,KEY]] [--no-cpu-baseline] [--markers]
+                    [--only KEY[,KEY]] [--details FILE] [--no-cpu-baseline] [--markers]
 
 Headline (the JSON line's metric / value / roofline / cpu_baseline): the first
 configuration named in --configs, by default c5 = configs[4], the largest one
@@ -18,9 +18,10 @@ The other configurations (c2 = configs[1] 1-head fp32 GAT, c3 = configs[2] RGCN
 fp32 and bf16, c4 = configs[3] HGT bf16, c1 = configs[0] the 2-layer GCN that the
 configuration list assigns to the host cores, timed there and on the GPU) are measured
 in the same run and reported as objects under "configs" of the same line: layer time, edges/s and, per operator,
-launch time (HIP events on the launch stream), algorithmic bytes, effective GB/s,
-fraction of the 8 TB/s HBM peak and, for the matrix kernels, TFLOP/s against the
-MFMA peak and against min(MFMA peak, intensity x HBM peak).
+[launch time in ms (HIP events on the launch stream), fraction of the 8 TB/s HBM peak].
+--details FILE writes the full records: algorithmic bytes, effective GB/s, counted traffic
+and, for the matrix kernels, TFLOP/s against the MFMA peak and against min(MFMA peak,
+intensity x HBM peak).
 
 Algorithmic bytes credit one gathered row per edge and no cache reuse.  An operator
 whose gathered table fits the 256 MB Infinity Cache, or whose algorithmic bytes flow
@@ -35,7 +36,7 @@ operator writes cannot be that operator's and is refused.
 dispatches between two such passes are exactly one operator's calls (the line's
 "profile_segments" lists key and number of calls in order), and the passes themselves
 calibrate the counters.
-Prints ONE JSON line.
+Prints ONE JSON line, short enough for a reader that keeps the last few kilobytes.
 """
 import argparse
 import json
@@ -65,6 +66,18 @@ def load_traffic():
     return table
 
 
+def brief(rec):
+    """A configuration's record as it stands in the JSON line: times and rates, and
+    [ms, fraction of the HBM peak] per operator."""
+    out = {k: rec[k] for k in ("dtype", "num_pairs", "ms_per_step", "edges_per_s",
+                               "host_ms_over_gpu_ms") if rec.get(k) is not None}
+    if "variants" in rec:
+        out["variants"] = {k: brief(v) for k, v in rec["variants"].items()}
+    if rec.get("ops"):
+        out["ops"] = {k: [v["ms"], v["frac"]] for k, v in rec["ops"].items()}
+    return out
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -76,9 +89,10 @@ def main():
                     help="comma-separated operator keys (c4.hgt_layer, c2.segment_softmax, ...): time "
                          "only these, skip the network steps and the CPU legs (short profiler runs)")
     ap.add_argument("--reps", type=int, default=30, help="timed calls per operator")
+    ap.add_argument("--details", metavar="FILE", help="write the full records of all configurations there")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--gather-ceiling", "--reference-points", dest="gather_ceiling", action="store_true",
-                    help="configs[4]: also run its aggregation kernels on graphs with the same "
+                    help="(results in --details) configs[4]: also run its aggregation kernels on graphs with the same "
                          "destinations and uniformly random sources over tables of several sizes (HBM, "
                          "Infinity Cache, L2): what the memory system gives a gather of 512-byte rows; "
                          "configs[1] and [4]: u_add_v next to plain gathers of the same rows (torch's "
@@ -807,9 +821,12 @@ def main():
         "roofline": roofline,
         "cpu_baseline": cpu,
         "peak_measured_copy_GBps": measured_copy,
-        "configs": results,
+        "configs": {c: brief(r) for c, r in results.items()},
     }
     line.update(extra)
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(dict(line, configs=results), f, indent=1)
     print(json.dumps(line))
 
 

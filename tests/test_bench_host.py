@@ -51,3 +51,22 @@ def test_traffic_table_has_a_count_for_every_benchmarked_operator():
     assert table["c4.segment_mm_gather"] >= 2_000_000 * 256
     assert table["c4.hgt_layer"] >= 100_000 * 256
     assert table["c5.gat_aggregate_from_z"] >= 2_449_029 * 512
+
+
+def test_a_configuration_in_the_line_is_short():
+    """The line has to stay within the few kilobytes of output that are kept of a run: twice
+    the operators of today's five configurations, in full width, next to 2 KB of the rest."""
+    import json
+
+    import bench
+    op = {"ms": 1234.5678, "algorithmic_bytes": 10 ** 11, "written_bytes": 10 ** 11, "frac": 0.1234,
+          "effective_GBps": 12345.6, "frac_basis": "min(counted traffic, algorithmic bytes)"}
+    rec = {"workload": "x" * 200, "dtype": "bf16", "ms_per_step": 1234.5678, "edges_per_s": 9281522882.6,
+           "ops": {"segment_mm_node_qkv_128_%d" % i: dict(op) for i in range(10)}, "roofline": dict(op)}
+    typed = {"workload": "x" * 200, "variants": {"f32": dict(rec), "bf16": dict(rec)}}
+    got = bench.brief(rec)
+    assert got["ops"]["segment_mm_node_qkv_128_0"] == [1234.5678, 0.1234]
+    assert "roofline" not in got and "workload" not in got
+    assert bench.brief(typed)["variants"]["bf16"] == got
+    line = json.dumps({c: bench.brief(typed if c == "c3" else rec) for c in ("c1", "c2", "c3", "c4", "c5")})
+    assert len(line) < 5000
