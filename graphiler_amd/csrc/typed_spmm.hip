@@ -29,7 +29,8 @@
 //     touches.  The messages enter as bf16: rounded to nearest for bf16 tensors (the
 //     values the two-operator chain stores), as three truncated terms of 8 bits each for
 //     fp32 (their sum is the fp32 message to 2^-24; products with 0 / 1 are exact and the
-//     accumulation is fp32), two of them to a product.  No LDS, no atomics: a run gives the same bits every time.
+//     accumulation is fp32), two of them to a product.  No LDS, no atomics: a run gives the
+//     same bits every time.
 //     Messages that are not finite would turn the zeros of S_b into NaN for their
 //     neighbours: they are replaced by zero and remembered as one bit per element and
 //     kind (+inf, -inf, NaN), which the final write adds back in.
