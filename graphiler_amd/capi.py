@@ -16,6 +16,7 @@ LIB_PATH = os.path.join(_HERE, "lib", "libgraphiler_hip.so")
 GA_OK = 0
 GA_EINVAL, GA_EUNSUPPORTED, GA_EWORKSPACE, GA_EALIGN, GA_ESCRATCH = -1, -2, -3, -4, -5
 GA_STATIC_SCRATCH_BYTES = 32 << 20
+GA_DEGREE_BUCKETS = 31
 GA_ACT_NONE, GA_ACT_RELU, GA_ACT_ELU = 0, 1, 2
 GA_F32, GA_BF16 = 0, 1
 GA_COPY_U, GA_COPY_E, GA_U_MUL_E, GA_U_ADD_E, GA_U_SUB_E, GA_U_DIV_E = 0, 1, 2, 3, 4, 5
@@ -39,6 +40,12 @@ SIGNATURES = {
     "ga_spmm_scaled_workspace_bytes": (_sz, [_i64, _i64]),
     "ga_spmm_csr_scaled": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64,
                                   _int, _int, _vp, _sz, _vp]),
+    "ga_spmm_source_classes": (_i64, [_vp, _vp, _i64, _i64, _i64, _int]),
+    "ga_source_classes_workspace_bytes": (_sz, [_i64, _i64]),
+    "ga_source_classes_build": (_int, [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "ga_spmm_classes_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),
+    "ga_spmm_classes": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _int,
+                               _vp, _sz, _vp]),
     "ga_spmm_arg_workspace_bytes": (_sz, [_i64, _i64]),
     "ga_spmm_csr_arg": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64,
                                _i64, _i64, _int, _int, _int, _vp, _sz, _vp]),

@@ -64,6 +64,102 @@ __global__ __launch_bounds__(kBlock) void fill_zero_kernel(int32_t *p, int64_t n
   if (i < n) p[i] = 0;
 }
 
+// ---- slots ordered by classes of their sources ---------------------------------
+// A stable partition of the in-adjacency's slots into up to kMaxClasses classes of source
+// nodes: every wavefront counts the classes of kPartSlots consecutive slots (ballots),
+// one workgroup turns the counts into positions, every wavefront writes its slots.  A
+// class is made of blocks of kClassRows node ids, so that the rows of a class spread over
+// all memory channels (with src % classes every class of 256-byte rows lies in two of
+// sixteen), and the blocks are dealt by a multiplicative hash, so that popular ids, which
+// graph generators and loaders put side by side, meet all classes.
+constexpr int kMaxClasses = 8;
+constexpr int kPartSlots = 4096;
+constexpr int kClassRowsShift = 6;
+__device__ __forceinline__ int source_class(int32_t src, int class_shift) {
+  return (int)((((uint32_t)src >> kClassRowsShift) * 0x9E3779B1u) >> (32 - class_shift));
+}
+
+__global__ __launch_bounds__(kBlock) void class_count_kernel(
+    const int32_t *__restrict__ nbr, int64_t n_edges, int class_shift, int64_t n_units,
+    int32_t *__restrict__ counts) {
+  const int64_t unit = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
+  if (unit >= n_units) return;
+  const int lane = threadIdx.x & (kWave - 1);
+  int n[kMaxClasses] = {};
+  for (int i = 0; i < kPartSlots; i += kWave) {
+    const int64_t j = unit * kPartSlots + i + lane;
+    const int c = j < n_edges ? source_class(nbr[j], class_shift) : -1;
+#pragma unroll
+    for (int k = 0; k < kMaxClasses; ++k) n[k] += __popcll(__ballot(c == k));
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int k = 0; k < kMaxClasses; ++k)
+      if (k >> class_shift == 0) counts[k * n_units + unit] = n[k];
+  }
+}
+
+// counts <- their exclusive prefix sums, in place, by one workgroup
+__global__ __launch_bounds__(1024) void class_scan_kernel(int32_t *__restrict__ counts, int64_t n) {
+  __shared__ int32_t wave_sum[1024 / kWave];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  int32_t before = 0;                    // all items of earlier rounds
+  for (int64_t base = 0; base < n; base += 1024) {
+    const int64_t i = base + threadIdx.x;
+    const int32_t v = i < n ? counts[i] : 0;
+    int32_t incl = v;
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int32_t o = __shfl_up(incl, off);
+      if (lane >= off) incl += o;
+    }
+    if (lane == kWave - 1) wave_sum[wave] = incl;
+    __syncthreads();
+    int32_t in_front = before, all = 0;
+    for (int w = 0; w < 1024 / kWave; ++w) {
+      if (w < wave) in_front += wave_sum[w];
+      all += wave_sum[w];
+    }
+    if (i < n) counts[i] = in_front + incl - v;
+    before += all;
+    __syncthreads();
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void class_scatter_kernel(
+    const int32_t *__restrict__ row_of_slot, const int32_t *__restrict__ nbr, int64_t n_rows,
+    int64_t n_edges, int class_shift, int64_t n_units, const int32_t *__restrict__ first,
+    int32_t *__restrict__ rows_out, int32_t *__restrict__ nbr_out) {
+  const int64_t unit = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
+  if (unit >= n_units) return;
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint64_t below = ((uint64_t)1 << lane) - 1;
+  int32_t pos[kMaxClasses];
+#pragma unroll
+  for (int k = 0; k < kMaxClasses; ++k)
+    pos[k] = k >> class_shift == 0 ? first[k * n_units + unit] : 0;
+  for (int i = 0; i < kPartSlots; i += kWave) {
+    const int64_t j = unit * kPartSlots + i + lane;
+    int32_t src = 0, row = 0;
+    int c = -1;
+    if (j < n_edges) {
+      src = nbr[j];
+      row = row_of_slot[j];
+      c = source_class(src, class_shift);
+    }
+    int32_t p = 0;
+#pragma unroll
+    for (int k = 0; k < kMaxClasses; ++k) {
+      const uint64_t m = __ballot(c == k);
+      if (c == k) p = pos[k] + __popcll(m & below);
+      pos[k] += __popcll(m);
+    }
+    if (c >= 0) {
+      rows_out[p] = (int32_t)(c * n_rows + row);
+      nbr_out[p] = src;
+    }
+  }
+}
+
 inline size_t round_up(size_t v) { return (v + 255) & ~(size_t)255; }
 
 struct PrepLayout {
@@ -150,6 +246,40 @@ int ga_group_edges(const int64_t *key, const int64_t *other, int64_t n_keys,
     hipLaunchKernelGGL(gather_other_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, other,
                        eid, n_items, nbr);
   }
+  return launch_status();
+}
+
+size_t ga_source_classes_workspace_bytes(int64_t n_edges, int64_t n_classes) {
+  if (n_edges < 0 || n_edges > 0x7fffffff || n_classes < 2 || n_classes > ga::kMaxClasses) return 0;
+  const size_t units = (size_t)((n_edges + ga::kPartSlots - 1) / ga::kPartSlots);
+  return ga::round_up(units * (size_t)n_classes * 4 + 4);
+}
+
+int ga_source_classes_build(const int32_t *row_of_slot, const int32_t *nbr, int64_t n_rows,
+                            int64_t n_edges, int64_t n_classes, int32_t *pointer, int32_t *rows,
+                            int32_t *nbr_out, void *workspace, size_t workspace_bytes,
+                            ga_stream_t stream) {
+  using namespace ga;
+  if (n_rows <= 0 || n_edges <= 0 || n_edges > 0x7fffffff) return GA_EINVAL;
+  if (n_classes != 2 && n_classes != 4 && n_classes != 8) return GA_EINVAL;
+  if (n_rows * n_classes > 0x7ffffffe) return GA_EUNSUPPORTED;
+  if (!row_of_slot || !nbr || !pointer || !rows || !nbr_out) return GA_EINVAL;
+  if (!workspace || workspace_bytes < ga_source_classes_workspace_bytes(n_edges, n_classes) ||
+      !aligned(workspace, 4))
+    return GA_EWORKSPACE;
+  hipStream_t s = (hipStream_t)stream;
+  const int shift = ilog2_floor((uint64_t)n_classes);
+  const int64_t units = (n_edges + kPartSlots - 1) / kPartSlots;
+  const unsigned blocks = (unsigned)((units + kBlock / kWave - 1) / (kBlock / kWave));
+  int32_t *counts = (int32_t *)workspace;
+  hipLaunchKernelGGL(class_count_kernel, dim3(blocks), dim3(kBlock), 0, s, nbr, n_edges, shift,
+                     units, counts);
+  hipLaunchKernelGGL(class_scan_kernel, dim3(1), dim3(1024), 0, s, counts, units * n_classes);
+  hipLaunchKernelGGL(class_scatter_kernel, dim3(blocks), dim3(kBlock), 0, s, row_of_slot, nbr,
+                     n_rows, n_edges, shift, units, counts, rows, nbr_out);
+  const int64_t n_keys = n_rows * n_classes;
+  hipLaunchKernelGGL(pointer_kernel, dim3((unsigned)((n_keys + 1 + kBlock - 1) / kBlock)),
+                     dim3(kBlock), 0, s, rows, n_keys, n_edges, pointer);
   return launch_status();
 }
 

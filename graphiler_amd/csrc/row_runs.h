@@ -224,6 +224,25 @@ __device__ __forceinline__ void fold_chain(float (&acc)[Policy::kState], const f
   for (; w < w1; ++w, src += stride) Policy::merge(acc, src);
 }
 
+// Workgroups are handed to the eight XCDs in turn.  A policy whose slots are ordered by
+// what they gather (RunOrder specialised) has XCD x walk the x-th eighth of them, so that
+// an L2 holds the rows of its own eighth; everything indexed by workgroup below is in
+// slot order.
+template <class Policy>
+struct RunOrder {
+  static constexpr bool kByXcd = false;
+};
+constexpr int kXcdShift = 3;
+template <class Policy>
+__device__ __forceinline__ int64_t slot_block(int64_t n_wg) {
+  const int64_t b = blockIdx.x;
+  if constexpr (RunOrder<Policy>::kByXcd) {
+    const int64_t per = n_wg >> kXcdShift;
+    if (b < per << kXcdShift) return (b & ((1 << kXcdShift) - 1)) * per + (b >> kXcdShift);
+  }
+  return b;
+}
+
 template <class Policy>
 __global__ __launch_bounds__(kBlock) void runs_kernel(
     typename Policy::Args args, const int32_t *__restrict__ pointer,
@@ -249,7 +268,8 @@ __global__ __launch_bounds__(kBlock) void runs_kernel(
   const int G = kBlock >> geo.tpr_shift;
   const int grp = threadIdx.x >> geo.tpr_shift;
   const int lane = threadIdx.x & (tpr - 1);
-  const int64_t k = (int64_t)blockIdx.x * G + grp;
+  const int64_t block = slot_block<Policy>(geo.n_wg);
+  const int64_t k = block * G + grp;
   const int flane = (int)blockIdx.y * tpr + lane;   // feature lane index
   const int f0 = lane_first_feature<Policy>((int)blockIdx.y, lane, geo.tpr_shift);
   // lanes past the row's features take part in the walk where the group's lanes read the
@@ -356,8 +376,8 @@ __global__ __launch_bounds__(kBlock) void runs_kernel(
     fold_chain<Policy>(acc, state_of(j + 1, 0), (int64_t)2 * tpr * SF, j + 1, i + 1);
     return starts_inside;
   };
-  float *const gp = partial + (int64_t)blockIdx.x * 2 * geo.lanes_total * SF;
-  const int64_t runs_left = geo.n_runs - (int64_t)blockIdx.x * G;
+  float *const gp = partial + block * 2 * geo.lanes_total * SF;
+  const int64_t runs_left = geo.n_runs - block * G;
   const int last = (int)(runs_left < G ? runs_left : G) - 1;
 
   if (has_a && !a_open) {            // a row ends in my run

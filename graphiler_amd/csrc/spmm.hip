@@ -2,6 +2,8 @@
 // on the run-based row-reduction schedule of row_runs.h.
 #include "row_runs.h"
 
+#include <cmath>
+
 namespace ga {
 
 int run_shift_for(int64_t n_edges, int64_t feat) {
@@ -769,6 +771,84 @@ int launch_spmm_arg(int reduce, int bop, const int32_t *pointer,
 #undef GA_SPMM_ARG
 }
 
+// ---- sums over slots ordered by classes of their sources -----------------------
+// A sum whose table exceeds an L2 waits for the rows that miss it: all eight L2s hold the
+// same popular rows.  With the slots ordered by (source class, destination) -- see
+// ga_source_classes_build -- XCD x walks the x-th eighth of them (RunOrder), its L2 serves
+// an eighth of the table, and a destination has a partial sum per class, added in class
+// order by class_sum_kernel, which applies the tail.  What it costs is those partial rows,
+// written and read once; ga_spmm_source_classes says where that is the smaller part.
+// us, plain -> classes: 114.6 M R-MAT edges, 233 k nodes, 64 fp32 features 2006 -> 1643
+// (4 classes), 128 features 4282 -> 3133; uniform graphs: 100 k nodes and 20 M edges, 64
+// fp32 646 -> 370 (8 classes), 64 bf16 320 -> 235, 5 M edges, 32 fp32 87 -> 68.
+template <typename T, int VEC, int GL>
+struct ClassSumPolicy : SpmmPolicy<T, VEC, GA_SUM, 0, false, false, GA_ACT_NONE, GL> {
+  typedef SpmmPolicy<T, VEC, GA_SUM, 0, false, false, GA_ACT_NONE, GL> Base;
+  typedef typename Base::Args Args;
+  typedef float out_t;                 // partial sums stay fp32 whatever the rows are
+  static __device__ __forceinline__ void emit(const Args &, float *out, int64_t row, int feat,
+                                              int f0, const float (&st)[Base::kState]) {
+#pragma unroll
+    for (int v = 0; v < VEC; v += 4)
+      *reinterpret_cast<float4 *>(out + row * feat + f0 + v) =
+          make_float4(st[v], st[v + 1], st[v + 2], st[v + 3]);
+  }
+  static __device__ __forceinline__ void emit_empty(const Args &A, float *out, int64_t row,
+                                                    int feat, int f0) {
+    float st[Base::kState];
+    Base::init(st);
+    emit(A, out, row, feat, f0, st);
+  }
+};
+
+}  // namespace
+template <typename T, int VEC, int GL>
+struct RunOrder<ClassSumPolicy<T, VEC, GL>> {
+  static constexpr bool kByXcd = true;
+};
+namespace {
+
+// out[v] = act(row_scale[v] * (partial[0][v] + partial[1][v] + ...)), four features a thread
+template <typename T, int CLASSES>
+__global__ __launch_bounds__(kBlock) void class_sum_kernel(
+    const float4 *__restrict__ partial, const float *__restrict__ row_scale, int activation,
+    int64_t n_quads, int quads_per_row, T *__restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n_quads) return;
+  float4 x[CLASSES];
+#pragma unroll
+  for (int c = 0; c < CLASSES; ++c) x[c] = partial[c * n_quads + i];
+  float o[4] = {x[0].x, x[0].y, x[0].z, x[0].w};
+#pragma unroll
+  for (int c = 1; c < CLASSES; ++c) {
+    o[0] += x[c].x; o[1] += x[c].y; o[2] += x[c].z; o[3] += x[c].w;
+  }
+  if (row_scale) {
+    const float f = row_scale[i / quads_per_row];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) o[v] *= f;
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    if (activation == GA_ACT_RELU) o[v] = relu_keep_nan(o[v]);
+    if (activation == GA_ACT_ELU) o[v] = elu(o[v]);
+  }
+  if constexpr (sizeof(T) == 4)
+    reinterpret_cast<float4 *>(out)[i] = make_float4(o[0], o[1], o[2], o[3]);
+  else
+    reinterpret_cast<uint2 *>(out)[i] = make_uint2(pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3]));
+}
+
+template <typename T, int VEC, int GL>
+int launch_class_sums(const int32_t *pointer, const int32_t *rows, const int32_t *nbr,
+                      const void *u, float *partial, int64_t n_rows, int64_t n_edges, int feat,
+                      float *runs, size_t runs_bytes, hipStream_t s) {
+  typedef ClassSumPolicy<T, VEC, GL> P;
+  const bool ids_vec = aligned(rows, 16) && aligned(nbr, 16);
+  typename P::Args args{nbr, nullptr, (const T *)u, nullptr, 1, feat, ids_vec, 0, nullptr};
+  return launch_runs<P>(args, pointer, rows, partial, n_rows, n_edges, feat, runs, s, runs_bytes);
+}
+
 template <typename T, int VEC, int RED, bool SPREAD>
 int pick_w(int bop, const int32_t *pointer, const int32_t *row_of_slot,
            const int32_t *gidx, const int32_t *eid, const void *u,
@@ -807,6 +887,37 @@ int pick_red(int reduce, int bop, const int32_t *pointer,
                                     out, n_rows, n_edges, feat, heads, partial,
                                     stream);
   }
+}
+
+// Share of the gathers that hit a cache of `rows` rows with least-recently-used
+// replacement, when a node of out-degree d is gathered d times in no particular order:
+// a row is found if it was used within the time t in which `rows` different ones are
+// (Che, Tung and Wang, "Hierarchical Web caching systems", 2002):
+// sum_i (1 - exp(-d_i t)) = rows.  Degrees by powers of two: bucket b holds `nodes[b]`
+// nodes of degree 2^b .. 2^(b+1) - 1 with `edges[b]` edges together.
+constexpr double kL2Bytes = 4 << 20;       // of one XCD
+double cached_share(const int64_t *nodes, const int64_t *edges, double rows) {
+  double all_nodes = 0, all_edges = 0;
+  for (int b = 0; b < GA_DEGREE_BUCKETS; ++b) {
+    all_nodes += (double)nodes[b];
+    all_edges += (double)edges[b];
+  }
+  if (rows >= all_nodes || all_edges <= 0) return 1.0;
+  double lo = 1e-12, hi = 64, share = 0;
+  for (int i = 0; i < 60; ++i) {
+    const double t = sqrt(lo * hi);
+    double used = 0;
+    share = 0;
+    for (int b = 0; b < GA_DEGREE_BUCKETS; ++b) {
+      if (nodes[b] <= 0) continue;
+      const double p = 1.0 - exp(-(double)edges[b] / (double)nodes[b] * t);
+      used += (double)nodes[b] * p;
+      share += (double)edges[b] * p;
+    }
+    if (used > rows) hi = t;
+    else lo = t;
+  }
+  return share / all_edges;
 }
 
 __global__ __launch_bounds__(kBlock) void row_ids_kernel(
@@ -1008,6 +1119,105 @@ int ga_spmm_csr_scaled(const int32_t *pointer, const int32_t *row_of_slot,
   GA_SPMM_EPI(ga::bf16_t, 1, false);
 #undef GA_SPMM_EPI
 #undef GA_SPMM_EPI_ACT
+}
+
+// Time of the gathers from the share that an L2 serves, plus the partial rows, fitted to
+// 64 combinations of graph (R-MAT and uniform, 25 to 490 edges per node, 30 k to 233 k
+// nodes), width and type, with 1, 2, 4 and 8 classes each (us per GB of rows: 45 where all
+// hit, 135 where none does, bf16 rows 62 and 134; 450 per GB of partial rows for the
+// write and the read).  Six per cent are asked for: R-MAT, 100 k nodes, 200 edges per node,
+// 64 fp32 features, where four of five gathers hit anyway, 272 : 282 us, and 233 k nodes
+// with 50 edges per node 220 : 230, both left to the plain sum; uniform, 100 k nodes with
+// 25 edges per node, 64 features 94 : 98 (plain), with 50 173 : 146 (classes).
+int64_t ga_spmm_source_classes(const int64_t *nodes_of_degree, const int64_t *edges_of_degree,
+                               int64_t n_rows, int64_t n_edges, int64_t feat, int dtype) {
+  if (n_rows <= 0 || n_edges <= 0 || feat < 8 || (dtype != GA_F32 && dtype != GA_BF16)) return 0;
+  const bool half = dtype == GA_BF16;
+  const double row = (double)feat * (half ? 2 : 4);
+  if (feat % (half ? 8 : 4) || n_rows > 0x7ffffffe / 8 || n_edges < 16 * n_rows ||
+      (double)n_rows * row <= ga::kL2Bytes)
+    return 0;
+  if (!nodes_of_degree || !edges_of_degree) return 1;      // worth counting the degrees
+  const double gb = 1e-9 * (double)n_edges * (row < 128 ? 128 : row);
+  auto gathers = [&](int64_t classes) {                    // us
+    const double miss = 1.0 - ga::cached_share(nodes_of_degree, edges_of_degree,
+                                               (double)classes * ga::kL2Bytes / row);
+    return gb * (half ? 62.0 + 72.0 * pow(miss, 1.4) : 45.0 + 90.0 * pow(miss, 1.4));
+  };
+  const double plain = gathers(1);
+  double best = plain / 1.06;
+  int64_t classes = 0;
+  for (int64_t k = 2; k <= 8; k *= 2) {
+    const double t = gathers(k) + 450e-9 * (double)(k * n_rows) * (double)feat * 4 + 4.0;
+    if (t < best) {
+      best = t;
+      classes = k;
+    }
+  }
+  return classes;
+}
+
+size_t ga_spmm_classes_workspace_bytes(int64_t n_rows, int64_t n_edges, int64_t feat,
+                                       int64_t n_classes) {
+  if (n_rows <= 0 || n_edges <= 0 || feat <= 0 || n_classes <= 0) return 0;
+  return (size_t)n_rows * n_classes * feat * sizeof(float) + ga::runs_workspace_bytes(n_edges, feat, 1);
+}
+
+int ga_spmm_classes(const int32_t *pointer, const int32_t *rows, const int32_t *nbr, const void *u,
+                    void *out, const float *row_scale, int activation, int64_t n_rows,
+                    int64_t n_edges, int64_t feat, int64_t n_classes, int dtype, void *workspace,
+                    size_t workspace_bytes, ga_stream_t stream) {
+  using namespace ga;
+  if (n_rows <= 0 || n_edges <= 0 || feat <= 0 || n_edges > 0x7fffffff || feat > 0x7fffffff)
+    return GA_EINVAL;
+  if (n_classes != 2 && n_classes != 4 && n_classes != 8) return GA_EINVAL;
+  if (n_rows > 0x7ffffffe / n_classes) return GA_EUNSUPPORTED;
+  if (activation < GA_ACT_NONE || activation > GA_ACT_ELU) return GA_EINVAL;
+  if (dtype != GA_F32 && dtype != GA_BF16) return GA_EINVAL;
+  if (!pointer || !rows || !nbr || !u || !out) return GA_EINVAL;
+  if (feat % (dtype == GA_F32 ? 4 : 8) || !aligned(u, 16) || !aligned(out, 16))
+    return GA_EUNSUPPORTED;
+  if (row_scale && !aligned(row_scale, 4)) return GA_EALIGN;
+  if (!workspace || !aligned(workspace, 16) ||
+      workspace_bytes < ga_spmm_classes_workspace_bytes(n_rows, n_edges, feat, n_classes))
+    return GA_EWORKSPACE;
+  const int64_t n_quads = n_rows * feat / 4;
+  const int64_t blocks = (n_quads + kBlock - 1) / kBlock;
+  if (blocks > 0x7fffffff) return GA_EUNSUPPORTED;
+  hipStream_t s = (hipStream_t)stream;
+  float *const partial = (float *)workspace;
+  float *const runs = partial + n_rows * n_classes * feat;
+  const size_t runs_bytes = workspace_bytes - (size_t)n_rows * n_classes * feat * sizeof(float);
+  int rc;
+  // the lanes that share column reads: as the plain sum (launch_spmm)
+#define GA_CLASS_SUMS(T, VEC, GL)                                                            \
+  rc = launch_class_sums<T, VEC, GL>(pointer, rows, nbr, u, partial, n_rows * n_classes,     \
+                                     n_edges, (int)feat, runs, runs_bytes, s)
+  if (dtype == GA_F32) {
+    if (feat > 32) GA_CLASS_SUMS(float, 4, 16);
+    else if (feat > 16) GA_CLASS_SUMS(float, 4, 8);
+    else GA_CLASS_SUMS(float, 4, 0);
+  } else {
+    if (feat > 128) GA_CLASS_SUMS(bf16_t, 8, 16);
+    else GA_CLASS_SUMS(bf16_t, 8, 0);
+  }
+#undef GA_CLASS_SUMS
+  if (rc != GA_OK) return rc;
+#define GA_CLASS_SUM(T, N)                                                                   \
+  hipLaunchKernelGGL((class_sum_kernel<T, N>), dim3((unsigned)blocks), dim3(kBlock), 0, s,   \
+                     (const float4 *)partial, row_scale, activation, n_quads, (int)(feat / 4), \
+                     (T *)out)
+#define GA_CLASS_SUM_T(T)                       \
+  do {                                          \
+    if (n_classes == 2) GA_CLASS_SUM(T, 2);     \
+    else if (n_classes == 4) GA_CLASS_SUM(T, 4); \
+    else GA_CLASS_SUM(T, 8);                    \
+  } while (0)
+  if (dtype == GA_F32) GA_CLASS_SUM_T(float);
+  else GA_CLASS_SUM_T(bf16_t);
+#undef GA_CLASS_SUM_T
+#undef GA_CLASS_SUM
+  return launch_status();
 }
 
 size_t ga_spmm_arg_workspace_bytes(int64_t n_edges, int64_t feat) {

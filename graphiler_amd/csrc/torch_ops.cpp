@@ -13,8 +13,10 @@
 #include <torch/custom_class.h>
 #include <torch/script.h>
 
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
+#include <map>
 #include <mutex>
 
 #include "../../include/graphiler_amd.h"
@@ -264,6 +266,67 @@ struct DGLGraph : torch::CustomClassHolder {
     }
     return pairs_;
   }
+  // The slots of the in-adjacency ordered by classes of their sources, where a sum of
+  // rows of `feat` features is faster over them (ga_spmm_source_classes).  Degrees are
+  // read and a layout is built on first use, neither while the stream is captured; a
+  // layout that does not fit the memory is done without.
+  struct SourceClasses {
+    int64_t num_classes = 0;           // 0: the plain sum
+    torch::Tensor pointer, rows, nbr;  // int32
+  };
+  SourceClasses source_classes(int64_t feat, int dtype) {
+    if (!ga_spmm_source_classes(nullptr, nullptr, num_nodes, num_edges, feat, dtype)) return {};
+    const Side in = side(false);
+    std::lock_guard<std::mutex> lock(mu_);
+    const bool capturing = c10::hip::currentStreamCaptureStatusMayInitCtx() !=
+                           c10::hip::CaptureStatus::None;
+    const auto key = std::make_pair(feat, dtype);
+    auto it = class_count_.find(key);
+    if (it == class_count_.end()) {
+      if (capturing) return {};
+      if (source_degrees_.empty()) {
+        torch::Tensor deg = torch::diff(out_pointer);
+        deg = deg.index({deg.gt(0)}).to(at::kDouble);
+        const torch::Tensor bucket = torch::log2(deg).floor().to(at::kLong);
+        const torch::Tensor both =
+            torch::stack({torch::bincount(bucket, {}, GA_DEGREE_BUCKETS).to(at::kDouble),
+                          torch::bincount(bucket, deg, GA_DEGREE_BUCKETS)})
+                .to(at::kLong).cpu().contiguous();
+        const int64_t *p = both.data_ptr<int64_t>();
+        source_degrees_.assign(p, p + 2 * GA_DEGREE_BUCKETS);
+      }
+      const int64_t k = ga_spmm_source_classes(source_degrees_.data(),
+                                               source_degrees_.data() + GA_DEGREE_BUCKETS,
+                                               num_nodes, num_edges, feat, dtype);
+      it = class_count_.emplace(key, k).first;
+    }
+    const int64_t k = it->second;
+    if (k == 0) return {};
+    auto at = classes_.find(k);
+    if (at == classes_.end()) {
+      if (capturing) return {};
+      try {
+        const auto i32 = in_pointer.options();
+        SourceClasses c;
+        c.num_classes = k;
+        c.pointer = torch::empty({k * num_nodes + 1}, i32);
+        c.rows = torch::empty({num_edges}, i32);
+        c.nbr = torch::empty({num_edges}, i32);
+        const size_t bytes = ga_source_classes_workspace_bytes(num_edges, k);
+        torch::Tensor ws = torch::empty({(int64_t)bytes}, i32.dtype(at::kByte));
+        check_ga(ga_source_classes_build(
+                     in.rows.data_ptr<int>(), in_node_indices.data_ptr<int>(), num_nodes, num_edges,
+                     k, c.pointer.data_ptr<int>(), c.rows.data_ptr<int>(), c.nbr.data_ptr<int>(),
+                     ws.data_ptr(), bytes, current_stream(in_pointer)),
+                 "ga_source_classes_build");
+        at = classes_.emplace(k, c).first;
+      } catch (const c10::OutOfMemoryError &) {
+        it->second = 0;
+        return {};
+      }
+    }
+    return at->second;
+  }
   // Scratch shared by the operators called on this graph: calls that use it must be
   // ordered on one stream (two streams working on one graph object race on it).  It
   // grows on demand; a buffer that was handed out is never freed while the graph
@@ -271,9 +334,10 @@ struct DGLGraph : torch::CustomClassHolder {
   torch::Tensor workspace(size_t bytes) {
     std::lock_guard<std::mutex> lock(mu_);
     if (!ws_.defined() || (size_t)ws_.numel() < bytes) {
+      torch::Tensor larger = torch::empty({(int64_t)std::max<size_t>(bytes, 256)},
+                                          in_pointer.options().dtype(at::kByte));
       if (ws_.defined()) retired_ws_.push_back(ws_);
-      ws_ = torch::empty({(int64_t)std::max<size_t>(bytes, 256)},
-                         in_pointer.options().dtype(at::kByte));
+      ws_ = larger;
     }
     return ws_;
   }
@@ -283,6 +347,9 @@ struct DGLGraph : torch::CustomClassHolder {
   Side in_side_, out_side_;
   TypedTiles tiles_;
   RelationPairs pairs_;
+  std::vector<int64_t> source_degrees_;
+  std::map<std::pair<int64_t, int>, int64_t> class_count_;
+  std::map<int64_t, SourceClasses> classes_;
   torch::Tensor ws_;
   std::vector<torch::Tensor> retired_ws_;
 };
@@ -290,6 +357,27 @@ struct DGLGraph : torch::CustomClassHolder {
 using GraphPtr = c10::intrusive_ptr<DGLGraph>;
 
 namespace {
+
+// The sum of source rows over slots ordered by source classes, where that is the faster
+// order; false (nothing launched) elsewhere.
+bool sum_by_classes(const GraphPtr &g, const torch::Tensor &u, torch::Tensor &out,
+                    const float *row_scale, int activation, int64_t feat, int dt) {
+  if (((uintptr_t)u.data_ptr() | (uintptr_t)out.data_ptr()) % 16) return false;
+  const DGLGraph::SourceClasses c = g->source_classes(feat, dt);
+  if (c.num_classes == 0) return false;
+  torch::Tensor ws;
+  try {
+    ws = g->workspace(ga_spmm_classes_workspace_bytes(g->num_nodes, g->num_edges, feat, c.num_classes));
+  } catch (const c10::OutOfMemoryError &) {
+    return false;
+  }
+  check_ga(ga_spmm_classes(c.pointer.data_ptr<int>(), c.rows.data_ptr<int>(), c.nbr.data_ptr<int>(),
+                           u.data_ptr(), out.data_ptr(), row_scale, activation, g->num_nodes,
+                           g->num_edges, feat, c.num_classes, dt, ws.data_ptr(),
+                           (size_t)ws.numel(), current_stream(u)),
+           "ga_spmm_classes");
+  return true;
+}
 
 // edge_rows: u is per-edge in edge-id order and is read through the edge-id
 // column in place of the neighbour column (u[e] op w[e])
@@ -317,6 +405,9 @@ torch::Tensor spmm(const GraphPtr &g, int op, int reduce, const torch::Tensor &u
   TORCH_CHECK(u.size(0) == (op == GA_COPY_E || edge_rows ? g->num_edges : g->num_nodes),
               "features have the wrong number of rows");
   torch::Tensor out = torch::empty(out_shape(g->num_nodes, u), u.options());
+  if (op == GA_COPY_U && reduce == GA_SUM && !reverse &&
+      sum_by_classes(g, u, out, nullptr, GA_ACT_NONE, feat, dt))
+    return out;
   const size_t ws_bytes = ga_spmm_workspace_bytes(g->num_edges, feat);
   torch::Tensor ws = g->workspace(ws_bytes);
   check_ga(ga_spmm_csr(ptr.data_ptr<int>(), side.rows.data_ptr<int>(),
@@ -382,6 +473,9 @@ torch::Tensor SpMMScaled(torch::Tensor features, at::optional<torch::Tensor> row
   torch::Tensor factor;
   if (per_row) factor = row_scale.value().contiguous();
   torch::Tensor out = torch::empty(out_shape(n, features), features.options());
+  if (!edge_rows && sum_by_classes(graph, features, out, per_row ? factor.data_ptr<float>() : nullptr,
+                                   (int)activation, feat, dt))
+    return out;
   torch::Tensor ws = graph->workspace(ga_spmm_scaled_workspace_bytes(graph->num_edges, feat));
   check_ga(ga_spmm_csr_scaled(
                graph->in_pointer.data_ptr<int>(), side.rows.data_ptr<int>(),

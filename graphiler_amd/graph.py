@@ -219,6 +219,49 @@ class DGLGraph:
             self._cache["pairs"] = _build_relation_pairs(self)
         return self._cache["pairs"]
 
+    def _source_degrees(self):
+        """(nodes, edges) by the power of two below the out-degree, as host int64 arrays."""
+        if "source_degrees" not in self._cache:
+            deg = torch.diff(self.out_pointer)
+            deg = deg[deg > 0].double()
+            bucket = torch.log2(deg).floor().long()
+            both = torch.stack([torch.bincount(bucket, minlength=capi.GA_DEGREE_BUCKETS).double(),
+                                torch.bincount(bucket, deg, minlength=capi.GA_DEGREE_BUCKETS)])
+            self._cache["source_degrees"] = both.long().cpu().numpy()
+        return self._cache["source_degrees"]
+
+    def source_classes(self, feat: int, dtype: int) -> Optional["SourceClasses"]:
+        """The slots of the in-adjacency ordered by classes of their sources, where a sum
+        of rows of ``feat`` features is faster over them (``ga_spmm_source_classes``),
+        else None.  Degrees are read and a layout is built on first use, neither while the
+        stream is captured; a layout that does not fit the memory is done without."""
+        lib = capi.load()
+        key = ("source_classes", feat, dtype)
+        n = self._cache.get(key)
+        if n is None:
+            if not lib.ga_spmm_source_classes(None, None, self.num_nodes, self.num_edges, feat, dtype):
+                n = 0
+            elif torch.cuda.is_current_stream_capturing():
+                return None
+            else:
+                nodes, edges = self._source_degrees()
+                n = int(lib.ga_spmm_source_classes(nodes.ctypes.data, edges.ctypes.data,
+                                                   self.num_nodes, self.num_edges, feat, dtype))
+            self._cache[key] = n
+        if n == 0:
+            return None
+        layout = self._cache.get(("classes", n))
+        if layout is None:
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            try:
+                layout = _build_source_classes(self, n)
+            except torch.OutOfMemoryError:
+                self._cache[key] = 0
+                return None
+            self._cache[("classes", n)] = layout
+        return layout
+
     def workspace(self, nbytes: int) -> torch.Tensor:
         """Scratch buffer shared by the operators called on this graph (grows on
         demand).  Calls that use it must be ordered on one stream: two streams
@@ -227,11 +270,11 @@ class DGLGraph:
         replay launches that write to it."""
         ws = self._cache.get("ws")
         if ws is None or ws.numel() < nbytes:
+            larger = torch.empty(max(int(nbytes), 256), dtype=torch.uint8,
+                                 device=self.device)
             if ws is not None:
                 self._cache.setdefault("retired_ws", []).append(ws)
-            ws = torch.empty(max(int(nbytes), 256), dtype=torch.uint8,
-                             device=self.device)
-            self._cache["ws"] = ws
+            self._cache["ws"] = ws = larger
         return ws
 
 
@@ -291,6 +334,29 @@ def _build_relation_pairs(g: "DGLGraph") -> Optional[RelationPairs]:
         dst_by_type=pair_dst[by_type].contiguous())
     pairs.max_slots = int(largest.item())      # read behind all launches: the host waits once
     return pairs
+
+
+@dataclass
+class SourceClasses:
+    """Slots of the in-adjacency ordered by (class of the source, destination)."""
+    num_classes: int
+    pointer: torch.Tensor           # (classes * N + 1) int32
+    rows: torch.Tensor              # (E) int32: class * N + destination
+    nbr: torch.Tensor               # (E) int32: source
+
+
+def _build_source_classes(g: "DGLGraph", n: int) -> SourceClasses:
+    lib = capi.load()
+    i32 = dict(dtype=torch.int32, device=g.device)
+    out = SourceClasses(n, torch.empty(n * g.num_nodes + 1, **i32),
+                        torch.empty(g.num_edges, **i32), torch.empty(g.num_edges, **i32))
+    ws = torch.empty(int(lib.ga_source_classes_workspace_bytes(g.num_edges, n)),
+                     dtype=torch.uint8, device=g.device)
+    capi.check(lib.ga_source_classes_build(
+        g.in_row_of_slot.data_ptr(), g.in_node_indices.data_ptr(), g.num_nodes, g.num_edges, n,
+        out.pointer.data_ptr(), out.rows.data_ptr(), out.nbr.data_ptr(), ws.data_ptr(),
+        ws.numel(), torch.cuda.current_stream(g.device).cuda_stream), "ga_source_classes_build")
+    return out
 
 
 def group_on_device(key: torch.Tensor, other: Optional[torch.Tensor], n_keys: int):

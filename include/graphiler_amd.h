@@ -133,6 +133,34 @@ int ga_spmm_csr_scaled(const int32_t *pointer, const int32_t *row_of_slot,
                        int64_t n_edges, int64_t feat, int op, int dtype, void *workspace,
                        size_t workspace_bytes, ga_stream_t stream);
 
+/* The same sum (GA_COPY_U, with the tail) over slots ordered by classes of their sources:
+ * dense graphs whose table exceeds an L2.  ga_spmm_source_classes (host arithmetic): the
+ * classes to use, 0 where ga_spmm_csr[_scaled] is the faster call; from the nodes with
+ * out-degrees 2^b .. 2^(b+1) - 1 and their edges, b < GA_DEGREE_BUCKETS (host arrays;
+ * NULL: 0 if the answer is 0 whatever they hold, else 1).  ga_source_classes_build (once per graph
+ * and number of classes; 2, 4 or 8) partitions the in-adjacency:
+ *   pointer  (n_classes * n_rows + 1) int32    rows  (n_edges) int32: class * n_rows + row
+ *   nbr_out  (n_edges) int32: source of the slot
+ * stable, so slots ascend by (class, destination, original slot).  ga_spmm_classes takes
+ * rows that 16-byte accesses tile (feat % 4 fp32 / % 8 bf16, 16-byte aligned u and out;
+ * GA_EUNSUPPORTED otherwise); the partial sums of a destination's classes, fp32 in the
+ * workspace (16-byte aligned), are added in class order.
+ */
+#define GA_DEGREE_BUCKETS 31
+int64_t ga_spmm_source_classes(const int64_t *nodes_of_degree, const int64_t *edges_of_degree,
+                               int64_t n_rows, int64_t n_edges, int64_t feat, int dtype);
+size_t ga_source_classes_workspace_bytes(int64_t n_edges, int64_t n_classes);
+int ga_source_classes_build(const int32_t *row_of_slot, const int32_t *nbr, int64_t n_rows,
+                            int64_t n_edges, int64_t n_classes, int32_t *pointer, int32_t *rows,
+                            int32_t *nbr_out, void *workspace, size_t workspace_bytes,
+                            ga_stream_t stream);
+size_t ga_spmm_classes_workspace_bytes(int64_t n_rows, int64_t n_edges, int64_t feat,
+                                       int64_t n_classes);
+int ga_spmm_classes(const int32_t *pointer, const int32_t *rows, const int32_t *nbr, const void *u,
+                    void *out, const float *row_scale, int activation, int64_t n_rows,
+                    int64_t n_edges, int64_t feat, int64_t n_classes, int dtype, void *workspace,
+                    size_t workspace_bytes, ga_stream_t stream);
+
 /* SpMM with max / min and the position of each extremum: the arg_u / arg_e
  * outputs of the reference's generic kernel (SpMMCsrKernel, spmm.cuh:30-71,
  * reducers functor.cuh:148-213: strict comparison, so the first extremum in
