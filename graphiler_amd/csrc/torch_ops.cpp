@@ -213,6 +213,7 @@ struct DGLGraph : torch::CustomClassHolder {
     torch::Tensor pair_pointer, pair_of_slot, pair_dst, dst_pointer, type_pointer;   // int32
     torch::Tensor by_type, dst_by_type;                                              // int64
     torch::Tensor rank, rank_of_slot;                                                // int32
+    torch::Tensor rows, tiles;         // (-, 4) int32, ga_pair_tiles_build
     bool valid = false;
     bool ready = false;
   };
@@ -259,6 +260,14 @@ struct DGLGraph : torch::CustomClassHolder {
           pairs_.dst_by_type = pair_dst.index_select(0, by_type).contiguous();
           pairs_.rank = rank.to(at::kInt).contiguous();
           pairs_.rank_of_slot = rank.index_select(0, pair_of_slot).to(at::kInt).contiguous();
+          pairs_.rows = torch::empty({P, 4}, in_pointer.options());
+          pairs_.tiles = torch::empty({ga_pair_tiles_capacity(P, num_etypes), 4}, in_pointer.options());
+          check_ga(ga_pair_tiles_build(
+                       pairs_.type_pointer.data_ptr<int>(), num_etypes,
+                       pairs_.by_type.data_ptr<int64_t>(), pairs_.dst_by_type.data_ptr<int64_t>(),
+                       pairs_.pair_pointer.data_ptr<int>(), P, pairs_.rows.data_ptr<int>(),
+                       pairs_.tiles.data_ptr<int>(), current_stream(in_pointer)),
+                   "ga_pair_tiles_build");
           pairs_.max_slots = largest.item<int64_t>();     // behind all launches: the host waits once
           pairs_.valid = true;
         }
@@ -1280,15 +1289,17 @@ torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::T
   const int dt = feat_dtype(k, "k");
   const auto stream = current_stream(k);
   if (!relation_att.is_contiguous()) return per_edge();
-  // the matrices as the query side needs them: transposed, times scale / divisor
-  torch::Tensor att_t = torch::empty_like(relation_att);
   torch::Tensor sc;
   if (scale.has_value()) sc = scale.value().to(at::kFloat).contiguous();
-  check_ga(ga_transpose_scale_blocks(relation_att.data_ptr(),
-                                     sc.defined() ? sc.data_ptr<float>() : nullptr,
-                                     (float)(1.0 / divisor), att_t.data_ptr(),
-                                     graph->num_etypes * heads, d, dt, stream),
-           "ga_transpose_scale_blocks");
+  const float *const scp = sc.defined() ? sc.data_ptr<float>() : nullptr;
+  // the matrices as the query side needs them: transposed, times scale / divisor
+  auto transposed = [&]() {
+    torch::Tensor att_t = torch::empty_like(relation_att);
+    check_ga(ga_transpose_scale_blocks(relation_att.data_ptr(), scp, (float)(1.0 / divisor),
+                                       att_t.data_ptr(), graph->num_etypes * heads, d, dt, stream),
+             "ga_transpose_scale_blocks");
+    return att_t;
+  };
   auto typed_rows = [&](const torch::Tensor &x, const torch::Tensor &index,
                         const torch::Tensor &w, torch::Tensor &y) {
     return ga_segment_mm_gather(pairs.type_pointer.data_ptr<int>(), graph->num_etypes,
@@ -1301,18 +1312,29 @@ torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::T
   if (ga_pair_attention_preferred(P, e, pairs.max_slots, heads, d, dt)) {
     torch::Tensor m_pair = torch::empty({P, hid}, k.options());
     torch::Tensor lse = torch::empty({P, heads}, k.options().dtype(at::kFloat));
-    const int rc = ga_pair_attention(
-        pairs.type_pointer.data_ptr<int>(), graph->num_etypes, pairs.by_type.data_ptr<int64_t>(),
-        pairs.dst_by_type.data_ptr<int64_t>(), pairs.pair_pointer.data_ptr<int>(),
+    const size_t bytes = ga_pair_weights_bytes(graph->num_etypes, heads, d, dt);
+    torch::Tensor att, msg = relation_msg;
+    if (bytes > 0) {                     // both matrices as the products read them
+      att = torch::empty({(int64_t)bytes}, k.options().dtype(at::kByte));
+      msg = torch::empty({(int64_t)bytes}, k.options().dtype(at::kByte));
+      check_ga(ga_pair_weights(relation_att.data_ptr<float>(), scp, GA_F32, (float)(1.0 / divisor),
+                               relation_msg.data_ptr<float>(), att.data_ptr(), msg.data_ptr(),
+                               graph->num_etypes, heads, d, stream),
+               "ga_pair_weights");
+    } else {
+      att = transposed();
+    }
+    const int rc = ga_pair_attention_tiles(
+        pairs.rows.data_ptr<int>(), pairs.tiles.data_ptr<int>(), graph->num_etypes,
         graph->in_node_indices.data_ptr<int>(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-        att_t.data_ptr(), relation_msg.data_ptr(), m_pair.data_ptr(), lse.data_ptr<float>(), P,
+        att.data_ptr(), msg.data_ptr(), m_pair.data_ptr(), lse.data_ptr<float>(), P, n,
         pairs.max_slots, heads, d, dt, stream);
     if (rc != GA_EUNSUPPORTED) {
-      check_ga(rc, "ga_pair_attention");
+      check_ga(rc, "ga_pair_attention_tiles");
       torch::Tensor ws = graph->workspace(ga_gat_workspace_bytes(P, hid, heads));
       torch::Tensor out = torch::empty({n, hid}, k.options());
       check_ga(ga_edge_softmax_sum(pairs.dst_pointer.data_ptr<int>(), pairs.pair_dst.data_ptr<int>(),
-                                   nullptr, lse.data_ptr<float>(), m_pair.data_ptr(),
+                                   pairs.rank.data_ptr<int>(), lse.data_ptr<float>(), m_pair.data_ptr(),
                                    out.data_ptr(), n, P, heads, d, dt, ws.data_ptr(),
                                    (size_t)ws.numel(), stream),
                "ga_edge_softmax_sum");
@@ -1320,7 +1342,7 @@ torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::T
     }
   }
   torch::Tensor q_pair = torch::empty({P, hid}, k.options());
-  int rc = typed_rows(q, pairs.dst_by_type, att_t, q_pair);
+  int rc = typed_rows(q, pairs.dst_by_type, transposed(), q_pair);
   if (rc == GA_EUNSUPPORTED) return per_edge();
   check_ga(rc, "ga_segment_mm_gather");
   // both passes share the scratch; the bytes are not monotonic in the number of items

@@ -294,6 +294,8 @@ class RelationPairs:
     rank: torch.Tensor              # (P) int32: position of a pair in by_type
     rank_of_slot: torch.Tensor      # (E) int32: rank[pair_of_slot]
     dst_by_type: torch.Tensor       # (P) int64: pair_dst[by_type]
+    rows: torch.Tensor              # (P, 4) int32 in by_type order: first slot, end slot, destination, 0
+    tiles: torch.Tensor             # (-, 4) int32: type (-1: none), first row, end row, 0
 
 
 def _build_relation_pairs(g: "DGLGraph") -> Optional[RelationPairs]:
@@ -331,7 +333,14 @@ def _build_relation_pairs(g: "DGLGraph") -> Optional[RelationPairs]:
         by_type=by_type.contiguous(),
         rank=rank.int().contiguous(),
         rank_of_slot=rank[pair_of_slot].int().contiguous(),
-        dst_by_type=pair_dst[by_type].contiguous())
+        dst_by_type=pair_dst[by_type].contiguous(),
+        rows=torch.empty((n_pairs, 4), dtype=torch.int32, device=dev),
+        tiles=torch.empty((int(capi.load().ga_pair_tiles_capacity(n_pairs, n_types)), 4),
+                          dtype=torch.int32, device=dev))
+    capi.check(capi.load().ga_pair_tiles_build(
+        pairs.type_pointer.data_ptr(), n_types, pairs.by_type.data_ptr(),
+        pairs.dst_by_type.data_ptr(), pairs.pair_pointer.data_ptr(), n_pairs, pairs.rows.data_ptr(),
+        pairs.tiles.data_ptr(), torch.cuda.current_stream(dev).cuda_stream), "ga_pair_tiles_build")
     pairs.max_slots = int(largest.item())      # read behind all launches: the host waits once
     return pairs
 

@@ -1033,14 +1033,17 @@ def relation_pair_attention(k, q, v, relation_att, relation_msg, relation_scale,
         if tuple(relation_scale.shape) != (n_types, heads) \
                 or relation_scale.dtype not in (torch.float32, torch.bfloat16):
             raise RuntimeError("relation_scale must be (edge types, heads) float32 or bfloat16")
-    # the matrices as the query side needs them: transposed, times the scale (an fp32
-    # product rounded once to the features' dtype)
-    att_t = torch.empty_like(relation_att)
     scale_dt = capi.GA_BF16 if relation_scale is not None and relation_scale.dtype == torch.bfloat16 \
         else capi.GA_F32
-    capi.check(lib.ga_transpose_scale_blocks_as(
-        relation_att.data_ptr(), _ptr(relation_scale), scale_dt, float(factor), att_t.data_ptr(),
-        n_types * heads, d, dt, stream), "ga_transpose_scale_blocks_as")
+
+    def transposed():
+        # the matrices as the query side needs them: transposed, times the scale (an fp32
+        # product rounded once to the features' dtype)
+        att_t = torch.empty_like(relation_att)
+        capi.check(lib.ga_transpose_scale_blocks_as(
+            relation_att.data_ptr(), _ptr(relation_scale), scale_dt, float(factor), att_t.data_ptr(),
+            n_types * heads, d, dt, stream), "ga_transpose_scale_blocks_as")
+        return att_t
 
     def typed_rows(x, index, w):        # row r = x[index[r]] @ w[relation of pair by_type[r]]
         y = torch.empty((P, hid), dtype=x.dtype, device=dev)
@@ -1055,25 +1058,32 @@ def relation_pair_attention(k, q, v, relation_att, relation_msg, relation_scale,
     # log-sum-exps (the softmax-weighted sum of per-"edge" rows, with the pairs as the
     # edges), which makes the weights the softmax over all its in-edges
     if lib.ga_pair_attention_preferred(P, e, pairs.max_slots, heads, d, dt):
-        m_pair = torch.empty((P, hid), dtype=v.dtype, device=dev)            # pair order
+        m_pair = torch.empty((P, hid), dtype=v.dtype, device=dev)            # by_type order
         lse = torch.empty((P, heads), dtype=torch.float32, device=dev)
-        rc = lib.ga_pair_attention(
-            pairs.type_pointer.data_ptr(), n_types, pairs.by_type.data_ptr(),
-            pairs.dst_by_type.data_ptr(), pairs.pair_pointer.data_ptr(),
-            graph.in_node_indices.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-            att_t.data_ptr(), relation_msg.data_ptr(), m_pair.data_ptr(), lse.data_ptr(), P,
-            pairs.max_slots, heads, d, dt, stream)
+        nbytes = int(lib.ga_pair_weights_bytes(n_types, heads, d, dt))
+        if nbytes:                      # both matrices as the products read them
+            att, msg = (torch.empty(nbytes, dtype=torch.uint8, device=dev) for _ in range(2))
+            capi.check(lib.ga_pair_weights(
+                relation_att.data_ptr(), _ptr(relation_scale), scale_dt, float(factor),
+                relation_msg.data_ptr(), att.data_ptr(), msg.data_ptr(), n_types, heads, d, stream),
+                "ga_pair_weights")
+        else:
+            att, msg = transposed(), relation_msg
+        rc = lib.ga_pair_attention_tiles(
+            pairs.rows.data_ptr(), pairs.tiles.data_ptr(), n_types, graph.in_node_indices.data_ptr(),
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), att.data_ptr(), msg.data_ptr(),
+            m_pair.data_ptr(), lse.data_ptr(), P, n, pairs.max_slots, heads, d, dt, stream)
         if rc != capi.GA_EUNSUPPORTED:
-            capi.check(rc, "ga_pair_attention")
+            capi.check(rc, "ga_pair_attention_tiles")
             ws = graph.workspace(lib.ga_gat_workspace_bytes(P, hid, heads))
             out = torch.empty((n, hid), dtype=v.dtype, device=dev)
             capi.check(lib.ga_edge_softmax_sum(
-                pairs.dst_pointer.data_ptr(), pairs.pair_dst.data_ptr(), None, lse.data_ptr(),
-                m_pair.data_ptr(), out.data_ptr(), n, P, heads, d, dt, ws.data_ptr(), ws.numel(),
-                stream), "ga_edge_softmax_sum")
+                pairs.dst_pointer.data_ptr(), pairs.pair_dst.data_ptr(), pairs.rank.data_ptr(),
+                lse.data_ptr(), m_pair.data_ptr(), out.data_ptr(), n, P, heads, d, dt, ws.data_ptr(),
+                ws.numel(), stream), "ga_edge_softmax_sum")
             return out
         del m_pair, lse
-    q_pair = typed_rows(q, pairs.dst_by_type, att_t)
+    q_pair = typed_rows(q, pairs.dst_by_type, transposed())
     # both passes share the scratch; the bytes are not monotonic in the number of items
     # (longer runs from a threshold on), so the pairs are asked for as well
     ws = graph.workspace(max(lib.ga_softmax_workspace_bytes(e, heads),

@@ -198,3 +198,65 @@ def test_more_than_a_million_pairs(device, heads, d, bf16):
     three = ops.relation_pair_attention(*args)
     tol = 2 * (2 * TOL_BF16 if bf16 else 2 * TOL_F32)       # each within its own of the exact value
     assert_close(one.float().cpu().numpy(), three.float().cpu().numpy(), tol, f"{heads}x{d}")
+
+
+@pytest.mark.parametrize("heads,d,bf16", [(1, 64, False), (2, 32, False), (4, 16, False), (1, 64, True),
+                                          (2, 64, False), (8, 16, True)])
+@pytest.mark.parametrize("per", [[1], [63, 0, 65], [64, 1, 0, 129, 300] + [3] * 70])
+def test_prepared_tiles(device, heads, d, bf16, per):
+    """Tiles, rows and matrices prepared for the pass: the pass by itself over them gives what
+    it gives without them, in by_type order, and both are within rounding of float64; more
+    types than a wavefront has lanes."""
+    rng = np.random.default_rng(len(per) + d)
+    g, *_, n = _typed_graph(rng, per, 30, device)
+    pairs, lib, T = g.relation_pairs(), capi.load(), len(per)
+    tiles = pairs.tiles.cpu().numpy()
+    want = [(t, lo, min(lo + 64, hi), 0) for t, (lo, hi) in enumerate(zip(
+        pairs.type_pointer.tolist(), pairs.type_pointer.tolist()[1:])) for lo in range(lo, hi, 64)]
+    assert [tuple(x) for x in tiles[:len(want)]] == want and (tiles[len(want):, 0] == -1).all()
+    by_type = pairs.by_type
+    assert torch.equal(pairs.rows[:, 0], pairs.pair_pointer[by_type])
+    assert torch.equal(pairs.rows[:, 1], pairs.pair_pointer[by_type + 1])
+    assert torch.equal(pairs.rows[:, 2].long(), pairs.dst_by_type)
+    dt, code = (torch.bfloat16, capi.GA_BF16) if bf16 else (torch.float32, capi.GA_F32)
+    rand = lambda *s: torch.from_numpy(rng.standard_normal(s, dtype=np.float32)).to(device).to(dt)
+    k, q, v = (rand(n, heads * d) for _ in range(3))
+    att, msg = (rand(T, heads, d, d) / d ** 0.5 for _ in range(2))
+    rc, m, lse = _one_pass(g, k, q, v, att, msg)
+    assert rc == capi.GA_OK
+    m2, lse2 = torch.empty_like(m), torch.empty_like(lse)
+    a, b = att, msg
+    nbytes = lib.ga_pair_weights_bytes(T, heads, d, code)
+    assert (nbytes > 0) == (not bf16 and heads * d == 64 and d >= 32)
+    if nbytes:
+        a, b = (torch.empty(nbytes, dtype=torch.uint8, device=device) for _ in range(2))
+        scale = torch.full((T, heads), 2.0, device=device)
+        capi.check(lib.ga_pair_weights(
+            att.transpose(2, 3).contiguous().data_ptr(), scale.data_ptr(), capi.GA_F32, 0.5,
+            msg.data_ptr(), a.data_ptr(), b.data_ptr(), T, heads, d, 0), "weights")
+    run = lambda nodes: lib.ga_pair_attention_tiles(
+        pairs.rows.data_ptr(), pairs.tiles.data_ptr(), T, g.in_node_indices.data_ptr(), q.data_ptr(),
+        k.data_ptr(), v.data_ptr(), a.data_ptr(), b.data_ptr(), m2.data_ptr(), lse2.data_ptr(),
+        pairs.num_pairs, nodes, pairs.max_slots, heads, d, code, torch.cuda.current_stream().cuda_stream)
+    assert run(2 ** 31 - 1) == capi.GA_EUNSUPPORTED       # offsets past 4 GB
+    capi.check(run(n), "tiles")
+    if not nbytes:
+        assert torch.equal(m[by_type], m2) and torch.equal(lse[by_type], lse2)
+        return
+    ref_m, ref_lse = _by_pair(g, k, q, v, att, msg)
+    at = by_type.cpu()
+    assert_close(m2.cpu().numpy(), ref_m[at].numpy(), 2 * TOL_F32, "m")
+    assert_close(lse2.cpu().numpy(), ref_lse[at].numpy(), 2 * TOL_F32, "lse")
+    # rows with values that are not finite: the same rows as the fp32 products give
+    src, e = g.in_node_indices.long(), g.num_edges
+    q[pairs.pair_dst[0].long(), 5] = float("inf")
+    v[src[e - 1], 7], v[src[e // 2], :] = -float("inf"), float("nan")
+    rc, m, lse = _one_pass(g, k, q, v, att, msg)
+    capi.check(run(n), "tiles")
+    for x, y in ((m[by_type], m2), (lse[by_type], lse2)):
+        assert torch.equal(torch.isnan(x), torch.isnan(y)) and torch.equal(x == float("inf"), y == float("inf"))
+        both = torch.isfinite(x)
+        assert torch.equal(both, torch.isfinite(y))
+        if bool(both.any()):
+            assert_close(x[both].cpu().numpy(), y[both].cpu().numpy(), 4 * TOL_F32, "finite")
+    assert not bool(torch.isfinite(m2).all())
