@@ -64,6 +64,27 @@ __global__ __launch_bounds__(kBlock) void fill_zero_kernel(int32_t *p, int64_t n
   if (i < n) p[i] = 0;
 }
 
+// Pointer of items that are already sorted by key: item i writes the entries of the keys
+// after its predecessor's up to its own, the last item those after its own as well.  No
+// sort, no search: every key is read once (672,884 keys: a stable sort and the comparison
+// behind it took 185 us of launches and two waits).  status[0]: a key outside [0, n_keys),
+// status[1]: a key below its predecessor; nothing is written for such an item.
+__global__ __launch_bounds__(kBlock) void sorted_pointer_kernel(
+    const int64_t *__restrict__ key, int64_t n_keys, int64_t n_items,
+    int32_t *__restrict__ pointer, int32_t *__restrict__ status) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (n_items == 0 && i <= n_keys) pointer[i] = 0;
+  if (i >= n_items) return;
+  const int64_t k = key[i], before = i > 0 ? key[i - 1] : -1;
+  const bool outside = k < 0 || k >= n_keys, unsorted = i > 0 && k < before;
+  if (outside) status[0] = 1;       // every writer stores the same value
+  if (unsorted) status[1] = 1;
+  if (outside || unsorted) return;
+  for (int64_t v = before < -1 ? 0 : before + 1; v <= k; ++v) pointer[v] = (int32_t)i;
+  if (i == n_items - 1)
+    for (int64_t v = k + 1; v <= n_keys; ++v) pointer[v] = (int32_t)n_items;
+}
+
 // ---- slots ordered by classes of their sources ---------------------------------
 // A stable partition of the in-adjacency's slots into up to kMaxClasses classes of source
 // nodes: every wavefront counts the classes of kPartSlots consecutive slots (ballots),
@@ -280,6 +301,19 @@ int ga_source_classes_build(const int32_t *row_of_slot, const int32_t *nbr, int6
   const int64_t n_keys = n_rows * n_classes;
   hipLaunchKernelGGL(pointer_kernel, dim3((unsigned)((n_keys + 1 + kBlock - 1) / kBlock)),
                      dim3(kBlock), 0, s, rows, n_keys, n_edges, pointer);
+  return launch_status();
+}
+
+int ga_sorted_pointer(const int64_t *key, int64_t n_keys, int64_t n_items, int32_t *pointer,
+                      int32_t *status, ga_stream_t stream) {
+  using namespace ga;
+  if (n_keys < 0 || n_items < 0 || n_keys > 0x7ffffffe || n_items > 0x7fffffff) return GA_EINVAL;
+  if (!pointer || !status || (n_items > 0 && !key)) return GA_EINVAL;
+  hipStream_t s = (hipStream_t)stream;
+  hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(kBlock), 0, s, status, (int64_t)2);
+  const int64_t threads = n_items > 0 ? n_items : n_keys + 1;
+  hipLaunchKernelGGL(sorted_pointer_kernel, dim3((unsigned)((threads + kBlock - 1) / kBlock)),
+                     dim3(kBlock), 0, s, key, n_keys, n_items, pointer, status);
   return launch_status();
 }
 

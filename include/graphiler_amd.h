@@ -91,6 +91,14 @@ int ga_group_edges(const int64_t *key, const int64_t *other, int64_t n_keys,
                    int32_t *status, void *workspace, size_t workspace_bytes,
                    ga_stream_t stream);
 
+/* The pointer of items whose keys ascend already (type columns: ids of one type are
+ * contiguous, include/dglgraph.h:68-71), one pass over the keys.  key (n_items) int64,
+ * pointer (n_keys + 1) int32; status two int32 on the device: [0] 1 when a key lies outside
+ * [0, n_keys), [1] 1 when a key is below the one before it (pointer is then meaningless).
+ */
+int ga_sorted_pointer(const int64_t *key, int64_t n_keys, int64_t n_items, int32_t *pointer,
+                      int32_t *status, ga_stream_t stream);
+
 /* ------------------------------------------------------------------- SpMM --
  * out[v, h, d] = reduce_{i in [pointer[v], pointer[v+1])} msg_i[h, d]
  * Replaces SpMMSrc (spmm.cu:375-389; op GA_COPY_U, gather by nbr),

@@ -1,0 +1,58 @@
+"""Graph preparation: uploads in page-locked pieces and pointers of sorted type columns,
+against numpy."""
+import numpy as np
+import pytest
+import torch
+
+from graphiler_amd import prepare_graph
+from graphiler_amd import graph as G
+
+pytestmark = pytest.mark.gpu
+
+
+# a piece holds 524,288 ids; arrays below 131,072 ids go over directly; the ring has three
+@pytest.mark.parametrize("sizes", [(0,), (1, 131_071, 131_072), (524_288, 524_289),
+                                   (2_000_003, 5, 1_700_000)])
+def test_upload(device, sizes):
+    rng = np.random.default_rng(sum(sizes))
+    arrays = [rng.integers(-2 ** 62, 2 ** 62, n) for n in sizes]
+    for got, want in zip(G._upload(arrays, device), arrays):
+        assert got.dtype == torch.int64 and np.array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("n,keys", [(0, 5), (1, 1), (255, 3), (257, 1000), (100_000, 7), (70_000, 70_001)])
+def test_sorted_pointer(device, n, keys):
+    rng = np.random.default_rng(n + keys)
+    key = np.sort(rng.integers(0, keys, n)).astype(np.int64)
+    pointer, status = G._sorted_pointer(torch.from_numpy(key).to(device), keys)
+    assert status.tolist() == [0, 0]
+    assert np.array_equal(pointer.cpu().numpy(), np.searchsorted(key, np.arange(keys + 1)))
+    if n > 2:
+        for at, value, want in ((n - 1, keys, [1, 0]), (0, -1, [1, 0]), (n // 2, -5, [1, 1])):
+            bad = key.copy()
+            bad[at] = value
+            assert G._sorted_pointer(torch.from_numpy(bad).to(device), keys)[1].tolist() == want
+
+
+@pytest.mark.parametrize("n,e", [(7, 20), (3000, 140_000), (9000, 600_000)])
+def test_typed_graph(device, n, e):
+    rng = np.random.default_rng(e)
+    src, dst = rng.integers(0, n, e), rng.integers(0, n, e)
+    nt, et = np.sort(rng.integers(0, 4, n)), np.sort(rng.integers(1, 30, e))
+    g = prepare_graph(src, dst, n, device=device, ntype_of=nt, num_ntypes=5, etype_of=et, num_etypes=31)
+    want = G.build_graph_arrays(src, dst, n)
+    for name in ("in_pointer", "in_node_indices", "in_edge_indices", "out_pointer",
+                 "out_node_indices", "out_edge_indices", "COO_src", "COO_dst"):
+        assert np.array_equal(getattr(g, name).cpu().numpy(), getattr(want, name)), name
+    assert np.array_equal(g.ntype_pointer.cpu().numpy(), G.type_pointer(nt, 5))
+    assert np.array_equal(g.etype_pointer.cpu().numpy(), G.type_pointer(et, 31))
+    assert np.array_equal(g.ntype_COO.cpu().numpy(), nt) and np.array_equal(g.etype_COO.cpu().numpy(), et)
+    typed = dict(ntype_of=nt, num_ntypes=5, etype_of=et, num_etypes=31)
+    with pytest.raises(ValueError, match="endpoint"):       # reported before a bad type
+        prepare_graph(np.where(np.arange(e) == 3, n, src), dst, n, device=device, **{**typed, "etype_of": et[::-1]})
+    with pytest.raises(ValueError, match="sorted by type"):
+        prepare_graph(src, dst, n, device=device, **{**typed, "etype_of": et[::-1]})
+    with pytest.raises(ValueError, match="type outside"):
+        prepare_graph(src, dst, n, device=device, **{**typed, "num_ntypes": int(nt.max())})
+    with pytest.raises(RuntimeError, match="one entry per node"):
+        prepare_graph(src, dst, n, device=device, **{**typed, "ntype_of": nt[1:]})
