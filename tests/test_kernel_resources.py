@@ -26,3 +26,19 @@ def test_pair_attention_builds_spill_nothing(tmp_path):
     assert len(spills) == len(waves) == 16
     assert not any(spills), spills
     assert min(waves) >= 4, waves
+
+
+@pytest.mark.skipif(not (os.path.exists(HIPCC) or shutil.which("hipcc")), reason="no hipcc")
+def test_pair_tiles_builds_spill_nothing(tmp_path):
+    r = subprocess.run([HIPCC if os.path.exists(HIPCC) else "hipcc", "--offload-arch=gfx950", "-O3",
+                        "-std=c++17", "-fPIC", "-Xclang", "-target-feature", "-Xclang",
+                        "-packed-fp32-ops", "-Rpass-analysis=kernel-resource-usage", "-c",
+                        "pair_tiles.hip", "-o", str(tmp_path / "pair_tiles.o")],
+                       cwd=CSRC, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert "failed to meet occupancy" not in r.stderr
+    spills = [int(x) for x in re.findall(r"VGPRs Spill: (\d+)", r.stderr)]
+    waves = [int(x) for x in re.findall(r"Occupancy \[waves/SIMD\]: (\d+)", r.stderr)]
+    assert len(spills) == len(waves) == 21      # 16 of the pass, tiles, four of the matrices
+    assert not any(spills), spills
+    assert min(waves) >= 4, waves
