@@ -54,6 +54,34 @@ __device__ __forceinline__ float lanes_sum(float v, int lanes) {
   return v;
 }
 
+// d[t] of the GL lanes of a head, summed over them: lane i gets the sum of slot (i & 7).
+// Halving the slots a lane keeps at every step costs as many instructions as summing all
+// eight in every lane, and leaves each sum in one lane.
+template <int CTRL>
+__device__ __forceinline__ float plus_other(float v) {      // v plus the DPP partner's
+  return v + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+template <int GL>
+__device__ __forceinline__ float sum_by_slot(float (&d)[kUnroll], int sub) {
+  if constexpr (GL == 16) {
+#pragma unroll
+    for (int t = 0; t < kUnroll; ++t) d[t] = plus_other<0x140>(d[t]);         // row_mirror
+  }
+  float e[4], f[2];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {                                               // row_half_mirror
+    const float lo = plus_other<0x141>(d[t]), hi = plus_other<0x141>(d[4 + t]);
+    e[t] = sub & 4 ? hi : lo;
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {                                               // quad_perm [2,3,0,1]
+    const float lo = plus_other<0x4E>(e[t]), hi = plus_other<0x4E>(e[2 + t]);
+    f[t] = sub & 2 ? hi : lo;
+  }
+  const float lo = plus_other<0xB1>(f[0]), hi = plus_other<0xB1>(f[1]);       // quad_perm [1,0,3,2]
+  return sub & 1 ? hi : lo;
+}
+
 // SPREAD: the lane's features lie a lane-group width apart (rows that 16-byte
 // accesses do not tile); they share the lane's one (m, l) pair, i.e. one head.
 // ACT: the activation compiled into the row store (GA_ACT_RELU / GA_ACT_ELU), or
@@ -83,6 +111,7 @@ struct GatPolicy {
     int head_lanes; // kGatFromZ: lanes that share a head (dph / VEC)
     int stride_shift;   // SPREAD: log2 of the lanes per group, set by the launcher
     int act;            // GA_ACT_*: applied to the finished row before it is stored
+    int64_t z_stride;   // elements from a row of z to the next
   };
   static __device__ __forceinline__ void init(float (&st)[VEC + 2]) {
 #pragma unroll
@@ -150,7 +179,9 @@ struct GatPolicy {
       for (int64_t j = a; j < b; j += kUnroll) {
         typename IO::raw_t x[kUnroll];
         float sv;                   // lane i holds the logit of slot (i & 7)
-        if constexpr (MODE == kGatEdge) {
+        if constexpr (MODE == kGatFromZ) {
+          sv = A.er[(int64_t)ids.my_row(sub) * A.heads + h];
+        } else if constexpr (MODE == kGatEdge) {
           if constexpr (GL == 16) {     // lanes 8 .. 15 hold the indices
             sv = A.el[(int64_t)(sub & 8 ? ids.row : 0) * A.heads + h];
             const float o = other_half(sv);
@@ -166,13 +197,26 @@ struct GatPolicy {
                      A.slope);
         }
         static_for<kUnroll>([&](auto t) {
-          x[t] = IO::load(A.z + (int64_t)ids.template index_of<t>() * feat + f0, ln);
+          x[t] = IO::load(A.z + (int64_t)ids.template index_of<t>() * A.z_stride + f0, ln);
         });
         // the columns of the next batch arrive while this batch's rows are added; asked for
         // after the gathers (GroupIds)
         __builtin_amdgcn_sched_barrier(0);
         next.load(row_of_slot, A.nbr, j + kUnroll, b, sub);
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (MODE == kGatFromZ) {
+          // every live lane of a head runs this together (heads tile the row)
+          float d[kUnroll];
+#pragma unroll
+          for (int t = 0; t < kUnroll; ++t) {
+            float xf[VEC];
+            IO::widen(x[t], xf);
+            d[t] = 0.0f;
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) d[t] = fmaf(xf[v], al[v], d[t]);
+          }
+          sv = leaky(sum_by_slot<GL>(d, sub) + sv, A.slope);
+        }
         const bool one_row = j + kUnroll <= b && ids.template row_of<0>() == cur &&
                              ids.template row_of<kUnroll - 1>() == cur;
         if (one_row) {
@@ -233,7 +277,7 @@ struct GatPolicy {
       }
 #pragma unroll
       for (int t = 0; t < kUnroll; ++t) {
-        x[t] = IO::load(A.z + (int64_t)g[t] * feat + f0, ln);
+        x[t] = IO::load(A.z + (int64_t)g[t] * A.z_stride + f0, ln);
         if constexpr (MODE == kGatEdge)
           s[t] = A.el[(int64_t)g[t] * A.heads + h];
         else if constexpr (MODE == kGatNode)
@@ -438,21 +482,22 @@ int launch_gat(const int32_t *pointer, const int32_t *row_of_slot,
                const int32_t *nbr, const float *el, const float *er,
                const void *z, void *out, int64_t n_rows, int64_t n_edges,
                int heads, int dim, float slope, float *ws, hipStream_t stream,
-               size_t ws_bytes = SIZE_MAX, int act = GA_ACT_NONE, size_t *size_only = nullptr) {
+               size_t ws_bytes = SIZE_MAX, int act = GA_ACT_NONE, size_t *size_only = nullptr,
+               int64_t z_stride = 0) {      // 0: rows of z side by side
   // the 16-byte lane layouts of the node forms (every benchmarked shape) get a build per
   // activation; everything else reads it from the arguments
   if constexpr (ACT == kActRuntime && !SPREAD && MODE != kGatEdge && VEC > 1) {
     if (act == GA_ACT_NONE)
       return launch_gat<T, VEC, MODE, SPREAD, GA_ACT_NONE>(pointer, row_of_slot, nbr, el, er, z, out,
                                                            n_rows, n_edges, heads, dim, slope, ws,
-                                                           stream, ws_bytes, act, size_only);
+                                                           stream, ws_bytes, act, size_only, z_stride);
     if (act == GA_ACT_RELU)
       return launch_gat<T, VEC, MODE, SPREAD, GA_ACT_RELU>(pointer, row_of_slot, nbr, el, er, z, out,
                                                            n_rows, n_edges, heads, dim, slope, ws,
-                                                           stream, ws_bytes, act, size_only);
+                                                           stream, ws_bytes, act, size_only, z_stride);
     return launch_gat<T, VEC, MODE, SPREAD, GA_ACT_ELU>(pointer, row_of_slot, nbr, el, er, z, out,
                                                         n_rows, n_edges, heads, dim, slope, ws, stream,
-                                                        ws_bytes, act, size_only);
+                                                        ws_bytes, act, size_only, z_stride);
   }
   if constexpr (GL == 0 && VEC > 1 && MODE != kGatFromZ) {
     // lane groups of eight lanes and more share the columns and the logits they form from
@@ -463,7 +508,7 @@ int launch_gat(const int32_t *pointer, const int32_t *row_of_slot,
 #define GA_GAT_GL(N)                                                                            \
   return launch_gat<T, VEC, MODE, SPREAD, ACT, N>(pointer, row_of_slot, nbr, el, er, z, out,    \
                                                   n_rows, n_edges, heads, dim, slope, ws, stream, \
-                                                  ws_bytes, act, size_only)
+                                                  ws_bytes, act, size_only, z_stride)
     // per-edge rows stream: where they fill the lane group sharing gives nothing (108,368
     // uniform edges, fp32 rows of 128 and 512: 0.95 times the speed; 1 M edges: 1.03 .. 1.08)
     const bool streams = MODE == kGatEdge && !SPREAD && (lanes & (lanes - 1)) == 0;
@@ -477,7 +522,20 @@ int launch_gat(const int32_t *pointer, const int32_t *row_of_slot,
   if (MODE == kGatFromZ &&
       (dim % VEC != 0 || head_lanes > 16 || (head_lanes & (head_lanes - 1)) != 0))
     return GA_EUNSUPPORTED;
-  typename P::Args args{nbr, el, er, (const T *)z, heads, dim, slope, ids_vec, head_lanes, 0, act};
+  if constexpr (GL == 0 && VEC > 1 && MODE == kGatFromZ) {
+#define GA_GAT_GL(N)                                                                            \
+  return launch_gat<T, VEC, MODE, SPREAD, ACT, N>(pointer, row_of_slot, nbr, el, er, z, out,    \
+                                                  n_rows, n_edges, heads, dim, slope, ws, stream, \
+                                                  ws_bytes, act, size_only, z_stride)
+    // the lanes of a head of 8 or 16 lanes form a slot's logit and exponential once (rows
+    // kept apart as ga_gather_row_stride says, against every lane for itself: 4 x 64 bf16 on
+    // 64 M edges, ids shuffled, 4870 -> 4616 us, 3 x 64 4507 -> 3924; uniform 6153 -> 5965)
+    if (head_lanes == 16) GA_GAT_GL(16);
+    if (head_lanes == 8) GA_GAT_GL(8);
+#undef GA_GAT_GL
+  }
+  typename P::Args args{nbr, el, er, (const T *)z, heads, dim, slope, ids_vec, head_lanes, 0, act,
+                        z_stride ? z_stride : (int64_t)heads * dim};
   return launch_runs<P>(args, pointer, row_of_slot, out, n_rows, n_edges,
                         heads * dim, ws, stream, ws_bytes, size_only);
 }
@@ -489,26 +547,27 @@ int gat_aggregate_dispatch(const int32_t *pointer, const int32_t *row_of_slot,
                            const void *z, void *out, int64_t n_rows, int64_t n_edges,
                            int heads, int dim, float slope, int dtype, float *ws,
                            size_t ws_bytes, hipStream_t s, int act = GA_ACT_NONE,
-                           size_t *size_only = nullptr) {
+                           size_t *size_only = nullptr, int64_t z_stride = 0) {
+  // (a stride is whole 16-byte pieces: checked where it comes in)
   const bool vec_ok = aligned(out, 16) && (!z || aligned(z, 16));
   if (dtype == GA_F32) {
     if (vec_ok && dim % 4 == 0)
       return launch_gat<float, 4>(pointer, row_of_slot, nbr, el, er, z, out, n_rows, n_edges,
-                                  heads, dim, slope, ws, s, ws_bytes, act, size_only);
+                                  heads, dim, slope, ws, s, ws_bytes, act, size_only, z_stride);
     if (heads == 1 && dim >= 3 && dim <= 256)   // rows that 16-byte accesses do not tile
       return launch_gat<float, 4, kGatNode, true>(pointer, row_of_slot, nbr, el, er, z, out,
-                                                  n_rows, n_edges, 1, dim, slope, ws, s, ws_bytes, act, size_only);
+                                                  n_rows, n_edges, 1, dim, slope, ws, s, ws_bytes, act, size_only, z_stride);
     return launch_gat<float, 1>(pointer, row_of_slot, nbr, el, er, z, out, n_rows, n_edges,
-                                heads, dim, slope, ws, s, ws_bytes, act, size_only);
+                                heads, dim, slope, ws, s, ws_bytes, act, size_only, z_stride);
   }
   if (vec_ok && dim % 8 == 0)
     return launch_gat<bf16_t, 8>(pointer, row_of_slot, nbr, el, er, z, out, n_rows, n_edges,
-                                 heads, dim, slope, ws, s, ws_bytes, act, size_only);
+                                 heads, dim, slope, ws, s, ws_bytes, act, size_only, z_stride);
   if (heads == 1 && dim >= 3 && dim <= 256)
     return launch_gat<bf16_t, 4, kGatNode, true>(pointer, row_of_slot, nbr, el, er, z, out,
-                                                 n_rows, n_edges, 1, dim, slope, ws, s, ws_bytes, act, size_only);
+                                                 n_rows, n_edges, 1, dim, slope, ws, s, ws_bytes, act, size_only, z_stride);
   return launch_gat<bf16_t, 1>(pointer, row_of_slot, nbr, el, er, z, out, n_rows, n_edges,
-                               heads, dim, slope, ws, s, ws_bytes, act, size_only);
+                               heads, dim, slope, ws, s, ws_bytes, act, size_only, z_stride);
 }
 
 // Argument checks shared by ga_gat_aggregate and ga_gat_aggregate_static
@@ -731,12 +790,11 @@ int ga_gat_aggregate_from_z(const int32_t *pointer, const int32_t *row_of_slot,
                                      workspace_bytes, stream);
 }
 
-int ga_gat_aggregate_from_z_act(const int32_t *pointer, const int32_t *row_of_slot,
-                                const int32_t *nbr, const float *a_l, const float *er,
-                                const void *z, void *out, int64_t n_rows, int64_t n_edges,
-                                int64_t heads, int64_t dim, float slope, int activation,
-                                int dtype, void *workspace, size_t workspace_bytes,
-                                ga_stream_t stream) {
+static int gat_from_z(const int32_t *pointer, const int32_t *row_of_slot, const int32_t *nbr,
+                      const float *a_l, const float *er, const void *z, int64_t z_stride, void *out,
+                      int64_t n_rows, int64_t n_edges, int64_t heads, int64_t dim, float slope,
+                      int activation, int dtype, void *workspace, size_t workspace_bytes,
+                      ga_stream_t stream) {
   if (activation < GA_ACT_NONE || activation > GA_ACT_ELU) return GA_EINVAL;
   if (n_rows < 0 || n_edges < 0 || heads <= 0 || dim <= 0) return GA_EINVAL;
   if (n_rows > 0x7fffffff || n_edges > 0x7fffffff || heads * dim > 0x7fffffff)
@@ -762,15 +820,72 @@ int ga_gat_aggregate_from_z_act(const int32_t *pointer, const int32_t *row_of_sl
   if (dtype == GA_F32) {
     if (vec_ok && dim % 4 == 0)
       return ga::launch_gat<float, 4, ga::kGatFromZ>(pointer, row_of_slot, nbr, a_l, er, z, out,
-                                                     n_rows, n_edges, h, d, slope, ws, s, SIZE_MAX, activation);
+                                                     n_rows, n_edges, h, d, slope, ws, s, SIZE_MAX, activation,
+                                                     nullptr, z_stride);
     return ga::launch_gat<float, 1, ga::kGatFromZ>(pointer, row_of_slot, nbr, a_l, er, z, out,
-                                                   n_rows, n_edges, h, d, slope, ws, s, SIZE_MAX, activation);
+                                                   n_rows, n_edges, h, d, slope, ws, s, SIZE_MAX, activation,
+                                                     nullptr, z_stride);
   }
   if (vec_ok && dim % 8 == 0)
     return ga::launch_gat<ga::bf16_t, 8, ga::kGatFromZ>(pointer, row_of_slot, nbr, a_l, er, z,
-                                                        out, n_rows, n_edges, h, d, slope, ws, s, SIZE_MAX, activation);
+                                                        out, n_rows, n_edges, h, d, slope, ws, s, SIZE_MAX, activation,
+                                                     nullptr, z_stride);
   return ga::launch_gat<ga::bf16_t, 1, ga::kGatFromZ>(pointer, row_of_slot, nbr, a_l, er, z, out,
-                                                      n_rows, n_edges, h, d, slope, ws, s, SIZE_MAX, activation);
+                                                      n_rows, n_edges, h, d, slope, ws, s, SIZE_MAX, activation,
+                                                     nullptr, z_stride);
+}
+
+int ga_gat_aggregate_from_z_act(const int32_t *pointer, const int32_t *row_of_slot,
+                                const int32_t *nbr, const float *a_l, const float *er,
+                                const void *z, void *out, int64_t n_rows, int64_t n_edges,
+                                int64_t heads, int64_t dim, float slope, int activation,
+                                int dtype, void *workspace, size_t workspace_bytes,
+                                ga_stream_t stream) {
+  return gat_from_z(pointer, row_of_slot, nbr, a_l, er, z, 0, out, n_rows, n_edges, heads, dim,
+                    slope, activation, dtype, workspace, workspace_bytes, stream);
+}
+
+// Rows of whole multiples of 256 bytes are kept 128 bytes further apart where their table is
+// larger than an L2.  Graph generators and loaders give popular nodes ids with structure
+// (many zero bits in R-MAT), and with rows a power of two apart those ids' rows meet in a
+// few of the memory channels, which change every 128 bytes.  The fused aggregation, rows
+// side by side -> 128 bytes further apart, us (64 or 256 bytes: slower):
+//   R-MAT, 2.4 M nodes, 64 M edges: 4 x 64 bf16 6259 -> 4472 (4616 with the ids shuffled),
+//     8 x 64 12721 -> 8817, 1 x 64 fp32 3808 -> 2791
+//   R-MAT, 233 k nodes, 11.6 M edges: 1 x 64 fp32 330 -> 262, 4 x 64 bf16 884 -> 747
+//   uniform, the same sizes: 5963 -> 5953, 498 -> 498; 20 k nodes, 400 k edges: level
+int64_t ga_gather_row_stride(int64_t n_rows, int64_t feat, int dtype) {
+  if (n_rows < 0 || feat <= 0 || (dtype != GA_F32 && dtype != GA_BF16)) return 0;
+  const int64_t esz = dtype == GA_F32 ? 4 : 2;
+  return feat * esz % 256 == 0 && n_rows > (4 << 20) / (feat * esz) ? feat + 128 / esz : feat;
+}
+
+int ga_gat_aggregate_strided(const int32_t *pointer, const int32_t *row_of_slot,
+                             const int32_t *nbr, const float *source, const float *er,
+                             const void *z, int64_t z_stride, void *out, int64_t n_rows,
+                             int64_t n_edges, int64_t heads, int64_t dim, float slope, int from_z,
+                             int activation, int dtype, void *workspace, size_t workspace_bytes,
+                             ga_stream_t stream) {
+  if (activation < GA_ACT_NONE || activation > GA_ACT_ELU) return GA_EINVAL;
+  bool nothing = false;
+  const int rc = ga::gat_aggregate_check(pointer, row_of_slot, nbr, source, er, z, out, n_rows,
+                                         n_edges, heads, dim, dtype, &nothing);
+  if (rc != GA_OK || nothing) return rc;
+  const int64_t piece = dtype == GA_F32 ? 4 : 8;
+  if (z_stride < heads * dim) return GA_EINVAL;
+  if (dim % piece || z_stride % piece || !ga::aligned(z, 16) || !ga::aligned(out, 16))
+    return GA_EUNSUPPORTED;
+  if (from_z)
+    return gat_from_z(pointer, row_of_slot, nbr, source, er, z, z_stride, out, n_rows, n_edges,
+                      heads, dim, slope, activation, dtype, workspace, workspace_bytes, stream);
+  if (n_edges > 0 &&
+      (!workspace || !ga::aligned(workspace, 16) ||
+       ga_gat_workspace_bytes(n_edges, heads * dim, heads) > workspace_bytes))
+    return GA_EWORKSPACE;
+  return ga::gat_aggregate_dispatch(pointer, row_of_slot, nbr, source, er, z, out, n_rows, n_edges,
+                                    (int)heads, (int)dim, slope, dtype, (float *)workspace,
+                                    workspace_bytes, (hipStream_t)stream, activation, nullptr,
+                                    z_stride);
 }
 
 }  // extern "C"

@@ -97,7 +97,7 @@ linear_attn_kernel(
     const float *__restrict__ X, const float *__restrict__ W,
     const float *__restrict__ a_l, const float *__restrict__ a_r,
     float *__restrict__ Z, float *__restrict__ el, float *__restrict__ er,
-    const float *__restrict__ row_scale, int64_t rows, int K, int M, int heads) {
+    const float *__restrict__ row_scale, int64_t rows, int K, int M, int heads, int ldz) {
   static_assert(NCB == kCB || !HAS_ATTN, "the attention epilogue pairs up all four column blocks");
   using xvec_t = typename XVec<VK>::type;
   __shared__ __attribute__((aligned(16))) float xs[kWgRows * kXs];   // wave-private rows, one buffer
@@ -279,7 +279,7 @@ linear_attn_kernel(
 #pragma unroll
       for (int cb = 0; cb < NCB; ++cb) {
         const int c = col0 + cb * 16 + lr;
-        if (live && c < M) Z[row * M + c] = acc[t][cb][r];
+        if (live && c < M) Z[row * ldz + c] = acc[t][cb][r];
       }
       if constexpr (HAS_ATTN) {
         // lane-local products, blocks of one head added, then one 16-lane tree
@@ -317,9 +317,10 @@ namespace ga {
 namespace {
 int launch_linear(const float *X, const float *W, const float *a_l, const float *a_r, float *Z,
                   float *el, float *er, const float *row_scale, int64_t rows, int64_t K,
-                  int64_t M, int64_t heads, ga_stream_t stream) {
+                  int64_t M, int64_t heads, int64_t ldz, ga_stream_t stream) {
   if (rows < 0 || K <= 0 || M <= 0 || heads <= 0 || M % heads) return GA_EINVAL;
   if (rows > 0x7fffffff || K > 0x7fffffff || M > 0x7fffffff) return GA_EINVAL;
+  if (ldz < M || ldz > 0x7fffffff) return GA_EINVAL;
   if (rows == 0) return GA_OK;
   if (!X || !W || !Z) return GA_EINVAL;
   // 32-bit byte offsets: 128 rows of K floats, and all of W
@@ -339,7 +340,7 @@ int launch_linear(const float *X, const float *W, const float *a_l, const float 
 #define GA_LAUNCH_LINEAR_NCB(ATTN, VK, WAVES, NCB)                                  \
   hipLaunchKernelGGL((linear_attn_kernel<ATTN, VK, WAVES, NCB>),                   \
                      dim3((unsigned)gx, (unsigned)gy), dim3(kBlock), 0, s, X, W, a_l, a_r, Z, el, \
-                     er, row_scale, rows, (int)K, (int)M, (int)heads)
+                     er, row_scale, rows, (int)K, (int)M, (int)heads, (int)ldz)
 #define GA_LAUNCH_LINEAR(ATTN, VK, WAVES)                           \
   do {                                                              \
     if (!ATTN && M <= 16) GA_LAUNCH_LINEAR_NCB(false, VK, WAVES, 1); \
@@ -378,12 +379,19 @@ extern "C" int ga_linear_attn(const float *X, const float *W, const float *a_l,
                               const float *a_r, float *Z, float *el, float *er,
                               int64_t rows, int64_t K, int64_t M, int64_t heads,
                               ga_stream_t stream) {
-  return ga::launch_linear(X, W, a_l, a_r, Z, el, er, nullptr, rows, K, M, heads, stream);
+  return ga::launch_linear(X, W, a_l, a_r, Z, el, er, nullptr, rows, K, M, heads, M, stream);
+}
+
+extern "C" int ga_linear_attn_strided(const float *X, const float *W, const float *a_l,
+                                      const float *a_r, float *Z, int64_t ldz, float *el,
+                                      float *er, int64_t rows, int64_t K, int64_t M,
+                                      int64_t heads, ga_stream_t stream) {
+  return ga::launch_linear(X, W, a_l, a_r, Z, el, er, nullptr, rows, K, M, heads, ldz, stream);
 }
 
 extern "C" int ga_linear_rows_scaled(const float *X, const float *W, const float *row_scale,
                                      float *Z, int64_t rows, int64_t K, int64_t M,
                                      ga_stream_t stream) {
   return ga::launch_linear(X, W, nullptr, nullptr, Z, nullptr, nullptr, row_scale, rows, K, M, 1,
-                           stream);
+                           M, stream);
 }

@@ -1096,6 +1096,40 @@ int launch_dense_attn(const T *X, const T *W, T *Z, const float *a_l, const floa
 }  // namespace
 }  // namespace ga
 
+namespace ga {
+namespace {
+// bf16, whole groups of 128 columns holding whole heads: one pass over X for all of them;
+// rows of Z ldz elements apart
+int project_wide(const void *X, const void *W, const float *a_l, const float *a_r, void *Z,
+                 int64_t ldz, float *el, float *er, int64_t rows, int64_t K, int64_t M,
+                 int64_t heads, hipStream_t s) {
+  const int64_t dph = M / heads;
+  if (M % kWideGroupCols != 0 || !(dph == 32 || dph == 64 || dph == 128) ||
+      !wide_mm_fits((int)K, (int)(M / kWideGroupCols)))
+    return GA_EUNSUPPORTED;
+  WideMm p = {};
+  p.n_types = 1;
+  p.rows = rows;
+  p.X = (const bf16_t *)X;
+  p.K = (int)K;
+  p.n_groups = (int)(M / kWideGroupCols);
+  p.ldd = heads;
+  p.dph = (int)dph;
+  for (int g = 0; g < p.n_groups; ++g) {
+    p.W[g] = (const bf16_t *)W + g * kWideGroupCols;
+    p.ldw[g] = M;
+    p.Y[g] = (bf16_t *)Z + g * kWideGroupCols;
+    p.ldy[g] = ldz;
+    p.a_l[g] = a_l + g * kWideGroupCols;
+    p.a_r[g] = a_r + g * kWideGroupCols;
+    p.el[g] = el + g * (kWideGroupCols / dph);
+    p.er[g] = er + g * (kWideGroupCols / dph);
+  }
+  return wide_mm_launch(p, s);
+}
+}  // namespace
+}  // namespace ga
+
 extern "C" int ga_project_attn(const void *X, const void *W, const float *a_l,
                                const float *a_r, void *Z, float *el, float *er,
                                int64_t rows, int64_t K, int64_t M, int64_t heads,
@@ -1121,33 +1155,8 @@ extern "C" int ga_project_attn(const void *X, const void *W, const float *a_l,
     return GA_EUNSUPPORTED;
   }
   if ((M & 1) || !aligned(Z, 4)) return GA_EUNSUPPORTED;      // packed bf16 pair stores
-  {
-    // whole groups of 128 columns holding whole heads: one pass over X for all of them
-    const int64_t dph = M / heads;
-    if (M % kWideGroupCols == 0 && (dph == 32 || dph == 64 || dph == 128) &&
-        wide_mm_fits((int)K, (int)(M / kWideGroupCols))) {
-      WideMm p = {};
-      p.n_types = 1;
-      p.rows = rows;
-      p.X = (const bf16_t *)X;
-      p.K = (int)K;
-      p.n_groups = (int)(M / kWideGroupCols);
-      p.ldd = heads;
-      p.dph = (int)dph;
-      for (int g = 0; g < p.n_groups; ++g) {
-        p.W[g] = (const bf16_t *)W + g * kWideGroupCols;
-        p.ldw[g] = M;
-        p.Y[g] = (bf16_t *)Z + g * kWideGroupCols;
-        p.ldy[g] = M;
-        p.a_l[g] = a_l + g * kWideGroupCols;
-        p.a_r[g] = a_r + g * kWideGroupCols;
-        p.el[g] = el + g * (kWideGroupCols / dph);
-        p.er[g] = er + g * (kWideGroupCols / dph);
-      }
-      const int rc = wide_mm_launch(p, s);
-      if (rc != GA_EUNSUPPORTED) return rc;
-    }
-  }
+  const int rc = project_wide(X, W, a_l, a_r, Z, M, el, er, rows, K, M, heads, s);
+  if (rc != GA_EUNSUPPORTED) return rc;
   if (aligned(X, 16) && K % 8 == 0)
     return launch_dense_attn<bf16_t, 32>((const bf16_t *)X, (const bf16_t *)W, (bf16_t *)Z,
                                          a_l, a_r, el, er, rows, (int)K, (int)M, (int)heads, s);
@@ -1155,6 +1164,26 @@ extern "C" int ga_project_attn(const void *X, const void *W, const float *a_l,
     return launch_dense_attn<bf16_t, 16>((const bf16_t *)X, (const bf16_t *)W, (bf16_t *)Z,
                                          a_l, a_r, el, er, rows, (int)K, (int)M, (int)heads, s);
   return GA_EUNSUPPORTED;
+}
+
+extern "C" int ga_project_attn_strided(const void *X, const void *W, const float *a_l,
+                                       const float *a_r, void *Z, int64_t ldz, float *el,
+                                       float *er, int64_t rows, int64_t K, int64_t M,
+                                       int64_t heads, int dtype, ga_stream_t stream) {
+  using namespace ga;
+  if (rows < 0 || K <= 0 || M <= 0 || heads <= 0 || M % heads || ldz < M) return GA_EINVAL;
+  if (dtype != GA_F32 && dtype != GA_BF16) return GA_EINVAL;
+  if (rows > 0x7fffffff || K > 0x7fffffff || M > 0x7fffffff || ldz > 0x7fffffff) return GA_EINVAL;
+  if (rows == 0) return GA_OK;
+  if (!X || !W || !a_l || !a_r || !Z || !el || !er) return GA_EINVAL;
+  const size_t esz = dtype == GA_F32 ? 4 : 2;
+  if (!aligned(X, esz) || !aligned(W, esz) || !aligned(Z, esz) || !aligned(a_l, 4) ||
+      !aligned(a_r, 4) || !aligned(el, 4) || !aligned(er, 4))
+    return GA_EALIGN;
+  if (dtype == GA_F32)
+    return ga_linear_attn_strided((const float *)X, (const float *)W, a_l, a_r, (float *)Z, ldz, el,
+                                  er, rows, K, M, heads, stream);
+  return project_wide(X, W, a_l, a_r, Z, ldz, el, er, rows, K, M, heads, (hipStream_t)stream);
 }
 
 namespace ga {

@@ -88,6 +88,13 @@ def gat_layer(g: DGLGraph, h, fc_weight, attn_weight, heads: int = 1,
     gathered rows instead of gathering them as well.  ``activation`` ("relu" |
     "elu"; the ``F.elu`` between the layers of examples/GAT/GAT.py) is applied by
     the fused pass to the rows it stores, by a separate call otherwise."""
+    if fused and h.is_cuda and fc_weight.dtype == h.dtype and fc_weight.is_contiguous() \
+            and h.is_contiguous() and h.dtype in (torch.float32, torch.bfloat16):
+        out = ops.gat_project_and_aggregate(
+            h, fc_weight, attn_weight[0].float().contiguous(), attn_weight[1].float().contiguous(),
+            g, negative_slope, activation, 4 * g.num_nodes * heads >= SOURCE_TERM_TABLE_LIMIT)
+        if out is not None:
+            return out
     z, el, er = gat_project(h, fc_weight, attn_weight, heads)
     if fused:
         if el.numel() * el.element_size() >= SOURCE_TERM_TABLE_LIMIT:

@@ -937,6 +937,50 @@ def gat_aggregate_from_z(a_l, er, z, graph: DGLGraph, negative_slope: float = 0.
     return out
 
 
+def gat_project_and_aggregate(h, weight, a_l, a_r, graph: DGLGraph, negative_slope: float = 0.01,
+                              activation=None, from_z: bool = False):
+    """``linear_attn`` and ``gat_aggregate`` (``from_z``: ``gat_aggregate_from_z``) with the
+    projected rows kept apart where side by side they would meet in few memory channels
+    (``ga_gather_row_stride``): the layer's z is read by nobody else.  None, nothing launched,
+    where rows lie side by side anyway or the projection does not take the shape."""
+    act = _activation(activation)
+    for name, x in (("h", h), ("weight", weight), ("a_l", a_l), ("a_r", a_r)):
+        _check_input(x, name)
+    dt = _feat_dtype(h, "h")
+    if weight.dtype != h.dtype or h.dim() != 2 or weight.dim() != 2 or weight.shape[0] != h.shape[1]:
+        return None
+    rows, k, m = int(h.shape[0]), int(h.shape[1]), int(weight.shape[1])
+    heads = int(a_l.shape[0])
+    if a_l.dtype != torch.float32 or a_r.dtype != torch.float32 or a_l.numel() != m \
+            or a_r.numel() != m or m % heads or rows != graph.num_nodes:
+        return None
+    lib = capi.load()
+    stride = int(lib.ga_gather_row_stride(rows, m, dt))
+    piece = 4 if dt == capi.GA_F32 else 8
+    dim = m // heads
+    lanes = dim // piece
+    if stride == m or dim % piece or (from_z and (lanes > 16 or lanes & (lanes - 1))):
+        return None
+    z = torch.empty((rows, stride), dtype=h.dtype, device=h.device)
+    el = torch.empty((rows, heads), dtype=torch.float32, device=h.device)
+    er = torch.empty((rows, heads), dtype=torch.float32, device=h.device)
+    rc = lib.ga_project_attn_strided(
+        h.data_ptr(), weight.data_ptr(), a_l.data_ptr(), a_r.data_ptr(), z.data_ptr(), stride,
+        el.data_ptr(), er.data_ptr(), rows, k, m, heads, dt, _stream(h))
+    if rc == capi.GA_EUNSUPPORTED:
+        return None
+    capi.check(rc, "ga_project_attn_strided")
+    out = torch.empty((rows, m), dtype=h.dtype, device=h.device)
+    ws = graph.workspace(lib.ga_gat_workspace_bytes(graph.num_edges, m, heads))
+    capi.check(lib.ga_gat_aggregate_strided(
+        graph.in_pointer.data_ptr(), graph.in_row_of_slot.data_ptr(),
+        graph.in_node_indices.data_ptr(), (a_l if from_z else el).data_ptr(), er.data_ptr(),
+        z.data_ptr(), stride, out.data_ptr(), graph.num_nodes, graph.num_edges, heads, dim,
+        float(negative_slope), int(from_z), act, dt, ws.data_ptr(), ws.numel(), _stream(out)),
+        "ga_gat_aggregate_strided")
+    return out
+
+
 def edge_softmax_sum(logits, messages, graph: DGLGraph) -> torch.Tensor:
     """out[v] = sum over in-edges e of softmax_v(logits)[e] * messages[e]: the
     SegmentSoftmax -> mul -> SpMMEdge tail of the reference's HGT plan

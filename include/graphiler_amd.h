@@ -532,6 +532,21 @@ int ga_gat_aggregate_from_z_act(const int32_t *pointer, const int32_t *row_of_sl
                                 int dtype, void *workspace, size_t workspace_bytes,
                                 ga_stream_t stream);
 
+/* Either form over rows of z that lie z_stride elements apart (from_z: `source` is a_l,
+ * else el): what a layer that writes z for this alone passes between ga_project_attn_strided
+ * and here, with the stride ga_gather_row_stride names (more than the row where rows
+ * are a multiple of 256 bytes and more than an L2 holds: they would meet in few memory
+ * channels).  GA_EUNSUPPORTED, having
+ * launched nothing, unless rows, heads and the stride are whole 16-byte pieces and z and out
+ * 16-byte aligned, and where ga_gat_aggregate_from_z says so. */
+int64_t ga_gather_row_stride(int64_t n_rows, int64_t feat, int dtype);
+int ga_gat_aggregate_strided(const int32_t *pointer, const int32_t *row_of_slot,
+                             const int32_t *nbr, const float *source, const float *er,
+                             const void *z, int64_t z_stride, void *out, int64_t n_rows,
+                             int64_t n_edges, int64_t heads, int64_t dim, float slope, int from_z,
+                             int activation, int dtype, void *workspace, size_t workspace_bytes,
+                             ga_stream_t stream);
+
 /* Dot-product attention over an adjacency, in one pass:
  *   s_i[h]       = <k[nbr[i], h, :], q[qrow[i], h, :]>      for the slots i of row r,
  *   out[r, h, :] = sum_i softmax_r(s)[i, h] * v[nbr[i], h, :],
@@ -663,6 +678,16 @@ int ga_project_attn(const void *X, const void *W, const float *a_l,
                     const float *a_r, void *Z, float *el, float *er,
                     int64_t rows, int64_t K, int64_t M, int64_t heads, int dtype,
                     ga_stream_t stream);
+
+/* ga_linear_attn / ga_project_attn with the rows of Z ldz >= M elements apart (what lies
+ * between them is not written).  ga_project_attn_strided: GA_EUNSUPPORTED, having launched
+ * nothing, for bf16 other than whole groups of 128 columns of heads of 32, 64 or 128. */
+int ga_linear_attn_strided(const float *X, const float *W, const float *a_l, const float *a_r,
+                           float *Z, int64_t ldz, float *el, float *er, int64_t rows, int64_t K,
+                           int64_t M, int64_t heads, ga_stream_t stream);
+int ga_project_attn_strided(const void *X, const void *W, const float *a_l, const float *a_r,
+                            void *Z, int64_t ldz, float *el, float *er, int64_t rows, int64_t K,
+                            int64_t M, int64_t heads, int dtype, ga_stream_t stream);
 
 #ifdef __cplusplus
 }
