@@ -111,7 +111,7 @@ struct GatPolicy {
     int head_lanes; // kGatFromZ: lanes that share a head (dph / VEC)
     int stride_shift;   // SPREAD: log2 of the lanes per group, set by the launcher
     int act;            // GA_ACT_*: applied to the finished row before it is stored
-    int64_t z_stride;   // elements from a row of z to the next
+    int z_stride;       // elements from a row of z to the next
   };
   static __device__ __forceinline__ void init(float (&st)[VEC + 2]) {
 #pragma unroll
@@ -483,7 +483,7 @@ int launch_gat(const int32_t *pointer, const int32_t *row_of_slot,
                const void *z, void *out, int64_t n_rows, int64_t n_edges,
                int heads, int dim, float slope, float *ws, hipStream_t stream,
                size_t ws_bytes = SIZE_MAX, int act = GA_ACT_NONE, size_t *size_only = nullptr,
-               int64_t z_stride = 0) {      // 0: rows of z side by side
+               int z_stride = 0) {      // 0: rows of z side by side
   // the 16-byte lane layouts of the node forms (every benchmarked shape) get a build per
   // activation; everything else reads it from the arguments
   if constexpr (ACT == kActRuntime && !SPREAD && MODE != kGatEdge && VEC > 1) {
@@ -535,7 +535,7 @@ int launch_gat(const int32_t *pointer, const int32_t *row_of_slot,
 #undef GA_GAT_GL
   }
   typename P::Args args{nbr, el, er, (const T *)z, heads, dim, slope, ids_vec, head_lanes, 0, act,
-                        z_stride ? z_stride : (int64_t)heads * dim};
+                        z_stride ? z_stride : heads * dim};
   return launch_runs<P>(args, pointer, row_of_slot, out, n_rows, n_edges,
                         heads * dim, ws, stream, ws_bytes, size_only);
 }
@@ -547,7 +547,7 @@ int gat_aggregate_dispatch(const int32_t *pointer, const int32_t *row_of_slot,
                            const void *z, void *out, int64_t n_rows, int64_t n_edges,
                            int heads, int dim, float slope, int dtype, float *ws,
                            size_t ws_bytes, hipStream_t s, int act = GA_ACT_NONE,
-                           size_t *size_only = nullptr, int64_t z_stride = 0) {
+                           size_t *size_only = nullptr, int z_stride = 0) {
   // (a stride is whole 16-byte pieces: checked where it comes in)
   const bool vec_ok = aligned(out, 16) && (!z || aligned(z, 16));
   if (dtype == GA_F32) {
@@ -791,7 +791,7 @@ int ga_gat_aggregate_from_z(const int32_t *pointer, const int32_t *row_of_slot,
 }
 
 static int gat_from_z(const int32_t *pointer, const int32_t *row_of_slot, const int32_t *nbr,
-                      const float *a_l, const float *er, const void *z, int64_t z_stride, void *out,
+                      const float *a_l, const float *er, const void *z, int z_stride, void *out,
                       int64_t n_rows, int64_t n_edges, int64_t heads, int64_t dim, float slope,
                       int activation, int dtype, void *workspace, size_t workspace_bytes,
                       ga_stream_t stream) {
@@ -872,11 +872,11 @@ int ga_gat_aggregate_strided(const int32_t *pointer, const int32_t *row_of_slot,
                                          n_edges, heads, dim, dtype, &nothing);
   if (rc != GA_OK || nothing) return rc;
   const int64_t piece = dtype == GA_F32 ? 4 : 8;
-  if (z_stride < heads * dim) return GA_EINVAL;
+  if (z_stride < heads * dim || z_stride > 0x7fffffff) return GA_EINVAL;
   if (dim % piece || z_stride % piece || !ga::aligned(z, 16) || !ga::aligned(out, 16))
     return GA_EUNSUPPORTED;
   if (from_z)
-    return gat_from_z(pointer, row_of_slot, nbr, source, er, z, z_stride, out, n_rows, n_edges,
+    return gat_from_z(pointer, row_of_slot, nbr, source, er, z, (int)z_stride, out, n_rows, n_edges,
                       heads, dim, slope, activation, dtype, workspace, workspace_bytes, stream);
   if (n_edges > 0 &&
       (!workspace || !ga::aligned(workspace, 16) ||
@@ -885,7 +885,7 @@ int ga_gat_aggregate_strided(const int32_t *pointer, const int32_t *row_of_slot,
   return ga::gat_aggregate_dispatch(pointer, row_of_slot, nbr, source, er, z, out, n_rows, n_edges,
                                     (int)heads, (int)dim, slope, dtype, (float *)workspace,
                                     workspace_bytes, (hipStream_t)stream, activation, nullptr,
-                                    z_stride);
+                                    (int)z_stride);
 }
 
 }  // extern "C"
