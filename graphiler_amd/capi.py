@@ -59,6 +59,7 @@ SIGNATURES = {
     "ga_sddmm_bcast": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _int, _int, _vp, _vp, _i64, _i64,
                               _i64, _i64, _int, _vp]),
     "ga_sddmm_u_op_v_adj": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
+    "ga_sddmm_u_dot_v_adj": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
     "ga_typed_tile_rows": (_i64, [_i64]),
     "ga_typed_tiles_chunk_capacity": (_i64, [_i64, _i64, _i64, _i64]),
     "ga_typed_tiles_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),

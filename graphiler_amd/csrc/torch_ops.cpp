@@ -757,6 +757,18 @@ torch::Tensor u_dot_v(torch::Tensor src_feature, torch::Tensor dst_feature,
   const int64_t dim = src_feature.size(src_feature.dim() - 1);
   torch::Tensor out = torch::empty({graph->num_edges, heads},
                                    src_feature.options().dtype(at::kFloat));
+  if (graph->num_edges >= (1 << 15)) {     // from there the walk over the adjacency is faster
+    const auto side = graph->side(false);
+    const int rc = ga_sddmm_u_dot_v_adj(
+        side.rows.data_ptr<int>(), graph->in_node_indices.data_ptr<int>(),
+        side.identity ? nullptr : graph->in_edge_indices.data_ptr<int>(), src_feature.data_ptr(),
+        dst_feature.data_ptr(), out.data_ptr<float>(), graph->num_edges, heads, dim, dt,
+        current_stream(out));
+    if (rc != GA_EUNSUPPORTED) {           // else: the two-column kernel
+      check_ga(rc, "ga_sddmm_u_dot_v_adj");
+      return out;
+    }
+  }
   const EdgeColumns c = edge_columns(graph);
   check_ga(ga_sddmm_u_dot_v(c.lhs, c.rhs, c.bits, src_feature.data_ptr(),
                             dst_feature.data_ptr(), out.data_ptr<float>(),

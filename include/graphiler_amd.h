@@ -226,6 +226,13 @@ int ga_sddmm_u_op_v(const void *lhs, const void *rhs, int idx_bits,
                     const void *u, const void *v, float *out, int64_t n_edges,
                     int64_t feat, int op, int dtype, ga_stream_t stream);
 
+/* ga_sddmm_u_dot_v over a grouped adjacency: out[eid[i], h] = <u[nbr[i], h, :], v[row(i), h, :]>
+ * for every slot i (eid NULL: i).  GA_EUNSUPPORTED unless u and v are 16-byte aligned, a
+ * row is 5 to 64 16-byte pieces and a head 1, 2, 4, 8 or 16 of them. */
+int ga_sddmm_u_dot_v_adj(const int32_t *row_of_slot, const int32_t *nbr, const int32_t *eid,
+                         const void *u, const void *v, float *out, int64_t n_edges, int64_t heads,
+                         int64_t dim, int dtype, ga_stream_t stream);
+
 /* The same operators over a grouped adjacency, for graphs whose edge ids are slot
  * numbers (eid[i] == i, e.g. edges stored by destination): out[i, k] =
  * u[nbr[i], k] (op) v[row(i), k] for every slot i, i.e. the reference's
