@@ -975,7 +975,10 @@ def gat_project_and_aggregate(h, weight, a_l, a_r, graph: DGLGraph, negative_slo
     lanes = dim // piece
     if stride == m or dim % piece or (from_z and (lanes > 16 or lanes & (lanes - 1))):
         return None
-    z = torch.empty((rows, stride), dtype=h.dtype, device=h.device)
+    try:
+        z = torch.empty((rows, stride), dtype=h.dtype, device=h.device)
+    except torch.OutOfMemoryError:       # the rows side by side may still fit
+        return None
     el = torch.empty((rows, heads), dtype=torch.float32, device=h.device)
     er = torch.empty((rows, heads), dtype=torch.float32, device=h.device)
     rc = lib.ga_project_attn_strided(
@@ -984,12 +987,19 @@ def gat_project_and_aggregate(h, weight, a_l, a_r, graph: DGLGraph, negative_slo
     if rc == capi.GA_EUNSUPPORTED:
         return None
     capi.check(rc, "ga_project_attn_strided")
-    out = torch.empty((rows, m), dtype=h.dtype, device=h.device)
-    ws = graph.workspace(lib.ga_gat_workspace_bytes(graph.num_edges, m, heads))
+    return _aggregate_rows(a_l if from_z else el, er, z, m, heads, graph, negative_slope, act, dt, from_z)
+
+
+def _aggregate_rows(source, er, z, feat: int, heads: int, graph: DGLGraph, negative_slope: float,
+                    act: int, dt: int, from_z: bool) -> torch.Tensor:
+    """The fused aggregation over the first ``feat`` values of every row of z."""
+    out = torch.empty((int(z.shape[0]), feat), dtype=z.dtype, device=z.device)
+    lib = capi.load()
+    ws = graph.workspace(lib.ga_gat_workspace_bytes(graph.num_edges, feat, heads))
     capi.check(lib.ga_gat_aggregate_strided(
         graph.in_pointer.data_ptr(), graph.in_row_of_slot.data_ptr(),
-        graph.in_node_indices.data_ptr(), (a_l if from_z else el).data_ptr(), er.data_ptr(),
-        z.data_ptr(), stride, out.data_ptr(), graph.num_nodes, graph.num_edges, heads, dim,
+        graph.in_node_indices.data_ptr(), source.data_ptr(), er.data_ptr(), z.data_ptr(),
+        int(z.shape[1]), out.data_ptr(), graph.num_nodes, graph.num_edges, heads, feat // heads,
         float(negative_slope), int(from_z), act, dt, ws.data_ptr(), ws.numel(), _stream(out)),
         "ga_gat_aggregate_strided")
     return out
