@@ -135,38 +135,47 @@ struct Block<bf16_t, D> {
   }
 };
 
-// x = p0 + p1 + p2 exactly, each piece a bf16 (the top eight significant bits of what the
-// pieces before it leave), packed in pairs.  What is not finite stays in p0, with NaN in the
-// others.
+// x = p0 + p1 / 2^8 + p2 / 2^16 exactly for every finite x, each piece a bf16 rounded to
+// nearest from what the pieces before it leave, packed in pairs.  Rounded, the pieces and what
+// a product of them leaves out have either sign (cut off, all have that of x); scaled, they
+// stay in bf16's range as long as x does in float's (side by side the third leaves it below
+// 2^-110).  The first two stop at the largest bf16, which the values next to the largest
+// float round past.  An x that is not finite leaves a third piece that is not.
 template <int N>
 __device__ __forceinline__ void split(const float (&x)[N], uint32_t (&p)[3][N / 2]) {
+  constexpr float kMost = 0x1.fep127f;
 #pragma unroll
   for (int j = 0; j < N; j += 2) {
-    float lo = __builtin_canonicalizef(x[j]), hi = __builtin_canonicalizef(x[j + 1]);
+    float lo = x[j], hi = x[j + 1];
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const uint32_t a = __float_as_uint(lo), b = __float_as_uint(hi);
-      p[q][j / 2] = __builtin_amdgcn_perm(b, a, 0x07060302u);       // the upper halves
-      lo -= __uint_as_float(a & 0xffff0000u);
-      hi -= __uint_as_float(b & 0xffff0000u);
+    for (int q = 0; q < 2; ++q) {
+      const uint32_t w = pack_bf16(__builtin_amdgcn_fmed3f(lo, -kMost, kMost),
+                                   __builtin_amdgcn_fmed3f(hi, -kMost, kMost));
+      p[q][j / 2] = w;
+      lo = (lo - bf16_lo(w)) * 256.0f;
+      hi = (hi - bf16_hi(w)) * 256.0f;
     }
+    p[2][j / 2] = pack_bf16(lo, hi);
   }
 }
+constexpr float kPieceScale = 1.0f / 256.0f;
 // the value of three pieces
 __device__ __forceinline__ float joined(bf16_t p0, bf16_t p1, bf16_t p2) {
-  const float x = bf16_lo(p0);
-  return fabsf(x) < INFINITY ? x + (bf16_lo(p1) + bf16_lo(p2)) : x;
+  return fmaf(fmaf(bf16_lo(p2), kPieceScale, bf16_lo(p1)), kPieceScale, bf16_lo(p0));
 }
 
 // Heads of 32 and 64 of rows of 64 fp32 features: the product on the bf16 instruction, at 16
-// times the fp32 one's rate.  Operands are split into three bf16 pieces, and six piece
-// products of weight >= 2^-16 are added in fp32, small ones first (the three left out are
-// below 2^-24 of |x||w|).  The tile's rows are kept split, three planes of 64 values side by
-// side: split when an operand is read, every value would be split by every wavefront.  The
-// matrices come split and in the order the lanes read them (pair_weights_kernel).
-// Messages of 1.2 M edges in 0.62 M pairs against float64, 2-norm / largest: heads of 64
-// 1.59e-7 / 4.57e-7 on the fp32 instruction, 1.26e-7 / 2.64e-7 here, heads of 32 1.16e-7 /
-// 2.55e-7 and 0.87e-7 / 1.69e-7.
+// times the fp32 one's rate.  Operands are split into three bf16 pieces; six piece products
+// are added in fp32, those of one weight (1, 2^-8, 2^-16) in an accumulator of their own.  The
+// three left out are together below 2^-24 of |x||w|.  The tile's rows are kept split, three
+// planes of 64 values side by side: split when an operand is read, every value would be split
+// by every wavefront.  The matrices come split and in the order the lanes read them
+// (pair_weights_kernel).  Messages of 1.2 M edges in 0.53 M pairs against float64, 2-norm /
+// largest, on the fp32 instruction and here: heads of 64 1.63e-7 / 3.8e-7 and 0.71e-7 / 1.5e-7,
+// of 32 1.20e-7 / 3.1e-7 and 0.61e-7 / 1.2e-7, heads of 64 of values in [0, 1) 1.19e-7 / 4.9e-7
+// and 0.57e-7 / 2.1e-7.  (Pieces cut off at eight bits and added in one accumulator: 1.30e-7 /
+// 4.7e-7, and up to 7.8 x 2^-24 of |x||w| left out; 636 us instead of 640 for the operator on
+// 1.95 M pairs, 1 x 64.)
 template <int D>
 struct SplitBlock {
   static constexpr int KB = D / 32;
@@ -182,8 +191,7 @@ struct SplitBlock {
   }
   // row: planes of 64 values
   __device__ __forceinline__ floatx4 mma(const bf16_t *row, int k0, int lk) const {
-    floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    constexpr int px[6] = {2, 1, 0, 1, 0, 0}, pw[6] = {0, 1, 2, 0, 1, 0};
+    floatx4 acc[3] = {};
 #pragma unroll
     for (int b = 0; b < KB; ++b) {
       uint4 x[3];
@@ -191,12 +199,18 @@ struct SplitBlock {
       for (int q = 0; q < 3; ++q)
         x[q] = *reinterpret_cast<const uint4 *>(row + 64 * q + k0 + 32 * b + 8 * lk);
 #pragma unroll
-      for (int i = 0; i < 6; ++i)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x[px[i]]),
-                                                      __builtin_bit_cast(bf16x8, w[b][pw[i]]),
-                                                      acc, 0, 0, 0);
+      for (int px = 0; px < 3; ++px)
+#pragma unroll
+        for (int pw = 0; pw < 3 - px; ++pw)
+          acc[px + pw] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8, x[px]), __builtin_bit_cast(bf16x8, w[b][pw]), acc[px + pw],
+              0, 0, 0);
     }
-    return acc;
+    floatx4 sum;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      sum[i] = fmaf(fmaf(acc[2][i], kPieceScale, acc[1][i]), kPieceScale, acc[0][i]);
+    return sum;
   }
   // the same product on the fp32 instruction, for operands that are not finite: their pieces
   // give NaN where fp32 products may give inf

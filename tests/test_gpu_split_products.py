@@ -1,10 +1,12 @@
 """fp32 products of the pair attention on the bf16 instruction (heads of 32 and 64 of 64
-features): the rows of a tile that no pair owns."""
+features): operands whose pieces do not cancel or lie far down in float's range, and the rows
+of a tile that no pair owns."""
 import numpy as np
 import pytest
 import torch
 
 from graphiler_amd import capi, prepare_graph
+from test_gpu_pair_attention import _by_pair
 
 pytestmark = pytest.mark.gpu
 
@@ -28,6 +30,48 @@ def _tiles_pass(g, k, q, v, att, msg):
         lse.data_ptr(), pairs.num_pairs, g.num_nodes, pairs.max_slots, heads, d, capi.GA_F32, stream),
         "tiles")
     return m, lse
+
+
+def _bits(word, *shape):
+    return torch.full(shape, word, dtype=torch.int32).view(torch.float32)
+
+
+@pytest.mark.parametrize("heads,d", [(1, 64), (2, 32)])
+@pytest.mark.parametrize("values", ["cut", "near_one", "one_sign", "both_signs", "small", "tiny", "large"])
+def test_products_against_float64(device, heads, d, values):
+    """Pairs of one slot: the softmax weight is 1, the message is v @ M alone.  No sum is
+    further from float64 than 2^-22 of the sum of its products' sizes: the products left out are
+    below 2^-24 of theirs, the others are added in fp32 (the fp32 instruction's own 16 dependent
+    sums are up to 6.2 x 2^-24 off on products of one sign).  Pieces that were cut off instead
+    of rounded left out up to 7.8 x 2^-24, all of one sign, and third pieces out of bf16's range
+    476 x 2^-24."""
+    rng = np.random.default_rng(7)
+    types, n = 3, 130
+    dst = np.concatenate([np.arange(n), np.arange(64), np.arange(5)])
+    et = np.repeat(np.arange(types), [n, 64, 5])
+    g = prepare_graph(rng.integers(0, n, dst.size), dst, n, device=device, etype_of=et, num_etypes=types)
+    normal = lambda *s: torch.from_numpy(rng.standard_normal(s, dtype=np.float32))
+    v, msg = normal(n, heads * d), normal(types, heads, d, d)
+    if values == "cut":                    # the most that cutting a significand in three loses
+        v, msg = _bits(0x3f80ffff, n, heads * d), _bits(0x3f80ffff, types, heads, d, d)
+    elif values == "near_one":             # significands around 1 + 2^-7
+        v, msg = (1 + 2.0 ** -7 + 2.0 ** -8 * torch.sigmoid(x) for x in (v, msg))
+    elif values == "one_sign":
+        v, msg = v.abs(), msg.abs()
+    elif values == "small":
+        v = v * 2.0 ** -112
+    elif values == "tiny":
+        v, msg = v * 2.0 ** -118, msg * 2.0 ** 20
+    elif values == "large":                # next to the largest float and what rounds past bf16's
+        v, msg = _bits(0x7f7fffff, n, heads * d) * torch.sign(v), msg * 2.0 ** -20
+    q, k = normal(n, heads * d) / d, normal(n, heads * d)
+    att = normal(types, heads, d, d) / d ** 0.5
+    m, _ = _tiles_pass(g, *(x.to(device) for x in (k, q, v, att, msg)))
+    ref, _ = _by_pair(g, *(x.to(device) for x in (k, q, v, att, msg)))
+    size, _ = _by_pair(g, *(x.to(device) for x in (k, q, v.abs(), att, msg.abs())))
+    at = g.relation_pairs().by_type.cpu()
+    err = (m.cpu().double() - ref[at]).abs() / size[at]
+    assert float(err.max()) < 2.0 ** -22, f"{values}: {float(err.max()) * 2 ** 24:.2f} x 2^-24"
 
 
 @pytest.mark.parametrize("heads,d", [(1, 64), (2, 32)])
