@@ -42,6 +42,7 @@ SIGNATURES = {
     "ga_spmm_csr_scaled": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64,
                                   _int, _int, _vp, _sz, _vp]),
     "ga_spmm_source_classes": (_i64, [_vp, _vp, _i64, _i64, _i64, _int]),
+    "ga_degree_buckets": (_int, [_vp, _i64, _vp, _vp]),
     "ga_source_classes_workspace_bytes": (_sz, [_i64, _i64]),
     "ga_source_classes_build": (_int, [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _sz, _vp]),
     "ga_spmm_classes_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),

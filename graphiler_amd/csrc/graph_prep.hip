@@ -181,6 +181,26 @@ __global__ __launch_bounds__(kBlock) void class_scatter_kernel(
   }
 }
 
+// Rows and their items by the power of two below a row's length: integers, so the order in
+// which the workgroups add them does not matter.
+__global__ __launch_bounds__(kBlock) void degree_buckets_kernel(
+    const int32_t *__restrict__ pointer, int64_t n_rows, unsigned long long *__restrict__ buckets) {
+  __shared__ unsigned long long all[2 * GA_DEGREE_BUCKETS];
+  if (threadIdx.x < 2 * GA_DEGREE_BUCKETS) all[threadIdx.x] = 0;
+  __syncthreads();
+  for (int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x; v < n_rows;
+       v += (int64_t)gridDim.x * kBlock) {
+    const int32_t d = pointer[v + 1] - pointer[v];
+    if (d <= 0) continue;
+    const int b = 31 - __clz(d);
+    atomicAdd(&all[b], 1ull);
+    atomicAdd(&all[GA_DEGREE_BUCKETS + b], (unsigned long long)d);
+  }
+  __syncthreads();
+  if (threadIdx.x < 2 * GA_DEGREE_BUCKETS && all[threadIdx.x])
+    atomicAdd(&buckets[threadIdx.x], all[threadIdx.x]);
+}
+
 inline size_t round_up(size_t v) { return (v + 255) & ~(size_t)255; }
 
 struct PrepLayout {
@@ -267,6 +287,20 @@ int ga_group_edges(const int64_t *key, const int64_t *other, int64_t n_keys,
     hipLaunchKernelGGL(gather_other_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, other,
                        eid, n_items, nbr);
   }
+  return launch_status();
+}
+
+int ga_degree_buckets(const int32_t *pointer, int64_t n_rows, int64_t *buckets, ga_stream_t stream) {
+  using namespace ga;
+  if (n_rows < 0 || n_rows > 0x7ffffffe || !buckets || (n_rows > 0 && !pointer)) return GA_EINVAL;
+  if (!aligned(buckets, 8) || !aligned(pointer, 4)) return GA_EALIGN;
+  hipStream_t s = (hipStream_t)stream;
+  hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(kBlock), 0, s, (int32_t *)buckets,
+                     (int64_t)(4 * GA_DEGREE_BUCKETS));
+  const int64_t blocks = (n_rows + kBlock - 1) / kBlock;
+  if (blocks > 0)
+    hipLaunchKernelGGL(degree_buckets_kernel, dim3((unsigned)(blocks < 1024 ? blocks : 1024)),
+                       dim3(kBlock), 0, s, pointer, n_rows, (unsigned long long *)buckets);
   return launch_status();
 }
 

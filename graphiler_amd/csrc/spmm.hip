@@ -1137,18 +1137,23 @@ int64_t ga_spmm_source_classes(const int64_t *nodes_of_degree, const int64_t *ed
   if (feat % (half ? 8 : 4) || n_rows > 0x7ffffffe / 8 || n_edges < 16 * n_rows ||
       (double)n_rows * row <= ga::kL2Bytes)
     return 0;
-  if (!nodes_of_degree || !edges_of_degree) return 1;      // worth counting the degrees
   const double gb = 1e-9 * (double)n_edges * (row < 128 ? 128 : row);
+  const double hit = half ? 62.0 : 45.0, missed = half ? 72.0 : 90.0;
+  auto partial_rows = [&](int64_t classes) {
+    return 450e-9 * (double)(classes * n_rows) * (double)feat * 4 + 4.0;
+  };
+  if (!nodes_of_degree || !edges_of_degree)       // the most that two classes could give
+    return gb * hit + partial_rows(2) < gb * (hit + missed) / 1.06;
   auto gathers = [&](int64_t classes) {                    // us
     const double miss = 1.0 - ga::cached_share(nodes_of_degree, edges_of_degree,
                                                (double)classes * ga::kL2Bytes / row);
-    return gb * (half ? 62.0 + 72.0 * pow(miss, 1.4) : 45.0 + 90.0 * pow(miss, 1.4));
+    return gb * (hit + missed * pow(miss, 1.4));
   };
   const double plain = gathers(1);
   double best = plain / 1.06;
   int64_t classes = 0;
   for (int64_t k = 2; k <= 8; k *= 2) {
-    const double t = gathers(k) + 450e-9 * (double)(k * n_rows) * (double)feat * 4 + 4.0;
+    const double t = gathers(k) + partial_rows(k);
     if (t < best) {
       best = t;
       classes = k;

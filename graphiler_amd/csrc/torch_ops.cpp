@@ -294,13 +294,11 @@ struct DGLGraph : torch::CustomClassHolder {
     if (it == class_count_.end()) {
       if (capturing) return {};
       if (source_degrees_.empty()) {
-        torch::Tensor deg = torch::diff(out_pointer);
-        deg = deg.index({deg.gt(0)}).to(at::kDouble);
-        const torch::Tensor bucket = torch::log2(deg).floor().to(at::kLong);
-        const torch::Tensor both =
-            torch::stack({torch::bincount(bucket, {}, GA_DEGREE_BUCKETS).to(at::kDouble),
-                          torch::bincount(bucket, deg, GA_DEGREE_BUCKETS)})
-                .to(at::kLong).cpu().contiguous();
+        torch::Tensor both = torch::empty({2 * GA_DEGREE_BUCKETS}, in_pointer.options().dtype(at::kLong));
+        check_ga(ga_degree_buckets(out_pointer.data_ptr<int>(), num_nodes, both.data_ptr<int64_t>(),
+                                   current_stream(in_pointer)),
+                 "ga_degree_buckets");
+        both = both.cpu();
         const int64_t *p = both.data_ptr<int64_t>();
         source_degrees_.assign(p, p + 2 * GA_DEGREE_BUCKETS);
       }

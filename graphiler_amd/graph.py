@@ -222,12 +222,11 @@ class DGLGraph:
     def _source_degrees(self):
         """(nodes, edges) by the power of two below the out-degree, as host int64 arrays."""
         if "source_degrees" not in self._cache:
-            deg = torch.diff(self.out_pointer)
-            deg = deg[deg > 0].double()
-            bucket = torch.log2(deg).floor().long()
-            both = torch.stack([torch.bincount(bucket, minlength=capi.GA_DEGREE_BUCKETS).double(),
-                                torch.bincount(bucket, deg, minlength=capi.GA_DEGREE_BUCKETS)])
-            self._cache["source_degrees"] = both.long().cpu().numpy()
+            both = torch.empty((2, capi.GA_DEGREE_BUCKETS), dtype=torch.int64, device=self.device)
+            capi.check(capi.load().ga_degree_buckets(
+                self.out_pointer.data_ptr(), self.num_nodes, both.data_ptr(),
+                torch.cuda.current_stream(self.device).cuda_stream), "ga_degree_buckets")
+            self._cache["source_degrees"] = both.cpu().numpy()
         return self._cache["source_degrees"]
 
     def source_classes(self, feat: int, dtype: int) -> Optional["SourceClasses"]:

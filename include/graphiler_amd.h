@@ -145,7 +145,9 @@ int ga_spmm_csr_scaled(const int32_t *pointer, const int32_t *row_of_slot,
  * dense graphs whose table exceeds an L2.  ga_spmm_source_classes (host arithmetic): the
  * classes to use, 0 where ga_spmm_csr[_scaled] is the faster call; from the nodes with
  * out-degrees 2^b .. 2^(b+1) - 1 and their edges, b < GA_DEGREE_BUCKETS (host arrays;
- * NULL: 0 if the answer is 0 whatever they hold, else 1).  ga_source_classes_build (once per graph
+ * NULL: 0 if the answer is 0 whatever they hold, else 1).  ga_degree_buckets counts both on
+ * the device from a row pointer: buckets (2 * GA_DEGREE_BUCKETS) int64, 8-byte aligned, rows
+ * before items.  ga_source_classes_build (once per graph
  * and number of classes; 2, 4 or 8) partitions the in-adjacency:
  *   pointer  (n_classes * n_rows + 1) int32    rows  (n_edges) int32: class * n_rows + row
  *   nbr_out  (n_edges) int32: source of the slot
@@ -157,6 +159,7 @@ int ga_spmm_csr_scaled(const int32_t *pointer, const int32_t *row_of_slot,
 #define GA_DEGREE_BUCKETS 31
 int64_t ga_spmm_source_classes(const int64_t *nodes_of_degree, const int64_t *edges_of_degree,
                                int64_t n_rows, int64_t n_edges, int64_t feat, int dtype);
+int ga_degree_buckets(const int32_t *pointer, int64_t n_rows, int64_t *buckets, ga_stream_t stream);
 size_t ga_source_classes_workspace_bytes(int64_t n_edges, int64_t n_classes);
 int ga_source_classes_build(const int32_t *row_of_slot, const int32_t *nbr, int64_t n_rows,
                             int64_t n_edges, int64_t n_classes, int32_t *pointer, int32_t *rows,

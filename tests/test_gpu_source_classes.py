@@ -157,3 +157,35 @@ def test_boundary_operators_take_the_order_where_it_is_faster():
     assert torch.equal(torch.ops.my_ops.SpMMScaled(x, scale, capi.GA_ACT_RELU, False, t),
                        ops.spmm_scaled(x, g, scale, "relu"))
     assert g.source_classes(64, capi.GA_F32).num_classes > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lengths", [[1], [0, 0, 0], [1, 2, 3, 4, 7, 8, 0, 255, 256, 2 ** 20 + 1],
+                                     list(range(257)), [2 ** 31 - 1], [3] * 300_001])
+def test_degrees_counted_on_the_device(lengths):
+    deg = np.asarray(lengths, np.int64)
+    pointer = torch.from_numpy(np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)).cuda()
+    out = torch.full((2, capi.GA_DEGREE_BUCKETS), -1, dtype=torch.int64, device="cuda")
+    capi.check(capi.load().ga_degree_buckets(pointer.data_ptr(), deg.size, out.data_ptr(),
+                                             torch.cuda.current_stream().cuda_stream), "buckets")
+    nodes, edges = _degrees(deg)
+    assert (out.cpu().numpy() == np.stack([nodes, edges])).all()
+
+
+@pytest.mark.gpu
+def test_sums_of_dense_graphs_under_deterministic_algorithms():
+    """Counting the degrees asks torch for nothing it refuses there."""
+    from graphiler_amd import torch_boundary
+    torch_boundary.load()
+    g = _graph(40_000, 6_000_000, 7)
+    t = torch_boundary.script_graph(g)
+    x = torch.randn(40_000, 64, device="cuda")
+    torch.use_deterministic_algorithms(True)
+    try:
+        out = ops.SpMMSrc(x, [1], False, None, g)
+        same = torch.ops.my_ops.SpMMSrc(x, [1], False, None, t)
+    finally:
+        torch.use_deterministic_algorithms(False)
+    assert g.source_classes(64, capi.GA_F32).num_classes > 0
+    assert torch.equal(out, same)
+    assert bool(((out.double() - _sum64(g, x)).abs() <= _sum64(g, x.abs()) * (64 * 2.0 ** -24)).all())
