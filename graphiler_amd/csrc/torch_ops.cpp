@@ -282,6 +282,7 @@ struct DGLGraph : torch::CustomClassHolder {
   struct SourceClasses {
     int64_t num_classes = 0;           // 0: the plain sum
     torch::Tensor pointer, rows, nbr;  // int32
+    bool used = false;                 // handed to a launch
   };
   SourceClasses source_classes(int64_t feat, int dtype) {
     if (!ga_spmm_source_classes(nullptr, nullptr, num_nodes, num_edges, feat, dtype)) return {};
@@ -334,6 +335,19 @@ struct DGLGraph : torch::CustomClassHolder {
     }
     return at->second;
   }
+  // What became of the scratch of such a sum.  Where it does not fit, that width takes the
+  // plain sum from then on, and a layout that no launch has read is given back; one that has
+  // been read stays, a recorded HIP graph may replay launches over it.
+  void source_classes_scratch(int64_t feat, int dtype, int64_t classes, bool fits) {
+    std::lock_guard<std::mutex> lock(mu_);
+    const auto at = classes_.find(classes);
+    if (fits) {
+      if (at != classes_.end()) at->second.used = true;
+      return;
+    }
+    class_count_[std::make_pair(feat, dtype)] = 0;
+    if (at != classes_.end() && !at->second.used) classes_.erase(at);
+  }
   // Scratch shared by the operators called on this graph: calls that use it must be
   // ordered on one stream (two streams working on one graph object race on it).  It
   // grows on demand; a buffer that was handed out is never freed while the graph
@@ -376,8 +390,10 @@ bool sum_by_classes(const GraphPtr &g, const torch::Tensor &u, torch::Tensor &ou
   try {
     ws = g->workspace(ga_spmm_classes_workspace_bytes(g->num_nodes, g->num_edges, feat, c.num_classes));
   } catch (const c10::OutOfMemoryError &) {
+    g->source_classes_scratch(feat, dt, c.num_classes, false);
     return false;
   }
+  if (!c.used) g->source_classes_scratch(feat, dt, c.num_classes, true);
   check_ga(ga_spmm_classes(c.pointer.data_ptr<int>(), c.rows.data_ptr<int>(), c.nbr.data_ptr<int>(),
                            u.data_ptr(), out.data_ptr(), row_scale, activation, g->num_nodes,
                            g->num_edges, feat, c.num_classes, dt, ws.data_ptr(),

@@ -261,6 +261,14 @@ class DGLGraph:
             self._cache[("classes", n)] = layout
         return layout
 
+    def refuse_source_classes(self, feat: int, dtype: int) -> None:
+        """The scratch of ``feat`` features over source classes does not fit: the plain sum
+        from now on.  A layout that no launch has read is given back; one that has been
+        read stays, a recorded HIP graph may replay launches over it."""
+        n, self._cache[("source_classes", feat, dtype)] = self._cache[("source_classes", feat, dtype)], 0
+        if not self._cache[("classes", n)].used:
+            del self._cache[("classes", n)]
+
     def workspace(self, nbytes: int) -> torch.Tensor:
         """Scratch buffer shared by the operators called on this graph (grows on
         demand).  Calls that use it must be ordered on one stream: two streams
@@ -351,6 +359,7 @@ class SourceClasses:
     pointer: torch.Tensor           # (classes * N + 1) int32
     rows: torch.Tensor              # (E) int32: class * N + destination
     nbr: torch.Tensor               # (E) int32: source
+    used: bool = False              # a launch has read it
 
 
 def _build_source_classes(g: "DGLGraph", n: int) -> SourceClasses:

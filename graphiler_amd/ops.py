@@ -163,7 +163,9 @@ def _sum_by_classes(g: DGLGraph, u, out, row_scale, act: int, feat: int, dt: int
         ws = g.workspace(lib.ga_spmm_classes_workspace_bytes(g.num_nodes, g.num_edges, feat,
                                                              layout.num_classes))
     except torch.OutOfMemoryError:
+        g.refuse_source_classes(feat, dt)
         return False
+    layout.used = True
     capi.check(lib.ga_spmm_classes(
         layout.pointer.data_ptr(), layout.rows.data_ptr(), layout.nbr.data_ptr(), u.data_ptr(),
         out.data_ptr(), _ptr(row_scale), act, g.num_nodes, g.num_edges, feat,

@@ -1,4 +1,6 @@
 """Sums over slots ordered by source classes against the plain sum and float64."""
+import gc
+
 import numpy as np
 import pytest
 import torch
@@ -189,3 +191,52 @@ def test_sums_of_dense_graphs_under_deterministic_algorithms():
     assert g.source_classes(64, capi.GA_F32).num_classes > 0
     assert torch.equal(out, same)
     assert bool(((out.double() - _sum64(g, x)).abs() <= _sum64(g, x.abs()) * (64 * 2.0 ** -24)).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("boundary", [False, True])
+@pytest.mark.parametrize("used", [False, True])
+def test_scratch_that_does_not_fit_is_asked_for_once(boundary, used):
+    from graphiler_amd import torch_boundary
+    torch_boundary.load()
+    lib, n, e, feat = capi.load(), 40_000, 6_000_000, 512
+    gc.collect()            # no large segment of earlier tests to take blocks from
+    torch.cuda.empty_cache()
+    g = _graph(n, e, 8)
+    t = torch_boundary.script_graph(g)
+    x = torch.randn(n, feat, device="cuda")
+    call = (lambda y: torch.ops.my_ops.SpMMSrc(y, [1], False, None, t)) if boundary else \
+        (lambda y: ops.SpMMSrc(y, [1], False, None, g))
+    probe = _graph(n, e, 8)
+    k = probe.source_classes(feat, capi.GA_F32).num_classes
+    narrow = next(f for f in (256, 128, 64) if probe.source_classes(f, capi.GA_F32).num_classes == k)
+    plain = lib.ga_spmm_workspace_bytes(e, feat)
+    classes = lib.ga_spmm_classes_workspace_bytes(n, e, feat, k)
+    del probe
+    call(x.to(torch.float64).max(1).values.float().view(n, 1))      # row ids; no classes here
+    if used:                # the layout serves another width and stays
+        few = x[:, :narrow].contiguous()
+        before = call(few)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    room = 4 * n * feat * 2 + 10 * e + plain + (64 << 20)
+    assert classes > room
+    ooms = lambda: torch.cuda.memory_stats()["num_ooms"]
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + room) / total)
+        at = ooms()
+        first = call(x)
+        assert ooms() == at + 1
+        second = call(x)
+        assert ooms() == at + 1
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(first, second)
+    part = x[:, :16].contiguous()
+    err = (first[:, :16].double() - _sum64(g, part)).abs()
+    assert bool((err <= _sum64(g, part.abs()) * (64 * 2.0 ** -24)).all())
+    if not boundary:
+        assert (("classes", k) in g._cache) == used
+    if used:
+        assert torch.equal(call(few), before)
