@@ -95,6 +95,7 @@ SIGNATURES = {
     "ga_project_attn_strided": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64,
                                        _i64, _int, _vp]),
     "ga_gather_row_stride": (_i64, [_i64, _i64, _int]),
+    "ga_gat_from_z_shares_logits": (_int, [_i64, _i64, _i64, _i64, _int]),
     "ga_gat_aggregate_strided": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _i64, _i64,
                                         _i64, ctypes.c_float, _int, _int, _int, _vp, _sz, _vp]),
     "ga_gat_workspace_bytes": (_sz, [_i64, _i64, _i64]),

@@ -527,11 +527,10 @@ int launch_gat(const int32_t *pointer, const int32_t *row_of_slot,
   return launch_gat<T, VEC, MODE, SPREAD, ACT, N>(pointer, row_of_slot, nbr, el, er, z, out,    \
                                                   n_rows, n_edges, heads, dim, slope, ws, stream, \
                                                   ws_bytes, act, size_only, z_stride)
-    // the lanes of a head of 8 or 16 lanes form a slot's logit and exponential once (rows
-    // kept apart as ga_gather_row_stride says, against every lane for itself: 4 x 64 bf16 on
-    // 64 M edges, ids shuffled, 4870 -> 4616 us, 3 x 64 4507 -> 3924; uniform 6153 -> 5965)
-    if (head_lanes == 16) GA_GAT_GL(16);
-    if (head_lanes == 8) GA_GAT_GL(8);
+    if (ga_gat_from_z_shares_logits(n_rows, heads, dim, z_stride, sizeof(T) == 4 ? GA_F32 : GA_BF16)) {
+      if (head_lanes == 16) GA_GAT_GL(16);
+      GA_GAT_GL(8);
+    }
 #undef GA_GAT_GL
   }
   typename P::Args args{nbr, el, er, (const T *)z, heads, dim, slope, ids_vec, head_lanes, 0, act,
@@ -843,6 +842,30 @@ int ga_gat_aggregate_from_z_act(const int32_t *pointer, const int32_t *row_of_sl
                                 ga_stream_t stream) {
   return gat_from_z(pointer, row_of_slot, nbr, a_l, er, z, 0, out, n_rows, n_edges, heads, dim,
                     slope, activation, dtype, workspace, workspace_bytes, stream);
+}
+
+// Whether the lanes of a head (8 or 16 of them) form a slot's logit and exponential once, or
+// every lane for itself.  Once is a third fewer instructions and one more wavefront per
+// SIMD: faster where instructions bound the walk, slower where rows side by side meet in few
+// memory channels, which more wavefronts in flight make worse.  us, every lane -> once, R-MAT
+// and uniform graphs of 12 to 50 edges per node:
+//   rows apart, 64 M R-MAT edges     4 x 64 bf16 4864 -> 4466, 2 x 64 2968 -> 2718
+//   bf16 side by side, 128 to 384 and 640 bytes   0.67 .. 0.93 of the time at all sizes
+//     512 bytes    120 MB 830 -> 784, 360 MB 969 -> 911, 614 MB 2348 -> 2361, 1.25 GB 5705 -> 6186
+//     1024 bytes   100 MB 380 -> 321 (uniform 431 -> 440), 240 MB 1495 -> 1497 (1647 -> 1674),
+//                  720 MB 1762 -> 1843, 2.5 GB 12237 -> 12568
+//   fp32 side by side, 128 to 512 bytes   up to 60 MB 0.79 .. 1.03, from 120 MB on 0.98 .. 1.05
+//     384 and 768 bytes   up to 540 MB 0.75 .. 1.03, above 0.95 .. 1.05
+int ga_gat_from_z_shares_logits(int64_t n_rows, int64_t heads, int64_t dim, int64_t z_stride,
+                                int dtype) {
+  if (n_rows < 0 || heads <= 0 || dim <= 0 || (dtype != GA_F32 && dtype != GA_BF16)) return 0;
+  const int64_t esz = dtype == GA_F32 ? 4 : 2, piece = 16 / esz;
+  if (dim != 8 * piece && dim != 16 * piece) return 0;
+  if (z_stride > heads * dim) return 1;
+  const int64_t row = heads * dim * esz;
+  const bool power = (row & (row - 1)) == 0;
+  if (dtype == GA_F32) return n_rows <= ((power ? 64ll : 640ll) << 20) / row;
+  return row % 512 != 0 || n_rows <= ((row % 1024 != 0 ? 768ll : 192ll) << 20) / row;
 }
 
 // Rows of whole multiples of 256 bytes are kept 128 bytes further apart where their table is

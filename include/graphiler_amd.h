@@ -550,6 +550,10 @@ int ga_gat_aggregate_from_z_act(const int32_t *pointer, const int32_t *row_of_sl
  * launched nothing, unless rows, heads and the stride are whole 16-byte pieces and z and out
  * 16-byte aligned, and where ga_gat_aggregate_from_z says so. */
 int64_t ga_gather_row_stride(int64_t n_rows, int64_t feat, int dtype);
+/* 1 where the forms that take the source term from the rows (z_stride 0: side by side) let the
+ * lanes of a head share a slot's logit, 0 where every lane forms it (host arithmetic only). */
+int ga_gat_from_z_shares_logits(int64_t n_rows, int64_t heads, int64_t dim, int64_t z_stride,
+                                int dtype);
 int ga_gat_aggregate_strided(const int32_t *pointer, const int32_t *row_of_slot,
                              const int32_t *nbr, const float *source, const float *er,
                              const void *z, int64_t z_stride, void *out, int64_t n_rows,

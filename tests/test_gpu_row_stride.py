@@ -101,3 +101,50 @@ def test_layer(device, heads, dim, bf16, monkeypatch):
         with monkeypatch.context() as mp:
             mp.setattr(ops, "gat_project_and_aggregate", lambda *args: None)
             assert torch.equal(apart, layers.gat_layer(g, h, w, a, heads, 0.2, activation="elu"))
+
+
+def test_shared_logits_rule_on_the_host():
+    f, mb = capi.load().ga_gat_from_z_shares_logits, 1 << 20
+    # rows apart; heads of other than 8 or 16 lanes
+    assert f(1 << 22, 4, 64, 256 + 64, capi.GA_BF16) == 1 and f(1 << 22, 2, 64, 160, capi.GA_F32) == 1
+    for heads, dim, dt in ((4, 32, capi.GA_BF16), (2, 256, capi.GA_BF16), (4, 16, capi.GA_F32),
+                           (1, 128, capi.GA_F32), (1, 65, capi.GA_F32)):
+        assert f(1000, heads, dim, 0, dt) == 0
+    # side by side: the size of the table from which rows that share channels are left alone
+    for heads, dim, dt, limit in ((4, 64, capi.GA_BF16, 768), (2, 128, capi.GA_BF16, 768),
+                                  (8, 64, capi.GA_BF16, 192), (1, 64, capi.GA_F32, 64),
+                                  (4, 32, capi.GA_F32, 64), (3, 32, capi.GA_F32, 640),
+                                  (3, 64, capi.GA_F32, 640)):
+        rows = limit * mb // (heads * dim * (4 if dt == capi.GA_F32 else 2))
+        for stride in (0, heads * dim):
+            assert f(rows, heads, dim, stride, dt) == 1 and f(rows + 1, heads, dim, stride, dt) == 0
+    for heads in (1, 2, 3, 5):
+        assert f(1 << 30, heads, 64, 0, capi.GA_BF16) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,dim,bf16,n", [(1, 64, False, 262_145), (2, 32, False, 262_145),
+                                              (8, 64, True, 196_609)])
+def test_logits_of_every_lane(device, heads, dim, bf16, n):
+    """Side by side, one row past the line from which every lane forms its own logit: what the
+    shared form gives over rows apart, to the rounding of a logit's sum in another order."""
+    g, lib, feat, e = _graph(n, 2 * n, heads), capi.load(), heads * dim, 2 * n
+    dt, code = (torch.bfloat16, capi.GA_BF16) if bf16 else (torch.float32, capi.GA_F32)
+    assert not lib.ga_gat_from_z_shares_logits(n, heads, dim, 0, code)
+    gen = torch.Generator(device=device).manual_seed(feat)
+    z = torch.randn(n, feat, generator=gen, device=device).to(dt)
+    er = torch.randn(n, heads, generator=gen, device=device)
+    al = torch.randn(heads, dim, generator=gen, device=device) / 8
+    got = ops.gat_aggregate_from_z(al, er, z, g, 0.2)
+    wide = torch.zeros(n, feat + 128 // z.element_size(), dtype=dt, device=device)
+    wide[:, :feat] = z
+    out = torch.empty_like(z)
+    ws = g.workspace(lib.ga_gat_workspace_bytes(e, feat, heads))
+    capi.check(lib.ga_gat_aggregate_strided(
+        g.in_pointer.data_ptr(), g.in_row_of_slot.data_ptr(), g.in_node_indices.data_ptr(),
+        al.data_ptr(), er.data_ptr(), wide.data_ptr(), wide.shape[1], out.data_ptr(), n, e, heads, dim,
+        0.2, 1, capi.GA_ACT_NONE, code, ws.data_ptr(), ws.numel(), 0), "strided")
+    # logits of a few units, dim terms: weights move by less than 64 roundings of fp32; a bf16
+    # result next to a border between two values goes to the other, at most 2^-7 of it away
+    bound = out.double().abs() * (2.0 ** -7 if bf16 else 0) + 64 * 2.0 ** -24 * z.float().abs().max()
+    assert bool(((got.double() - out.double()).abs() <= bound).all())
