@@ -36,6 +36,14 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
+// The same instruction out of the compiler's sight: what it knows of the conversion it uses to
+// move code across the five row stores of a walk, which takes registers (GatOpaqueStore).
+__device__ __forceinline__ uint32_t pack_bf16_opaque(float lo, float hi) {
+  uint32_t r;
+  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(lo), "v"(hi));
+  return r;
+}
+
 // Sums over lane groups with DPP moves (all VALU, no LDS), result in every lane
 // of the group: swaps inside quads, then the half-row mirror (8 lanes:
 // 8j..8j+7) and the row mirror (16 lanes: 16j..16j+15).

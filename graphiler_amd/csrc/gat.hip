@@ -476,6 +476,32 @@ int launch_dot_attn(const int32_t *pointer, const int32_t *row_of_slot, const in
                         stream, ws_bytes);
 }
 
+// bf16 rows of several heads, the same values stored through pack_bf16_opaque: 124 registers and
+// four wavefronts per SIMD where the build above takes 150 to 168 and three (125 and four
+// while every value was rounded by five instructions).  Fewer wavefronts with more loads of
+// their own are the better form on large tables that fill their lane groups: 4 x 64 on 64 M
+// R-MAT edges 6737 (four) : 6539 us, on 8 M uniform edges 846 : 797, and of narrow rows (3 x 32 on
+// 64 M 3256 : 3157).  Rows of more than 16 lanes that do not (5 x 64 on 11.6 M R-MAT edges 943 :
+// 1050, on 12 M uniform edges 1804 : 1950, 3 x 64 on 16 M 936 : 1033) and short lists (4 x 64 on
+// 600 k uniform edges 56 : 59, 8 x 64 on 400 k 61 : 67) take this one.
+template <int ACT>
+struct GatOpaqueStore : GatPolicy<bf16_t, 8, kGatNode, false, ACT, 0> {
+  typedef GatPolicy<bf16_t, 8, kGatNode, false, ACT, 0> Base;
+  static __device__ __forceinline__ void emit(const typename Base::Args &, bf16_t *out, int64_t row,
+                                              int feat, int f0, const float (&st)[Base::kState]) {
+    float o[8];
+    Base::finish(st, o);
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      if (ACT == GA_ACT_ELU) o[v] = elu(o[v]);
+      if (ACT == GA_ACT_RELU) o[v] = relu_keep_nan(o[v]);
+    }
+    *reinterpret_cast<uint4 *>(out + row * feat + f0) =
+        make_uint4(pack_bf16_opaque(o[0], o[1]), pack_bf16_opaque(o[2], o[3]),
+                   pack_bf16_opaque(o[4], o[5]), pack_bf16_opaque(o[6], o[7]));
+  }
+};
+
 template <typename T, int VEC, int MODE = kGatNode, bool SPREAD = false, int ACT = kActRuntime,
           int GL = 0>
 int launch_gat(const int32_t *pointer, const int32_t *row_of_slot,
@@ -535,6 +561,13 @@ int launch_gat(const int32_t *pointer, const int32_t *row_of_slot,
   }
   typename P::Args args{nbr, el, er, (const T *)z, heads, dim, slope, ids_vec, head_lanes, 0, act,
                         z_stride ? z_stride : heads * dim};
+  if constexpr (sizeof(T) == 2 && VEC == 8 && MODE == kGatNode && !SPREAD && GL == 0 &&
+                ACT != kActRuntime) {
+    const int lanes = heads * dim / VEC;
+    if ((lanes > 16 && (lanes & (lanes - 1)) != 0) || n_edges < (1 << 20))
+      return launch_runs<GatOpaqueStore<ACT>>(args, pointer, row_of_slot, out, n_rows, n_edges,
+                                              heads * dim, ws, stream, ws_bytes, size_only);
+  }
   return launch_runs<P>(args, pointer, row_of_slot, out, n_rows, n_edges,
                         heads * dim, ws, stream, ws_bytes, size_only);
 }
