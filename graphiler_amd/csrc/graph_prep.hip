@@ -38,8 +38,9 @@ __global__ __launch_bounds__(kBlock) void prep_keys_kernel(
 }
 
 // pointer[v] = number of items with key < v, v in [0, n_keys]
+template <typename K>
 __global__ __launch_bounds__(kBlock) void pointer_kernel(
-    const int32_t *__restrict__ key_sorted, int64_t n_keys, int64_t n_items,
+    const K *__restrict__ key_sorted, int64_t n_keys, int64_t n_items,
     int32_t *__restrict__ pointer) {
   const int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (v > n_keys) return;
@@ -68,18 +69,22 @@ __global__ __launch_bounds__(kBlock) void fill_zero_kernel(int32_t *p, int64_t n
 // after its predecessor's up to its own, the last item those after its own as well.  No
 // sort, no search: every key is read once (672,884 keys: a stable sort and the comparison
 // behind it took 185 us of launches and two waits).  status[0]: a key outside [0, n_keys),
-// status[1]: a key below its predecessor; nothing is written for such an item.
+// status[1]: a key below its predecessor; nothing is written for such an item.  A lane writes
+// a gap between two keys alone, so there are at most kSerialKeys of them; above, WRITE is
+// false and pointer_kernel searches every entry.
+constexpr int64_t kSerialKeys = 4096;
+template <bool WRITE>
 __global__ __launch_bounds__(kBlock) void sorted_pointer_kernel(
     const int64_t *__restrict__ key, int64_t n_keys, int64_t n_items,
     int32_t *__restrict__ pointer, int32_t *__restrict__ status) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (n_items == 0 && i <= n_keys) pointer[i] = 0;
+  if (WRITE && n_items == 0 && i <= n_keys) pointer[i] = 0;
   if (i >= n_items) return;
   const int64_t k = key[i], before = i > 0 ? key[i - 1] : -1;
   const bool outside = k < 0 || k >= n_keys, unsorted = i > 0 && k < before;
   if (outside) status[0] = 1;       // every writer stores the same value
   if (unsorted) status[1] = 1;
-  if (outside || unsorted) return;
+  if (!WRITE || outside || unsorted) return;
   for (int64_t v = before < -1 ? 0 : before + 1; v <= k; ++v) pointer[v] = (int32_t)i;
   if (i == n_items - 1)
     for (int64_t v = k + 1; v <= n_keys; ++v) pointer[v] = (int32_t)n_items;
@@ -280,7 +285,7 @@ int ga_group_edges(const int64_t *key, const int64_t *other, int64_t n_keys,
     if (e != hipSuccess) return (int)e;
   }
   const int64_t pblocks = (n_keys + 1 + kBlock - 1) / kBlock;
-  hipLaunchKernelGGL(pointer_kernel, dim3((unsigned)pblocks), dim3(kBlock), 0, s, key_sorted,
+  hipLaunchKernelGGL(pointer_kernel<int32_t>, dim3((unsigned)pblocks), dim3(kBlock), 0, s, key_sorted,
                      n_keys, n_items, pointer);
   if (n_items > 0 && nbr) {
     const int64_t blocks = (n_items + kBlock - 1) / kBlock;
@@ -333,7 +338,7 @@ int ga_source_classes_build(const int32_t *row_of_slot, const int32_t *nbr, int6
   hipLaunchKernelGGL(class_scatter_kernel, dim3(blocks), dim3(kBlock), 0, s, row_of_slot, nbr,
                      n_rows, n_edges, shift, units, counts, rows, nbr_out);
   const int64_t n_keys = n_rows * n_classes;
-  hipLaunchKernelGGL(pointer_kernel, dim3((unsigned)((n_keys + 1 + kBlock - 1) / kBlock)),
+  hipLaunchKernelGGL(pointer_kernel<int32_t>, dim3((unsigned)((n_keys + 1 + kBlock - 1) / kBlock)),
                      dim3(kBlock), 0, s, rows, n_keys, n_edges, pointer);
   return launch_status();
 }
@@ -345,9 +350,17 @@ int ga_sorted_pointer(const int64_t *key, int64_t n_keys, int64_t n_items, int32
   if (!pointer || !status || (n_items > 0 && !key)) return GA_EINVAL;
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(kBlock), 0, s, status, (int64_t)2);
-  const int64_t threads = n_items > 0 ? n_items : n_keys + 1;
-  hipLaunchKernelGGL(sorted_pointer_kernel, dim3((unsigned)((threads + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, s, key, n_keys, n_items, pointer, status);
+  auto blocks = [](int64_t threads) { return dim3((unsigned)((threads + kBlock - 1) / kBlock)); };
+  if (n_keys <= kSerialKeys) {
+    hipLaunchKernelGGL(sorted_pointer_kernel<true>, blocks(n_items > 0 ? n_items : n_keys + 1),
+                       dim3(kBlock), 0, s, key, n_keys, n_items, pointer, status);
+    return launch_status();
+  }
+  if (n_items > 0)
+    hipLaunchKernelGGL(sorted_pointer_kernel<false>, blocks(n_items), dim3(kBlock), 0, s, key, n_keys,
+                       n_items, pointer, status);
+  hipLaunchKernelGGL(pointer_kernel<int64_t>, blocks(n_keys + 1), dim3(kBlock), 0, s, key, n_keys,
+                     n_items, pointer);
   return launch_status();
 }
 

@@ -56,3 +56,19 @@ def test_typed_graph(device, n, e):
         prepare_graph(src, dst, n, device=device, **{**typed, "num_ntypes": int(nt.max())})
     with pytest.raises(RuntimeError, match="one entry per node"):
         prepare_graph(src, dst, n, device=device, **{**typed, "ntype_of": nt[1:]})
+
+
+@pytest.mark.parametrize("key,keys", [([], 4096), ([], 5000), ([0], 4096), ([4095], 4097), ([3, 3, 4096], 4097),
+                                      ([7, 19_000_000], 20_000_000)])
+def test_sorted_pointer_of_few_items(device, key, keys):
+    """Far more keys than items: no lane walks a long gap by itself (20 M entries written one
+    by one take tens of milliseconds, searched they are a launch)."""
+    want = np.searchsorted(key, np.arange(keys + 1))
+    column = torch.tensor(key, dtype=torch.int64, device=device)
+    G._sorted_pointer(column, keys)
+    start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    start.record()
+    pointer, status = G._sorted_pointer(column, keys)
+    end.record()
+    assert status.tolist() == [0, 0] and np.array_equal(pointer.cpu().numpy(), want)
+    assert start.elapsed_time(end) < 5.0
