@@ -43,9 +43,13 @@ def gcn_layer(g: DGLGraph, h: torch.Tensor, weight: torch.Tensor,
 def gat_project(h, fc_weight, attn_weight, heads: int = 1):
     """Dense part of the GAT plan (GAT.py:25-29 after the split and reorder
     passes): z = h @ W, el = <z, a_l>, er = <z, a_r> per head."""
+    return _project(h, fc_weight, attn_weight, attn_weight[0].float().contiguous(),
+                    attn_weight[1].float().contiguous())
+
+
+def _project(h, fc_weight, attn_weight, a_l, a_r):
     try:        # one kernel: the GEMM with the attention terms in its epilogue
-        return ops.linear_attn(h, fc_weight, attn_weight[0].float().contiguous(),
-                               attn_weight[1].float().contiguous())
+        return ops.linear_attn(h, fc_weight, a_l, a_r)
     except capi.GraphilerError as err:
         if err.code != capi.GA_EUNSUPPORTED:
             raise
@@ -88,19 +92,21 @@ def gat_layer(g: DGLGraph, h, fc_weight, attn_weight, heads: int = 1,
     gathered rows instead of gathering them as well.  ``activation`` ("relu" |
     "elu"; the ``F.elu`` between the layers of examples/GAT/GAT.py) is applied by
     the fused pass to the rows it stores, by a separate call otherwise."""
-    if fused and h.is_cuda and fc_weight.dtype == h.dtype and fc_weight.is_contiguous() \
+    a_l, a_r = attn_weight[0].float().contiguous(), attn_weight[1].float().contiguous()
+    # rows apart are a matter of tables larger than an L2; asked further only there
+    if fused and h.is_cuda and g.num_nodes * fc_weight.shape[-1] * h.element_size() > ops.L2_BYTES \
+            and fc_weight.dtype == h.dtype and fc_weight.is_contiguous() \
             and h.is_contiguous() and h.dtype in (torch.float32, torch.bfloat16):
         out = ops.gat_project_and_aggregate(
-            h, fc_weight, attn_weight[0].float().contiguous(), attn_weight[1].float().contiguous(),
-            g, negative_slope, activation, 4 * g.num_nodes * heads >= SOURCE_TERM_TABLE_LIMIT)
+            h, fc_weight, a_l, a_r, g, negative_slope, activation,
+            4 * g.num_nodes * int(a_l.shape[0]) >= SOURCE_TERM_TABLE_LIMIT)
         if out is not None:
             return out
-    z, el, er = gat_project(h, fc_weight, attn_weight, heads)
+    z, el, er = _project(h, fc_weight, attn_weight, a_l, a_r)
     if fused:
         if el.numel() * el.element_size() >= SOURCE_TERM_TABLE_LIMIT:
             try:
-                return ops.gat_aggregate_from_z(attn_weight[0].float().contiguous(), er.float(),
-                                                z, g, negative_slope, activation)
+                return ops.gat_aggregate_from_z(a_l, er.float(), z, g, negative_slope, activation)
             except capi.GraphilerError as err:      # head width the variant does not take
                 if err.code != capi.GA_EUNSUPPORTED:
                     raise

@@ -954,6 +954,9 @@ def gat_aggregate_from_z(a_l, er, z, graph: DGLGraph, negative_slope: float = 0.
     return out
 
 
+L2_BYTES = 4 << 20       # of one XCD
+
+
 def gat_project_and_aggregate(h, weight, a_l, a_r, graph: DGLGraph, negative_slope: float = 0.01,
                               activation=None, from_z: bool = False):
     """``linear_attn`` and ``gat_aggregate`` (``from_z``: ``gat_aggregate_from_z``) with the

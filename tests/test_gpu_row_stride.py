@@ -148,3 +148,33 @@ def test_logits_of_every_lane(device, heads, dim, bf16, n):
     # result next to a border between two values goes to the other, at most 2^-7 of it away
     bound = out.double().abs() * (2.0 ** -7 if bf16 else 0) + 64 * 2.0 ** -24 * z.float().abs().max()
     assert bool(((got.double() - out.double()).abs() <= bound).all())
+
+
+def _layer_inputs(device, n, k, heads, dim, dt):
+    gen = torch.Generator(device=device).manual_seed(heads + dim)
+    h = torch.randn(n, k, generator=gen, device=device).to(dt)
+    w = (torch.randn(k, heads * dim, generator=gen, device=device) / k ** 0.5).to(dt)
+    return h, w, torch.randn(2, heads, dim, generator=gen, device=device) / 4
+
+
+@pytest.mark.gpu
+def test_small_layers_do_not_ask_for_rows_apart(device, monkeypatch):
+    """Tables that an L2 holds go straight to the two operators."""
+    g = _graph(300, 2000, 1)
+    want = layers.gat_layer(g, *_layer_inputs(device, 300, 48, 4, 64, torch.float32), 4, 0.2)
+    def asked(*args):
+        raise AssertionError("asked for rows apart")
+    monkeypatch.setattr(ops, "gat_project_and_aggregate", asked)
+    got = layers.gat_layer(g, *_layer_inputs(device, 300, 48, 4, 64, torch.float32), 4, 0.2)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+def test_layer_goes_by_the_heads_of_its_vectors(device, monkeypatch):
+    """``heads`` left at its default: the form of the source term follows the vectors, as the
+    table of terms does."""
+    n = 17_000
+    g = _graph(n, 60_000, 2)
+    inputs = _layer_inputs(device, n, 48, 4, 64, torch.bfloat16)
+    monkeypatch.setattr(layers, "SOURCE_TERM_TABLE_LIMIT", 4 * n * 4)
+    assert torch.equal(layers.gat_layer(g, *inputs, negative_slope=0.2), layers.gat_layer(g, *inputs, 4, 0.2))
