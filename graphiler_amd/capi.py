@@ -109,6 +109,7 @@ SIGNATURES = {
                                  _i64, _i64, _i64, _i64, _int, _vp]),
     "ga_pair_tiles_capacity": (_i64, [_i64, _i64]),
     "ga_pair_tiles_build": (_int, [_vp, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _vp]),
+    "ga_pair_tiles_fit": (_int, [_i64, _i64, _i64, _int]),
     "ga_pair_weights_bytes": (_sz, [_i64, _i64, _i64, _int]),
     "ga_pair_weights": (_int, [_vp, _vp, _int, ctypes.c_float, _vp, _vp, _vp, _i64, _i64, _i64, _vp]),
     "ga_pair_attention_tiles": (_int, [_vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64,

@@ -106,6 +106,14 @@ extern "C" int ga_pair_weights(const float *att, const void *scale, int scale_dt
   return launch_status();
 }
 
+// a slot's address is a 32-bit offset
+extern "C" int ga_pair_tiles_fit(int64_t n_nodes, int64_t heads, int64_t dim, int dtype) {
+  if (n_nodes < 0 || n_nodes > 0x7fffffff || heads <= 0 || dim <= 0 || heads > 0x7fffffff / dim ||
+      (dtype != GA_F32 && dtype != GA_BF16))
+    return 0;
+  return n_nodes <= 0xffffffffll / (heads * dim * (dtype == GA_F32 ? 4 : 2));
+}
+
 extern "C" int ga_pair_attention_tiles(const int32_t *rows, const int32_t *tiles, int64_t n_types,
                                        const int32_t *nbr, const void *q, const void *k,
                                        const void *v, const void *att, const void *msg, void *m,
@@ -121,10 +129,7 @@ extern "C" int ga_pair_attention_tiles(const int32_t *rows, const int32_t *tiles
                  q, k, v, att, msg, m, lse, (int)n_types};
   const int rc = ga::check_pairs(A, max_slots);
   if (rc != GA_OK) return rc;
-  // a slot's address is a 32-bit offset
-  if (n_nodes > 0x7fffffff ||
-      n_nodes > 0xffffffffll / (heads * dim * (dtype == GA_F32 ? 4 : 2)))
-    return GA_EUNSUPPORTED;
+  if (!ga_pair_tiles_fit(n_nodes, heads, dim, dtype)) return GA_EUNSUPPORTED;
   if (ga_pair_weights_bytes(n_types, heads, dim, dtype) > 0 &&
       (!ga::aligned(att, 16) || !ga::aligned(msg, 16)))
     return GA_EALIGN;

@@ -1276,8 +1276,8 @@ torch::Tensor dot_attention_sum(torch::Tensor k, torch::Tensor q, torch::Tensor 
 // per pair instead of per edge:
 //   score = <k[src], q[dst] (s A)^T>,  out[v] = sum_pairs (sum_{e in pair} a_e v[src]) M
 // with both products, the scores, the softmax inside the pair and its weighted sum in one
-// pass (ga_pair_attention) or, where ga_pair_attention_preferred says no, in three launches
-// around ga_dot_attention_sum; the pairs of a destination are weighed by the softmax of
+// pass (ga_pair_attention_tiles; ga_pair_attention where the tables reach 4 GB) or, where
+// ga_pair_attention_preferred says no, in three launches around ga_dot_attention_sum; the pairs of a destination are weighed by the softmax of
 // their log-sum-exps.  Graphs without such pairs and shapes outside those kernels run the
 // three per-edge operators.
 torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::Tensor v,
@@ -1339,7 +1339,9 @@ torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::T
   if (ga_pair_attention_preferred(P, e, pairs.max_slots, heads, d, dt)) {
     torch::Tensor m_pair = torch::empty({P, hid}, k.options());
     torch::Tensor lse = torch::empty({P, heads}, k.options().dtype(at::kFloat));
-    const size_t bytes = ga_pair_weights_bytes(graph->num_etypes, heads, d, dt);
+    // over prepared tiles, or over the pair columns where a slot's address takes 64 bits
+    const bool tiled = ga_pair_tiles_fit(n, heads, d, dt);
+    const size_t bytes = tiled ? ga_pair_weights_bytes(graph->num_etypes, heads, d, dt) : 0;
     torch::Tensor att, msg = relation_msg;
     if (bytes > 0) {                     // both matrices as the products read them
       att = torch::empty({(int64_t)bytes}, k.options().dtype(at::kByte));
@@ -1351,19 +1353,26 @@ torch::Tensor relation_pair_attention(torch::Tensor k, torch::Tensor q, torch::T
     } else {
       att = transposed();
     }
-    const int rc = ga_pair_attention_tiles(
-        pairs.rows.data_ptr<int>(), pairs.tiles.data_ptr<int>(), graph->num_etypes,
-        graph->in_node_indices.data_ptr<int>(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-        att.data_ptr(), msg.data_ptr(), m_pair.data_ptr(), lse.data_ptr<float>(), P, n,
-        pairs.max_slots, heads, d, dt, stream);
+    const int rc =
+        tiled ? ga_pair_attention_tiles(
+                    pairs.rows.data_ptr<int>(), pairs.tiles.data_ptr<int>(), graph->num_etypes,
+                    graph->in_node_indices.data_ptr<int>(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                    att.data_ptr(), msg.data_ptr(), m_pair.data_ptr(), lse.data_ptr<float>(), P, n,
+                    pairs.max_slots, heads, d, dt, stream)
+              : ga_pair_attention(
+                    pairs.type_pointer.data_ptr<int>(), graph->num_etypes,
+                    pairs.by_type.data_ptr<int64_t>(), pairs.dst_by_type.data_ptr<int64_t>(),
+                    pairs.pair_pointer.data_ptr<int>(), graph->in_node_indices.data_ptr<int>(),
+                    q.data_ptr(), k.data_ptr(), v.data_ptr(), att.data_ptr(), msg.data_ptr(),
+                    m_pair.data_ptr(), lse.data_ptr<float>(), P, pairs.max_slots, heads, d, dt, stream);
     if (rc != GA_EUNSUPPORTED) {
-      check_ga(rc, "ga_pair_attention_tiles");
+      check_ga(rc, tiled ? "ga_pair_attention_tiles" : "ga_pair_attention");
       torch::Tensor ws = graph->workspace(ga_gat_workspace_bytes(P, hid, heads));
       torch::Tensor out = torch::empty({n, hid}, k.options());
       check_ga(ga_edge_softmax_sum(pairs.dst_pointer.data_ptr<int>(), pairs.pair_dst.data_ptr<int>(),
-                                   pairs.rank.data_ptr<int>(), lse.data_ptr<float>(), m_pair.data_ptr(),
-                                   out.data_ptr(), n, P, heads, d, dt, ws.data_ptr(),
-                                   (size_t)ws.numel(), stream),
+                                   tiled ? pairs.rank.data_ptr<int>() : nullptr,
+                                   lse.data_ptr<float>(), m_pair.data_ptr(), out.data_ptr(), n, P,
+                                   heads, d, dt, ws.data_ptr(), (size_t)ws.numel(), stream),
                "ga_edge_softmax_sum");
       return out;
     }

@@ -1132,9 +1132,12 @@ def relation_pair_attention(k, q, v, relation_att, relation_msg, relation_scale,
     # log-sum-exps (the softmax-weighted sum of per-"edge" rows, with the pairs as the
     # edges), which makes the weights the softmax over all its in-edges
     if lib.ga_pair_attention_preferred(P, e, pairs.max_slots, heads, d, dt):
-        m_pair = torch.empty((P, hid), dtype=v.dtype, device=dev)            # by_type order
+        # over prepared tiles, which leave messages and log-sum-exps in by_type order, or over
+        # the pair columns and in pair order where a slot's address takes 64 bits
+        tiled = bool(lib.ga_pair_tiles_fit(n, heads, d, dt))
+        m_pair = torch.empty((P, hid), dtype=v.dtype, device=dev)
         lse = torch.empty((P, heads), dtype=torch.float32, device=dev)
-        nbytes = int(lib.ga_pair_weights_bytes(n_types, heads, d, dt))
+        nbytes = int(lib.ga_pair_weights_bytes(n_types, heads, d, dt)) if tiled else 0
         if nbytes:                      # both matrices as the products read them
             att, msg = (torch.empty(nbytes, dtype=torch.uint8, device=dev) for _ in range(2))
             capi.check(lib.ga_pair_weights(
@@ -1143,18 +1146,28 @@ def relation_pair_attention(k, q, v, relation_att, relation_msg, relation_scale,
                 "ga_pair_weights")
         else:
             att, msg = transposed(), relation_msg
-        rc = lib.ga_pair_attention_tiles(
-            pairs.rows.data_ptr(), pairs.tiles.data_ptr(), n_types, graph.in_node_indices.data_ptr(),
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), att.data_ptr(), msg.data_ptr(),
-            m_pair.data_ptr(), lse.data_ptr(), P, n, pairs.max_slots, heads, d, dt, stream)
+        if tiled:
+            rc = lib.ga_pair_attention_tiles(
+                pairs.rows.data_ptr(), pairs.tiles.data_ptr(), n_types,
+                graph.in_node_indices.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                att.data_ptr(), msg.data_ptr(), m_pair.data_ptr(), lse.data_ptr(), P, n,
+                pairs.max_slots, heads, d, dt, stream)
+        else:
+            rc = lib.ga_pair_attention(
+                pairs.type_pointer.data_ptr(), n_types, pairs.by_type.data_ptr(),
+                pairs.dst_by_type.data_ptr(), pairs.pair_pointer.data_ptr(),
+                graph.in_node_indices.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                att.data_ptr(), msg.data_ptr(), m_pair.data_ptr(), lse.data_ptr(), P,
+                pairs.max_slots, heads, d, dt, stream)
         if rc != capi.GA_EUNSUPPORTED:
-            capi.check(rc, "ga_pair_attention_tiles")
+            capi.check(rc, "ga_pair_attention_tiles" if tiled else "ga_pair_attention")
             ws = graph.workspace(lib.ga_gat_workspace_bytes(P, hid, heads))
             out = torch.empty((n, hid), dtype=v.dtype, device=dev)
             capi.check(lib.ga_edge_softmax_sum(
-                pairs.dst_pointer.data_ptr(), pairs.pair_dst.data_ptr(), pairs.rank.data_ptr(),
-                lse.data_ptr(), m_pair.data_ptr(), out.data_ptr(), n, P, heads, d, dt, ws.data_ptr(),
-                ws.numel(), stream), "ga_edge_softmax_sum")
+                pairs.dst_pointer.data_ptr(), pairs.pair_dst.data_ptr(),
+                pairs.rank.data_ptr() if tiled else None, lse.data_ptr(), m_pair.data_ptr(),
+                out.data_ptr(), n, P, heads, d, dt, ws.data_ptr(), ws.numel(), stream),
+                "ga_edge_softmax_sum")
             return out
         del m_pair, lse
     q_pair = typed_rows(q, pairs.dst_by_type, transposed())

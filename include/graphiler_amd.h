@@ -607,7 +607,7 @@ int ga_pair_attention(const int32_t *type_pointer, int64_t n_types, const int64_
  * (first slot, end slot, destination, 0), tiles (ga_pair_tiles_capacity, 4) int32 (type or
  * -1, first row, end row, 0), both 16-byte aligned.  Differences from ga_pair_attention: m
  * and lse are in by_type order; q, k and v have n_nodes rows of together less than 4 GB
- * each (GA_EUNSUPPORTED otherwise); and where ga_pair_weights_bytes is not 0 (fp32 heads
+ * each (ga_pair_tiles_fit 1; GA_EUNSUPPORTED otherwise); and where ga_pair_weights_bytes is not 0 (fp32 heads
  * of 32 and 64 of 64 features), att and msg are what ga_pair_weights wrote from the (n_types,
  * heads, dim, dim) matrices: att transposed, times scale[type, head] (fp32 or bf16, or NULL)
  * and factor, both cut into bf16 pieces; ga_pair_weights_bytes bytes each, 16-byte aligned. */
@@ -615,6 +615,7 @@ int64_t ga_pair_tiles_capacity(int64_t n_pairs, int64_t n_types);
 int ga_pair_tiles_build(const int32_t *type_pointer, int64_t n_types, const int64_t *by_type,
                         const int64_t *dst_by_type, const int32_t *pair_pointer, int64_t n_pairs,
                         int32_t *rows, int32_t *tiles, ga_stream_t stream);
+int ga_pair_tiles_fit(int64_t n_nodes, int64_t heads, int64_t dim, int dtype);
 size_t ga_pair_weights_bytes(int64_t n_types, int64_t heads, int64_t dim, int dtype);
 int ga_pair_weights(const float *att, const void *scale, int scale_dtype, float factor,
                     const float *msg, void *att_out, void *msg_out, int64_t n_types,
