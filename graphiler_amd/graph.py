@@ -169,19 +169,25 @@ class DGLGraph:
             rows.data_ptr(), stream), "ga_csr_row_ids")
         return rows
 
+    def _kept_row_ids(self, key: str, pointer: torch.Tensor) -> torch.Tensor:
+        rows = self._cache.get(key)
+        if rows is None:
+            rows = self._row_ids(pointer)
+            # inside a capture nothing runs yet and the memory is the recorded graph's: that
+            # graph fills its own column on every replay, the next eager call one to keep
+            if not torch.cuda.is_current_stream_capturing():
+                self._cache[key] = rows
+        return rows
+
     @property
     def in_row_of_slot(self) -> torch.Tensor:
         """Destination node of every slot of the in-adjacency (int32, E)."""
-        if "in_rows" not in self._cache:
-            self._cache["in_rows"] = self._row_ids(self.in_pointer)
-        return self._cache["in_rows"]
+        return self._kept_row_ids("in_rows", self.in_pointer)
 
     @property
     def out_row_of_slot(self) -> torch.Tensor:
         """Source node of every slot of the out-adjacency (int32, E)."""
-        if "out_rows" not in self._cache:
-            self._cache["out_rows"] = self._row_ids(self.out_pointer)
-        return self._cache["out_rows"]
+        return self._kept_row_ids("out_rows", self.out_pointer)
 
     def _identity(self, key: str, column: torch.Tensor) -> bool:
         if key not in self._cache:

@@ -67,3 +67,28 @@ def test_operators(device, e):
     for got in (ops.gsddmm_u_dot_v(u, v, g),
                 torch.ops.my_ops.gsddmm_u_dot_v(u, v, torch_boundary.script_graph(g))):
         assert bool(((got.double() - ref).abs() <= size * (16 * 2.0 ** -24)).all())
+
+
+def test_first_call_inside_a_capture(device):
+    """The destination column that the walk reads is not kept from a capture, where nothing
+    has run yet: replays fill their own, eager calls build theirs."""
+    rng = np.random.default_rng(4)
+    n, e = 3000, 40_000
+    g = prepare_graph(rng.integers(0, n, e), rng.integers(0, n, e), n, device=device)
+    u, v = (torch.randn(n, 4, 16, device=device) for _ in range(2))
+    assert not g.in_eid_is_identity and "in_rows" not in g._cache
+    torch.cuda.synchronize()
+    recorded = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(recorded):
+        captured = ops.gsddmm_u_dot_v(u, v, g)
+    assert "in_rows" not in g._cache
+    eager = ops.gsddmm_u_dot_v(u, v, g)
+    assert "in_rows" in g._cache
+    ref = (u.double()[g.COO_src] * v.double()[g.COO_dst]).sum(2)
+    assert float((eager.double() - ref).abs().max()) < 16 * 2.0 ** -23 * float(u.abs().max() * v.abs().max())
+    for _ in range(3):
+        captured.zero_()
+        recorded.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, eager)
+        assert torch.equal(ops.gsddmm_u_dot_v(u, v, g), eager)
