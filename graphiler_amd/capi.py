@@ -17,6 +17,7 @@ GA_OK = 0
 GA_EINVAL, GA_EUNSUPPORTED, GA_EWORKSPACE, GA_EALIGN, GA_ESCRATCH = -1, -2, -3, -4, -5
 GA_STATIC_SCRATCH_BYTES = 32 << 20
 GA_DEGREE_BUCKETS = 31
+GA_CLASSES_MIN_DEGREE = 16
 GA_ACT_NONE, GA_ACT_RELU, GA_ACT_ELU = 0, 1, 2
 GA_F32, GA_BF16 = 0, 1
 GA_COPY_U, GA_COPY_E, GA_U_MUL_E, GA_U_ADD_E, GA_U_SUB_E, GA_U_DIV_E = 0, 1, 2, 3, 4, 5

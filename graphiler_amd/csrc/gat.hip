@@ -536,7 +536,10 @@ int launch_gat(const int32_t *pointer, const int32_t *row_of_slot,
                                                   n_rows, n_edges, heads, dim, slope, ws, stream, \
                                                   ws_bytes, act, size_only, z_stride)
     // per-edge rows stream: where they fill the lane group sharing gives nothing (108,368
-    // uniform edges, fp32 rows of 128 and 512: 0.95 times the speed; 1 M edges: 1.03 .. 1.08)
+    // uniform edges, fp32 rows of 128 and 512: 0.95 times the speed; 1 M edges: 1.03 .. 1.08).
+    // The same holds where they are gathered through an id column (the pairs of a relation
+    // attention by rank): own -> shared reads 1 x 64 fp32 11.5 -> 11.8 us on 100 k rows, 24.5 ->
+    // 24.5 on 269 k, 37.8 -> 35.6 on 530 k, 114.7 -> 112.9 on 1.95 M, bf16 within 2 %
     const bool streams = MODE == kGatEdge && !SPREAD && (lanes & (lanes - 1)) == 0;
     if (lanes > 8 && !streams && (one_head || dim % (16 * VEC) == 0)) GA_GAT_GL(16);
     if (lanes > 4 && lanes <= 8 && !streams && one_head) GA_GAT_GL(8);
@@ -904,12 +907,17 @@ int ga_gat_from_z_shares_logits(int64_t n_rows, int64_t heads, int64_t dim, int6
 // Rows of whole multiples of 256 bytes are kept 128 bytes further apart where their table is
 // larger than an L2.  Graph generators and loaders give popular nodes ids with structure
 // (many zero bits in R-MAT), and with rows a power of two apart those ids' rows meet in a
-// few of the memory channels, which change every 128 bytes.  The fused aggregation, rows
-// side by side -> 128 bytes further apart, us (64 or 256 bytes: slower):
-//   R-MAT, 2.4 M nodes, 64 M edges: 4 x 64 bf16 6259 -> 4472 (4616 with the ids shuffled),
-//     8 x 64 12721 -> 8817, 1 x 64 fp32 3808 -> 2791
-//   R-MAT, 233 k nodes, 11.6 M edges: 1 x 64 fp32 330 -> 262, 4 x 64 bf16 884 -> 747
-//   uniform, the same sizes: 5963 -> 5953, 498 -> 498; 20 k nodes, 400 k edges: level
+// few of the memory channels, which change every 128 bytes; how many also depends on where
+// the table lies (1 x 64 fp32 on 11.6 M edges, the same table in four places: 264 to 320 us,
+// apart 245 to 272).  Side by side -> 128 bytes further apart (64 or 256 bytes: slower), us, the
+// projection and the aggregation over three buffers in turn, R-MAT:
+//   2.4 M nodes, 64 M edges      1 x 64 fp32 3575 -> 3075, 2 x 64 bf16 3298 -> 2627, 4 x 64 6207 -> 4604
+//   700 k nodes, 8 M edges       1 x 64 fp32 472 -> 420, 2 x 64 bf16 471 -> 447, 4 x 64 948 -> 810
+//   233 k nodes, 11.6 M edges    1 x 64 fp32 459 -> 440 (level, 431, in other runs), 2 x 64 bf16
+//                                446 -> 444, 4 x 64 fp32 1882 -> 1358
+//   100 k nodes, 3 M edges       1 x 64 fp32 106 -> 106, 2 x 64 202 -> 175, 4 x 64 398 -> 354
+// Uniform ids, tables below 32 MB and rows of 768 bytes: level (within 1.4 %).  The price is
+// memory: half as much z again at 256 bytes a row, a quarter at 512, an eighth at 1024.
 int64_t ga_gather_row_stride(int64_t n_rows, int64_t feat, int dtype) {
   if (n_rows < 0 || feat <= 0 || (dtype != GA_F32 && dtype != GA_BF16)) return 0;
   const int64_t esz = dtype == GA_F32 ? 4 : 2;

@@ -7,14 +7,15 @@
 //
 // Tall-skinny GEMM with fp32 operands and fp32 results on the bf16 matrix
 // instruction (v_mfma_f32_16x16x32_bf16, 16x the rate of the fp32 one): every
-// operand value is split exactly into three bf16 pieces, x = x0 + x1 + x2 (8
-// significant bits each, 24 in all), and the product is accumulated in fp32 from
-// the six piece products of weight >= 2^-16, x0w0 + x0w1 + x1w0 + x1w1 + x0w2 +
-// x2w0; each piece product is exact in fp32 and the three dropped ones are below
-// 2^-24 of |x||w|, i.e. below the rounding of an fp32 product.  Measured against
-// float64 the result is as close as the fp32 instruction's (max error / max |Z|
-// 8e-7 against 1.2e-6 at K = 602).  Non-finite inputs give NaN (inf - inf in the
-// split) where fp32 products may give inf.
+// operand value is split into three bf16 pieces, x = x0 + x1 + x2 (8 significant
+// bits each, 24 in all; exact down to 2^-110, below which the third leaves bf16's
+// range), and the product is accumulated in fp32 from the six piece products x0w0 +
+// x0w1 + x1w0 + x1w1 + x0w2 + x2w0; each is exact in fp32.  The pieces are cut off,
+// not rounded, so the three dropped products reach 7.8 x 2^-24 of |x||w| at the worst
+// significands (0.7 x 2^-24 on average) and have the product's sign.  Measured against
+// float64 on values of both signs the result is as close as the fp32 instruction's (max
+// error / max |Z| 8e-7 against 1.2e-6 at K = 602).  Non-finite inputs give NaN (inf -
+// inf in the split) where fp32 products may give inf.
 //
 // A workgroup (4 waves) owns 128 rows, each wave 32 rows (2 tiles of 16) x 64
 // columns per pass.  Both operands go global -> registers -> LDS in
@@ -45,8 +46,8 @@ namespace {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// x = p0 + p1 + p2 exactly, each piece a bf16 (the top 8 significant bits of
-// what the pieces before it leave); eight values -> three packed operands.
+// x = p0 + p1 + p2 (exactly from 2^-110 up), each piece a bf16 (the top 8 significant
+// bits of what the pieces before it leave); eight values -> three packed operands.
 __device__ __forceinline__ void split8(const float (&v)[8], uint4 &p0, uint4 &p1, uint4 &p2) {
   uint32_t a[8], b[8], c[8];
 #pragma unroll

@@ -25,14 +25,17 @@ extern "C" int ga_pair_attention(const int32_t *type_pointer, int64_t n_types,
 // taken as one and a half rows of the largest size on one group, between a lone large pair
 // and many side by side.  The three launches pay for the pairs' rows in memory and for
 // their own starts, but spread the slots evenly.  The figures (us; 0.72 per batch, 30 and
-// 33 per 100 k pairs and 1 M edges of 256-byte rows) are fitted to 500 to 1.95 M pairs of 1
-// to 256 slots; pair form against three launches, 1 x 64 fp32:
-//   500 pairs of 16 / 32 / 256      29 : 34,  40 : 34,  199 : 40 us    (7 tiles for 256 CUs)
-//   2,500 pairs of 16 / 32 / 100    30 : 36,  42 : 38,   91 : 48
-//   10,000 pairs of 32 / 64         41 : 48,  65 : 59
-//   40,000 pairs of 64 / 256       111 : 138, 359 : 378
-//   100,000 pairs of 3 on average, 0.3 % of 64 / 128 / 256   84 : 99, 115 : 99, 177 : 100
-//   1 M pairs of 3, 0.3 % of 128 / 256                      523 : 669, 656 : 696
+// 33 per 100 k pairs and 1 M edges of 256-byte rows) were fitted to the pass over pair columns.
+// Over prepared tiles it is faster, one head of 64 fp32 features most (a group walks two
+// rows, not four), so the line is on the launches' side: of 433 combinations of 500 to 1 M
+// pairs of 2 to 256 slots in five layouts 39 take a form that is more than 5 % slower than the
+// other, 37 of them the launches.  The operator as it runs, pass : launches, 1 x 64 fp32:
+//   500 pairs of 16 / 32 / 64 / 256       23 : 34,   30 : 34,   45 : 36,  131 : 48
+//   2,500 pairs of 32 / 64 / 256          35 : 44,   48 : 49,  131 : 73
+//   10,000 pairs of 32 / 64 / 256         38 : 59,   52 : 73,  140 : 169
+//   40,000 pairs of 64 / 256             141 : 181, 489 : 563
+//   100,000 pairs of 3 on average, 0.3 % of 64 / 128 / 256    78 : 102,  87 : 103, 125 : 103
+//   1 M pairs of 3, 0.3 % of 64 / 128 / 256                  392 : 653, 442 : 667, 585 : 690
 extern "C" int ga_pair_attention_preferred(int64_t n_pairs, int64_t n_edges, int64_t max_slots,
                                            int64_t heads, int64_t dim, int dtype) {
   if (n_pairs <= 0 || n_edges < n_pairs || heads <= 0 || dim <= 0 || max_slots > 256) return 0;

@@ -1128,13 +1128,16 @@ int ga_spmm_csr_scaled(const int32_t *pointer, const int32_t *row_of_slot,
 // write and the read).  Six per cent are asked for: R-MAT, 100 k nodes, 200 edges per node,
 // 64 fp32 features, where four of five gathers hit anyway, 272 : 282 us, and 233 k nodes
 // with 50 edges per node 220 : 230, both left to the plain sum; uniform, 100 k nodes with
-// 25 edges per node, 64 features 94 : 98 (plain), with 50 173 : 146 (classes).
+// 25 edges per node, 64 features 94 : 98 (plain), with 50 173 : 146 (classes).  In the model's
+// best case, every gather a hit instead of none, two classes pay for their partial rows from
+// 11 edges per row in fp32 and 28 in bf16: without degrees the answer is that case's, and
+// GA_CLASSES_MIN_DEGREE a first line that callers compare for themselves.
 int64_t ga_spmm_source_classes(const int64_t *nodes_of_degree, const int64_t *edges_of_degree,
                                int64_t n_rows, int64_t n_edges, int64_t feat, int dtype) {
   if (n_rows <= 0 || n_edges <= 0 || feat < 8 || (dtype != GA_F32 && dtype != GA_BF16)) return 0;
   const bool half = dtype == GA_BF16;
   const double row = (double)feat * (half ? 2 : 4);
-  if (feat % (half ? 8 : 4) || n_rows > 0x7ffffffe / 8 || n_edges < 16 * n_rows ||
+  if (feat % (half ? 8 : 4) || n_rows > 0x7ffffffe / 8 || n_edges < GA_CLASSES_MIN_DEGREE * n_rows ||
       (double)n_rows * row <= ga::kL2Bytes)
     return 0;
   const double gb = 1e-9 * (double)n_edges * (row < 128 ? 128 : row);

@@ -428,8 +428,8 @@ torch::Tensor spmm(const GraphPtr &g, int op, int reduce, const torch::Tensor &u
   TORCH_CHECK(u.size(0) == (op == GA_COPY_E || edge_rows ? g->num_edges : g->num_nodes),
               "features have the wrong number of rows");
   torch::Tensor out = torch::empty(out_shape(g->num_nodes, u), u.options());
-  if (op == GA_COPY_U && g->num_edges >= 16 * g->num_nodes && reduce == GA_SUM && !reverse &&
-      sum_by_classes(g, u, out, nullptr, GA_ACT_NONE, feat, dt))
+  if (op == GA_COPY_U && g->num_edges >= GA_CLASSES_MIN_DEGREE * g->num_nodes &&
+      reduce == GA_SUM && !reverse && sum_by_classes(g, u, out, nullptr, GA_ACT_NONE, feat, dt))
     return out;
   const size_t ws_bytes = ga_spmm_workspace_bytes(g->num_edges, feat);
   torch::Tensor ws = g->workspace(ws_bytes);
@@ -496,7 +496,7 @@ torch::Tensor SpMMScaled(torch::Tensor features, at::optional<torch::Tensor> row
   torch::Tensor factor;
   if (per_row) factor = row_scale.value().contiguous();
   torch::Tensor out = torch::empty(out_shape(n, features), features.options());
-  if (graph->num_edges >= 16 * graph->num_nodes && !edge_rows &&
+  if (graph->num_edges >= GA_CLASSES_MIN_DEGREE * graph->num_nodes && !edge_rows &&
       sum_by_classes(graph, features, out, per_row ? factor.data_ptr<float>() : nullptr,
                                    (int)activation, feat, dt))
     return out;

@@ -136,7 +136,8 @@ def spmm(g: DGLGraph, op: str, reduce: str, u: torch.Tensor,
             feat, heads, code, _REDUCE[reduce], dt, ws.data_ptr(), ws.numel(),
             _stream(u)), "ga_spmm_csr_arg")
         return out, arg_u, arg_e
-    if op == "copy_u" and g.num_edges >= 16 * g.num_nodes and reduce == "sum" and not reverse and \
+    if op == "copy_u" and g.num_edges >= capi.GA_CLASSES_MIN_DEGREE * g.num_nodes and \
+            reduce == "sum" and not reverse and \
             _sum_by_classes(g, u, out, None, capi.GA_ACT_NONE, feat, dt):
         return out
     ws_bytes = lib.ga_spmm_workspace_bytes(g.num_edges, feat)
@@ -225,7 +226,7 @@ def spmm_scaled(features, graph: DGLGraph, row_scale=None, activation=None,
             raise RuntimeError("row_scale must be (N,) or (N, 1) float32")
     feat = get_feat_dim(features)
     out = torch.empty(_out_shape(n, features), dtype=features.dtype, device=features.device)
-    if graph.num_edges >= 16 * graph.num_nodes and not edge_rows and \
+    if graph.num_edges >= capi.GA_CLASSES_MIN_DEGREE * graph.num_nodes and not edge_rows and \
             _sum_by_classes(graph, features, out, row_scale, act, feat, dt):
         return out
     lib = capi.load()

@@ -157,6 +157,9 @@ int ga_spmm_csr_scaled(const int32_t *pointer, const int32_t *row_of_slot,
  * workspace (16-byte aligned), are added in class order.
  */
 #define GA_DEGREE_BUCKETS 31
+/* graphs with fewer edges per row: 0 from ga_spmm_source_classes, which callers with many
+ * small calls compare for themselves */
+#define GA_CLASSES_MIN_DEGREE 16
 int64_t ga_spmm_source_classes(const int64_t *nodes_of_degree, const int64_t *edges_of_degree,
                                int64_t n_rows, int64_t n_edges, int64_t feat, int dtype);
 int ga_degree_buckets(const int32_t *pointer, int64_t n_rows, int64_t *buckets, ga_stream_t stream);
