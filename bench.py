@@ -25,7 +25,7 @@ intensity x HBM peak).
 
 Algorithmic bytes credit one gathered row per edge and no cache reuse.  An operator
 whose gathered table fits the 256 MB Infinity Cache, or whose algorithmic bytes flow
-faster than the HBM peak, is marked "cache_served": its fraction is then taken from the
+faster than the HBM peak (in the headline: than this run's copy of 1 GiB), is marked "cache_served": its fraction is then taken from the
 L2 <-> fabric traffic that rocprofv3 counted for the operator's own dispatches (read
 from profiles/hbm_traffic.md, separate counter runs of this script with --markers: not
 measured here), and is null when no such count exists.  A count below the bytes the
@@ -78,6 +78,19 @@ def brief(rec):
     return out
 
 
+def served_by_caches(roof, measured_copy):
+    """The roofline record with its fraction from the counted traffic where the algorithmic
+    bytes flow faster than a large copy does on this card: then the caches serve part of
+    them."""
+    if not measured_copy or roof.get("cache_served") or roof["effective_GBps"] <= measured_copy:
+        return roof
+    moved = roof.get("traffic")
+    return dict(roof, cache_served=True,
+                frac=round(min(moved, roof["algorithmic_bytes"]) / roof["ms"] / 1e6 / HBM_PEAK_GBS, 4)
+                if moved else None,
+                frac_basis="min(counted traffic, algorithmic bytes)" if moved else None)
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -117,7 +130,7 @@ def main():
     import torch
     import torch.nn.functional as F
 
-    from graphiler_amd import datasets, layers, ops, prepare_graph
+    from graphiler_amd import capi, datasets, layers, ops, prepare_graph
 
     if not torch.cuda.is_available():
         sys.exit("bench.py: no GPU visible")
@@ -361,6 +374,16 @@ def main():
         opsr["gat_aggregate_from_z"] = op_record(
             "c5.gat_aggregate_from_z", lambda: ops.gat_aggregate_from_z(a_l, er1, z1, g, slope),
             fused_bytes, gather=(N * Fw * b, E * Fw * b))
+        # the same operator as the layer runs it: over rows that it keeps apart
+        code = capi.GA_BF16
+        stride = int(capi.load().ga_gather_row_stride(N, Fw, code))
+        z1a = torch.zeros(N, stride, dtype=dt, device=dev)
+        z1a[:, :Fw] = z1
+        opsr["gat_aggregate_rows_apart"] = op_record(
+            "c5.gat_aggregate_rows_apart",
+            lambda: ops._aggregate_rows(a_l, er1, z1a, Fw, H, g, slope, capi.GA_ACT_NONE, code, True),
+            fused_bytes, gather=(N * Fw * b, E * Fw * b))
+        del z1a
         if not args.no_ops:
             opsr["gat_aggregate"] = op_record(
                 "c5.gat_aggregate", lambda: ops.gat_aggregate(el1, er1, z1, g, slope),
@@ -385,9 +408,9 @@ def main():
                     N * (k + Fw) * b + k * Fw * b + 2 * N * H * 4,
                     2.0 * N * k * Fw + 4.0 * N * Fw, "bf16")
         rec["ops"] = opsr = kept(opsr)
-        if "gat_aggregate_from_z" in opsr:
-            roof = dict(opsr["gat_aggregate_from_z"], kernel="gat_aggregate_from_z "
-                        "(runs_kernel<GatPolicy<bf16, 8, from z>> + fix-up)")
+        if "gat_aggregate_rows_apart" in opsr:
+            roof = dict(opsr["gat_aggregate_rows_apart"], kernel="gat_aggregate_rows_apart "
+                        "(runs_kernel<GatPolicy<bf16, 8, from z, rows apart>> + fix-up)")
             if inside:
                 # the headline figure is the operator's duration inside the network steps;
                 # "ms_back_to_back" keeps the repetitions of the operator on its own (its hot
@@ -400,6 +423,8 @@ def main():
                              "frac_algorithmic": round(fused_bytes / ms_in / 1e6 / HBM_PEAK_GBS, 4)})
                 if "traffic" in roof:
                     roof["traffic_GBps"] = round(roof["traffic"] / ms_in / 1e6, 1)
+                    if roof.get("cache_served"):
+                        roof["frac"] = round(min(roof["traffic"], fused_bytes) / ms_in / 1e6 / HBM_PEAK_GBS, 4)
             rec["roofline"] = roof
         if "project_attn_256_256" in opsr:
             rec["mfma"] = dict(opsr["project_attn_256_256"], kernel="project_attn 256 -> 256 bf16 "
@@ -791,7 +816,7 @@ def main():
         ms_step, eps, dtype = hv["ms_per_step"], hv["edges_per_s"], "f32"
     else:
         ms_step, eps, dtype = head["ms_per_step"], head["edges_per_s"], head["dtype"]
-    roof = head["roofline"]
+    roof = served_by_caches(head["roofline"], measured_copy)
     by_traffic = bool(roof.get("cache_served")) and roof.get("traffic") is not None
     roofline = {"kernel": roof["kernel"], "bound": "hbm",
                 "achieved": round(roof["frac"] * HBM_PEAK_GBS, 1) if by_traffic else roof["effective_GBps"],

@@ -70,3 +70,19 @@ def test_a_configuration_in_the_line_is_short():
     assert bench.brief(typed)["variants"]["bf16"] == got
     line = json.dumps({c: bench.brief(typed if c == "c3" else rec) for c in ("c1", "c2", "c3", "c4", "c5")})
     assert len(line) < 5000
+
+
+def test_bytes_faster_than_a_copy_are_served_by_caches():
+    import bench
+    roof = {"effective_GBps": 7800.0, "frac": 0.975, "frac_basis": "algorithmic bytes", "ms": 4.0,
+            "algorithmic_bytes": 31_200_000_000, "traffic": 24_000_000_000}
+    got = bench.served_by_caches(roof, 5000.0)
+    assert got["cache_served"] and got["frac"] == 0.75 and "traffic" in got["frac_basis"]
+    assert bench.served_by_caches(roof, 8000.0) is roof and bench.served_by_caches(roof, None) is roof
+    no_count = {k: v for k, v in roof.items() if k != "traffic"}
+    assert bench.served_by_caches(no_count, 5000.0)["frac"] is None
+
+
+def test_the_headline_divides_by_the_count_of_the_kernel_it_times():
+    import bench
+    assert bench.load_traffic()["c5.gat_aggregate_rows_apart"] >= 2_449_029 * 512
