@@ -91,6 +91,16 @@ int ga_group_edges(const int64_t *key, const int64_t *other, int64_t n_keys,
                    int32_t *status, void *workspace, size_t workspace_bytes,
                    ga_stream_t stream);
 
+/* Both adjacencies of an edge list at once, with half the launches: the in-columns are
+ * ga_group_edges(dst, src, ...), the out-columns ga_group_edges(src, dst, ...); status has two
+ * int32, for a dst and for a src outside [0, n_keys). */
+size_t ga_group_edges_both_workspace_bytes(int64_t n_keys, int64_t n_items);
+int ga_group_edges_both(const int64_t *src, const int64_t *dst, int64_t n_keys, int64_t n_items,
+                        int32_t *in_pointer, int32_t *in_nbr, int32_t *in_eid,
+                        int32_t *out_pointer, int32_t *out_nbr, int32_t *out_eid,
+                        int32_t *status, void *workspace, size_t workspace_bytes,
+                        ga_stream_t stream);
+
 /* The pointer of items whose keys ascend already (type columns: ids of one type are
  * contiguous, include/dglgraph.h:68-71), one pass over the keys.  key (n_items) int64,
  * pointer (n_keys + 1) int32; status two int32 on the device: [0] 1 when a key lies outside

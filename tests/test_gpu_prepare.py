@@ -72,3 +72,36 @@ def test_sorted_pointer_of_few_items(device, key, keys):
     end.record()
     assert status.tolist() == [0, 0] and np.array_equal(pointer.cpu().numpy(), want)
     assert start.elapsed_time(end) < 5.0
+
+
+# tiles of 2,048 (up to 700,000 items) and 4,096 items, digits of up to ten bits: one, two and
+# three passes; the library's sort above 16,777,216 items is what the large graphs' tests run
+@pytest.mark.parametrize("keys,n", [(1, 1), (2, 2048), (5, 2049), (1024, 4097), (1025, 70_000),
+                                    (1 << 20, 33_000), ((1 << 20) + 1, 33_001), ((1 << 30) + 7, 2047),
+                                    (94_806, 700_000), (94_806, 700_001), (3000, 1_000_003)])
+@pytest.mark.parametrize("kind", ["uniform", "hub", "ends"])
+def test_grouping_is_a_stable_sort(device, keys, n, kind):
+    rng = np.random.default_rng(n)
+    src, dst = rng.integers(0, keys, n), rng.integers(0, keys, n)
+    if kind == "hub":
+        dst[rng.random(n) < 0.9] = keys // 2
+    elif kind == "ends":
+        src, dst = (keys - 1) * rng.integers(0, 2, n), np.full(n, keys - 1)
+    dev = [torch.from_numpy(a).to(device) for a in (src, dst)]
+    status = torch.empty(2, dtype=torch.int32, device=device)
+    sides = G._group_both(*dev, keys, status) if keys <= 1 << 21 else \
+        [G.group_on_device(dev[1], dev[0], keys)[:3], G.group_on_device(dev[0], dev[1], keys)[:3]]
+    for (pointer, nbr, eid), key, other in zip(sides, (dst, src), (src, dst)):
+        order = np.argsort(key, kind="stable")
+        assert np.array_equal(eid.cpu().numpy(), order)
+        assert np.array_equal(nbr.cpu().numpy(), other[order])
+        at = np.unique(rng.integers(0, keys + 1, 1000))
+        want = np.searchsorted(key[order], at)
+        assert np.array_equal(pointer[torch.from_numpy(at).to(device)].cpu().numpy(), want)
+    if keys <= 1 << 21:
+        assert status.tolist() == [0, 0]
+        for bad, want in ((0, [0, 1]), (1, [1, 0])):
+            dev[bad][n // 2] = keys if bad else -1
+            G._group_both(*dev, keys, status)
+            assert status.tolist() == want
+            dev[bad][n // 2] = 0
