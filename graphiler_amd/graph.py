@@ -429,10 +429,13 @@ def _group_both(src: torch.Tensor, dst: torch.Tensor, num_nodes: int, status: to
     return sides
 
 
-# Host arrays go through page-locked pieces of this size, copied by all host threads while
-# the piece before is on its way: 17 MB of edges and types 330 us instead of 540 as pageable
-# memory (52 : 31 GB/s); arrays below a piece's quarter are not worth one.
-_UPLOAD_PIECE = 4 << 20
+# Host columns go to the device as 32-bit ids, which is all that a valid one holds, and are
+# widened there: the link moves half the bytes.  Pieces of this many ids go through page-locked
+# memory, narrowed and checked by all host threads while the piece before is on its way (82 us
+# for a full one).  The host's calls per piece bound small columns: 17 MB of edges and types in
+# pieces of 2 MB 330 us, of 4 MB 263, as 64-bit ids 460.  A column below a sixteenth of a piece
+# goes over directly.
+_UPLOAD_PIECE = 1 << 20
 _UPLOAD_PIECES = 3
 
 
@@ -441,24 +444,31 @@ def _upload(arrays, dev):
     torch's host allocator and are given back on return; one is written again only when
     the copy out of it is done."""
     outs = [torch.empty(a.shape, dtype=torch.int64, device=dev) for a in arrays]
-    step = _UPLOAD_PIECE // 8
     ring, used = [], 0
     for a, out in zip(arrays, outs):
         host, out = torch.from_numpy(a).view(-1), out.view(-1)
-        if a.nbytes < _UPLOAD_PIECE // 4:
+        if a.size < _UPLOAD_PIECE // 16:
             out.copy_(host)
             continue
-        for lo in range(0, a.size, step):
-            n = min(step, a.size - lo)
+        narrow = torch.empty(a.size, dtype=torch.int32, device=dev)
+        for lo in range(0, a.size, _UPLOAD_PIECE):
+            n = min(_UPLOAD_PIECE, a.size - lo)
             if len(ring) < _UPLOAD_PIECES:
-                ring.append((torch.empty(step, dtype=torch.int64, pin_memory=True), torch.cuda.Event()))
+                ring.append((torch.empty(_UPLOAD_PIECE, dtype=torch.int32, pin_memory=True),
+                             torch.cuda.Event()))
             piece, done = ring[used % _UPLOAD_PIECES]
             if used >= _UPLOAD_PIECES:
                 done.synchronize()
             piece[:n].copy_(host[lo:lo + n])
-            out[lo:lo + n].copy_(piece[:n], non_blocking=True)
+            narrow[lo:lo + n].copy_(piece[:n], non_blocking=True)
             done.record(torch.cuda.current_stream(dev))
             used += 1
+            least, most = torch.aminmax(host[lo:lo + n])
+            if int(least) < -2 ** 31 or int(most) >= 2 ** 31:
+                out.copy_(host)         # no id of a graph: whole, for whoever reports it
+                break
+        else:
+            out.copy_(narrow)
     return outs
 
 

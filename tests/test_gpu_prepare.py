@@ -105,3 +105,31 @@ def test_grouping_is_a_stable_sort(device, keys, n, kind):
             G._group_both(*dev, keys, status)
             assert status.tolist() == want
             dev[bad][n // 2] = 0
+
+
+# a piece holds 1,048,576 ids, columns below 65,536 go over directly, and a column with a value
+# that 32 bits do not hold goes over whole
+@pytest.mark.parametrize("sizes", [(65_535, 65_536), (1_048_576, 1_048_577, 70_000, 3_300_000)])
+@pytest.mark.parametrize("odd", [None, 2 ** 31, -2 ** 31 - 1, 2 ** 40 + 5])
+def test_upload_of_ids(device, sizes, odd):
+    rng = np.random.default_rng(sum(sizes))
+    arrays = [rng.integers(-2 ** 31, 2 ** 31, n) for n in sizes]
+    if odd is not None:
+        for a in arrays:
+            a[-1] = odd
+    for got, want in zip(G._upload(arrays, device), arrays):
+        assert got.dtype == torch.int64 and np.array_equal(got.cpu().numpy(), want)
+
+
+def test_ids_beyond_32_bits_are_reported(device):
+    n = 100_000
+    src = np.arange(n) % 50
+    bad = src.copy()
+    bad[7] += 2 ** 32            # a valid id in its lower half
+    for s, d in ((bad, src), (src, bad)):
+        with pytest.raises(ValueError, match="endpoint"):
+            prepare_graph(s, d, 50, device=device)
+    types = np.sort(src) * 0
+    types[-1] = 2 ** 32
+    with pytest.raises(ValueError, match="type outside"):
+        prepare_graph(src, src, 50, device=device, etype_of=types, num_etypes=3)
