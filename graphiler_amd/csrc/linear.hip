@@ -10,12 +10,13 @@
 // operand value is split into three bf16 pieces, x = x0 + x1 + x2 (8 significant
 // bits each, 24 in all; exact down to 2^-110, below which the third leaves bf16's
 // range), and the product is accumulated in fp32 from the six piece products x0w0 +
-// x0w1 + x1w0 + x1w1 + x0w2 + x2w0; each is exact in fp32.  The pieces are cut off,
-// not rounded, so the three dropped products reach 7.8 x 2^-24 of |x||w| at the worst
-// significands (0.7 x 2^-24 on average) and have the product's sign.  Measured against
-// float64 on values of both signs the result is as close as the fp32 instruction's (max
-// error / max |Z| 8e-7 against 1.2e-6 at K = 602).  Non-finite inputs give NaN (inf -
-// inf in the split) where fp32 products may give inf.
+// x0w1 + x1w0 + x1w1 + x0w2 + x2w0; each is exact in fp32.  The first piece is cut off (no
+// value of float's range overflows), the second rounded to nearest, so what the three dropped
+// products reach, below 2^-23 of |x||w|, has no sign of its own: with all three pieces cut off
+// it had the product's, which showed where all products are positive (error against float64,
+// 2-norm, 2,708 x 1433 -> 64: 1.3e-6 -> 0.8e-7, 10,000 x 600 3.2e-7 -> 0.8e-7, the vendor
+// GEMM 1.5e-7 and 3.7e-7; products of both signs 3.8e-7 -> 3.7e-7 at K = 602).  Non-finite
+// inputs give NaN (inf - inf in the split) where fp32 products may give inf.
 //
 // A workgroup (4 waves) owns 128 rows, each wave 32 rows (2 tiles of 16) x 64
 // columns per pass.  Both operands go global -> registers -> LDS in
@@ -46,23 +47,24 @@ namespace {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// x = p0 + p1 + p2 (exactly from 2^-110 up), each piece a bf16 (the top 8 significant
-// bits of what the pieces before it leave); eight values -> three packed operands.
+// x = p0 + p1 + p2 (exactly from 2^-110 up), each piece a bf16: the top 8 significant bits, what
+// they leave rounded to 8 bits, the rest (of either sign); eight values -> three packed operands.
 __device__ __forceinline__ void split8(const float (&v)[8], uint4 &p0, uint4 &p1, uint4 &p2) {
-  uint32_t a[8], b[8], c[8];
+  uint32_t a[8], b[4], c[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
+  for (int j = 0; j < 8; j += 2) {
     a[j] = __float_as_uint(v[j]);
-    const float r1 = v[j] - __uint_as_float(a[j] & 0xffff0000u);
-    b[j] = __float_as_uint(r1);
-    const float r2 = r1 - __uint_as_float(b[j] & 0xffff0000u);
-    c[j] = __float_as_uint(r2);
+    a[j + 1] = __float_as_uint(v[j + 1]);
+    const float r0 = v[j] - __uint_as_float(a[j] & 0xffff0000u);
+    const float r1 = v[j + 1] - __uint_as_float(a[j + 1] & 0xffff0000u);
+    b[j / 2] = pack_bf16(r0, r1);
+    c[j] = __float_as_uint(r0 - bf16_lo(b[j / 2]));
+    c[j + 1] = __float_as_uint(r1 - bf16_hi(b[j / 2]));
   }
   constexpr uint32_t hi = 0x07060302u;                   // high halves of (S1, S0)
   p0 = uint4{__builtin_amdgcn_perm(a[1], a[0], hi), __builtin_amdgcn_perm(a[3], a[2], hi),
              __builtin_amdgcn_perm(a[5], a[4], hi), __builtin_amdgcn_perm(a[7], a[6], hi)};
-  p1 = uint4{__builtin_amdgcn_perm(b[1], b[0], hi), __builtin_amdgcn_perm(b[3], b[2], hi),
-             __builtin_amdgcn_perm(b[5], b[4], hi), __builtin_amdgcn_perm(b[7], b[6], hi)};
+  p1 = uint4{b[0], b[1], b[2], b[3]};
   p2 = uint4{__builtin_amdgcn_perm(c[1], c[0], hi), __builtin_amdgcn_perm(c[3], c[2], hi),
              __builtin_amdgcn_perm(c[5], c[4], hi), __builtin_amdgcn_perm(c[7], c[6], hi)};
 }
@@ -311,11 +313,134 @@ linear_attn_kernel(
   }
 }
 
-}  // namespace
-}  // namespace ga
 
-namespace ga {
-namespace {
+// ---- few rows ------------------------------------------------------------------------------
+// A grid of 128-row workgroups that leaves most CUs idle takes as long as one workgroup's chain
+// of k slices.  Here a workgroup owns 16 rows and its KS wavefronts share out the slices: each
+// loads its operands straight into the layout of the matrix instruction (two 16-byte loads of a
+// row and eight of W per column block and slice, the next slice's behind this one's), splits
+// them as above, and the partial tiles are added through LDS in the order of the wavefronts.
+// Shorter chains also round less: error against float64 at K = 1433 5.5e-7 -> 2.0e-7.
+// us before (128-row workgroups) -> here: 2,708 x 1433 -> 64 73 -> 10, 5,000 x 300 -> 64 15 -> 7,
+// 19,717 x 500 -> 16 17.7 -> 8.7, 100,000 x 300 -> 32 39 -> 32.  16 columns of many rows run at
+// the rate X is read at (232,965 x 602, 4.4 TB/s, both forms).
+template <bool HAS_ATTN, int KS, int NCB>
+__global__ __launch_bounds__(KS * kWave) void linear_few_rows_kernel(
+    const float *__restrict__ X, const float *__restrict__ W, const float *__restrict__ a_l,
+    const float *__restrict__ a_r, float *__restrict__ Z, float *__restrict__ el,
+    float *__restrict__ er, const float *__restrict__ row_scale, int64_t rows, int K, int M,
+    int heads, int ldz) {
+  constexpr int kRows = 16, kCols = NCB * 16, kTile = kRows * kCols;
+  __shared__ float part[KS][kTile];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int lr = lane & 15, lk = lane >> 4;
+  const int col0 = blockIdx.y * kCols;
+  const int64_t row0 = (int64_t)blockIdx.x * kRows;
+  const int n_slices = (K + kSliceK - 1) / kSliceK;
+  const rsrc_t xrs = make_rsrc(X + row0 * K, (uint64_t)min((int64_t)kRows, rows - row0) * K * 4);
+  const rsrc_t wrs = make_rsrc(W, (uint64_t)K * M * 4);
+  const uint32_t xoff = (uint32_t)((min(row0 + lr, rows - 1) - row0) * K + lk * 8) * 4u;
+  uint32_t woff[NCB];
+#pragma unroll
+  for (int cb = 0; cb < NCB; ++cb)
+    woff[cb] = ((uint32_t)(lk * 8) * M + min(col0 + cb * 16 + lr, M - 1)) * 4u;
+  floatx4 acc[NCB];
+#pragma unroll
+  for (int cb = 0; cb < NCB; ++cb) acc[cb] = floatx4{0, 0, 0, 0};
+  struct Slice {
+    float4 x[2];
+    float w[NCB][8];
+  };
+  // Loads past the end of X and of W give 0 (the lane offsets are range-checked; W's columns are
+  // clamped, so an offset past K rows is past its end); what the last slice reads of the row
+  // behind it is cleared before it is multiplied.
+  auto fetch = [&](int sl, Slice &s) __attribute__((always_inline)) {
+    const uint32_t xs = xoff + (uint32_t)sl * (kSliceK * 4);
+    const uint32_t ws = (uint32_t)sl * kSliceK * (uint32_t)M * 4u;
+    s.x[0] = BufLoad<4>::at(xrs, xs, 0);
+    s.x[1] = BufLoad<4>::at(xrs, xs + 16, 0);
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb)
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        s.w[cb][j] = BufLoad<1>::at(wrs, woff[cb] + ws + (uint32_t)(j * M) * 4u, 0);
+  };
+  auto multiply = [&](int sl, const Slice &s) __attribute__((always_inline)) {
+    float v[8] = {s.x[0].x, s.x[0].y, s.x[0].z, s.x[0].w, s.x[1].x, s.x[1].y, s.x[1].z, s.x[1].w};
+    if (sl * kSliceK + kSliceK > K) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = sl * kSliceK + lk * 8 + j < K ? v[j] : 0.0f;
+    }
+    uint4 xp[3];
+    split8(v, xp[0], xp[1], xp[2]);
+    constexpr int px[6] = {2, 0, 1, 1, 0, 0}, pw[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb) {
+      uint4 wp[3];
+      split8(s.w[cb], wp[0], wp[1], wp[2]);
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+        acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xp[px[q]]),
+                                                          __builtin_bit_cast(bf16x8, wp[pw[q]]),
+                                                          acc[cb], 0, 0, 0);
+    }
+  };
+  if (wave < n_slices) {
+    Slice a, b;
+    fetch(wave, a);
+    for (int sl = wave; sl < n_slices; sl += 2 * KS) {
+      if (sl + KS < n_slices) fetch(sl + KS, b);
+      multiply(sl, a);
+      if (sl + KS >= n_slices) break;
+      if (sl + 2 * KS < n_slices) fetch(sl + 2 * KS, a);
+      multiply(sl + KS, b);
+    }
+  }
+#pragma unroll
+  for (int cb = 0; cb < NCB; ++cb)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) part[wave][(lk * 4 + r) * kCols + cb * 16 + lr] = acc[cb][r];
+  __syncthreads();
+  const int dph = M / heads;
+#pragma unroll
+  for (int i = threadIdx.x; i < kTile; i += KS * kWave) {   // lane = column, or several rows of them
+    float z = 0.0f;
+#pragma unroll
+    for (int w = 0; w < KS; ++w) z += part[w][i];
+    const int64_t row = row0 + i / kCols;
+    const int c = col0 + i % kCols;
+    const bool live = row < rows && c < M;
+    if (!HAS_ATTN && row_scale && live) z *= row_scale[row];
+    if (live) Z[row * ldz + c] = z;
+    if constexpr (HAS_ATTN) {             // a head's columns lie in one wavefront
+      float l = row16_sum(c < M ? z * a_l[c] : 0.0f), r = row16_sum(c < M ? z * a_r[c] : 0.0f);
+      if (dph >= 32) { l += __shfl_xor(l, 16); r += __shfl_xor(r, 16); }
+      if (dph == 64) { l += __shfl_xor(l, 32); r += __shfl_xor(r, 32); }
+      if (live && c % dph == 0) {
+        el[row * heads + c / dph] = l;
+        er[row * heads + c / dph] = r;
+      }
+    }
+  }
+}
+
+// Where the form above is the faster one, from 16 to 232,965 rows of 16 to 1,433 values.  Up to
+// 32 columns: small grids, and long rows up to where both wait for X (us here : there; 40,000 x
+// 32 -> 32 7.7 : 6.3, 40,000 x 128 -> 16 6.1 : 8.5, 100,000 x 300 -> 32 32 : 39, 232,965 x 602 ->
+// 32 180 : 155).  64 columns: W is read and split once per 16 rows, so the time grows with tiles
+// and slices, while the other form's, on a grid of one round, is its chain; the attention terms
+// cost up to 3 us here and 1.3 there (with them 10,000 x 64 8.9 : 7.4, 16,000 x 128 10.4 : 9.8,
+// 10,000 x 600 17.7 : 25.9; without 30,000 x 600 33 : 26, 16,000 x 1433 39 : 73).  One line for
+// both, so that Z does not depend on whether they are asked for.
+bool few_rows(int64_t rows, int64_t K, int64_t M) {
+  if ((K + kSliceK) * M >= ((int64_t)1 << 29)) return false;       // 32-bit offsets into W
+  const int64_t slices = (K + kSliceK - 1) / kSliceK;
+  if (M <= 32) return rows <= 20'000 || (slices >= 4 && rows <= 150'000);
+  const double tiles = (double)((rows + 15) / 16) * (double)((M + 63) / 64);
+  return tiles <= 2048 && tiles * (6e-3 + 0.68e-3 * slices) < 1.0 + 1.15 * slices;
+}
+
 int launch_linear(const float *X, const float *W, const float *a_l, const float *a_r, float *Z,
                   float *el, float *er, const float *row_scale, int64_t rows, int64_t K,
                   int64_t M, int64_t heads, int64_t ldz, ga_stream_t stream) {
@@ -338,6 +463,29 @@ int launch_linear(const float *X, const float *W, const float *a_l, const float 
   const int64_t gy = (M + kPassCols - 1) / kPassCols;
   if (gx > 0x7fffffff || gy > 65535) return GA_EUNSUPPORTED;
   hipStream_t s = (hipStream_t)stream;
+  if (few_rows(rows, K, M)) {
+    const int ncb = M > 32 ? 4 : M > 16 ? 2 : 1;
+    const dim3 grid((unsigned)((rows + 15) / 16), (unsigned)((M + 16 * ncb - 1) / (16 * ncb)));
+#define GA_LAUNCH_FEW(ATTN, KS, NCB)                                                               \
+  hipLaunchKernelGGL((linear_few_rows_kernel<ATTN, KS, NCB>), grid, dim3(KS * kWave), 0, s, X, W,  \
+                     a_l, a_r, Z, el, er, row_scale, rows, (int)K, (int)M, (int)heads, (int)ldz)
+#define GA_LAUNCH_FEW_NCB(ATTN, KS)                 \
+  do {                                              \
+    if (ncb == 4) GA_LAUNCH_FEW(ATTN, KS, 4);       \
+    else if (ncb == 2) GA_LAUNCH_FEW(ATTN, KS, 2);  \
+    else GA_LAUNCH_FEW(ATTN, KS, 1);                \
+  } while (0)
+    // at most a workgroup per CU: eight wavefronts halve the chain (2,708 x 1433 -> 64 13.8 ->
+    // 10.2 us); with more they crowd each other (19,717 x 500 -> 64 20 -> 24)
+    const bool crowded = grid.x * grid.y > 256;
+    if (attn && crowded) GA_LAUNCH_FEW_NCB(true, 4);
+    else if (attn) GA_LAUNCH_FEW_NCB(true, 8);
+    else if (crowded) GA_LAUNCH_FEW_NCB(false, 4);
+    else GA_LAUNCH_FEW_NCB(false, 8);
+#undef GA_LAUNCH_FEW_NCB
+#undef GA_LAUNCH_FEW
+    return launch_status();
+  }
 #define GA_LAUNCH_LINEAR_NCB(ATTN, VK, WAVES, NCB)                                  \
   hipLaunchKernelGGL((linear_attn_kernel<ATTN, VK, WAVES, NCB>),                   \
                      dim3((unsigned)gx, (unsigned)gy), dim3(kBlock), 0, s, X, W, a_l, a_r, Z, el, \

@@ -1218,12 +1218,23 @@ def relation_pair_attention(k, q, v, relation_att, relation_msg, relation_scale,
 
 
 # ------------------------------------------------------ dense projection ----
-# fp32 projections with at most this many output columns and at least this many rows
-# run on the library's own kernel (one pass over the rows, 1.2-2.1x the rate of the
-# vendor GEMM on an MI355X at these tall-and-narrow shapes); wider or shorter ones
-# are the vendor GEMM's ground (several column passes / too few workgroups here).
+# fp32 projections with at most this many output columns run on the library's own kernels:
+# with at least this many rows (one pass over the rows, 1.2-2.1x the rate of the vendor GEMM
+# on an MI355X at these tall-and-narrow shapes), and with fewer where 16 rows a workgroup are
+# the faster form (ga_linear_attn; 2,708 x 1433 -> 64 10 us against the vendor GEMM's 13, whose
+# call also costs the host 19 us instead of 9; 8,000 x 1433 22 against 17).  Wider ones are the
+# vendor GEMM's ground (several column passes here).
 LINEAR_MAX_COLS = 64
 LINEAR_MIN_ROWS = 16384
+LINEAR_FEW_ROWS_MAX_K = 2048
+LINEAR_FEW_ROWS_MAX_SIZE = 8 << 20      # values of x, with more than 32 output columns
+
+
+def _own_linear(rows: int, k: int, m: int) -> bool:
+    if m > LINEAR_MAX_COLS:
+        return False
+    return rows >= LINEAR_MIN_ROWS or (k <= LINEAR_FEW_ROWS_MAX_K
+                                       and (m <= 32 or rows * k <= LINEAR_FEW_ROWS_MAX_SIZE))
 
 
 def linear(x, weight, row_scale=None):
@@ -1239,7 +1250,8 @@ def linear(x, weight, row_scale=None):
         raise RuntimeError("row_scale must be (rows,) or (rows, 1) float32")
     if (x.dtype == torch.float32 and weight.dtype == torch.float32 and x.dim() == 2
             and weight.dim() == 2 and x.is_cuda and x.is_contiguous() and weight.is_contiguous()
-            and weight.shape[1] <= LINEAR_MAX_COLS and x.shape[0] >= LINEAR_MIN_ROWS):
+            and weight.shape[0] > 0 and weight.shape[1] > 0 and x.shape[0] > 0
+            and _own_linear(int(x.shape[0]), int(weight.shape[0]), int(weight.shape[1]))):
         if row_scale is None:
             return linear_attn(x, weight)
         _check_input(row_scale, "row_scale")

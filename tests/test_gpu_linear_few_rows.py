@@ -1,0 +1,50 @@
+"""The projection in tiles of 16 rows (ga_linear_attn on small grids and few columns): edges of
+its tiles, k slices and column blocks against float64, the attention terms and the row factor."""
+import numpy as np
+import pytest
+import torch
+
+from graphiler_amd import ops
+from helpers import TOL_F32, assert_close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 4097])
+@pytest.mark.parametrize("k", [1, 7, 31, 32, 33, 256, 259, 545])
+@pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 64])
+def test_plain(device, rows, k, m):
+    """k up to 17 slices: four and eight wavefronts with none, one, two and three each."""
+    gen = torch.Generator(device=device).manual_seed(rows + 100 * k + m)
+    x = torch.randn(rows, k, device=device, generator=gen)
+    w = torch.randn(k, m, device=device, generator=gen)
+    s = torch.rand(rows, device=device, generator=gen)
+    got = ops.linear(x, w)
+    want, size = x.double() @ w.double(), x.double().abs() @ w.double().abs()
+    assert_close(got.cpu().numpy(), want.cpu().numpy(), TOL_F32, "z", mag=size.cpu().numpy())
+    assert torch.equal(ops.linear(x, w, row_scale=s), got * s[:, None])
+    # a row that is not finite stays alone, and so does a column of the weights
+    x[rows // 2, k - 1] = float("inf")
+    bad = torch.isfinite(ops.linear(x, w)).all(1)
+    assert not bad[rows // 2] and bad.sum() == rows - 1
+    x[rows // 2, k - 1] = 1.0
+    w[0, m - 1] = float("nan")
+    cols = torch.isfinite(ops.linear(x, w)).all(0)
+    assert not cols[m - 1] and cols[:m - 1].all()
+
+
+@pytest.mark.parametrize("rows,k", [(1, 5), (17, 64), (4096, 130), (4113, 300)])
+@pytest.mark.parametrize("heads,dim", [(1, 16), (1, 32), (2, 16), (1, 64), (2, 32), (4, 16), (3, 16), (2, 64), (8, 16)])
+def test_attention_terms(device, rows, k, heads, dim):
+    rng = np.random.default_rng(rows + k + heads)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    w = rng.standard_normal((k, heads * dim)).astype(np.float32) / np.float32(np.sqrt(k))
+    a = rng.standard_normal((2, heads, dim)).astype(np.float32)
+    dev = [torch.from_numpy(t).to(device) for t in (x, w, a[0], a[1])]
+    z, el, er = ops.linear_attn(*dev)
+    zr = (x.astype(np.float64) @ w).reshape(rows, heads, dim)
+    zm = (np.abs(x).astype(np.float64) @ np.abs(w)).reshape(rows, heads, dim)
+    assert_close(z.cpu().numpy(), zr.reshape(rows, -1), TOL_F32, "z", mag=zm.reshape(rows, -1))
+    for got, v in ((el, a[0]), (er, a[1])):
+        assert_close(got.cpu().numpy(), (zr * v).sum(2), TOL_F32, "terms", mag=(zm * np.abs(v)).sum(2))
+    assert torch.equal(ops.linear_attn(*dev[:2]), z)
