@@ -38,6 +38,7 @@ SIGNATURES = {
     "ga_group_edges_both_workspace_bytes": (_sz, [_i64, _i64]),
     "ga_group_edges_both": (_int, [_vp, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                    _sz, _vp]),
+    "ga_row_lengths": (_int, [_vp, _i64, ctypes.c_float, _vp, _vp]),
     "ga_sorted_pointer": (_int, [_vp, _i64, _i64, _vp, _vp, _vp]),
     "ga_spmm_workspace_bytes": (_sz, [_i64, _i64]),
     "ga_spmm_csr": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64,

@@ -200,6 +200,14 @@ __global__ __launch_bounds__(kBlock) void class_scatter_kernel(
   }
 }
 
+// Row lengths as fp32, at least `least`: the degrees a layer's norm is made of, one launch
+// instead of a subtraction, a conversion and a clamp (5 us each on 2,708 nodes, host included).
+__global__ __launch_bounds__(kBlock) void row_lengths_kernel(
+    const int32_t *__restrict__ pointer, int64_t n_rows, float least, float *__restrict__ out) {
+  const int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (v < n_rows) out[v] = fmaxf((float)(pointer[v + 1] - pointer[v]), least);
+}
+
 // Rows and their items by the power of two below a row's length: integers, so the order in
 // which the workgroups add them does not matter.
 __global__ __launch_bounds__(kBlock) void degree_buckets_kernel(
@@ -588,6 +596,17 @@ int ga_group_edges_both(const int64_t *src, const int64_t *dst, int64_t n_keys, 
   S[1].key = src; S[1].other = dst;
   S[1].pointer = out_pointer; S[1].nbr = out_nbr; S[1].eid = out_eid; S[1].status = status + 1;
   return group_sides(S, 2, n_keys, n_items, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int ga_row_lengths(const int32_t *pointer, int64_t n_rows, float least, float *out,
+                   ga_stream_t stream) {
+  using namespace ga;
+  if (n_rows < 0 || n_rows > 0x7ffffffe || (n_rows > 0 && (!pointer || !out))) return GA_EINVAL;
+  if (!aligned(pointer, 4) || !aligned(out, 4)) return GA_EALIGN;
+  if (n_rows == 0) return GA_OK;
+  hipLaunchKernelGGL(row_lengths_kernel, dim3((unsigned)((n_rows + kBlock - 1) / kBlock)), dim3(kBlock),
+                     0, (hipStream_t)stream, pointer, n_rows, least, out);
+  return launch_status();
 }
 
 int ga_degree_buckets(const int32_t *pointer, int64_t n_rows, int64_t *buckets, ga_stream_t stream) {

@@ -1039,8 +1039,11 @@ torch::Tensor SegmentMMEdgeGather(torch::Tensor features, torch::Tensor weights,
 // and reduce steps (examples/RGCN/RGCN.py:25-33).  One pass without the per-edge
 // messages where that kernel is the faster one (the small products: K * M up to 2048,
 // e.g. 16 -> 64 and 64 -> 8), the two operators elsewhere.
-torch::Tensor TypedSpMMEdge(torch::Tensor features, torch::Tensor weights,
-                            at::optional<torch::Tensor> row_scale, const GraphPtr &graph) {
+// `activation`: of the fp32 sums before they are stored, afterwards on the operators' route.
+torch::Tensor TypedSpMMEdgeAct(torch::Tensor features, torch::Tensor weights,
+                               at::optional<torch::Tensor> row_scale, int64_t activation,
+                               const GraphPtr &graph) {
+  TORCH_CHECK(activation >= GA_ACT_NONE && activation <= GA_ACT_ELU, "unknown activation");
   const MmShape s = edge_mm_shape(features, weights, graph);
   const torch::Tensor factor = kernel_row_factor(row_scale, graph->num_edges, features);
   const float *rs = factor.defined() ? factor.data_ptr<float>() : nullptr;
@@ -1054,19 +1057,25 @@ torch::Tensor TypedSpMMEdge(torch::Tensor features, torch::Tensor weights,
       s.K * s.M <= 2048 && accurate) {
     const DGLGraph::TypedTiles &t = graph->typed_tiles();
     torch::Tensor out = torch::empty({graph->num_nodes, s.M}, features.options());
-    const int rc = ga_typed_spmm(
+    const int rc = ga_typed_spmm_act(
         t.tile_chunk_pointer.data_ptr<int>(), t.chunk_type.data_ptr<int>(),
         t.slot_src.data_ptr<int>(), t.slot_dst.data_ptr<uint8_t>(), t.slot_edge.data_ptr<int>(),
         features.data_ptr(), weights.data_ptr(), rs, out.data_ptr(), graph->num_nodes,
-        features.size(0), graph->num_edges, graph->num_etypes, t.tile_rows, s.K, s.M, s.dt,
-        current_stream(out));
+        features.size(0), graph->num_edges, graph->num_etypes, t.tile_rows, s.K, s.M,
+        (int)activation, s.dt, current_stream(out));
     if (rc != GA_EUNSUPPORTED) {
-      check_ga(rc, "ga_typed_spmm");
+      check_ga(rc, "ga_typed_spmm_act");
       return out;
     }
   }
-  return spmm(graph, GA_COPY_E, GA_SUM, SegmentMMEdgeGather(features, weights, 0, row_scale, graph),
-              at::nullopt, false);
+  torch::Tensor out = spmm(graph, GA_COPY_E, GA_SUM,
+                           SegmentMMEdgeGather(features, weights, 0, row_scale, graph), at::nullopt, false);
+  return activation == GA_ACT_RELU ? at::relu(out) : activation == GA_ACT_ELU ? at::elu(out) : out;
+}
+
+torch::Tensor TypedSpMMEdge(torch::Tensor features, torch::Tensor weights,
+                            at::optional<torch::Tensor> row_scale, const GraphPtr &graph) {
+  return TypedSpMMEdgeAct(features, weights, row_scale, GA_ACT_NONE, graph);
 }
 
 // out[e, h] = <features[endpoint(e)] @ weights[type(e)], other[other_endpoint(e)]>
@@ -1576,6 +1585,9 @@ static auto registry =
         .op("my_ops::TypedSpMMEdge(Tensor x, Tensor w, Tensor? row_scale, " GRAPH_T
             " g) -> Tensor z",
             &TypedSpMMEdge)
+        .op("my_ops::TypedSpMMEdgeAct(Tensor x, Tensor w, Tensor? row_scale, int activation, " GRAPH_T
+            " g) -> Tensor z",
+            &TypedSpMMEdgeAct)
         .op("my_ops::SegmentMMNodeStacked(Tensor x, Tensor[] ws, " GRAPH_T " g) -> Tensor[] zs",
             &SegmentMMNodeStacked)
         .op("my_ops::SegmentMMNodeScaled(Tensor x, Tensor w, Tensor row_scale, " GRAPH_T

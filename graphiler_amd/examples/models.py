@@ -38,6 +38,7 @@ def plan(name: str, level: int):
             "GCN": (udf.gcn_message, udf.gcn_reduce, None),
             "GAT": (udf.gat_message, udf.gat_reduce, None),
             "RGCN": (udf.rgcn_message, udf.rgcn_reduce, None),
+            "RGCN+relu": (udf.rgcn_message, udf.rgcn_reduce_relu, None),
             "HGT": (udf.hgt_message, udf.hgt_reduce, udf.hgt_update),
         }[name]
         _PLANS[key] = mpdfg_builder(*fns, opt_level=level)
@@ -100,9 +101,10 @@ class GCN:
 
     def __call__(self, g: GraphData, features, mode=2):
         ptr = g.graph.in_pointer
-        g.ndata['degree'] = (ptr[1:] - ptr[:-1]).float().clamp(min=1).unsqueeze(1)
-        x = F.relu(self._layer(g, features, self.w1, mode))
-        return self._layer(g, x, self.w2, mode)
+        g.ndata['degree'] = (ptr[1:] - ptr[:-1]).float().clamp(min=1).unsqueeze(1) \
+            if mode in EAGER else ops.in_degrees(g.graph, at_least=1)
+        # a layer ends in the relu of its reduce function: one between the layers changes nothing
+        return self._layer(g, self._layer(g, features, self.w1, mode), self.w2, mode)
 
 
 # ---- GAT (one head) ------------------------------------------------------------------
@@ -137,18 +139,19 @@ class RGCN:
         self.w1 = _param(rng, (num_rels, in_dim, hidden_dim), device)
         self.w2 = _param(rng, (num_rels, hidden_dim, out_dim), device)
 
-    def _layer(self, g, x, w, norm, mode):
+    def _layer(self, g, x, w, norm, mode, relu):
         g.ndata['h'], g.edata['norm'], g.etype_data['weight'] = x, norm, w
         if mode in EAGER:
             msg = _typed_rows(x[g.graph.COO_src], w, g.graph.etype_COO) * norm
-            g.ndata['h'] = _sum_by_dst(g, msg, mode)
+            h = _sum_by_dst(g, msg, mode)
+            g.ndata['h'] = F.relu(h) if relu else h
         else:
-            update_all(g, plan("RGCN", mode))
+            update_all(g, plan("RGCN+relu" if relu else "RGCN", mode))
         return g.ndata.pop('h')
 
     def __call__(self, g: GraphData, features, norm, mode=2):
-        x = F.relu(self._layer(g, features, self.w1, norm, mode))
-        return self._layer(g, x, self.w2, norm, mode)
+        x = self._layer(g, features, self.w1, norm, mode, relu=True)
+        return self._layer(g, x, self.w2, norm, mode, relu=False)
 
 
 # ---- HGT (single head) -------------------------------------------------------------------

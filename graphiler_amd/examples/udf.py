@@ -69,6 +69,11 @@ def rgcn_reduce(nodes: NodeBatchDummy):
     return {'h': torch.sum(nodes.mailbox['m'], dim=1)}
 
 
+def rgcn_reduce_relu(nodes: NodeBatchDummy):
+    """A layer that another one follows (examples/RGCN/RGCN.py:69)."""
+    return {'h': torch.relu(torch.sum(nodes.mailbox['m'], dim=1))}
+
+
 # ---- HGT (single head, as the reference's simplified layer) ----------------------
 def hgt_message(edges: EdgeBatchDummy, sqrt_dk: float):
     k = torch.bmm(edges.src['h'].unsqueeze(1), edges.srctype['k_weight']).squeeze()

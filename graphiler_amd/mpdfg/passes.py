@@ -520,11 +520,27 @@ class _Rewriter:
         # last: only the sums no other rewrite has taken
         for n in list(self.G.nodes()):
             if n.kind() in ("aten::relu", "aten::elu"):
-                changed |= self._fuse_spmm_tail(n)
+                changed |= self._fuse_typed_tail(n) or self._fuse_spmm_tail(n)
         for n in list(self.G.nodes()):
             if n.kind() == "aten::mul":
                 changed |= self._fuse_spmm_tail(n)
         return changed
+
+    def _fuse_typed_tail(self, n) -> bool:
+        """relu(TypedSpMMEdge(x, w, s)) -> TypedSpMMEdgeAct(x, w, s, 1): the activation between
+        two RGCN layers (examples/RGCN/RGCN.py:69) where the sums are stored."""
+        top = n.inputsAt(0)
+        sp = top.node()
+        if n.kind() != "aten::relu" or sp.kind() != "my_ops::TypedSpMMEdge" or not self.single_use(top) \
+                or _mutated(top):
+            return False
+        out = self.make("my_ops::TypedSpMMEdgeAct",
+                        [sp.inputsAt(0), sp.inputsAt(1), sp.inputsAt(2), self.const(1, n),
+                         self.dglgraph], n, NODE)
+        n.output().replaceAllUsesWith(out)
+        n.destroy()
+        sp.destroy()
+        return True
 
     def _fuse_spmm_tail(self, n) -> bool:
         """relu | elu (SpMMSrc | SpMMEdge (x) [* s]) and SpMMSrc | SpMMEdge (x) * s, s

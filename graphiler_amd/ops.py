@@ -1237,6 +1237,16 @@ def _own_linear(rows: int, k: int, m: int) -> bool:
                                        and (m <= 32 or rows * k <= LINEAR_FEW_ROWS_MAX_SIZE))
 
 
+def in_degrees(graph: DGLGraph, at_least: float = 0.0) -> torch.Tensor:
+    """(N, 1) fp32 in-degrees of the graph, none below ``at_least`` (the degree column that
+    examples/GCN/GCN.py:21-27 normalises by)."""
+    ptr = graph.in_pointer
+    out = torch.empty((graph.num_nodes, 1), dtype=torch.float32, device=ptr.device)
+    capi.check(capi.load().ga_row_lengths(ptr.data_ptr(), graph.num_nodes, float(at_least),
+                                          out.data_ptr(), _stream(out)), "ga_row_lengths")
+    return out
+
+
 def linear(x, weight, row_scale=None):
     """x @ weight for a (rows, K) node feature matrix and a (K, M) weight: the
     dense operator in front of the graph operators of a layer

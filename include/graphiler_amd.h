@@ -101,6 +101,10 @@ int ga_group_edges_both(const int64_t *src, const int64_t *dst, int64_t n_keys, 
                         int32_t *status, void *workspace, size_t workspace_bytes,
                         ga_stream_t stream);
 
+/* out[v] = max(pointer[v + 1] - pointer[v], least) as fp32: the in- or out-degrees of a graph. */
+int ga_row_lengths(const int32_t *pointer, int64_t n_rows, float least, float *out,
+                   ga_stream_t stream);
+
 /* The pointer of items whose keys ascend already (type columns: ids of one type are
  * contiguous, include/dglgraph.h:68-71), one pass over the keys.  key (n_items) int64,
  * pointer (n_keys + 1) int32; status two int32 on the device: [0] 1 when a key lies outside

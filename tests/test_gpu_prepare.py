@@ -133,3 +133,14 @@ def test_ids_beyond_32_bits_are_reported(device):
     types[-1] = 2 ** 32
     with pytest.raises(ValueError, match="type outside"):
         prepare_graph(src, src, 50, device=device, etype_of=types, num_etypes=3)
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 3000])
+def test_in_degrees(device, n):
+    from graphiler_amd import ops
+    rng = np.random.default_rng(n)
+    dst = rng.integers(0, n, 2 * n) // 2
+    g = prepare_graph(rng.integers(0, n, 2 * n), dst, n, device=device)
+    want = np.bincount(dst, minlength=n).astype(np.float32)[:, None]
+    assert np.array_equal(ops.in_degrees(g).cpu().numpy(), want)
+    assert np.array_equal(ops.in_degrees(g, at_least=1).cpu().numpy(), np.maximum(want, 1))

@@ -319,3 +319,10 @@ def test_every_operator_the_passes_emit_is_registered():
     assert len(names) > 20
     for name in sorted(names):
         assert len(torch._C._jit_get_schemas_for_operator(name)) == 1, name
+
+
+def test_relu_behind_an_rgcn_sum_rides_on_its_store():
+    from graphiler_amd.examples import models
+    kinds = [n.kind() for n in models.plan("RGCN+relu", 2).graph.nodes()]
+    assert [k for k in kinds if k.startswith("my_ops::")] == ["my_ops::TypedSpMMEdgeAct"]
+    assert "aten::relu" not in kinds
