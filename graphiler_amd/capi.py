@@ -126,6 +126,13 @@ SIGNATURES = {
     "ga_gat_aggregate": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64,
                                 _i64, _i64, ctypes.c_float, _int, _vp, _sz,
                                 _vp]),
+    "ga_gat_rows_longest": (_i64, [_i64]),
+    "ga_gat_rows_workspace_bytes": (_sz, [_i64, _i64]),
+    "ga_gat_rows_build": (_int, [_vp, _i64, _i64, _vp, _vp, _vp, _sz, _vp]),
+    "ga_gat_pieces_build": (_int, [_vp, _i64, _i64, _vp, _vp, _vp]),
+    "ga_gat_inputs_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
+    "ga_gat_inputs": (_int, [_vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64,
+                             _i64, _i64, ctypes.c_float, _int, _vp, _sz, _vp]),
     "ga_gat_aggregate_act": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64,
                                     ctypes.c_float, _int, _int, _vp, _sz, _vp]),
     "ga_gat_aggregate_from_z_act": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64,

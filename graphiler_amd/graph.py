@@ -267,6 +267,21 @@ class DGLGraph:
             self._cache[("classes", n)] = layout
         return layout
 
+    def rows_by_length(self) -> Optional["RowsByLength"]:
+        """The order in which a GAT layer over its inputs walks the destinations: built on the
+        device at first use and kept with the graph; None where that would have to happen while a
+        stream is captured, or does not fit the memory."""
+        rows = self._cache.get("rows_by_length")
+        if rows is None and "rows_by_length" not in self._cache:
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            try:
+                rows = _build_rows_by_length(self)
+            except torch.OutOfMemoryError:
+                rows = None
+            self._cache["rows_by_length"] = rows
+        return rows
+
     def refuse_source_classes(self, feat: int, dtype: int) -> None:
         """The scratch of ``feat`` features over source classes does not fit: the plain sum
         from now on.  A layout that no launch has read is given back; one that has been
@@ -356,6 +371,37 @@ def _build_relation_pairs(g: "DGLGraph") -> Optional[RelationPairs]:
         pairs.tiles.data_ptr(), torch.cuda.current_stream(dev).cuda_stream), "ga_pair_tiles_build")
     pairs.max_slots = int(largest.item())      # read behind all launches: the host waits once
     return pairs
+
+
+@dataclass
+class RowsByLength:
+    """Destinations ordered by their number of in-edges, long ones cut into pieces."""
+    rows: torch.Tensor              # (N, 4) int32: node, first slot, end slot, 0
+    n_light: int                    # rows of at most `longest` slots, in front
+    n_pieces: int                   # capacity of `pieces`
+    piece_first: torch.Tensor       # (long rows + 1) int32
+    pieces: torch.Tensor            # (n_pieces, 2) int32: first and end slot
+
+
+def _build_rows_by_length(g: "DGLGraph") -> RowsByLength:
+    lib, dev, n = capi.load(), g.device, g.num_nodes
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    i32 = dict(dtype=torch.int32, device=dev)
+    longest = int(lib.ga_gat_rows_longest(g.num_edges))
+    rows, light = torch.empty((n, 4), **i32), torch.empty(1, **i32)
+    ws = torch.empty(int(lib.ga_gat_rows_workspace_bytes(n, longest)), dtype=torch.uint8, device=dev)
+    capi.check(lib.ga_gat_rows_build(g.in_pointer.data_ptr(), n, longest, rows.data_ptr(), light.data_ptr(),
+                                     ws.data_ptr(), ws.numel(), stream), "ga_gat_rows_build")
+    n_light = int(light.item())
+    n_long = n - n_light
+    n_pieces = g.num_edges // longest + n_long if n_long else 0
+    out = RowsByLength(rows, n_light, n_pieces, torch.empty(n_long + 1, **i32),
+                       torch.empty((max(n_pieces, 1), 2), **i32))
+    if n_long:
+        capi.check(lib.ga_gat_pieces_build(rows[n_light:].data_ptr(), n_long, longest,
+                                           out.piece_first.data_ptr(), out.pieces.data_ptr(), stream),
+                   "ga_gat_pieces_build")
+    return out
 
 
 @dataclass

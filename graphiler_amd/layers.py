@@ -89,10 +89,17 @@ def gat_layer(g: DGLGraph, h, fc_weight, attn_weight, heads: int = 1,
     """One GAT layer forward; ``fused`` runs the chain as a single pass.  When
     the (N, heads) table of source terms is too large to stay cached
     (``SOURCE_TERM_TABLE_LIMIT`` bytes), the pass recomputes them from the
-    gathered rows instead of gathering them as well.  ``activation`` ("relu" |
+    gathered rows instead of gathering them as well.  A bf16 layer whose inputs are narrower
+    than half its outputs gathers the inputs and projects their sums (``ops.gat_inputs``).  ``activation`` ("relu" |
     "elu"; the ``F.elu`` between the layers of examples/GAT/GAT.py) is applied by
     the fused pass to the rows it stores, by a separate call otherwise."""
     a_l, a_r = attn_weight[0].float().contiguous(), attn_weight[1].float().contiguous()
+    if fused and h.is_cuda and h.dim() == 2 and h.is_contiguous() and fc_weight.is_contiguous() \
+            and h.dtype == fc_weight.dtype == torch.bfloat16 \
+            and ops.gat_inputs_preferred(int(h.shape[1]), int(a_l.shape[0]), int(fc_weight.shape[-1]), g.num_edges):
+        out = ops.gat_inputs(h, fc_weight, a_l, a_r, g, negative_slope, activation)
+        if out is not None:
+            return out
     # rows apart are a matter of tables larger than an L2; asked further only there
     if fused and h.is_cuda and g.num_nodes * fc_weight.shape[-1] * h.element_size() > ops.L2_BYTES \
             and fc_weight.dtype == h.dtype and fc_weight.is_contiguous() \

@@ -997,6 +997,54 @@ def gat_project_and_aggregate(h, weight, a_l, a_r, graph: DGLGraph, negative_slo
     return _aggregate_rows(a_l if from_z else el, er, z, m, heads, graph, negative_slope, act, dt, from_z)
 
 
+# Bytes of gathered rows that a GAT layer over its inputs has to save: below, what the order of its
+# rows costs once per graph (80-200 us) and its launches are not worth it (layer before : there,
+# us: 1.1 M edges, 100 inputs, four heads of 64, 0.28 GB less 148 : 130, 420,000 edges, 37 inputs,
+# eight heads of 64, 0.38 GB less 250 : 149).
+GAT_INPUTS_MIN_SAVING = 384 << 20
+
+
+def gat_inputs_preferred(k: int, heads: int, feat: int, n_edges: int) -> bool:
+    """Where an edge moves at most half the bytes as a row of inputs (whole 128-byte lines with the
+    source terms at their end) of what it moves as a projected row."""
+    row = -(-(2 * k + 4 * heads) // 128) * 128
+    return 2 * feat >= 2 * row and (2 * feat - row) * n_edges >= GAT_INPUTS_MIN_SAVING
+
+
+def gat_inputs(h, weight, a_l, a_r, graph: DGLGraph, negative_slope: float = 0.01, activation=None):
+    """A bf16 GAT layer with its product behind the sum over the edges (``ga_gat_inputs``): an edge
+    moves a row of h instead of a row of heads x dim.  None, nothing launched, for a shape the
+    kernels do not take, or where the order of the rows that they walk would have to be built
+    while a stream is captured."""
+    act = _activation(activation)
+    for name, x in (("h", h), ("weight", weight), ("a_l", a_l), ("a_r", a_r)):
+        _check_input(x, name)
+    if h.dtype != torch.bfloat16 or weight.dtype != h.dtype or h.dim() != 2 or weight.dim() != 2 \
+            or weight.shape[0] != h.shape[1] or a_l.dtype != torch.float32 or a_r.dtype != torch.float32:
+        return None
+    rows, k, m, heads = int(h.shape[0]), int(h.shape[1]), int(weight.shape[1]), int(a_l.shape[0])
+    if a_l.numel() != m or a_r.numel() != m or m % heads or rows != graph.num_nodes or graph.num_edges == 0:
+        return None
+    lib = capi.load()
+    if lib.ga_gat_inputs_workspace_bytes(rows, k, heads, m // heads, 0) == 0:
+        return None
+    order = graph.rows_by_length()
+    if order is None:
+        return None
+    try:
+        ws = torch.empty(int(lib.ga_gat_inputs_workspace_bytes(rows, k, heads, m // heads, order.n_pieces)),
+                         dtype=torch.uint8, device=h.device)
+    except torch.OutOfMemoryError:
+        return None
+    out = torch.empty((rows, m), dtype=h.dtype, device=h.device)
+    capi.check(lib.ga_gat_inputs(
+        order.rows.data_ptr(), order.n_light, order.piece_first.data_ptr(), order.pieces.data_ptr(),
+        order.n_pieces, graph.in_node_indices.data_ptr(), h.data_ptr(), weight.data_ptr(),
+        a_l.data_ptr(), a_r.data_ptr(), out.data_ptr(), rows, k, heads, m // heads,
+        float(negative_slope), act, ws.data_ptr(), ws.numel(), _stream(out)), "ga_gat_inputs")
+    return out
+
+
 def _aggregate_rows(source, er, z, feat: int, heads: int, graph: DGLGraph, negative_slope: float,
                     act: int, dt: int, from_z: bool) -> torch.Tensor:
     """The fused aggregation over the first ``feat`` values of every row of z."""

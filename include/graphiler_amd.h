@@ -559,6 +559,36 @@ int ga_gat_aggregate_from_z_act(const int32_t *pointer, const int32_t *row_of_sl
                                 int dtype, void *workspace, size_t workspace_bytes,
                                 ga_stream_t stream);
 
+/* A GAT layer over its inputs (bf16): out[v, h, :] = act((sum over the in-edges e of v of
+ * alpha[e, h] X[nbr(e), :]) @ W[:, h, :]), alpha the softmax over v's in-edges of
+ * leaky_relu(<X[nbr] @ W_h, a_l[h]> + <X[v] @ W_h, a_r[h]>): the layer of ga_project_attn +
+ * ga_gat_aggregate_act with the product behind the sum, which gathers K values an edge instead of
+ * heads * dim.  Everything is fp32 between X, W and out.  X (n_rows, K), W (K, heads * dim), out
+ * (n_rows, heads * dim) bf16, a_l / a_r (heads, dim) fp32.
+ *
+ * Once per graph: rows (n_rows, 4) int32, the nodes with their first and end slot, those of at
+ * most `longest` slots first by falling length, then the longer ones; n_light (one int32 on the
+ * device) counts the former.  `longest` is ga_gat_rows_longest(n_edges).  The longer rows are
+ * walked in pieces of `longest` slots: ga_gat_pieces_build(rows + 4 n_light, n_rows - n_light, ...)
+ * fills piece_first (n_long + 1) and pieces (at most n_edges / longest + n_long, 2); that capacity
+ * goes to the other calls as n_pieces (0 without longer rows).
+ *
+ * GA_EUNSUPPORTED (workspace bytes 0) unless heads is 1, 2, 4 or 8, dim 16, 32, 64, 128, 192 or 256,
+ * K at most 128 - 2 heads and the gathered table below 2 GiB. */
+int64_t ga_gat_rows_longest(int64_t n_edges);
+size_t ga_gat_rows_workspace_bytes(int64_t n_rows, int64_t longest);
+int ga_gat_rows_build(const int32_t *pointer, int64_t n_rows, int64_t longest, int32_t *rows,
+                      int32_t *n_light, void *workspace, size_t workspace_bytes, ga_stream_t stream);
+int ga_gat_pieces_build(const int32_t *long_rows, int64_t n_long, int64_t longest,
+                        int32_t *piece_first, int32_t *pieces, ga_stream_t stream);
+size_t ga_gat_inputs_workspace_bytes(int64_t n_rows, int64_t K, int64_t heads, int64_t dim,
+                                     int64_t n_pieces);
+int ga_gat_inputs(const int32_t *rows, int64_t n_light, const int32_t *piece_first,
+                  const int32_t *pieces, int64_t n_pieces, const int32_t *nbr, const void *X,
+                  const void *W, const float *a_l, const float *a_r, void *out, int64_t n_rows,
+                  int64_t K, int64_t heads, int64_t dim, float slope, int activation,
+                  void *workspace, size_t workspace_bytes, ga_stream_t stream);
+
 /* Either form over rows of z that lie z_stride elements apart (from_z: `source` is a_l,
  * else el): what a layer that writes z for this alone passes between ga_project_attn_strided
  * and here, with the stride ga_gather_row_stride names (more than the row where rows
