@@ -1162,8 +1162,10 @@ torch::Tensor BroadcastEdgeType(torch::Tensor features, const GraphPtr &graph) {
 int64_t get_feat_dim(torch::Tensor features) { return feat_dim(features); }
 
 // fused u_add_v -> leaky_relu -> SegmentSoftmax -> src_mul_e_sum
-torch::Tensor gat_aggregate(torch::Tensor el, torch::Tensor er, torch::Tensor z,
-                            double negative_slope, const GraphPtr &graph) {
+// (activation: of the fp32 rows before they are stored)
+torch::Tensor gat_aggregate_act(torch::Tensor el, torch::Tensor er, torch::Tensor z,
+                                double negative_slope, int64_t activation, const GraphPtr &graph) {
+  TORCH_CHECK(activation >= GA_ACT_NONE && activation <= GA_ACT_ELU, "unknown activation");
   check_input(el, "el");
   check_input(er, "er");
   check_input(z, "z");
@@ -1181,25 +1183,32 @@ torch::Tensor gat_aggregate(torch::Tensor el, torch::Tensor er, torch::Tensor z,
   const auto &side = graph->side(false);
   torch::Tensor out = torch::empty(out_shape(graph->num_nodes, z), z.options());
   torch::Tensor ws = graph->workspace(ga_gat_workspace_bytes(graph->num_edges, feat, heads));
-  check_ga(ga_gat_aggregate(graph->in_pointer.data_ptr<int>(),
-                            side.rows.data_ptr<int>(),
-                            graph->in_node_indices.data_ptr<int>(),
-                            el.data_ptr<float>(), er.data_ptr<float>(), z.data_ptr(),
-                            out.data_ptr(), graph->num_nodes, graph->num_edges, heads,
-                            feat / heads, (float)negative_slope, dt, ws.data_ptr(),
-                            (size_t)ws.numel(), current_stream(out)),
-           "ga_gat_aggregate");
+  check_ga(ga_gat_aggregate_act(graph->in_pointer.data_ptr<int>(),
+                                side.rows.data_ptr<int>(),
+                                graph->in_node_indices.data_ptr<int>(),
+                                el.data_ptr<float>(), er.data_ptr<float>(), z.data_ptr(),
+                                out.data_ptr(), graph->num_nodes, graph->num_edges, heads,
+                                feat / heads, (float)negative_slope, (int)activation, dt,
+                                ws.data_ptr(), (size_t)ws.numel(), current_stream(out)),
+           "ga_gat_aggregate_act");
   return out;
+}
+
+torch::Tensor gat_aggregate(torch::Tensor el, torch::Tensor er, torch::Tensor z,
+                            double negative_slope, const GraphPtr &graph) {
+  return gat_aggregate_act(el, er, z, negative_slope, GA_ACT_NONE, graph);
 }
 
 // gat_aggregate that may recompute the source term from the gathered rows: with
 // a_l (heads * dim elements) at hand, a table of source terms of 16 MB or more
 // (it no longer stays cached, and gathering it costs a memory sector per edge)
 // is not read at all; smaller tables take the ordinary pass.
-torch::Tensor gat_aggregate_al(torch::Tensor a_l, torch::Tensor el, torch::Tensor er,
-                               torch::Tensor z, double negative_slope, const GraphPtr &graph) {
+torch::Tensor gat_aggregate_al_act(torch::Tensor a_l, torch::Tensor el, torch::Tensor er,
+                                   torch::Tensor z, double negative_slope, int64_t activation,
+                                   const GraphPtr &graph) {
   constexpr int64_t kTableLimit = 16 << 20;
-  if (el.numel() * 4 < kTableLimit) return gat_aggregate(el, er, z, negative_slope, graph);
+  if (el.numel() * 4 < kTableLimit) return gat_aggregate_act(el, er, z, negative_slope, activation, graph);
+  TORCH_CHECK(activation >= GA_ACT_NONE && activation <= GA_ACT_ELU, "unknown activation");
   check_input(er, "er");
   check_input(z, "z");
   TORCH_CHECK(a_l.is_cuda(), "a_l must be a CUDA tensor");
@@ -1214,14 +1223,19 @@ torch::Tensor gat_aggregate_al(torch::Tensor a_l, torch::Tensor el, torch::Tenso
   const auto &side = graph->side(false);
   torch::Tensor out = torch::empty(out_shape(graph->num_nodes, z), z.options());
   torch::Tensor ws = graph->workspace(ga_gat_workspace_bytes(graph->num_edges, feat, heads));
-  const int rc = ga_gat_aggregate_from_z(
+  const int rc = ga_gat_aggregate_from_z_act(
       graph->in_pointer.data_ptr<int>(), side.rows.data_ptr<int>(),
       graph->in_node_indices.data_ptr<int>(), al.data_ptr<float>(), er.data_ptr<float>(),
       z.data_ptr(), out.data_ptr(), graph->num_nodes, graph->num_edges, heads, feat / heads,
-      (float)negative_slope, dt, ws.data_ptr(), (size_t)ws.numel(), current_stream(out));
-  if (rc == GA_EUNSUPPORTED) return gat_aggregate(el, er, z, negative_slope, graph);
-  check_ga(rc, "ga_gat_aggregate_from_z");
+      (float)negative_slope, (int)activation, dt, ws.data_ptr(), (size_t)ws.numel(), current_stream(out));
+  if (rc == GA_EUNSUPPORTED) return gat_aggregate_act(el, er, z, negative_slope, activation, graph);
+  check_ga(rc, "ga_gat_aggregate_from_z_act");
   return out;
+}
+
+torch::Tensor gat_aggregate_al(torch::Tensor a_l, torch::Tensor el, torch::Tensor er,
+                               torch::Tensor z, double negative_slope, const GraphPtr &graph) {
+  return gat_aggregate_al_act(a_l, el, er, z, negative_slope, GA_ACT_NONE, graph);
 }
 
 // SegmentSoftmax -> mul -> SpMMEdge (examples/HGT/HGT.py:50-53) in one pass:
@@ -1607,6 +1621,12 @@ static auto registry =
         .op("my_ops::gat_aggregate(Tensor el, Tensor er, Tensor z, float slope, " GRAPH_T
             " g) -> Tensor y",
             &gat_aggregate)
+        .op("my_ops::gat_aggregate_act(Tensor el, Tensor er, Tensor z, float slope, int activation, " GRAPH_T
+            " g) -> Tensor y",
+            &gat_aggregate_act)
+        .op("my_ops::gat_aggregate_al_act(Tensor a_l, Tensor el, Tensor er, Tensor z, float slope, "
+            "int activation, " GRAPH_T " g) -> Tensor y",
+            &gat_aggregate_al_act)
         .op("my_ops::gat_aggregate_al(Tensor a_l, Tensor el, Tensor er, Tensor z, float slope, "
             GRAPH_T " g) -> Tensor y",
             &gat_aggregate_al)

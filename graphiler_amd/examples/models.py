@@ -37,6 +37,7 @@ def plan(name: str, level: int):
         fns = {
             "GCN": (udf.gcn_message, udf.gcn_reduce, None),
             "GAT": (udf.gat_message, udf.gat_reduce, None),
+            "GAT+elu": (udf.gat_message, udf.gat_reduce_elu, None),
             "RGCN": (udf.rgcn_message, udf.rgcn_reduce, None),
             "RGCN+relu": (udf.rgcn_message, udf.rgcn_reduce_relu, None),
             "HGT": (udf.hgt_message, udf.hgt_reduce, udf.hgt_update),
@@ -116,20 +117,21 @@ class GAT:
             self.layers.append((_param(rng, (a, b), device),
                                 _param(rng, (2 * b, 1), device)))
 
-    def _layer(self, g, x, fc, attn, mode):
+    def _layer(self, g, x, fc, attn, mode, elu):
         g.ndata['h'] = x
         if mode in EAGER:
             z = torch.mm(x, fc)
             z_src, z_dst = z[g.graph.COO_src], z[g.graph.COO_dst]
             e = F.leaky_relu(torch.mm(torch.cat([z_src, z_dst], dim=1), attn), 0.2)
-            g.ndata['h'] = _sum_by_dst(g, _softmax_by_dst(g, e, mode) * z_src, mode)
+            h = _sum_by_dst(g, _softmax_by_dst(g, e, mode) * z_src, mode)
+            g.ndata['h'] = F.elu(h) if elu else h
         else:
-            update_all(g, plan("GAT", mode), msg_params=(fc, attn))
+            update_all(g, plan("GAT+elu" if elu else "GAT", mode), msg_params=(fc, attn))
         return g.ndata.pop('h')
 
     def __call__(self, g: GraphData, features, mode=2):
-        h = F.elu(self._layer(g, features, *self.layers[0], mode))
-        return self._layer(g, h, *self.layers[1], mode)
+        h = self._layer(g, features, *self.layers[0], mode, elu=True)
+        return self._layer(g, h, *self.layers[1], mode, elu=False)
 
 
 # ---- RGCN ------------------------------------------------------------------------------

@@ -32,6 +32,12 @@ def gat_reduce(nodes: NodeBatchDummy):
     return {'h': torch.sum(alpha * nodes.mailbox['z'], dim=1)}
 
 
+def gat_reduce_elu(nodes: NodeBatchDummy):
+    """A layer that another one follows (the F.elu of examples/GAT/GAT.py)."""
+    alpha = torch.softmax(nodes.mailbox['e'], dim=1)
+    return {'h': F.elu(torch.sum(alpha * nodes.mailbox['z'], dim=1))}
+
+
 # ---- GAT, four heads of width 16 (the shape literals must be constants for the
 # compiler to see that the view keeps one row per edge) -----------------------------
 def gat4_message(edges: EdgeBatchDummy, fc_weight, attn_l, attn_r):

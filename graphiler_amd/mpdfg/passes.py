@@ -520,23 +520,28 @@ class _Rewriter:
         # last: only the sums no other rewrite has taken
         for n in list(self.G.nodes()):
             if n.kind() in ("aten::relu", "aten::elu"):
-                changed |= self._fuse_typed_tail(n) or self._fuse_spmm_tail(n)
+                changed |= self._fuse_kernel_tail(n) or self._fuse_spmm_tail(n)
         for n in list(self.G.nodes()):
             if n.kind() == "aten::mul":
                 changed |= self._fuse_spmm_tail(n)
         return changed
 
-    def _fuse_typed_tail(self, n) -> bool:
-        """relu(TypedSpMMEdge(x, w, s)) -> TypedSpMMEdgeAct(x, w, s, 1): the activation between
-        two RGCN layers (examples/RGCN/RGCN.py:69) where the sums are stored."""
+    def _fuse_kernel_tail(self, n) -> bool:
+        """relu | elu of TypedSpMMEdge, gat_aggregate or gat_aggregate_al -> the operator with the
+        activation where it stores its rows: what stands between two RGCN or GAT layers
+        (examples/RGCN/RGCN.py:69, the F.elu of examples/GAT/GAT.py)."""
         top = n.inputsAt(0)
         sp = top.node()
-        if n.kind() != "aten::relu" or sp.kind() != "my_ops::TypedSpMMEdge" or not self.single_use(top) \
-                or _mutated(top):
+        fused = {"my_ops::TypedSpMMEdge": "my_ops::TypedSpMMEdgeAct",
+                 "my_ops::gat_aggregate": "my_ops::gat_aggregate_act",
+                 "my_ops::gat_aggregate_al": "my_ops::gat_aggregate_al_act"}.get(sp.kind())
+        if fused is None or not self.single_use(top) or _mutated(top):
             return False
-        out = self.make("my_ops::TypedSpMMEdgeAct",
-                        [sp.inputsAt(0), sp.inputsAt(1), sp.inputsAt(2), self.const(1, n),
-                         self.dglgraph], n, NODE)
+        if n.kind() == "aten::elu" and \
+                any(self.const_of(n.inputsAt(i)) not in (1, 1.0) for i in (1, 2, 3)):
+            return False
+        act = self.const(1 if n.kind() == "aten::relu" else 2, n)
+        out = self.make(fused, list(sp.inputs())[:-1] + [act, self.dglgraph], n, NODE)
         n.output().replaceAllUsesWith(out)
         n.destroy()
         sp.destroy()

@@ -326,3 +326,10 @@ def test_relu_behind_an_rgcn_sum_rides_on_its_store():
     kinds = [n.kind() for n in models.plan("RGCN+relu", 2).graph.nodes()]
     assert [k for k in kinds if k.startswith("my_ops::")] == ["my_ops::TypedSpMMEdgeAct"]
     assert "aten::relu" not in kinds
+
+
+def test_elu_behind_an_attention_sum_rides_on_its_store():
+    from graphiler_amd.examples import models
+    kinds = [n.kind() for n in models.plan("GAT+elu", 2).graph.nodes()]
+    assert [k for k in kinds if k.startswith("my_ops::")] == ["my_ops::gat_project", "my_ops::gat_aggregate_act"]
+    assert "aten::elu" not in kinds
