@@ -32,6 +32,7 @@
 // (HGT's sum(k * q)), in which case Y never reaches memory.
 #include "common.h"
 #include "typed_chunks.h"
+#include "typed_rows.h"
 #include "wide_mm.h"
 
 #include <type_traits>
@@ -981,11 +982,38 @@ int wide_typed(const int32_t *type_pointer, int64_t n_types, const void *X,
   return wide_mm_launch(p, s);
 }
 
+// fp32 rows by typed_rows_kernel: up to four tensors, a factor per row or a gate per type
+int rows_typed(const int32_t *type_pointer, int64_t n_types, const void *X, const void *const *W,
+               void *const *Y, int n_weights, int64_t rows, int64_t K, int64_t M,
+               const float *row_scale, const float *gate, bool sigmoid, hipStream_t s) {
+  if (K > 128 || M > 65536) return GA_EUNSUPPORTED;
+  TypedRows p = {};
+  p.tp = type_pointer;
+  p.n_types = (int)n_types;
+  p.X = (const float *)X;
+  p.rows = rows;
+  p.K = (int)K;
+  p.M = (int)M;
+  p.n_weights = n_weights;
+  for (int i = 0; i < n_weights; ++i) {
+    p.W[i] = (const float *)W[i];
+    p.Y[i] = (float *)Y[i];
+  }
+  p.row_scale = row_scale;
+  p.gate = gate;
+  p.gate_sigmoid = sigmoid;
+  return typed_rows_launch(p, s);
+}
+
 int segment_mm_any(const int32_t *type_pointer, int64_t n_types, const void *X,
                    const void *W, void *Y, int64_t rows, int64_t heads, int64_t K,
                    int64_t M, int dtype, const MmExt &ext, hipStream_t s) {
   const bool fused = ext.x_index || ext.Q;
   int rc = GA_EUNSUPPORTED;
+  if (dtype == GA_F32 && heads == 1 && !fused && Y) {
+    rc = rows_typed(type_pointer, n_types, X, &W, &Y, 1, rows, K, M, ext.row_scale, nullptr, false, s);
+    if (rc != GA_EUNSUPPORTED) return rc;
+  }
   if (dtype == GA_BF16 && heads == 1 && !fused && Y) {
     rc = wide_typed(type_pointer, n_types, X, &W, &Y, 1, rows, K, M, ext.row_scale, s);
     if (rc != GA_EUNSUPPORTED) return rc;
@@ -1278,6 +1306,10 @@ extern "C" int ga_segment_mm_stacked(const int32_t *type_pointer, int64_t n_type
     const int rc = wide_typed(type_pointer, n_types, X, W, Y, (int)n_weights, rows, K, M, nullptr, s);
     if (rc != GA_EUNSUPPORTED) return rc;
   }
+  if (dtype == GA_F32) {
+    const int rc = rows_typed(type_pointer, n_types, X, W, Y, (int)n_weights, rows, K, M, nullptr, nullptr, false, s);
+    if (rc != GA_EUNSUPPORTED) return rc;
+  }
   // any other shape: one product per weight tensor
   MmExt ext = {};
   for (int64_t i = 0; i < n_weights; ++i) {
@@ -1298,7 +1330,9 @@ extern "C" int ga_segment_mm_gated(const int32_t *type_pointer, int64_t n_types,
   if (!type_pointer || !X || !W || !Y || !gate) return GA_EINVAL;
   const size_t esz = dtype == GA_F32 ? 4 : 2;
   if (!aligned(X, esz) || !aligned(W, esz) || !aligned(Y, esz) || !aligned(gate, 4)) return GA_EALIGN;
-  if (dtype != GA_BF16) return GA_EUNSUPPORTED;
+  if (dtype == GA_F32)
+    return rows_typed(type_pointer, n_types, X, &W, &Y, 1, rows, K, M, nullptr, gate, gate_sigmoid != 0,
+                      (hipStream_t)stream);
   return wide_typed(type_pointer, n_types, X, &W, &Y, 1, rows, K, M, nullptr, (hipStream_t)stream,
                     gate, gate_sigmoid != 0);
 }

@@ -894,9 +894,9 @@ torch::Tensor SegmentMMNodeGated(torch::Tensor features, torch::Tensor weights, 
               "gate must have one entry per node type");
   // (a gate that would promote the product, e.g. fp32 on bf16 features, keeps the
   // meaning of the expression: it multiplies the result afterwards, below)
-  if (features.is_cuda() && features.scalar_type() == at::kBFloat16 &&
+  if (features.is_cuda() && (features.scalar_type() == at::kBFloat16 || features.scalar_type() == at::kFloat) &&
       at::promote_types(features.scalar_type(), gate.scalar_type()) == features.scalar_type() &&
-      weights.scalar_type() == at::kBFloat16 && features.dim() == 2 && weights.dim() == 3 &&
+      weights.scalar_type() == features.scalar_type() && features.dim() == 2 && weights.dim() == 3 &&
       features.size(0) == graph->num_nodes && weights.size(0) == graph->num_ntypes &&
       features.size(1) == weights.size(1) && gate.is_floating_point() &&
       graph->ntype_pointer.has_value()) {
@@ -908,7 +908,8 @@ torch::Tensor SegmentMMNodeGated(torch::Tensor features, torch::Tensor weights, 
     const int rc = ga_segment_mm_gated(
         graph->ntype_pointer.value().data_ptr<int>(), graph->num_ntypes, features.data_ptr(),
         weights.data_ptr(), out.data_ptr(), g32.data_ptr<float>(), sigmoid ? 1 : 0,
-        graph->num_nodes, weights.size(1), weights.size(2), GA_BF16, current_stream(out));
+        graph->num_nodes, weights.size(1), weights.size(2), feat_dtype(features, "features"),
+        current_stream(out));
     if (rc != GA_EUNSUPPORTED) {
       check_ga(rc, "ga_segment_mm_gated");
       return out;

@@ -575,7 +575,7 @@ def SegmentMMNodeGated(features, weights, gate, graph: DGLGraph, sigmoid: bool =
     """``SegmentMMNode(features, weights) * g(BroadcastNodeType(gate))`` with g the sigmoid
     (or the identity): the output projection of an HGT layer with its per-node-type gate
     (examples/HGT/HGT.py:58-60).  ``gate`` (T,) fp32.  The factor is applied to the fp32 sums
-    in the product's kernel where that kernel takes it (bf16, wide outputs); otherwise it is
+    in the product's kernel where that kernel takes it (bf16, wide outputs; fp32); otherwise it is
     formed per row first and goes in as ``row_scale`` of SegmentMMNode."""
     _check_input(features, "features")
     _check_input(weights, "weights")
@@ -584,7 +584,7 @@ def SegmentMMNodeGated(features, weights, gate, graph: DGLGraph, sigmoid: bool =
         raise RuntimeError("the graph has no type pointer for this operator")
     if gate.dtype != torch.float32 or gate.numel() != graph.num_ntypes:
         raise RuntimeError("gate must be one float32 per node type")
-    if features.dtype == torch.bfloat16 and weights.dtype == torch.bfloat16 and weights.dim() == 3 \
+    if features.dtype in (torch.bfloat16, torch.float32) and weights.dtype == features.dtype and weights.dim() == 3 \
             and int(weights.shape[0]) == graph.num_ntypes and features.dim() == 2 \
             and int(features.shape[0]) == graph.num_nodes \
             and int(features.shape[1]) == int(weights.shape[1]):
@@ -593,7 +593,7 @@ def SegmentMMNodeGated(features, weights, gate, graph: DGLGraph, sigmoid: bool =
         rc = capi.load().ga_segment_mm_gated(
             graph.ntype_pointer.data_ptr(), graph.num_ntypes, features.data_ptr(),
             weights.data_ptr(), out.data_ptr(), gate.data_ptr(), 1 if sigmoid else 0,
-            graph.num_nodes, K, M, capi.GA_BF16, _stream(out))
+            graph.num_nodes, K, M, _feat_dtype(features, "features"), _stream(out))
         if rc != capi.GA_EUNSUPPORTED:
             capi.check(rc, "ga_segment_mm_gated")
             return out

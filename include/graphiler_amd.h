@@ -390,8 +390,9 @@ int ga_segment_mm(const int32_t *type_pointer, int64_t n_types, const void *X,
  * (examples/HGT/HGT.py:35-44, three calls of segment_mm.cu:29-33 on one input) read X
  * once this way.  bf16 with K % 8 == 0, K <= 256 (or K % 4 == 0, K <= 128, two groups
  * at most), M % 128 == 0 and n_weights * M / 128 groups of 128 columns within the LDS
- * of a CU runs as one launch; every other shape ga_segment_mm takes runs as n_weights
- * launches with the same results. */
+ * of a CU runs as one launch, and so does fp32 with K % 4 == 0, K <= 128 and M 16, 32 or a
+ * multiple of 64; every other shape ga_segment_mm takes runs as n_weights launches with the
+ * same results. */
 int ga_segment_mm_stacked(const int32_t *type_pointer, int64_t n_types, const void *X,
                           const void *const *W, void *const *Y, int64_t n_weights,
                           int64_t rows, int64_t K, int64_t M, int dtype, ga_stream_t stream);
@@ -401,7 +402,8 @@ int ga_segment_mm_stacked(const int32_t *type_pointer, int64_t n_types, const vo
  * examples/HGT/HGT.py:58-60 (`trans_out * sigmoid(skip[ntype])`) applied to the fp32 sums
  * before they are rounded, so that neither the sigmoid, nor its copy to the nodes
  * (BroadcastNodeType, broadcast.cu:67-72), nor the multiplication is a pass of its own.
- * gate: (n_types,) fp32.  bf16 shapes of the wide kernel only (see ga_segment_mm_stacked);
+ * gate: (n_types,) fp32.  bf16 shapes of the wide kernel only (see ga_segment_mm_stacked), fp32 with
+ * K a multiple of 4 up to 128 and M 16, 32 or a multiple of 64;
  * GA_EUNSUPPORTED, having launched nothing, otherwise: the caller then forms the per-row
  * factor itself and passes it as row_scale of ga_segment_mm_gather. */
 int ga_segment_mm_gated(const int32_t *type_pointer, int64_t n_types, const void *X,
