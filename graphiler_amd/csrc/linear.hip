@@ -76,17 +76,96 @@ constexpr int kCB = 4;                                   // 16-column blocks per
 constexpr int kPassCols = kCB * 16;                      // 64
 constexpr int kSliceK = 32;                              // k per LDS slice
 constexpr int kXs = kSliceK + 4;                         // LDS row stride of the X tile
+constexpr int kAhead = 2;                                // slices of X on their way (odd rows)
 constexpr int kWb = kSliceK / 2 + 4;                      // LDS column stride of a W piece, in bf16 pairs
+
+// The k of element j of lane group lk where X goes straight to its operand: 4 lk .. 4 lk + 3 and
+// those 16 further on, so that the four lanes of a row read 64 bytes side by side.
+__device__ __forceinline__ int k_of(int lk, int j) { return 4 * lk + (j & 3) + 4 * (j & 4); }
+
+// What follows the k loop of a wavefront's 32 rows and NCB column blocks.
+template <bool HAS_ATTN, int NCB>
+__device__ __forceinline__ void store_tile(floatx4 (&acc)[kRT][NCB], const float *__restrict__ a_l,
+                                           const float *__restrict__ a_r, float *__restrict__ Z,
+                                           float *__restrict__ el, float *__restrict__ er,
+                                           const float *__restrict__ row_scale, int64_t rows, int M,
+                                           int heads, int ldz, int64_t wrow0, int col0) {
+  const int lane = threadIdx.x & (kWave - 1), lr = lane & 15, lk = lane >> 4;
+  // lane holds rows wrow0 + t*16 + 4*lk + r, column col0 + cb*16 + lr
+  // the row factors of the plain projection, all requested before the first store
+  float rsv[kRT][4];
+  if (!HAS_ATTN) {
+#pragma unroll
+    for (int t = 0; t < kRT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t row = wrow0 + t * 16 + lk * 4 + r;
+        rsv[t][r] = row_scale && row < rows ? row_scale[row] : 1.0f;
+      }
+  }
+  float al[kCB], ar[kCB];
+  const int dph = M / heads;
+  const int bph = dph >> 4;                              // column blocks per head
+  if constexpr (HAS_ATTN) {
+#pragma unroll
+    for (int cb = 0; cb < kCB; ++cb) {
+      const int c = col0 + cb * 16 + lr;
+      al[cb] = c < M ? a_l[c] : 0.0f;                    // (heads, dph) is (M,) flat
+      ar[cb] = c < M ? a_r[c] : 0.0f;
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < kRT; ++t) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t row = wrow0 + t * 16 + lk * 4 + r;
+      const bool live = row < rows;
+      if (!HAS_ATTN && row_scale) {                      // the plain projection only
+#pragma unroll
+        for (int cb = 0; cb < NCB; ++cb) acc[t][cb][r] *= rsv[t][r];
+      }
+#pragma unroll
+      for (int cb = 0; cb < NCB; ++cb) {
+        const int c = col0 + cb * 16 + lr;
+        if (live && c < M) Z[row * ldz + c] = acc[t][cb][r];
+      }
+      if constexpr (HAS_ATTN) {
+        // lane-local products, blocks of one head added, then one 16-lane tree
+        float pl[kCB], pr[kCB];
+#pragma unroll
+        for (int cb = 0; cb < kCB; ++cb) {
+          pl[cb] = acc[t][cb][r] * al[cb];
+          pr[cb] = acc[t][cb][r] * ar[cb];
+        }
+        if (bph >= 2) {
+          pl[0] += pl[1]; pr[0] += pr[1];
+          pl[2] += pl[3]; pr[2] += pr[3];
+        }
+        if (bph == 4) { pl[0] += pl[2]; pr[0] += pr[2]; }
+#pragma unroll
+        for (int cb = 0; cb < kCB; ++cb) {
+          if (cb % bph == 0) {                           // first block of a head
+            const float sl_ = row16_sum(pl[cb]), sr_ = row16_sum(pr[cb]);
+            const int head = (col0 + cb * 16) / dph;
+            if (live && lr == 0 && head < heads) {
+              el[row * heads + head] = sl_;
+              er[row * heads + head] = sr_;
+            }
+          }
+        }
+      }
+    }
+  }
+}
 
 template <int VK> struct XVec;
 template <> struct XVec<4> { using type = float4; };
 template <> struct XVec<2> { using type = float2; };
-template <> struct XVec<1> { using type = float; };
 
 // HAS_ATTN: also produce el / er; requires heads to tile a pass exactly
 // (dph = M / heads in {16, 32, 64}).
 // VK = widest aligned vector (floats) of a row of X: 4 when K % 4 == 0, 2 when
-// K % 2 == 0, else 1.  K % VK == 0, so such a vector lies wholly inside or
+// K % 2 == 0.  K % VK == 0, so such a vector lies wholly inside or
 // wholly outside a row: ragged edges clamp the address at fetch time (a valid
 // one, the row's last vector) and zero by select at commit time, where the
 // value is consumed anyway; no lane is ever predicated off in the k loop.
@@ -246,73 +325,146 @@ linear_attn_kernel(
   }
   if (sl < n_slices) step(sl, sb);
 
-  // epilogue: lane holds rows wrow0 + t*16 + 4*lk + r, column col0 + cb*16 + lr
-  // the row factors of the plain projection, all requested before the first store
-  float rsv[kRT][4];
-  if (!HAS_ATTN) {
-#pragma unroll
-    for (int t = 0; t < kRT; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t row = wrow0 + t * 16 + lk * 4 + r;
-        rsv[t][r] = row_scale && row < rows ? row_scale[row] : 1.0f;
-      }
-  }
-  float al[kCB], ar[kCB];
-  const int dph = M / heads;
-  const int bph = dph >> 4;                              // column blocks per head
-  if constexpr (HAS_ATTN) {
-#pragma unroll
-    for (int cb = 0; cb < kCB; ++cb) {
-      const int c = col0 + cb * 16 + lr;
-      al[cb] = c < M ? a_l[c] : 0.0f;                    // (heads, dph) is (M,) flat
-      ar[cb] = c < M ? a_r[c] : 0.0f;
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < kRT; ++t) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t row = wrow0 + t * 16 + lk * 4 + r;
-      const bool live = row < rows;
-      if (!HAS_ATTN && row_scale) {                      // the plain projection only
-#pragma unroll
-        for (int cb = 0; cb < NCB; ++cb) acc[t][cb][r] *= rsv[t][r];
-      }
-#pragma unroll
-      for (int cb = 0; cb < NCB; ++cb) {
-        const int c = col0 + cb * 16 + lr;
-        if (live && c < M) Z[row * ldz + c] = acc[t][cb][r];
-      }
-      if constexpr (HAS_ATTN) {
-        // lane-local products, blocks of one head added, then one 16-lane tree
-        float pl[kCB], pr[kCB];
-#pragma unroll
-        for (int cb = 0; cb < kCB; ++cb) {
-          pl[cb] = acc[t][cb][r] * al[cb];
-          pr[cb] = acc[t][cb][r] * ar[cb];
-        }
-        if (bph >= 2) {
-          pl[0] += pl[1]; pr[0] += pr[1];
-          pl[2] += pl[3]; pr[2] += pr[3];
-        }
-        if (bph == 4) { pl[0] += pl[2]; pr[0] += pr[2]; }
-#pragma unroll
-        for (int cb = 0; cb < kCB; ++cb) {
-          if (cb % bph == 0) {                           // first block of a head
-            const float sl_ = row16_sum(pl[cb]), sr_ = row16_sum(pr[cb]);
-            const int head = (col0 + cb * 16) / dph;
-            if (live && lr == 0 && head < heads) {
-              el[row * heads + head] = sl_;
-              er[row * heads + head] = sr_;
-            }
-          }
-        }
-      }
-    }
-  }
+  store_tile<HAS_ATTN, NCB>(acc, a_l, a_r, Z, el, er, row_scale, rows, M, heads, ldz, wrow0, col0);
 }
 
+// Rows of an odd number of values, which only four-byte accesses tile: staged through LDS one
+// float at a time they took 32 staged registers and two workgroups a CU.  Here the rows go
+// straight to the operand of the matrix instruction with 16-byte loads of 4-byte alignment, 64
+// bytes of a row side by side (few_rows' order of k); W as above.  Four workgroups per CU.  us:
+// 300,000 x 37 -> 64 38.5 -> 27, 100,000 x 101 26.5 -> 21, 40,000 x 1433 94 -> 66, 60,000 x 1433
+// 105 -> 93.  Rows that wider accesses tile are no faster this way (232,965 x 602 162 : 165,
+// 1 M x 100 164 : 182).
+template <bool HAS_ATTN, int WAVES, int NCB = kCB>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void
+linear_odd_kernel(
+    const float *__restrict__ X, const float *__restrict__ W,
+    const float *__restrict__ a_l, const float *__restrict__ a_r,
+    float *__restrict__ Z, float *__restrict__ el, float *__restrict__ er,
+    const float *__restrict__ row_scale, int64_t rows, int K, int M, int heads, int ldz) {
+  static_assert(NCB == kCB || !HAS_ATTN, "the attention epilogue pairs up all four column blocks");
+  __shared__ __attribute__((aligned(16))) uint32_t wb[2][3][kPassCols * kWb];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // in a scalar register
+  const int lr = lane & 15, lk = lane >> 4;
+  const int col0 = blockIdx.y * kPassCols;               // first column of the pass
+  const int64_t wg_row0 = (int64_t)blockIdx.x * kWgRows;
+  const int64_t wrow0 = wg_row0 + wave * kWaveRows;
+  const int n_slices = (K + kSliceK - 1) / kSliceK;
+
+  struct Rows { float4 x[kRT][2]; };
+  const rsrc_t xrs = make_rsrc(X + wg_row0 * K, (uint64_t)(rows - wg_row0) * K * 4);
+  const rsrc_t wrs = make_rsrc(W, (uint64_t)K * M * 4);
+  uint32_t xoff[kRT];                                    // byte offset in slice 0
+#pragma unroll
+  for (int t = 0; t < kRT; ++t)
+    xoff[t] = (uint32_t)((min(wrow0 + t * 16 + lr, rows - 1) - wg_row0) * K + 4 * lk) * 4u;
+  const int wc = threadIdx.x & 63, wkg = wave;           // column, lk of the eight k
+  const uint32_t woff = (uint32_t)min(col0 + wc, M - 1) * 4u;
+  const bool w_cols_full = col0 + kPassCols <= M;        // uniform
+
+  // The last slice, if it is not whole, keeps its k together (8 lk .. 8 lk + 7): fewer of the
+  // instruction's partial sums are rounded (error at K = 45 1.07e-7 -> 0.83e-7).
+  auto k_in = [&](int sl, int lane_k, int j) __attribute__((always_inline)) {
+    return sl * kSliceK + (sl * kSliceK + kSliceK <= K ? k_of(lane_k, j) : 8 * lane_k + j);
+  };
+  // What lies past the end of X reads as 0 (lane offsets are range-checked); what the last
+  // slice reads of the row behind is cleared when it is multiplied.  Slices past the last are
+  // fetched too and never multiplied.
+  auto fetch_x = [&](int sl, Rows &r) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < kRT; ++t) {
+      const bool whole = sl * kSliceK + kSliceK <= K;    // uniform
+      const uint32_t at = xoff[t] + (uint32_t)sl * (kSliceK * 4) + (whole ? 0u : 16u * lk);
+      r.x[t][0] = BufLoad<4>::at(xrs, at, 0);
+      r.x[t][1] = BufLoad<4>::at(xrs, at + (whole ? 64u : 16u), 0);
+    }
+  };
+  // the row of W is the scalar offset: no address arithmetic
+  auto fetch_w = [&](int sl, float (&w)[8]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      w[j] = BufLoad<1>::at(wrs, woff, (uint32_t)min(k_in(sl, wkg, j), K - 1) * (uint32_t)M * 4u);
+  };
+  auto commit_w = [&](int sl, const float (&w)[8]) __attribute__((always_inline)) {
+    const int buf = sl & 1;
+    float wv[8];
+    if (sl * kSliceK + kSliceK <= K && w_cols_full) {    // uniform
+#pragma unroll
+      for (int j = 0; j < 8; ++j) wv[j] = w[j];
+    } else {
+      const bool cin = col0 + wc < M;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) wv[j] = cin && k_in(sl, wkg, j) < K ? w[j] : 0.0f;
+    }
+    uint4 p0, p1, p2;
+    split8(wv, p0, p1, p2);
+    *reinterpret_cast<uint4 *>(&wb[buf][0][wc * kWb + wkg * 4]) = p0;
+    *reinterpret_cast<uint4 *>(&wb[buf][1][wc * kWb + wkg * 4]) = p1;
+    *reinterpret_cast<uint4 *>(&wb[buf][2][wc * kWb + wkg * 4]) = p2;
+  };
+
+  floatx4 acc[kRT][NCB];
+#pragma unroll
+  for (int t = 0; t < kRT; ++t)
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb) acc[t][cb] = floatx4{0, 0, 0, 0};
+
+  const int wl_ofs = lr * kWb + lk * 4;                  // in uint32 (pairs of bf16)
+  float wn[8];                                           // W of the next slice
+  auto step = [&](int sl, Rows &now) __attribute__((always_inline)) {
+    const int buf = sl & 1;
+    uint4 wf[2][3];
+    auto read_w = [&](int cb, uint4 (&f)[3]) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        f[p] = *reinterpret_cast<const uint4 *>(&wb[buf][p][wl_ofs + cb * 16 * kWb]);
+    };
+    read_w(0, wf[0]);
+    commit_w(sl + 1, wn);
+    fetch_w(sl + 2, wn);
+    uint4 xp[kRT][3];
+#pragma unroll
+    for (int t = 0; t < kRT; ++t) {
+      float v[8] = {now.x[t][0].x, now.x[t][0].y, now.x[t][0].z, now.x[t][0].w,
+                    now.x[t][1].x, now.x[t][1].y, now.x[t][1].z, now.x[t][1].w};
+      if (sl * kSliceK + kSliceK > K) {                  // uniform
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = k_in(sl, lk, j) < K ? v[j] : 0.0f;
+      }
+      split8(v, xp[t][0], xp[t][1], xp[t][2]);
+    }
+    fetch_x(sl + kAhead, now);
+    constexpr int px[6] = {2, 0, 1, 1, 0, 0}, pw[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb) {
+      if (cb + 1 < NCB) read_w(cb + 1, wf[(cb + 1) & 1]);
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+#pragma unroll
+        for (int t = 0; t < kRT; ++t)
+          acc[t][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8, xp[t][px[q]]), __builtin_bit_cast(bf16x8, wf[cb & 1][pw[q]]),
+              acc[t][cb], 0, 0, 0);
+    }
+    __syncthreads();
+  };
+
+  Rows x[kAhead];
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) fetch_x(i, x[i]);
+  fetch_w(0, wn);
+  commit_w(0, wn);
+  fetch_w(1, wn);
+  __syncthreads();
+  for (int sl = 0; sl < n_slices; sl += kAhead) {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i)
+      if (i == 0 || sl + i < n_slices) step(sl + i, x[i]);
+  }
+
+  store_tile<HAS_ATTN, NCB>(acc, a_l, a_r, Z, el, er, row_scale, rows, M, heads, ldz, wrow0, col0);
+}
 
 // ---- few rows ------------------------------------------------------------------------------
 // A grid of 128-row workgroups that leaves most CUs idle takes as long as one workgroup's chain
@@ -340,11 +492,11 @@ __global__ __launch_bounds__(KS * kWave) void linear_few_rows_kernel(
   const int n_slices = (K + kSliceK - 1) / kSliceK;
   const rsrc_t xrs = make_rsrc(X + row0 * K, (uint64_t)min((int64_t)kRows, rows - row0) * K * 4);
   const rsrc_t wrs = make_rsrc(W, (uint64_t)K * M * 4);
-  const uint32_t xoff = (uint32_t)((min(row0 + lr, rows - 1) - row0) * K + lk * 8) * 4u;
+  const uint32_t xoff = (uint32_t)((min(row0 + lr, rows - 1) - row0) * K + lk * 4) * 4u;
   uint32_t woff[NCB];
 #pragma unroll
   for (int cb = 0; cb < NCB; ++cb)
-    woff[cb] = ((uint32_t)(lk * 8) * M + min(col0 + cb * 16 + lr, M - 1)) * 4u;
+    woff[cb] = ((uint32_t)(lk * 4) * M + min(col0 + cb * 16 + lr, M - 1)) * 4u;
   floatx4 acc[NCB];
 #pragma unroll
   for (int cb = 0; cb < NCB; ++cb) acc[cb] = floatx4{0, 0, 0, 0};
@@ -359,18 +511,18 @@ __global__ __launch_bounds__(KS * kWave) void linear_few_rows_kernel(
     const uint32_t xs = xoff + (uint32_t)sl * (kSliceK * 4);
     const uint32_t ws = (uint32_t)sl * kSliceK * (uint32_t)M * 4u;
     s.x[0] = BufLoad<4>::at(xrs, xs, 0);
-    s.x[1] = BufLoad<4>::at(xrs, xs + 16, 0);
+    s.x[1] = BufLoad<4>::at(xrs, xs + 64, 0);
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb)
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        s.w[cb][j] = BufLoad<1>::at(wrs, woff[cb] + ws + (uint32_t)(j * M) * 4u, 0);
+        s.w[cb][j] = BufLoad<1>::at(wrs, woff[cb] + ws + (uint32_t)(k_of(0, j) * M) * 4u, 0);
   };
   auto multiply = [&](int sl, const Slice &s) __attribute__((always_inline)) {
     float v[8] = {s.x[0].x, s.x[0].y, s.x[0].z, s.x[0].w, s.x[1].x, s.x[1].y, s.x[1].z, s.x[1].w};
     if (sl * kSliceK + kSliceK > K) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = sl * kSliceK + lk * 8 + j < K ? v[j] : 0.0f;
+      for (int j = 0; j < 8; ++j) v[j] = sl * kSliceK + k_of(lk, j) < K ? v[j] : 0.0f;
     }
     uint4 xp[3];
     split8(v, xp[0], xp[1], xp[2]);
@@ -498,17 +650,23 @@ int launch_linear(const float *X, const float *W, const float *a_l, const float 
 #define GA_LAUNCH_LINEAR_VK(ATTN, WAVES)                 \
   do {                                                   \
     if (vk == 4) GA_LAUNCH_LINEAR(ATTN, 4, WAVES);       \
-    else if (vk == 2) GA_LAUNCH_LINEAR(ATTN, 2, WAVES);  \
-    else GA_LAUNCH_LINEAR(ATTN, 1, 2);                   \
+    else GA_LAUNCH_LINEAR(ATTN, 2, WAVES);               \
   } while (0)
   // three workgroups per CU once there is at least one per CU to start with; below
   // that the kernel is latency-bound and the build with the larger register budget
-  // (two per CU) has the shorter dependent chain per slice.  Rows that are only
-  // 4-byte aligned (odd K) are staged one float per load: that build holds 32 staged
-  // registers per lane, does not fit the three-workgroup budget without spilling
-  // (measured 4x slower there), and always runs two per CU.
+  // (two per CU) has the shorter dependent chain per slice.
   constexpr int64_t kDeviceCUs = 256;                    // MI355X
   const bool dense_grid = gx * gy >= kDeviceCUs;
+  if (vk == 1) {
+#define GA_LAUNCH_ODD(ATTN, NCB)                                                                    \
+  hipLaunchKernelGGL((linear_odd_kernel<ATTN, 4, NCB>), dim3((unsigned)gx, (unsigned)gy), dim3(kBlock), \
+                     0, s, X, W, a_l, a_r, Z, el, er, row_scale, rows, (int)K, (int)M, (int)heads, (int)ldz)
+    if (attn) GA_LAUNCH_ODD(true, kCB);
+    else if (M <= 16) GA_LAUNCH_ODD(false, 1);
+    else GA_LAUNCH_ODD(false, kCB);
+#undef GA_LAUNCH_ODD
+    return launch_status();
+  }
   if (attn) {
     if (dense_grid) GA_LAUNCH_LINEAR_VK(true, 3);
     else GA_LAUNCH_LINEAR_VK(true, 2);

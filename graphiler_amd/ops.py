@@ -1278,11 +1278,9 @@ LINEAR_FEW_ROWS_MAX_K = 2048
 LINEAR_FEW_ROWS_MAX_SIZE = 8 << 20      # values of x, with more than 32 output columns
 
 
-def _own_linear(rows: int, k: int, m: int) -> bool:
-    if m > LINEAR_MAX_COLS:
-        return False
-    return rows >= LINEAR_MIN_ROWS or (k <= LINEAR_FEW_ROWS_MAX_K
-                                       and (m <= 32 or rows * k <= LINEAR_FEW_ROWS_MAX_SIZE))
+def _few_rows(rows: int, k: int, m: int) -> bool:
+    return 0 < k <= LINEAR_FEW_ROWS_MAX_K and m > 0 and rows > 0 \
+        and (m <= 32 or rows * k <= LINEAR_FEW_ROWS_MAX_SIZE)
 
 
 def in_degrees(graph: DGLGraph, at_least: float = 0.0) -> torch.Tensor:
@@ -1308,8 +1306,8 @@ def linear(x, weight, row_scale=None):
         raise RuntimeError("row_scale must be (rows,) or (rows, 1) float32")
     if (x.dtype == torch.float32 and weight.dtype == torch.float32 and x.dim() == 2
             and weight.dim() == 2 and x.is_cuda and x.is_contiguous() and weight.is_contiguous()
-            and weight.shape[0] > 0 and weight.shape[1] > 0 and x.shape[0] > 0
-            and _own_linear(int(x.shape[0]), int(weight.shape[0]), int(weight.shape[1]))):
+            and weight.shape[1] <= LINEAR_MAX_COLS
+            and (x.shape[0] >= LINEAR_MIN_ROWS or _few_rows(x.shape[0], *weight.shape))):
         if row_scale is None:
             return linear_attn(x, weight)
         _check_input(row_scale, "row_scale")

@@ -48,3 +48,25 @@ def test_attention_terms(device, rows, k, heads, dim):
     for got, v in ((el, a[0]), (er, a[1])):
         assert_close(got.cpu().numpy(), (zr * v).sum(2), TOL_F32, "terms", mag=(zm * np.abs(v)).sum(2))
     assert torch.equal(ops.linear_attn(*dev[:2]), z)
+
+
+@pytest.mark.parametrize("rows,k,m", [(20_001, 33, 64), (40_000, 37, 17), (33_000, 45, 130), (20_480, 1433, 64),
+                                      (150_001, 1, 5), (151_000, 127, 16), (40_000, 31, 33)])
+def test_rows_of_an_odd_number_of_values(device, rows, k, m):
+    """Grids of 128-row workgroups whose rows only four-byte accesses tile: whole and broken last
+    slices, the last rows of x, columns beyond a pass, against float64."""
+    gen = torch.Generator(device=device).manual_seed(rows + k + m)
+    x = torch.randn(rows, k, device=device, generator=gen)
+    w = torch.randn(k, m, device=device, generator=gen)
+    want, size = x.double() @ w.double(), x.double().abs() @ w.double().abs()
+    z = ops.linear_attn(x, w)
+    assert_close(z.cpu().numpy(), want.cpu().numpy(), TOL_F32, "z", mag=size.cpu().numpy())
+    x[rows - 1, k - 1] = float("nan")
+    fin = torch.isfinite(ops.linear_attn(x, w)).all(1)
+    assert fin[:-1].all() and not fin[-1]
+    if m in (64, 16):
+        a = torch.randn(2, 1, m, device=device, generator=gen)
+        _, el, er = ops.linear_attn(x[:-1].contiguous(), w, a[0], a[1])
+        for got, v in ((el, a[0]), (er, a[1])):
+            assert_close(got.cpu().numpy(), (want[:-1] @ v.double().T).cpu().numpy(), TOL_F32, "terms",
+                         mag=(size[:-1] @ v.double().abs().T).cpu().numpy())
