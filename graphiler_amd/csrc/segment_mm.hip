@@ -1330,11 +1330,24 @@ extern "C" int ga_segment_mm_gated(const int32_t *type_pointer, int64_t n_types,
   if (!type_pointer || !X || !W || !Y || !gate) return GA_EINVAL;
   const size_t esz = dtype == GA_F32 ? 4 : 2;
   if (!aligned(X, esz) || !aligned(W, esz) || !aligned(Y, esz) || !aligned(gate, 4)) return GA_EALIGN;
-  if (dtype == GA_F32)
-    return rows_typed(type_pointer, n_types, X, &W, &Y, 1, rows, K, M, nullptr, gate, gate_sigmoid != 0,
-                      (hipStream_t)stream);
+  if (dtype == GA_F32) return GA_EUNSUPPORTED;
   return wide_typed(type_pointer, n_types, X, &W, &Y, 1, rows, K, M, nullptr, (hipStream_t)stream,
                     gate, gate_sigmoid != 0);
+}
+
+extern "C" int ga_segment_mm_gated_f32(const int32_t *type_pointer, int64_t n_types, const float *X,
+                                       const float *W, float *Y, const float *gate, int gate_sigmoid,
+                                       int64_t rows, int64_t K, int64_t M, ga_stream_t stream) {
+  using namespace ga;
+  const int bad = check_mm_args(n_types, rows, 1, K, M, GA_F32);
+  if (bad != GA_OK) return bad;
+  if (rows == 0 || n_types == 0) return GA_OK;
+  if (!type_pointer || !X || !W || !Y || !gate) return GA_EINVAL;
+  if (!aligned(X, 4) || !aligned(W, 4) || !aligned(Y, 4) || !aligned(gate, 4)) return GA_EALIGN;
+  const void *w = W;
+  void *y = Y;
+  return rows_typed(type_pointer, n_types, X, &w, &y, 1, rows, K, M, nullptr, gate, gate_sigmoid != 0,
+                    (hipStream_t)stream);
 }
 
 extern "C" int ga_segment_mm_gather(const int32_t *type_pointer, int64_t n_types,

@@ -886,15 +886,17 @@ torch::Tensor BroadcastNodeType(torch::Tensor features, const GraphPtr &graph);
 // SegmentMMNode(features, weights) * g(BroadcastNodeType(gate.unsqueeze(1))) with g the
 // sigmoid (or the identity): the output projection of examples/HGT/HGT.py:58-60 with its
 // per-node-type gate.  The product's kernel takes the per-type factor where it runs the
-// shape (ga_segment_mm_gated: bf16, wide outputs); otherwise the factor is formed per row
-// and handed to SegmentMMNodeScaled.
+// shape (ga_segment_mm_gated: bf16, wide outputs; ga_segment_mm_gated_f32); otherwise the
+// factor is formed per row and handed to SegmentMMNodeScaled.
 torch::Tensor SegmentMMNodeGated(torch::Tensor features, torch::Tensor weights, torch::Tensor gate,
                                  bool sigmoid, const GraphPtr &graph) {
   TORCH_CHECK(gate.dim() == 1 && gate.size(0) == graph->num_ntypes,
               "gate must have one entry per node type");
   // (a gate that would promote the product, e.g. fp32 on bf16 features, keeps the
   // meaning of the expression: it multiplies the result afterwards, below)
-  if (features.is_cuda() && (features.scalar_type() == at::kBFloat16 || features.scalar_type() == at::kFloat) &&
+  // (in fp32 the sigmoid is the expression's own only of an fp32 gate)
+  const bool f32 = features.scalar_type() == at::kFloat && gate.scalar_type() == at::kFloat;
+  if (features.is_cuda() && (features.scalar_type() == at::kBFloat16 || f32) &&
       at::promote_types(features.scalar_type(), gate.scalar_type()) == features.scalar_type() &&
       weights.scalar_type() == features.scalar_type() && features.dim() == 2 && weights.dim() == 3 &&
       features.size(0) == graph->num_nodes && weights.size(0) == graph->num_ntypes &&
@@ -905,11 +907,16 @@ torch::Tensor SegmentMMNodeGated(torch::Tensor features, torch::Tensor weights, 
     torch::Tensor g32 = gate.to(at::kFloat).contiguous();
     check_input(g32, "gate");
     torch::Tensor out = torch::empty({graph->num_nodes, weights.size(2)}, features.options());
-    const int rc = ga_segment_mm_gated(
-        graph->ntype_pointer.value().data_ptr<int>(), graph->num_ntypes, features.data_ptr(),
-        weights.data_ptr(), out.data_ptr(), g32.data_ptr<float>(), sigmoid ? 1 : 0,
-        graph->num_nodes, weights.size(1), weights.size(2), feat_dtype(features, "features"),
-        current_stream(out));
+    const int *types = graph->ntype_pointer.value().data_ptr<int>();
+    const int rc =
+        f32 ? ga_segment_mm_gated_f32(types, graph->num_ntypes, features.data_ptr<float>(),
+                                      weights.data_ptr<float>(), out.data_ptr<float>(),
+                                      g32.data_ptr<float>(), sigmoid ? 1 : 0, graph->num_nodes,
+                                      weights.size(1), weights.size(2), current_stream(out))
+            : ga_segment_mm_gated(types, graph->num_ntypes, features.data_ptr(), weights.data_ptr(),
+                                  out.data_ptr(), g32.data_ptr<float>(), sigmoid ? 1 : 0,
+                                  graph->num_nodes, weights.size(1), weights.size(2),
+                                  feat_dtype(features, "features"), current_stream(out));
     if (rc != GA_EUNSUPPORTED) {
       check_ga(rc, "ga_segment_mm_gated");
       return out;

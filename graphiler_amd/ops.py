@@ -590,10 +590,12 @@ def SegmentMMNodeGated(features, weights, gate, graph: DGLGraph, sigmoid: bool =
             and int(features.shape[1]) == int(weights.shape[1]):
         K, M = int(weights.shape[1]), int(weights.shape[2])
         out = torch.empty((graph.num_nodes, M), dtype=features.dtype, device=features.device)
-        rc = capi.load().ga_segment_mm_gated(
-            graph.ntype_pointer.data_ptr(), graph.num_ntypes, features.data_ptr(),
-            weights.data_ptr(), out.data_ptr(), gate.data_ptr(), 1 if sigmoid else 0,
-            graph.num_nodes, K, M, _feat_dtype(features, "features"), _stream(out))
+        lib = capi.load()
+        args = (graph.ntype_pointer.data_ptr(), graph.num_ntypes, features.data_ptr(),
+                weights.data_ptr(), out.data_ptr(), gate.data_ptr(), 1 if sigmoid else 0,
+                graph.num_nodes, K, M)
+        rc = lib.ga_segment_mm_gated_f32(*args, _stream(out)) if features.dtype == torch.float32 else \
+            lib.ga_segment_mm_gated(*args, capi.GA_BF16, _stream(out))
         if rc != capi.GA_EUNSUPPORTED:
             capi.check(rc, "ga_segment_mm_gated")
             return out

@@ -402,13 +402,16 @@ int ga_segment_mm_stacked(const int32_t *type_pointer, int64_t n_types, const vo
  * examples/HGT/HGT.py:58-60 (`trans_out * sigmoid(skip[ntype])`) applied to the fp32 sums
  * before they are rounded, so that neither the sigmoid, nor its copy to the nodes
  * (BroadcastNodeType, broadcast.cu:67-72), nor the multiplication is a pass of its own.
- * gate: (n_types,) fp32.  bf16 shapes of the wide kernel only (see ga_segment_mm_stacked), fp32 with
- * K a multiple of 4 up to 128 and M 16, 32 or a multiple of 64;
+ * gate: (n_types,) fp32.  bf16 shapes of the wide kernel only (see ga_segment_mm_stacked);
  * GA_EUNSUPPORTED, having launched nothing, otherwise: the caller then forms the per-row
- * factor itself and passes it as row_scale of ga_segment_mm_gather. */
+ * factor itself and passes it as row_scale of ga_segment_mm_gather.  The second form is the same
+ * of fp32 rows, with K a multiple of 4 up to 128 and M 16, 32 or a multiple of 64. */
 int ga_segment_mm_gated(const int32_t *type_pointer, int64_t n_types, const void *X,
                         const void *W, void *Y, const float *gate, int gate_sigmoid,
                         int64_t rows, int64_t K, int64_t M, int dtype, ga_stream_t stream);
+int ga_segment_mm_gated_f32(const int32_t *type_pointer, int64_t n_types, const float *X,
+                            const float *W, float *Y, const float *gate, int gate_sigmoid,
+                            int64_t rows, int64_t K, int64_t M, ga_stream_t stream);
 
 /* out[b, j, i] = W[b, i, j] * scale[b] * factor over n_blocks square D x D blocks (scale
  * NULL: 1), computed in fp32 and rounded once to `dtype`: the relation matrices of
