@@ -384,6 +384,13 @@ def main():
             lambda: ops._aggregate_rows(a_l, er1, z1a, Fw, H, g, slope, capi.GA_ACT_NONE, code, True),
             fused_bytes, gather=(N * Fw * b, E * Fw * b))
         del z1a
+        # the first layer as the network runs it: inputs are gathered, their sums projected
+        (w0, a0), K0 = params[0], 100
+        opsr["gat_inputs_100_256"] = op_record(
+            "c5.gat_inputs_100_256",
+            lambda: ops.gat_inputs(x0, w0, a0[0].contiguous(), a0[1].contiguous(), g, slope, "elu"),
+            4 * (N + 1) + E * (4 + H * 4 + K0 * b) + N * (K0 * b + H * 4 + Fw * b),
+            2.0 * N * K0 * Fw, "bf16", gather=(N * (K0 * b + H * 4), E * (K0 * b + H * 4)))
         if not args.no_ops:
             opsr["gat_aggregate"] = op_record(
                 "c5.gat_aggregate", lambda: ops.gat_aggregate(el1, er1, z1, g, slope),
