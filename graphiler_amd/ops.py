@@ -19,6 +19,7 @@ from typing import Optional, Sequence
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from . import capi
 from .bcast import calc_bcast_off
@@ -1285,6 +1286,17 @@ def _few_rows(rows: int, k: int, m: int) -> bool:
         and (m <= 32 or rows * k <= LINEAR_FEW_ROWS_MAX_SIZE)
 
 
+def _plain(*tensors) -> bool:
+    """True where nothing of torch would take part in a product of these tensors: no gradient, tangent
+    or transform, no trace, no autocast, no mode or tensor class that sees its operators."""
+    return (not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+            and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+            and forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._get_tracing_state() is None and not torch.compiler.is_compiling()
+            and not torch.is_autocast_enabled("cuda")
+            and not torch._C._len_torch_dispatch_stack() and not torch._C._len_torch_function_stack())
+
+
 def in_degrees(graph: DGLGraph, at_least: float = 0.0) -> torch.Tensor:
     """(N, 1) fp32 in-degrees of the graph, none below ``at_least`` (the degree column that
     examples/GCN/GCN.py:21-27 normalises by)."""
@@ -1301,7 +1313,8 @@ def linear(x, weight, row_scale=None):
     (examples/GCN/GCN.py:39 ``torch.mm(feature, self.weight)``).  ``row_scale``
     ((rows,) or (rows, 1) fp32): a factor per row of the product, the source-side
     norm of the GCN message (GCN.py:22-23), applied by the library's kernel to the
-    rows it stores and by a multiplication afterwards on the ``torch.mm`` route."""
+    rows it stores and by a multiplication afterwards on the ``torch.mm`` route.  Below
+    LINEAR_MIN_ROWS that route also keeps whatever torch does with a product besides its values."""
     if row_scale is not None and (row_scale.dtype != torch.float32
                                   or row_scale.numel() != x.shape[0]
                                   or row_scale.shape[0] != x.shape[0]):
@@ -1309,7 +1322,12 @@ def linear(x, weight, row_scale=None):
     if (x.dtype == torch.float32 and weight.dtype == torch.float32 and x.dim() == 2
             and weight.dim() == 2 and x.is_cuda and x.is_contiguous() and weight.is_contiguous()
             and weight.shape[1] <= LINEAR_MAX_COLS
-            and (x.shape[0] >= LINEAR_MIN_ROWS or _few_rows(x.shape[0], *weight.shape))):
+            and (x.shape[0] >= LINEAR_MIN_ROWS
+                 or (_few_rows(x.shape[0], *weight.shape) and weight.shape[0] == x.shape[1]
+                     and weight.device == x.device
+                     and (_plain(x, weight) if row_scale is None else
+                          row_scale.device == x.device and row_scale.is_contiguous()
+                          and _plain(x, weight, row_scale))))):
         if row_scale is None:
             return linear_attn(x, weight)
         _check_input(row_scale, "row_scale")

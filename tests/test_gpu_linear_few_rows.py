@@ -70,3 +70,31 @@ def test_rows_of_an_odd_number_of_values(device, rows, k, m):
         for got, v in ((el, a[0]), (er, a[1])):
             assert_close(got.cpu().numpy(), (want[:-1] @ v.double().T).cpu().numpy(), TOL_F32, "terms",
                          mag=(size[:-1] @ v.double().abs().T).cpu().numpy())
+
+
+def test_what_torch_does_with_a_product_is_kept(device):
+    """Few rows are a product of torch's where it has more to do than multiply."""
+    import torch.autograd.forward_ad as fwd
+    x, w = torch.randn(500, 40, device=device), torch.randn(40, 24, device=device)
+    s = torch.rand(500, 2, device=device)
+    want = x @ w
+    # fp32 products of 40 values: 40 roundings of 2^-24 each against |x| |w|
+    near = lambda got, ref: bool(((got - ref).abs() <= 80 * 2 ** -24 * (x.abs() @ w.abs())).all())
+    assert not ops.linear(x, w).requires_grad and near(ops.linear(x, w), want)
+    p = torch.nn.Parameter(w)
+    ops.linear(x, p, s[:, 1:].contiguous()).sum().backward()
+    assert torch.allclose(p.grad, x.t() @ s[:, 1:].expand(-1, 24), rtol=1e-4, atol=1e-3)
+    with torch.no_grad():
+        assert near(ops.linear(x, p), want)
+    assert torch.equal(ops.linear(x, w, s[:, 1]), want * s[:, 1:])              # a strided factor
+    assert torch.allclose(torch.vmap(lambda a: ops.linear(a, w))(x[None].expand(3, -1, -1))[2], want, atol=1e-4)
+    with fwd.dual_level():
+        assert fwd.unpack_dual(ops.linear(fwd.make_dual(x, torch.ones_like(x)), w)).tangent is not None
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert ops.linear(x, w).dtype == torch.bfloat16
+    traced = torch.jit.trace(lambda a: ops.linear(a, w), (x,), check_trace=False)
+    assert torch.allclose(traced(2 * x), 2 * want, atol=1e-4)
+    with pytest.raises(RuntimeError):
+        ops.linear(x, w[:39].contiguous())
+    with pytest.raises(RuntimeError):
+        ops.linear(x, w.cpu())
