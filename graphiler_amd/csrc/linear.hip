@@ -470,14 +470,18 @@ linear_odd_kernel(
 // A grid of 128-row workgroups that leaves most CUs idle takes as long as one workgroup's chain
 // of k slices.  Here a workgroup owns 16 rows and its KS wavefronts share out the slices: each
 // loads its operands straight into the layout of the matrix instruction (two 16-byte loads of a
-// row and eight of W per column block and slice, the next slice's behind this one's), splits
-// them as above, and the partial tiles are added through LDS in the order of the wavefronts.
-// Shorter chains also round less: error against float64 at K = 1433 5.5e-7 -> 2.0e-7.
-// us before (128-row workgroups) -> here: 2,708 x 1433 -> 64 73 -> 10, 5,000 x 300 -> 64 15 -> 7,
-// 19,717 x 500 -> 16 17.7 -> 8.7, 100,000 x 300 -> 32 39 -> 32.  16 columns of many rows run at
-// the rate X is read at (232,965 x 602, 4.4 TB/s, both forms).
+// row and eight of W per column block and slice, the next slice's behind this one's), and the
+// partial tiles are added through LDS in the order of the wavefronts.
+// The product is the fp32 instruction's: W is used for 16 rows only, so that splitting it, as
+// above, takes as long as the matrix time it saves, and this form stands where a product of
+// torch's would: infinities, products that overflow and operands near the end of the range come
+// out as they do there.  Two or four sums a block, so that a chain of roundings is short: 2-norm
+// against float64, values of both signs / of one, here, torch's product and the split: 2,708 x 1433
+// -> 64 1.8e-7, 3.4e-7, 2.0e-7 / 0.6e-7, 1.5e-7, 0.8e-7; 16,000 x 16 0.6e-7, 0.7e-7, 0.4e-7.
+// us, 128-row workgroups -> here (split: -): 2,708 x 1433 -> 64 50 -> 11.3 (11.8), 5,000 x 300 14.6
+// -> 7.0 (7.2), 19,717 x 500 -> 16 17.2 -> 8.5 (8.7), 100,000 x 300 -> 32 39 -> 36 (33).
 template <bool HAS_ATTN, int KS, int NCB>
-__global__ __launch_bounds__(KS * kWave) void linear_few_rows_kernel(
+__global__ __launch_bounds__(KS * kWave, NCB == 2 ? 3 : 2) void linear_few_rows_kernel(
     const float *__restrict__ X, const float *__restrict__ W, const float *__restrict__ a_l,
     const float *__restrict__ a_r, float *__restrict__ Z, float *__restrict__ el,
     float *__restrict__ er, const float *__restrict__ row_scale, int64_t rows, int K, int M,
@@ -497,9 +501,12 @@ __global__ __launch_bounds__(KS * kWave) void linear_few_rows_kernel(
 #pragma unroll
   for (int cb = 0; cb < NCB; ++cb)
     woff[cb] = ((uint32_t)(lk * 4) * M + min(col0 + cb * 16 + lr, M - 1)) * 4u;
-  floatx4 acc[NCB];
+  constexpr int kSums = NCB == 4 ? 2 : 4;
+  floatx4 acc[NCB][kSums];
 #pragma unroll
-  for (int cb = 0; cb < NCB; ++cb) acc[cb] = floatx4{0, 0, 0, 0};
+  for (int cb = 0; cb < NCB; ++cb)
+#pragma unroll
+    for (int i = 0; i < kSums; ++i) acc[cb][i] = floatx4{0, 0, 0, 0};
   struct Slice {
     float4 x[2];
     float w[NCB][8];
@@ -524,19 +531,12 @@ __global__ __launch_bounds__(KS * kWave) void linear_few_rows_kernel(
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] = sl * kSliceK + k_of(lk, j) < K ? v[j] : 0.0f;
     }
-    uint4 xp[3];
-    split8(v, xp[0], xp[1], xp[2]);
-    constexpr int px[6] = {2, 0, 1, 1, 0, 0}, pw[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) {
-      uint4 wp[3];
-      split8(s.w[cb], wp[0], wp[1], wp[2]);
+    for (int j = 0; j < 8; ++j)
 #pragma unroll
-      for (int q = 0; q < 6; ++q)
-        acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xp[px[q]]),
-                                                          __builtin_bit_cast(bf16x8, wp[pw[q]]),
-                                                          acc[cb], 0, 0, 0);
-    }
+      for (int cb = 0; cb < NCB; ++cb)
+        acc[cb][j % kSums] =
+            __builtin_amdgcn_mfma_f32_16x16x4f32(v[j], s.w[cb][j], acc[cb][j % kSums], 0, 0, 0);
   };
   if (wave < n_slices) {
     Slice a, b;
@@ -552,7 +552,11 @@ __global__ __launch_bounds__(KS * kWave) void linear_few_rows_kernel(
 #pragma unroll
   for (int cb = 0; cb < NCB; ++cb)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) part[wave][(lk * 4 + r) * kCols + cb * 16 + lr] = acc[cb][r];
+    for (int r = 0; r < 4; ++r) {
+      float z = acc[cb][0][r] + acc[cb][1][r];
+      if constexpr (kSums == 4) z += acc[cb][2][r] + acc[cb][3][r];
+      part[wave][(lk * 4 + r) * kCols + cb * 16 + lr] = z;
+    }
   __syncthreads();
   const int dph = M / heads;
 #pragma unroll
@@ -577,20 +581,25 @@ __global__ __launch_bounds__(KS * kWave) void linear_few_rows_kernel(
   }
 }
 
-// Where the form above is the faster one, from 16 to 232,965 rows of 16 to 1,433 values.  Up to
-// 32 columns: small grids, and long rows up to where both wait for X (us here : there; 40,000 x
-// 32 -> 32 7.7 : 6.3, 40,000 x 128 -> 16 6.1 : 8.5, 100,000 x 300 -> 32 32 : 39, 232,965 x 602 ->
-// 32 180 : 155).  64 columns: W is read and split once per 16 rows, so the time grows with tiles
-// and slices, while the other form's, on a grid of one round, is its chain; the attention terms
-// cost up to 3 us here and 1.3 there (with them 10,000 x 64 8.9 : 7.4, 16,000 x 128 10.4 : 9.8,
-// 10,000 x 600 17.7 : 25.9; without 30,000 x 600 33 : 26, 16,000 x 1433 39 : 73).  One line for
-// both, so that Z does not depend on whether they are asked for.
-bool few_rows(int64_t rows, int64_t K, int64_t M) {
+// Where the form above is taken.  A plain product of a few thousand rows (`plain`, below kFewRows)
+// stands where a product of torch's would: always, whatever the other form takes (16,000 x 16 -> 64
+// 6.0 : 5.2 us).  Otherwise where it is the faster one, us here : there.  Up to 16 columns small
+// grids and long rows (40,000 x 128 6.2 : 8.3, 100,000 x 300 23 : 31, 100,000 x 16 9.2 : 7.5, 150,000
+// x 600 82 : 78), up to 32 with twice the matrix time a row (40,000 x 128 9.8 : 10.9, 70,000 x 128
+// 15.8 : 14.8, 100,000 x 600 56 : 64, 150,000 x 300 52 : 47).  64 columns: two workgroups of tiles a
+// CU at once (8,000 x 64 4.4 : 6.0, with attention terms 6.5 : 7.4; 10,000 x 64 with them 10.4 : 7.5),
+// twice as many of long rows (with them 13,000 x 600 23 : 26, x 128 11.6 : 9.8; 20,000 x 600 33 : 26).
+constexpr int64_t kFewRows = 16'384;
+bool few_rows(int64_t rows, int64_t K, int64_t M, bool plain) {
   if ((K + kSliceK) * M >= ((int64_t)1 << 29)) return false;       // 32-bit offsets into W
+  if (plain && M <= 64 && rows < kFewRows) return true;
   const int64_t slices = (K + kSliceK - 1) / kSliceK;
-  if (M <= 32) return rows <= 20'000 || (slices >= 4 && rows <= 150'000);
-  const double tiles = (double)((rows + 15) / 16) * (double)((M + 63) / 64);
-  return tiles <= 2048 && tiles * (6e-3 + 0.68e-3 * slices) < 1.0 + 1.15 * slices;
+  if (M <= 32) {
+    const int64_t most = M <= 16 ? 300'000 : slices >= 8 ? 100'000 : 40'000;
+    return rows <= 20'000 || (slices >= 4 && rows <= most && rows * K <= ((int64_t)64 << 20));
+  }
+  const int64_t tiles = (rows + 15) / 16 * ((M + 63) / 64);
+  return tiles <= 512 || (tiles <= 1024 && slices >= 10);
 }
 
 int launch_linear(const float *X, const float *W, const float *a_l, const float *a_r, float *Z,
@@ -615,7 +624,7 @@ int launch_linear(const float *X, const float *W, const float *a_l, const float 
   const int64_t gy = (M + kPassCols - 1) / kPassCols;
   if (gx > 0x7fffffff || gy > 65535) return GA_EUNSUPPORTED;
   hipStream_t s = (hipStream_t)stream;
-  if (few_rows(rows, K, M)) {
+  if (few_rows(rows, K, M, !attn)) {
     const int ncb = M > 32 ? 4 : M > 16 ? 2 : 1;
     const dim3 grid((unsigned)((rows + 15) / 16), (unsigned)((M + 16 * ncb - 1) / (16 * ncb)));
 #define GA_LAUNCH_FEW(ATTN, KS, NCB)                                                               \
@@ -627,8 +636,7 @@ int launch_linear(const float *X, const float *W, const float *a_l, const float 
     else if (ncb == 2) GA_LAUNCH_FEW(ATTN, KS, 2);  \
     else GA_LAUNCH_FEW(ATTN, KS, 1);                \
   } while (0)
-    // at most a workgroup per CU: eight wavefronts halve the chain (2,708 x 1433 -> 64 13.8 ->
-    // 10.2 us); with more they crowd each other (19,717 x 500 -> 64 20 -> 24)
+    // at most a workgroup per CU: eight wavefronts halve the chain; with more they crowd each other
     const bool crowded = grid.x * grid.y > 256;
     if (attn && crowded) GA_LAUNCH_FEW_NCB(true, 4);
     else if (attn) GA_LAUNCH_FEW_NCB(true, 8);

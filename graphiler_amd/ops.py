@@ -1271,19 +1271,21 @@ def relation_pair_attention(k, q, v, relation_att, relation_msg, relation_scale,
 # ------------------------------------------------------ dense projection ----
 # fp32 projections with at most this many output columns run on the library's own kernels:
 # with at least this many rows (one pass over the rows, 1.2-2.1x the rate of the vendor GEMM
-# on an MI355X at these tall-and-narrow shapes), and with fewer where 16 rows a workgroup are
-# the faster form (ga_linear_attn; 2,708 x 1433 -> 64 10 us against the vendor GEMM's 13, whose
-# call also costs the host 19 us instead of 9; 8,000 x 1433 22 against 17).  Wider ones are the
-# vendor GEMM's ground (several column passes here).
+# on an MI355X at these tall-and-narrow shapes), and with fewer on its kernel of few rows, whose
+# products are the fp32 instruction's, where that takes no longer than the vendor GEMM's call
+# costs the host (18 us instead of 9): 2,708 x 1433 -> 64 11 us against 12.5 of the vendor's
+# kernel, 16,383 x 366 -> 64 14 : 9, 16,383 x 732 -> 32 15.5 : 12, x 1433 -> 16 17 : 19.  Wider ones
+# are the vendor GEMM's ground (several column passes here).
 LINEAR_MAX_COLS = 64
 LINEAR_MIN_ROWS = 16384
 LINEAR_FEW_ROWS_MAX_K = 2048
-LINEAR_FEW_ROWS_MAX_SIZE = 8 << 20      # values of x, with more than 32 output columns
+LINEAR_FEW_ROWS_MAX_SIZE = 24 << 20     # values of x times blocks of 16 output columns (1, 2 or 4)
 
 
 def _few_rows(rows: int, k: int, m: int) -> bool:
+    blocks = 1 if m <= 16 else 2 if m <= 32 else 4
     return 0 < k <= LINEAR_FEW_ROWS_MAX_K and m > 0 and rows > 0 \
-        and (m <= 32 or rows * k <= LINEAR_FEW_ROWS_MAX_SIZE)
+        and rows * k * blocks <= LINEAR_FEW_ROWS_MAX_SIZE
 
 
 def _plain(*tensors) -> bool:

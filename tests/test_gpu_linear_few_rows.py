@@ -33,6 +33,45 @@ def test_plain(device, rows, k, m):
     assert not cols[m - 1] and cols[:m - 1].all()
 
 
+@pytest.mark.parametrize("rows,k", [(1, 1), (17, 33), (2000, 64), (4113, 545), (16383, 130), (16383, 512)])
+@pytest.mark.parametrize("m", [1, 16, 33, 64])
+def test_infinities_products_that_overflow_and_small_operands(device, rows, k, m):
+    """What a product of torch's below LINEAR_MIN_ROWS gives: infinities with their signs, the sign of
+    a product that overflows, and operands far below 1 with all their bits."""
+    gen = torch.Generator(device=device).manual_seed(rows + k + m)
+    x = torch.randn(rows, k, device=device, generator=gen)
+    w = torch.randn(k, m, device=device, generator=gen)
+    x[0, k - 1], x[rows // 2, 0], x[rows // 3, k // 2] = float("inf"), float("-inf"), float("nan")
+    w[k // 3, m // 2] = float("inf")
+    got, want = ops.linear(x, w), (x.double() @ w.double()).float()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    inf = torch.isinf(want)
+    assert torch.equal(got[inf], want[inf])
+    # one product that overflows a sum, next to products of any sign
+    x, w = torch.randn_like(x), torch.randn_like(w) / 64
+    x[rows - 1], w[0, m - 1] = 0.0, -3e38
+    x[rows - 1, 0], x[rows - 1, k // 2] = 3e38, 3e38
+    got, want = ops.linear(x, w)[rows - 1], (x[rows - 1].double() @ w.double()).float()
+    assert got[m - 1] == -float("inf") and not torch.isnan(got).any()
+    assert torch.equal(torch.isinf(got), torch.isinf(want))
+    # 2^-122 has all the bits of a float; the result's last one is 2^-149
+    x = torch.randn(rows, k, device=device, generator=gen) * 2.0 ** -122
+    w = torch.randn(k, m, device=device, generator=gen)
+    want, size = x.double() @ w.double(), x.double().abs() @ w.double().abs()
+    got = ops.linear(x, w).double()
+    assert ((got - want).abs() <= (k + 8) * 2.0 ** -24 * size + k * 2.0 ** -149).all()
+
+
+def test_a_single_product_is_rounded_once(device):
+    """Rows with one value that is not zero (bag-of-words features)."""
+    gen = torch.Generator(device=device).manual_seed(3)
+    x, w = torch.zeros(3000, 300, device=device), torch.randn(300, 64, device=device, generator=gen)
+    at = torch.randint(0, 300, (3000,), device=device, generator=gen)
+    v = torch.randn(3000, device=device, generator=gen)
+    x[torch.arange(3000, device=device), at] = v
+    assert torch.equal(ops.linear(x, w), v[:, None] * w[at])
+
+
 @pytest.mark.parametrize("rows,k", [(1, 5), (17, 64), (4096, 130), (4113, 300)])
 @pytest.mark.parametrize("heads,dim", [(1, 16), (1, 32), (2, 16), (1, 64), (2, 32), (4, 16), (3, 16), (2, 64), (8, 16)])
 def test_attention_terms(device, rows, k, heads, dim):
