@@ -135,30 +135,6 @@ struct Block<bf16_t, D> {
   }
 };
 
-// x = p0 + p1 / 2^8 + p2 / 2^16 exactly for every finite x, each piece a bf16 rounded to
-// nearest from what the pieces before it leave, packed in pairs.  Rounded, the pieces and what
-// a product of them leaves out have either sign (cut off, all have that of x); scaled, they
-// stay in bf16's range as long as x does in float's (side by side the third leaves it below
-// 2^-110).  The first two stop at the largest bf16, which the values next to the largest
-// float round past.  An x that is not finite leaves a third piece that is not.
-template <int N>
-__device__ __forceinline__ void split(const float (&x)[N], uint32_t (&p)[3][N / 2]) {
-  constexpr float kMost = 0x1.fep127f;
-#pragma unroll
-  for (int j = 0; j < N; j += 2) {
-    float lo = x[j], hi = x[j + 1];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const uint32_t w = pack_bf16(__builtin_amdgcn_fmed3f(lo, -kMost, kMost),
-                                   __builtin_amdgcn_fmed3f(hi, -kMost, kMost));
-      p[q][j / 2] = w;
-      lo = (lo - bf16_lo(w)) * 256.0f;
-      hi = (hi - bf16_hi(w)) * 256.0f;
-    }
-    p[2][j / 2] = pack_bf16(lo, hi);
-  }
-}
-constexpr float kPieceScale = 1.0f / 256.0f;
 // the value of three pieces
 __device__ __forceinline__ float joined(bf16_t p0, bf16_t p1, bf16_t p2) {
   return fmaf(fmaf(bf16_lo(p2), kPieceScale, bf16_lo(p1)), kPieceScale, bf16_lo(p0));

@@ -7,13 +7,15 @@
 // So the tensors are the second grid dimension of one launch, W goes to LDS once per chunk in
 // the order in which the matrix instruction reads it (one 16-byte read per lane and piece), the
 // rows go straight from memory to their operand, and a lane stores C neighbouring columns of a
-// row at once.  fp32 on the bf16 instruction as in the dense projection: three pieces a value
-// (cut off, rounded, rest), six of nine products; values that are not finite are multiplied
-// again without the split.
+// row at once.  fp32 on the bf16 instruction: three pieces a value, scaled so that they reach as
+// far down as floats do, eight of nine products (the ninth is below 2^-32 of the whole; two more
+// left out cost a lone product up to another rounding), those of one weight in a sum of their own.
+// What comes out not finite is multiplied again without the split.
 // us before (a launch a tensor, fp32 instruction, rows of two tiles a workgroup) -> here, one tensor
-// and three: 93,773 x 64 -> 64 19 -> 14, 57 -> 30; 128 -> 128 70 -> 39, 210 -> 86; 5,000 x 64 -> 64
-// 7.3 -> 6.5, 21 -> 7; 1 M x 64 -> 64, 200 types 141 -> 122, 403 -> 314; 5.6 M x 16 -> 64 378 -> 365.
-// Error against float64 1.4e-7 -> 0.96e-7 at K = 64 (positive products 1.2e-7 -> 0.74e-7).
+// and three: 93,773 x 64 -> 64 19 -> 15.9, 54 -> 31; 128 -> 128 69 -> 43, 208 -> 93; 5,000 x 64 -> 64
+// 7.2 -> 6.1, 21 -> 6.6; 1 M x 64 -> 64, 200 types 117 -> 116, 351 -> 324; 5.7 M x 16 -> 64 378 -> 367.
+// (This kernel on the fp32 instruction: 17.7 and 38, 46 and 117, 120 and 328.)  Error against
+// float64 at K = 64 1.44e-7 -> 0.45e-7, positive products 1.15e-7 -> 0.49e-7; K = 16 0.74e-7 -> 0.29e-7.
 #include "typed_chunks.h"
 #include "typed_rows.h"
 
@@ -25,34 +27,11 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kWaves = kBlock / kWave;
 
-// x = p0 + p1 + p2; eight values -> three packed operands
-__device__ __forceinline__ void split8(const float (&v)[8], uint4 &p0, uint4 &p1, uint4 &p2) {
-  uint32_t a[8], b[4], c[8];
-#pragma unroll
-  for (int j = 0; j < 8; j += 2) {
-    a[j] = __float_as_uint(v[j]);
-    a[j + 1] = __float_as_uint(v[j + 1]);
-    const float r0 = v[j] - __uint_as_float(a[j] & 0xffff0000u);
-    const float r1 = v[j + 1] - __uint_as_float(a[j + 1] & 0xffff0000u);
-    b[j / 2] = pack_bf16(r0, r1);
-    c[j] = __float_as_uint(r0 - bf16_lo(b[j / 2]));
-    c[j + 1] = __float_as_uint(r1 - bf16_hi(b[j / 2]));
-  }
-  constexpr uint32_t hi = 0x07060302u;
-  p0 = uint4{__builtin_amdgcn_perm(a[1], a[0], hi), __builtin_amdgcn_perm(a[3], a[2], hi),
-             __builtin_amdgcn_perm(a[5], a[4], hi), __builtin_amdgcn_perm(a[7], a[6], hi)};
-  p1 = uint4{b[0], b[1], b[2], b[3]};
-  p2 = uint4{__builtin_amdgcn_perm(c[1], c[0], hi), __builtin_amdgcn_perm(c[3], c[2], hi),
-             __builtin_amdgcn_perm(c[5], c[4], hi), __builtin_amdgcn_perm(c[7], c[6], hi)};
-}
-
 // KS steps of 32 k, C blocks of 16 columns a pass: block c holds the columns 16 C pass + n C + c
 template <int KS, int C>
-__global__ __launch_bounds__(kBlock, KS == 4 ? 2 : 3) void typed_rows_kernel(TypedRows p, int chunk_rows, int passes) {
+__global__ __launch_bounds__(kBlock, KS == 4 ? 2 : KS == 2 ? 3 : 6) void typed_rows_kernel(TypedRows p, int chunk_rows, int passes) {
   __shared__ __attribute__((aligned(16))) uint4 wp[KS][C][3][kWave];
-  __shared__ int odd;                 // W has values that are not finite
   int type, row0, row1;
-  if (threadIdx.x == 0) odd = 0;
   if (!locate_chunk(p.tp, p.n_types, chunk_rows, blockIdx.x, type, row0, row1)) return;
   const int which = blockIdx.y / passes, col0 = blockIdx.y % passes * 16 * C;
   const int K = p.K, M = p.M;
@@ -75,21 +54,20 @@ __global__ __launch_bounds__(kBlock, KS == 4 ? 2 : 3) void typed_rows_kernel(Typ
   Tile t;
   const int first = row0 + 16 * wave;
   if (first < row1) fetch(first, t);  // on its way while W is prepared
-  __syncthreads();
   for (int i = threadIdx.x; i < KS * C * kWave; i += kBlock) {
     const int l = i & (kWave - 1), c = i / kWave % C, ks = i / kWave / C;
     const int k0 = ks * 32 + (l >> 4) * 4;
     const float *w = W + (l & 15) * C + c;
-    float v[8], z = 0.0f;
+    float v[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int k = k0 + (j & 3) + 4 * (j & 4);
       v[j] = k < K ? w[(int64_t)k * M] : 0.0f;
     }
+    uint32_t p3[3][4];
+    split<8, false>(v, p3);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) z = fmaf(v[j], 0.0f, z);
-    if (z != 0.0f) odd = 1;           // NaN: every writer stores the same value
-    split8(v, wp[ks][c][0][l], wp[ks][c][1][l], wp[ks][c][2][l]);
+    for (int h = 0; h < 3; ++h) wp[ks][c][h][l] = make_uint4(p3[h][0], p3[h][1], p3[h][2], p3[h][3]);
   }
   __syncthreads();
   float gate = 1.0f;
@@ -97,43 +75,59 @@ __global__ __launch_bounds__(kBlock, KS == 4 ? 2 : 3) void typed_rows_kernel(Typ
     const float g = p.gate[type];
     gate = p.gate_sigmoid ? 1.0f / (1.0f + expf(-g)) : g;
   }
-  const bool w_odd = odd != 0;
   for (int r = first; r < row1; r += 16 * kWaves) {
     const Tile now = t;
     asm volatile("" ::: "memory");    // W is read from LDS every time: held, it takes 96 registers
     if (r + 16 * kWaves < row1) fetch(r + 16 * kWaves, t);
-    floatx4 acc[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c) acc[c] = floatx4{0, 0, 0, 0};
-    float z = 0.0f;
+    uint4 xf[KS][3];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const float4 lo = now.x[ks][0], up = now.x[ks][1];
       const float v[8] = {lo.x, lo.y, lo.z, lo.w, up.x, up.y, up.z, up.w};
+      uint32_t xp[3][4];
+      split<8, false>(v, xp);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) z = fmaf(v[j], 0.0f, z);
-      uint4 xp[3];
-      split8(v, xp[0], xp[1], xp[2]);
-      constexpr int px[6] = {2, 0, 1, 1, 0, 0}, pw[6] = {0, 2, 1, 0, 1, 0};
+      for (int h = 0; h < 3; ++h) xf[ks][h] = make_uint4(xp[h][0], xp[h][1], xp[h][2], xp[h][3]);
+    }
+    floatx4 acc[C];
+    bool finite = true;
 #pragma unroll
-      for (int c = 0; c < C; ++c) {
+    for (int c = 0; c < C; ++c) {
+      floatx4 part[4] = {};           // products of pieces of one weight together: 1, 2^-8, 2^-16, 2^-24
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
         const uint4 wf[3] = {wp[ks][c][0][lane], wp[ks][c][1][lane], wp[ks][c][2][lane]};
+        constexpr int px[8] = {0, 0, 1, 0, 1, 2, 1, 2}, pw[8] = {0, 1, 0, 2, 1, 0, 2, 1};
 #pragma unroll
-        for (int m = 0; m < 6; ++m)
-          acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xp[px[m]]),
-                                                           __builtin_bit_cast(bf16x8, wf[pw[m]]), acc[c], 0, 0, 0);
+        for (int m = 0; m < 8; ++m)
+          part[px[m] + pw[m]] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8, xf[ks][px[m]]), __builtin_bit_cast(bf16x8, wf[pw[m]]),
+              part[px[m] + pw[m]], 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        acc[c][i] = fmaf(fmaf(fmaf(part[3][i], kPieceScale, part[2][i]), kPieceScale, part[1][i]),
+                         kPieceScale, part[0][i]);
+        finite = finite && isfinite(acc[c][i]);
       }
     }
-    if (w_odd || __builtin_amdgcn_ballot_w64(z != 0.0f) != 0) {
+    // What is not finite is multiplied again without the split: pieces of an infinity are NaN,
+    // and those of a product that overflows may do so with either sign.
+    if (__builtin_amdgcn_ballot_w64(!finite) != 0) {
+      floatx4 again[C];
 #pragma unroll
-      for (int c = 0; c < C; ++c) acc[c] = floatx4{0, 0, 0, 0};
+      for (int c = 0; c < C; ++c) again[c] = floatx4{0, 0, 0, 0};
       for (int k = 0; k < K; ++k)
 #pragma unroll
         for (int c = 0; c < C; ++c)
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            acc[c][i] = fmaf(p.X[(int64_t)min(r + 4 * q + i, row1 - 1) * K + k],
-                             W[(int64_t)k * M + n * C + c], acc[c][i]);
+            again[c][i] = fmaf(p.X[(int64_t)min(r + 4 * q + i, row1 - 1) * K + k],
+                               W[(int64_t)k * M + n * C + c], again[c][i]);
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[c][i] = isfinite(acc[c][i]) ? acc[c][i] : again[c][i];
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -154,8 +148,10 @@ __global__ __launch_bounds__(kBlock, KS == 4 ? 2 : 3) void typed_rows_kernel(Typ
 template <int KS>
 int launch(const TypedRows &p, hipStream_t s) {
   const int C = p.M >= 64 ? 4 : p.M / 16, passes = p.M / (16 * C);
-  // chunks of whole rounds of the four wavefronts, about five workgroups to a CU
-  const int64_t want = (p.rows * p.n_weights * passes + 1279) / 1280;
+  // chunks of whole rounds of the four wavefronts, as many as the chip holds at a time (four a CU;
+  // of 128 values 1,280 are faster than 1,024 or 768: three tensors 93 : 103 us)
+  const int64_t target = KS == 4 ? 1280 : 1024;
+  const int64_t want = (p.rows * p.n_weights * passes + target - 1) / target;
   const int chunk = (int)(want < 64 ? 64 : want > 1024 ? 1024 : (want + 63) / 64 * 64);
   const int64_t chunks = p.rows / chunk + p.n_types;      // every type has a ragged last one
   if (chunks > 0x7fffffff) return GA_EUNSUPPORTED;

@@ -72,3 +72,38 @@ def test_values_that_are_not_finite(device, value, m):
     assert np.array_equal(np.isnan(got), np.isnan(want))
     assert np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)].astype(np.float32))
     assert np.abs(got[fin] - want[fin]).max() <= TOL_F32 * np.abs(want[fin]).max()
+
+
+@pytest.mark.parametrize("k", [4, 32, 64, 128])
+@pytest.mark.parametrize("m", [16, 32, 64])
+def test_products_that_overflow_small_operands_and_single_products(device, k, m):
+    """The range and the rounding of fp32 products: a product beyond the largest float is an infinity
+    with its sign, operands of 2^-122 keep their bits, a lone product has one rounding's error (its
+    pieces are added smallest first: what comes before the last addition is 2^-8 of it)."""
+    rng = np.random.default_rng(k + m)
+    rows, types = 700, 3
+    ntype, g = _nodes(rng, rows, types, device)
+    dev = lambda a: torch.from_numpy(a).to(device)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    w = rng.standard_normal((types, k, m)).astype(np.float32)
+    big, wide = x.copy(), w.copy()
+    big[[1, 300, 699]] = 0.0                 # one product a sum that overflows, at most
+    big[[1, 300, 699], [0, k - 1, k // 2]] = 3e38, -3e38, 3.3e38
+    wide[:, k - 1, 3], wide[:, 0, 5] = 3e38, -3.2e38
+    want, _ = _want(big, wide, ntype)
+    with np.errstate(over="ignore"):
+        want = want.astype(np.float32)
+    got = ops.SegmentMMNode(dev(big), dev(wide), g).cpu().numpy()
+    assert np.isinf(want).any() and not np.isnan(got).any()
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    assert np.isfinite(got[np.isfinite(want)]).all()
+    small = x * np.float32(2.0 ** -122)
+    want, size = _want(small, w, ntype)
+    got = ops.SegmentMMNode(dev(small), dev(w), g).cpu().numpy().astype(np.float64)
+    assert (np.abs(got - want) <= (k + 8) * 2.0 ** -24 * size + k * 2.0 ** -149).all()
+    lone = np.zeros_like(x)
+    at = rng.integers(0, k, rows)
+    lone[np.arange(rows), at] = x[:, 0]
+    got = ops.SegmentMMNode(dev(lone), dev(w), g).cpu().numpy()
+    want = x[:, :1].astype(np.float64) * w[ntype, at]
+    assert (np.abs(got - want) <= (1 + 2.0 ** -6) * 2.0 ** -24 * np.abs(want)).all()
