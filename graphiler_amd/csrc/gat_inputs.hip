@@ -367,6 +367,13 @@ __device__ __forceinline__ float activated(float v, int act) {
   return act == GA_ACT_RELU ? relu_keep_nan(v) : act == GA_ACT_ELU ? elu(v) : v;
 }
 
+// A row of the tile: its node, kNoEdges beside it where the node has none; or kNoRow.  The sums of
+// nothing are 0 whatever W holds, and a product of zeros with a W that is not finite is not.
+constexpr int kNoRow = -1, kNoEdges = (int)0x80000000;
+__device__ __forceinline__ int tile_row(int node, bool edges) {
+  return node < 0 ? kNoRow : edges ? node : node | kNoEdges;
+}
+
 template <int H, int C>
 __device__ __forceinline__ void project(const GatInputs &A, const float *sums, const int *nodes) {
   const int lane = threadIdx.x & (kWave - 1), n = lane & 15, q = lane >> 4;
@@ -400,12 +407,12 @@ __device__ __forceinline__ void project(const GatInputs &A, const float *sums, c
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int node = nodes[4 * q + i];
-      if (node < 0) continue;
-      bf16_t *o = A.out + (int64_t)node * M + ch * 16 * C + n * C;
+      const int row_of = nodes[4 * q + i];
+      if (row_of == kNoRow) continue;
+      bf16_t *o = A.out + (int64_t)(row_of & ~kNoEdges) * M + ch * 16 * C + n * C;
       float v[C];
 #pragma unroll
-      for (int c = 0; c < C; ++c) v[c] = activated(acc[c][i], A.act);
+      for (int c = 0; c < C; ++c) v[c] = row_of < 0 ? 0.0f : activated(acc[c][i], A.act);
       if constexpr (C == 4)
         *reinterpret_cast<uint2 *>(o) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
       else if constexpr (C == 2)
@@ -468,7 +475,7 @@ __global__ __launch_bounds__(kBlock, H == 8 ? 3 : 4) void gat_inputs_kernel(GatI
   const int at = (blockIdx.x - A.piece_blocks) * kTileRows + group;
   int4 row = make_int4(-1, 0, 0, 0);
   if (at < A.n_light) row = A.rows[at];
-  if (j == 0) nodes[group] = row.x;
+  if (j == 0) nodes[group] = tile_row(row.x, row.z > row.y);
   const float *er = A.er + (int64_t)(row.x < 0 ? 0 : row.x) * H;
   if (finite) walk<H, true>(A, table, row.y, row.z, er, slots, st);
   else walk<H, false>(A, table, row.y, row.z, er, slots, st);
@@ -539,7 +546,7 @@ __global__ __launch_bounds__(kBlock) void gat_inputs_long_kernel(GatInputs A) {
       });
     }
   }
-  if (j == 0) nodes[group] = node;
+  if (j == 0) nodes[group] = tile_row(node, true);
   put_state<H>(A, sums, st, node >= 0);
   __syncthreads();
   project_tile<H>(A, sums, nodes);

@@ -90,6 +90,28 @@ def test_inputs_that_are_not_finite_stay_with_their_rows(device, value, heads, d
     assert not torch.isfinite(got[torch.from_numpy(hit).to(device)]).any(1).all()
 
 
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("heads,dim", [(1, 16), (2, 32), (4, 64), (8, 64)])
+def test_weights_that_are_not_finite(device, value, heads, dim):
+    """A value of W that is not finite makes its head's logits so, and with them that head of every
+    destination that has in-edges; one without stays a row of zeros, and so do the other heads."""
+    rng = np.random.default_rng(heads + dim)
+    n, e, k = 500, 1200, 60             # a tenth of the nodes have no in-edges
+    src, dst, g = _graph(rng, n, e, device, hub=400)
+    x = torch.randn(n, k, device=device).bfloat16()
+    w = (torch.randn(k, heads * dim, device=device) / k ** 0.5).bfloat16()
+    a = torch.randn(2, heads, dim, device=device) / dim ** 0.5
+    want = _reference(src, dst, n, x, w, a, 0.2, "elu")
+    w[3, dim // 2] = value
+    got = ops.gat_inputs(x, w, a[0], a[1], g, 0.2, "elu").double()
+    fed = torch.zeros(n, dtype=torch.bool, device=device)
+    fed[torch.from_numpy(dst).to(device)] = True
+    assert (~fed).sum() > 16 and (got[~fed] == 0).all()
+    assert not torch.isfinite(got[fed, :dim]).any()
+    near = (got - want)[:, dim:].abs() <= 2 ** -8 * want[:, dim:].abs() + 1e-5 * want.abs().max()
+    assert near.all()
+
+
 def test_the_layer_takes_it_and_falls_back(device, monkeypatch):
     rng = np.random.default_rng(5)
     n, e, k = 3000, 600_000, 50
