@@ -385,7 +385,8 @@ class RowsByLength:
 
 def _build_rows_by_length(g: "DGLGraph") -> RowsByLength:
     lib, dev, n = capi.load(), g.device, g.num_nodes
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    current = torch.cuda.current_stream(dev)
+    stream = current.cuda_stream
     i32 = dict(dtype=torch.int32, device=dev)
     longest = int(lib.ga_gat_rows_longest(g.num_edges))
     rows, light = torch.empty((n, 4), **i32), torch.empty(1, **i32)
@@ -401,6 +402,7 @@ def _build_rows_by_length(g: "DGLGraph") -> RowsByLength:
         capi.check(lib.ga_gat_pieces_build(rows[n_light:].data_ptr(), n_long, longest,
                                            out.piece_first.data_ptr(), out.pieces.data_ptr(), stream),
                    "ga_gat_pieces_build")
+        current.synchronize()       # the next call may come on another stream, which waits for nothing
     return out
 
 
