@@ -270,16 +270,15 @@ class DGLGraph:
     def rows_by_length(self) -> Optional["RowsByLength"]:
         """The order in which a GAT layer over its inputs walks the destinations: built on the
         device at first use and kept with the graph; None where that would have to happen while a
-        stream is captured, or does not fit the memory."""
+        stream is captured, or does not fit the memory now."""
         rows = self._cache.get("rows_by_length")
-        if rows is None and "rows_by_length" not in self._cache:
+        if rows is None:
             if torch.cuda.is_current_stream_capturing():
                 return None
             try:
-                rows = _build_rows_by_length(self)
+                rows = self._cache["rows_by_length"] = _build_rows_by_length(self)
             except torch.OutOfMemoryError:
-                rows = None
-            self._cache["rows_by_length"] = rows
+                return None
         return rows
 
     def refuse_source_classes(self, feat: int, dtype: int) -> None:

@@ -52,3 +52,15 @@ def test_pieces_are_there_when_the_order_is_kept(monkeypatch, n_light):
     g, dev = _graph(monkeypatch, n_light)
     assert g.rows_by_length() is g.rows_by_length()
     assert dev.done == (["rows", "pieces", "waited"] if n_light < 2 else ["rows"])
+
+
+def test_an_order_that_did_not_fit_is_tried_again(monkeypatch):
+    g, dev = _graph(monkeypatch, 2)
+    build = dev.ga_gat_rows_workspace_bytes
+
+    def full(*args):
+        raise torch.OutOfMemoryError("full")
+    dev.ga_gat_rows_workspace_bytes = full
+    assert g.rows_by_length() is None
+    dev.ga_gat_rows_workspace_bytes = build
+    assert g.rows_by_length() is not None
