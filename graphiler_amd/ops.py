@@ -1288,15 +1288,24 @@ def _few_rows(rows: int, k: int, m: int) -> bool:
         and rows * k * blocks <= LINEAR_FEW_ROWS_MAX_SIZE
 
 
+# What torch has no public question for.  A torch that keeps one of these elsewhere multiplies itself.
+try:
+    _TRANSFORM = torch._C._functorch.peek_interpreter_stack
+    _TRACE = torch._C._get_tracing_state
+    _MODES = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+    _ASKED = isinstance(forward_ad._current_level, int)
+except AttributeError:
+    _ASKED = False
+
+
 def _plain(*tensors) -> bool:
     """True where nothing of torch would take part in a product of these tensors: no gradient, tangent
     or transform, no trace, no autocast, no mode or tensor class that sees its operators."""
-    return (not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+    return (_ASKED and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
             and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
-            and forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
-            and torch._C._get_tracing_state() is None and not torch.compiler.is_compiling()
-            and not torch.is_autocast_enabled("cuda")
-            and not torch._C._len_torch_dispatch_stack() and not torch._C._len_torch_function_stack())
+            and forward_ad._current_level < 0 and _TRANSFORM() is None
+            and _TRACE() is None and not torch.compiler.is_compiling()
+            and not torch.is_autocast_enabled("cuda") and not _MODES[0]() and not _MODES[1]())
 
 
 def in_degrees(graph: DGLGraph, at_least: float = 0.0) -> torch.Tensor:

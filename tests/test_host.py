@@ -2,6 +2,8 @@
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -290,3 +292,29 @@ def test_pair_attention_rule(n_pairs, n_edges, max_slots, want):
     for heads, d, dt in ((1, 64, capi.GA_F32), (8, 16, capi.GA_BF16)):
         assert lib.ga_pair_attention_preferred(n_pairs, n_edges, max_slots, heads, d, dt) == want
     assert lib.ga_pair_attention_preferred(n_pairs, n_edges, max_slots, 4, 64, capi.GA_F32) == 0
+
+
+_RENAMED = """
+import importlib, torch
+from torch.autograd import forward_ad
+from graphiler_amd import ops
+x = torch.ones(2, 2)
+assert ops._plain(x)
+for place, name in ((torch._C._functorch, "peek_interpreter_stack"), (torch._C, "_get_tracing_state"),
+                    (torch._C, "_len_torch_dispatch_stack"), (torch._C, "_len_torch_function_stack"),
+                    (forward_ad, "_current_level")):
+    kept = getattr(place, name)
+    delattr(place, name)
+    importlib.reload(ops)
+    assert not ops._plain(x), name
+    setattr(place, name, kept)
+importlib.reload(ops)
+assert ops._plain(x)
+"""
+
+
+def test_a_torch_that_renames_what_is_asked_of_it_multiplies_itself():
+    """ops.linear asks torch's internals whether a product has more to it than its values: where one
+    of them is not there, every product of few rows is torch's."""
+    r = subprocess.run([sys.executable, "-c", _RENAMED], cwd=ROOT, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr[-1000:]
