@@ -529,7 +529,8 @@ class _Rewriter:
     def _fuse_kernel_tail(self, n) -> bool:
         """relu | elu of TypedSpMMEdge, gat_aggregate or gat_aggregate_al -> the operator with the
         activation where it stores its rows: what stands between two RGCN or GAT layers
-        (examples/RGCN/RGCN.py:69, the F.elu of examples/GAT/GAT.py)."""
+        (examples/RGCN/RGCN.py:69, the F.elu of examples/GAT/GAT.py).  It stays where the sum was:
+        what stands in between may overwrite what the sum reads."""
         top = n.inputsAt(0)
         sp = top.node()
         fused = {"my_ops::TypedSpMMEdge": "my_ops::TypedSpMMEdgeAct",
@@ -540,8 +541,8 @@ class _Rewriter:
         if n.kind() == "aten::elu" and \
                 any(self.const_of(n.inputsAt(i)) not in (1, 1.0) for i in (1, 2, 3)):
             return False
-        act = self.const(1 if n.kind() == "aten::relu" else 2, n)
-        out = self.make(fused, list(sp.inputs())[:-1] + [act, self.dglgraph], n, NODE)
+        act = self.const(1 if n.kind() == "aten::relu" else 2, sp)
+        out = self.make(fused, list(sp.inputs())[:-1] + [act, self.dglgraph], sp, NODE)
         n.output().replaceAllUsesWith(out)
         n.destroy()
         sp.destroy()

@@ -333,3 +333,21 @@ def test_elu_behind_an_attention_sum_rides_on_its_store():
     kinds = [n.kind() for n in models.plan("GAT+elu", 2).graph.nodes()]
     assert [k for k in kinds if k.startswith("my_ops::")] == ["my_ops::gat_project", "my_ops::gat_aggregate_act"]
     assert "aten::elu" not in kinds
+
+
+def _sum_of_messages(edges: EdgeBatchDummy):
+    m = torch.bmm(edges.src['h'].unsqueeze(1), edges.type['weight']).squeeze()
+    return {'m': m * edges.data['norm']}
+
+
+def _relu_behind_an_overwrite(nodes: NodeBatchDummy):
+    s = torch.sum(nodes.mailbox['m'], dim=1)
+    h = nodes.data['h'].add_(1.0)
+    return {'h': torch.relu(s) + h}
+
+
+def test_a_sum_that_takes_its_activation_stays_where_it_was():
+    """The sum reads its rows before something behind it overwrites them."""
+    kinds = [n.kind() for n in mpdfg_builder(_sum_of_messages, _relu_behind_an_overwrite, opt_level=2).graph.nodes()]
+    assert "my_ops::TypedSpMMEdgeAct" in kinds and "aten::relu" not in kinds
+    assert kinds.index("my_ops::TypedSpMMEdgeAct") < kinds.index("aten::add_")
