@@ -1335,7 +1335,7 @@ def linear(x, weight, row_scale=None):
             and weight.shape[1] <= LINEAR_MAX_COLS
             and (x.shape[0] >= LINEAR_MIN_ROWS
                  or (_few_rows(x.shape[0], *weight.shape) and weight.shape[0] == x.shape[1]
-                     and weight.device == x.device
+                     and weight.device == x.device and x.get_device() == torch.cuda.current_device()
                      and (_plain(x, weight) if row_scale is None else
                           row_scale.device == x.device and row_scale.is_contiguous()
                           and _plain(x, weight, row_scale))))):

@@ -137,3 +137,14 @@ def test_what_torch_does_with_a_product_is_kept(device):
         ops.linear(x, w[:39].contiguous())
     with pytest.raises(RuntimeError):
         ops.linear(x, w.cpu())
+
+
+def test_a_product_of_another_device_is_torchs(device, monkeypatch):
+    """Kernels are launched on the current device; torch multiplies on that of its operands."""
+    x, w = torch.randn(500, 40, device=device), torch.randn(40, 24, device=device)
+    launched = []
+    monkeypatch.setattr(ops, "linear_attn", lambda *a: launched.append(a))
+    ops.linear(x, w)
+    assert len(launched) == 1
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: x.get_device() + 1)
+    assert torch.equal(ops.linear(x, w), torch.mm(x, w)) and len(launched) == 1
