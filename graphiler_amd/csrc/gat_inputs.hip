@@ -185,28 +185,6 @@ struct State {
   }
 };
 
-// x = p0 + p1 + p2, each piece a bf16: the split of the fp32 projection (the first piece cut
-// off, the second rounded, the rest).
-__device__ __forceinline__ void split8(const float (&v)[8], uint4 &p0, uint4 &p1, uint4 &p2) {
-  uint32_t a[8], b[4], c[8];
-#pragma unroll
-  for (int j = 0; j < 8; j += 2) {
-    a[j] = __float_as_uint(v[j]);
-    a[j + 1] = __float_as_uint(v[j + 1]);
-    const float r0 = v[j] - __uint_as_float(a[j] & 0xffff0000u);
-    const float r1 = v[j + 1] - __uint_as_float(a[j + 1] & 0xffff0000u);
-    b[j / 2] = pack_bf16(r0, r1);
-    c[j] = __float_as_uint(r0 - bf16_lo(b[j / 2]));
-    c[j + 1] = __float_as_uint(r1 - bf16_hi(b[j / 2]));
-  }
-  constexpr uint32_t hi = 0x07060302u;
-  p0 = uint4{__builtin_amdgcn_perm(a[1], a[0], hi), __builtin_amdgcn_perm(a[3], a[2], hi),
-             __builtin_amdgcn_perm(a[5], a[4], hi), __builtin_amdgcn_perm(a[7], a[6], hi)};
-  p1 = uint4{b[0], b[1], b[2], b[3]};
-  p2 = uint4{__builtin_amdgcn_perm(c[1], c[0], hi), __builtin_amdgcn_perm(c[3], c[2], hi),
-             __builtin_amdgcn_perm(c[5], c[4], hi), __builtin_amdgcn_perm(c[7], c[6], hi)};
-}
-
 // The weights of a batch on their way between lanes, and zeros for lanes of other rows.
 template <int H>
 struct WeightSlots {
@@ -343,7 +321,7 @@ __device__ __forceinline__ void walk(const GatInputs &A, rsrc_t table, int a, in
 }
 
 // The tile's sums, (row, head, k) with kPitch floats a head, through W and out.
-__host__ __device__ inline int head_pitch(int K) { return (K + 7) / 8 * 8 + 4; }
+__host__ __device__ constexpr int head_pitch(int K) { return (K + 7) / 8 * 8 + 4; }
 
 template <int H>
 __device__ __forceinline__ void put_state(const GatInputs &A, float *sums, const State<H> &st, bool any) {
@@ -658,12 +636,9 @@ int launch_inputs(const bf16_t *X, const bf16_t *W, const float *a_l, const floa
   else GA_ROWS(1);
 #undef GA_ROWS
   const size_t lds = (size_t)kTileRows * H * head_pitch(A.K) * sizeof(float);
-  if (lds > 64 * 1024) {
-    for (const void *k : {(const void *)gat_inputs_kernel<H>, (const void *)gat_inputs_long_kernel<H>}) {
-      const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (e != hipSuccess) return (int)e;
-    }
-  }
+  static_assert(kTileRows * H * head_pitch(kMaxK - 2 * H) * sizeof(float) + sizeof(WeightSlots<H>) +
+                        kTileRows * sizeof(int) <= 64 * 1024,
+                "more than a launch gets without asking");
   A.piece_blocks = (A.n_pieces + kTileRows - 1) / kTileRows;
   const int tiles = (A.n_light + kTileRows - 1) / kTileRows;
   if (A.piece_blocks + tiles > 0)

@@ -47,28 +47,6 @@ namespace {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// x = p0 + p1 + p2 (exactly from 2^-110 up), each piece a bf16: the top 8 significant bits, what
-// they leave rounded to 8 bits, the rest (of either sign); eight values -> three packed operands.
-__device__ __forceinline__ void split8(const float (&v)[8], uint4 &p0, uint4 &p1, uint4 &p2) {
-  uint32_t a[8], b[4], c[8];
-#pragma unroll
-  for (int j = 0; j < 8; j += 2) {
-    a[j] = __float_as_uint(v[j]);
-    a[j + 1] = __float_as_uint(v[j + 1]);
-    const float r0 = v[j] - __uint_as_float(a[j] & 0xffff0000u);
-    const float r1 = v[j + 1] - __uint_as_float(a[j + 1] & 0xffff0000u);
-    b[j / 2] = pack_bf16(r0, r1);
-    c[j] = __float_as_uint(r0 - bf16_lo(b[j / 2]));
-    c[j + 1] = __float_as_uint(r1 - bf16_hi(b[j / 2]));
-  }
-  constexpr uint32_t hi = 0x07060302u;                   // high halves of (S1, S0)
-  p0 = uint4{__builtin_amdgcn_perm(a[1], a[0], hi), __builtin_amdgcn_perm(a[3], a[2], hi),
-             __builtin_amdgcn_perm(a[5], a[4], hi), __builtin_amdgcn_perm(a[7], a[6], hi)};
-  p1 = uint4{b[0], b[1], b[2], b[3]};
-  p2 = uint4{__builtin_amdgcn_perm(c[1], c[0], hi), __builtin_amdgcn_perm(c[3], c[2], hi),
-             __builtin_amdgcn_perm(c[5], c[4], hi), __builtin_amdgcn_perm(c[7], c[6], hi)};
-}
-
 constexpr int kRT = 2;                                   // 16-row tiles per wave
 constexpr int kWaveRows = kRT * 16;                      // 32
 constexpr int kWgRows = kWaveRows * (kBlock / kWave);    // 128
