@@ -193,6 +193,17 @@ def test_sums_of_dense_graphs_under_deterministic_algorithms():
     assert bool(((out.double() - _sum64(g, x)).abs() <= _sum64(g, x.abs()) * (64 * 2.0 ** -24)).all())
 
 
+def _fill_free_blocks():
+    """Tensors in every free block of more than a megabyte that torch holds: what is asked for from
+    here on needs memory of the device, whatever earlier tests left between their allocations."""
+    held = []
+    for segment in torch.cuda.memory_snapshot():
+        if segment["stream"] == 0 and tuple(segment["segment_pool_id"]) == (0, 0) and segment["segment_type"] == "large":
+            held += [torch.empty(b["size"], dtype=torch.uint8, device="cuda") for b in segment["blocks"]
+                     if b["state"] == "inactive" and b["size"] > 1 << 20]
+    return held
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("boundary", [False, True])
 @pytest.mark.parametrize("used", [False, True])
@@ -219,6 +230,9 @@ def test_scratch_that_does_not_fit_is_asked_for_once(boundary, used):
         before = call(few)
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
+    reserved = torch.cuda.memory_reserved()
+    held = _fill_free_blocks()
+    assert torch.cuda.memory_reserved() == reserved
     total = torch.cuda.get_device_properties(0).total_memory
     room = 4 * n * feat * 2 + 10 * e + plain + (64 << 20)
     assert classes > room
@@ -232,6 +246,7 @@ def test_scratch_that_does_not_fit_is_asked_for_once(boundary, used):
         assert ooms() == at + 1
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
+    del held
     assert torch.equal(first, second)
     part = x[:, :16].contiguous()
     err = (first[:, :16].double() - _sum64(g, part)).abs()

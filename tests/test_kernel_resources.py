@@ -56,3 +56,24 @@ def test_opaque_row_stores_keep_four_wavefronts(tmp_path):
     waves = re.findall(r"Function Name: \S*11runs_kernelINS_12_GLOBAL__N_114GatOpaqueStore"
                        r".*?Occupancy \[waves/SIMD\]: (\d+)", r.stderr, re.S)
     assert len(waves) == 3 and min(map(int, waves)) >= 4, waves
+
+
+@pytest.mark.skipif(not (os.path.exists(HIPCC) or shutil.which("hipcc")), reason="no hipcc")
+@pytest.mark.parametrize("source,kernel,builds,waves", [
+    ("gat_inputs", "17gat_inputs_kernelILi", 4, {"8": 3, None: 4}),
+    ("typed_rows", "17typed_rows_kernelILi", 9, {"4": 3, "1": 5, None: 4}),
+    ("linear", "22linear_few_rows_kernelILb[01]ELi[48]ELi", 12, {"4": 2, "2": 3, None: 4})])
+def test_register_budgets(tmp_path, source, kernel, builds, waves):
+    """The layer over its inputs (by heads), typed fp32 rows (by k steps) and the projection of few
+    rows (by column blocks): no spills, the wavefronts per SIMD that their comments count on."""
+    r = subprocess.run([HIPCC if os.path.exists(HIPCC) else "hipcc", "--offload-arch=gfx950", "-O3",
+                        "-std=c++17", "-fPIC", "-Xclang", "-target-feature", "-Xclang",
+                        "-packed-fp32-ops", "-Rpass-analysis=kernel-resource-usage", "-c",
+                        source + ".hip", "-o", str(tmp_path / "kernel.o")],
+                       cwd=CSRC, capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stderr[-2000:]
+    found = re.findall(r"Function Name: \S*" + kernel + r"(\d+).*?Occupancy \[waves/SIMD\]: (\d+)"
+                       r".*?VGPRs Spill: (\d+)", r.stderr, re.S)
+    assert len(found) == builds, found
+    for build, occupancy, spilled in found:
+        assert int(occupancy) >= waves.get(build, waves[None]) and int(spilled) == 0, (build, occupancy, spilled)
