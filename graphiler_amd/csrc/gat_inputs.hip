@@ -408,7 +408,7 @@ __device__ __forceinline__ void project_tile(const GatInputs &A, const float *su
   else project<H, 1>(A, sums, nodes);
 }
 
-// Wavefronts per SIMD: four (114 registers with four heads; left to itself the compiler takes
+// Wavefronts per SIMD: four (116 registers with four heads; left to itself the compiler takes
 // enough for three, 3.45 against 3.18 ms on 64.3 M edges, and five spill), three for eight heads.
 template <int H>
 __global__ __launch_bounds__(kBlock, H == 8 ? 3 : 4) void gat_inputs_kernel(GatInputs A) {

@@ -11,12 +11,13 @@
 // bits each, 24 in all; exact down to 2^-110, below which the third leaves bf16's
 // range), and the product is accumulated in fp32 from the six piece products x0w0 +
 // x0w1 + x1w0 + x1w1 + x0w2 + x2w0; each is exact in fp32.  The first piece is cut off (no
-// value of float's range overflows), the second rounded to nearest, so what the three dropped
-// products reach, below 2^-23 of |x||w|, has no sign of its own: with all three pieces cut off
-// it had the product's, which showed where all products are positive (error against float64,
-// 2-norm, 2,708 x 1433 -> 64: 1.3e-6 -> 0.8e-7, 10,000 x 600 3.2e-7 -> 0.8e-7, the vendor
-// GEMM 1.5e-7 and 3.7e-7; products of both signs 3.8e-7 -> 3.7e-7 at K = 602).  Non-finite
-// inputs give NaN (inf - inf in the split) where fp32 products may give inf.
+// value of float's range overflows), the second rounded to nearest: a second piece reaches 2^-7
+// and a third 2^-16 of its value, so the three dropped products stay below 2^-22 of |x||w|
+// (3.94 x 2^-24 at x = w = 1.0078; 0.36 x 2^-24 root mean square) and have no sign of their own.
+// With all three pieces cut off they had the product's, which showed where all products are
+// positive (error against float64, 2-norm, 40,000 x 1433 -> 64 1.3e-6 -> 6.2e-7, the vendor GEMM
+// 5.8e-7; 232,965 x 602 3.3e-7 -> 3.1e-7, 3.7e-7; both signs 3.7e-7 -> 3.65e-7, 4.4e-7).
+// Non-finite inputs give NaN (inf - inf in the split) where fp32 products may give inf.
 //
 // A workgroup (4 waves) owns 128 rows, each wave 32 rows (2 tiles of 16) x 64
 // columns per pass.  Both operands go global -> registers -> LDS in

@@ -89,9 +89,10 @@ def gat_layer(g: DGLGraph, h, fc_weight, attn_weight, heads: int = 1,
     """One GAT layer forward; ``fused`` runs the chain as a single pass.  When
     the (N, heads) table of source terms is too large to stay cached
     (``SOURCE_TERM_TABLE_LIMIT`` bytes), the pass recomputes them from the
-    gathered rows instead of gathering them as well.  A bf16 layer whose inputs are narrower
-    than half its outputs gathers the inputs and projects their sums (``ops.gat_inputs``).  ``activation`` ("relu" |
-    "elu"; the ``F.elu`` between the layers of examples/GAT/GAT.py) is applied by
+    gathered rows instead of gathering them as well.  A bf16 layer whose gathered rows would be
+    at most half as long, source terms included, as whole 128-byte lines of inputs, gathers the
+    inputs and projects their sums, where that saves 384 MiB in all (``ops.gat_inputs_preferred``).
+    ``activation`` ("relu" | "elu"; the ``F.elu`` between the layers of examples/GAT/GAT.py) is applied by
     the fused pass to the rows it stores, by a separate call otherwise."""
     a_l, a_r = attn_weight[0].float().contiguous(), attn_weight[1].float().contiguous()
     if fused and h.is_cuda and h.dim() == 2 and h.is_contiguous() and fc_weight.is_contiguous() \
