@@ -709,9 +709,11 @@ int ga_edge_softmax_sum(const int32_t *pointer, const int32_t *row_of_slot,
  * src/optimizer/split.cpp:5-34); with el == er == NULL it is the plain node
  * projection of examples/GCN/GCN.py:39.  X (rows, K), W (K, M), Z (rows, M),
  * a_l / a_r (heads, M/heads), el / er (rows, heads), all fp32.
- * Every fp32 product is formed exactly, from bf16 pieces of its operands on the
- * matrix unit, and summed in fp32: the result is as close to the exact product
- * as plain fp32 arithmetic gets; a non-finite input gives NaN.
+ * Grids of many rows form an fp32 product from six products of bf16 pieces of its
+ * operands, which leave out less than 2^-22 of it, and sum in fp32: the result is as
+ * close to the exact one as plain fp32 arithmetic gets, an input that is not finite
+ * gives NaN, and operands below 2^-110 lose bits.  Few rows (without attention terms
+ * always below 16,384 with M <= 64) are multiplied on the fp32 matrix instruction.
  * GA_EUNSUPPORTED when the attention terms are requested with M/heads not in
  * {16, 32, 64}, when K > 2^22 or when K * M >= 2^30.
  */
