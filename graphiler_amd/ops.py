@@ -36,6 +36,13 @@ def _check_input(x: torch.Tensor, name: str) -> None:
         raise RuntimeError(f"{name} must be contiguous")
 
 
+def _check_nodes(graph: DGLGraph, *tensors: torch.Tensor) -> None:
+    """The kernels gather rows by node id."""
+    for x in tensors:
+        if x.dim() == 0 or x.shape[0] < graph.num_nodes:
+            raise RuntimeError("inputs must have one row per node")
+
+
 def _feat_dtype(x: torch.Tensor, name: str) -> int:
     if x.dtype not in _DTYPES:
         raise RuntimeError(f"{name} must be float32 or bfloat16")
@@ -303,6 +310,7 @@ def gsddmm_u_op_v(op: str, src_feature, dst_feature, graph: DGLGraph) -> torch.T
     dst_feature[dst[e]] in edge-id order, fp32 (E, feat).  fp32 operands of width
     2 or 4 on a graph whose edge ids are in-adjacency slots walk the adjacency
     (rows from the row pointer: one index column read instead of two)."""
+    _check_nodes(graph, src_feature, dst_feature)
     code = {"add": capi.GA_SDDMM_ADD, "sub": capi.GA_SDDMM_SUB, "mul": capi.GA_SDDMM_MUL,
             "div": capi.GA_SDDMM_DIV}[op]
     if (src_feature.dtype == torch.float32 and dst_feature.dtype == torch.float32
@@ -354,6 +362,7 @@ def gsddmm_u_dot_v(src_feature, dst_feature, graph: DGLGraph) -> torch.Tensor:
     if dst_feature.dtype != src_feature.dtype or \
             dst_feature.shape[1:] != src_feature.shape[1:]:
         raise RuntimeError("src_feature and dst_feature must share dtype and shape")
+    _check_nodes(graph, src_feature, dst_feature)
     if src_feature.dim() == 2:
         heads, dim = 1, int(src_feature.shape[1])
     elif src_feature.dim() == 3:
@@ -909,6 +918,7 @@ def gat_aggregate(el, er, z, graph: DGLGraph, negative_slope: float = 0.01, acti
     dt = _feat_dtype(z, "z")
     if not (el.is_floating_point() and er.is_floating_point()):
         raise RuntimeError("el and er must be floating point")
+    _check_nodes(graph, el, er, z)
     # bf16 attention terms (a bf16 plan's mm(z, attn_weight)): the logits are fp32 either way
     el, er = el.float().contiguous(), er.float().contiguous()
     heads = get_feat_dim(el)
@@ -940,6 +950,7 @@ def gat_aggregate_from_z(a_l, er, z, graph: DGLGraph, negative_slope: float = 0.
     _check_input(er, "er")
     _check_input(z, "z")
     dt = _feat_dtype(z, "z")
+    _check_nodes(graph, er, z)
     if a_l.dtype != torch.float32 or er.dtype != torch.float32:
         raise RuntimeError("a_l and er must be float32")
     heads = get_feat_dim(er)
